@@ -414,7 +414,9 @@ int pennant_end_cycle(pennant_problem* pb);
  * between their launches in every cycle (direct launches then, not the
  * captured graph).  For the pipelined mixed cycle the first entry is the
  * zone pass (corrector and next predictor), the third is 0 and the fourth
- * includes the predictor redo.
+ * includes the predictor redo.  Cycles that would run as tiles (tuning
+ * "tiles") are timed as separate passes when phase_ms is given: a tile cycle
+ * has no such phases.
  * Returns 0, PENNANT_EBADSIDES or a hipError_t. */
 int pennant_time_cycles(pennant_problem* pb, int ncycles, int mode, double* total_ms,
                         double* phase_ms);
@@ -441,11 +443,19 @@ int pennant_bench_copy(size_t nbytes, int reps, double* ms_per_copy);
  *                its index instead of reading mapsp1 and the slot map
  *                (default; pennant_get_tuning reports 1 only when the mesh
  *                qualifies), 0: they read the maps
+ *   "tiles"      1: on a structured mesh (rect, or pie of two rows or more, in
+ *                the generator's numbering) a cycle is one kernel over tiles of
+ *                zones (default; pennant_get_tuning reports 1 only when the
+ *                mesh qualifies), 0: separate passes.  Cycles for which
+ *                "k1_layout" 1, "pipeline" 1, "rect_maps" 0 (rect) or a capture
+ *                buffer is set, and the odd cycle of a launch, run as separate
+ *                passes
  * pennant_set_tuning returns PENNANT_EINVAL for an unknown key or value. */
 int pennant_set_tuning(pennant_problem* pb, const char* key, int value);
 int pennant_get_tuning(pennant_problem* pb, const char* key);
-/* Autotuner: times `cycles` cycles of `mode` at every launch shape (K1
- * layout for the FP64 form, grid cap 256..4096, XCD mapping) from one
+/* Autotuner: times `cycles` cycles of `mode` as tiles and at every launch
+ * shape of the separate passes (K1 layout for the FP64 form, grid cap
+ * 256..4096, XCD mapping, the pipelined cycle for the mixed forms) from one
  * snapshot of the state, keeps the fastest and restores the snapshot (the
  * problem does not advance).  best_ms (may be NULL) receives its time. */
 int pennant_autotune(pennant_problem* pb, int mode, int cycles, double* best_ms);

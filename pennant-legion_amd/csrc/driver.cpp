@@ -499,6 +499,13 @@ static bool pipelined(const pennant_problem* pb, int form) {
     return form != FORM_FP64 && pb->tune.pipeline && !pb->cap_buf;
 }
 
+// Whether cycles of `form` run as tile cycles: on structured meshes, unless a
+// tuning asks for one of the separate passes' own forms.
+static bool tiled(const pennant_problem* pb, int form) {
+    return pb->tile.nzx > 0 && pb->tune.tiles && pb->tune.k1_layout == 0 && !pb->cap_buf &&
+           (pb->tile.pie || pb->tune.rect_maps) && !pipelined(pb, form);
+}
+
 // One cycle of `form` (ev as for fused_cycle / fused_cycle_pipe).  A
 // pipelined cycle first computes the look-ahead predictor when it is not
 // current; any other cycle makes it stale.
@@ -526,11 +533,12 @@ static int ensure_lookahead(pennant_problem* pb, int form) {
 static int build_graph(pennant_problem* pb, int form) {
     drop_graph(pb);
     hipGraph_t g = nullptr;
-    const bool pipe = pipelined(pb, form);
+    const bool pipe = pipelined(pb, form), tile = tiled(pb, form);
     CK(hipStreamBeginCapture(pb->stream, hipStreamCaptureModeThreadLocal));
     int rc = 0;
     for (int k = 0; k < PN_GRAPH_CYCLES && !rc; ++k)
-        rc = pipe ? fused_cycle_pipe(pb, nullptr, form) : fused_cycle(pb, nullptr, form);
+        rc = pipe ? fused_cycle_pipe(pb, nullptr, form)
+                  : (tile ? tile_cycle(pb, form, k & 1) : fused_cycle(pb, nullptr, form));
     const int rc2 = (int)hipStreamEndCapture(pb->stream, &g);
     if (rc || rc2) {
         if (g) (void)hipGraphDestroy(g);
@@ -615,6 +623,11 @@ int pennant_launch_cycles(pennant_problem* pb, int ncycles, int mode) {
             for (; left >= PN_GRAPH_CYCLES; left -= PN_GRAPH_CYCLES) CK(hipGraphLaunch(pb->gexec, pb->stream));
         }
         if (left > 0) CK(ensure_lookahead(pb, form));
+        // tile cycles come in pairs; an odd cycle runs as separate passes
+        for (; left > 1 && tiled(pb, form); left -= 2) {
+            CK(tile_cycle(pb, form, 0));
+            CK(tile_cycle(pb, form, 1));
+        }
         for (; left > 0; --left) CK(one_cycle(pb, nullptr, form));
         return 0;
     }
@@ -720,6 +733,11 @@ int pennant_set_tuning(pennant_problem* pb, const char* key, int value) {
         pb->tune.xcd = value;
         return 0;
     }
+    if (!strcmp(key, "tiles")) {
+        if (value != 0 && value != 1) return PENNANT_EINVAL;
+        pb->tune.tiles = value;
+        return 0;
+    }
     if (!strcmp(key, "rect_maps")) {
         if (value != 0 && value != 1) return PENNANT_EINVAL;
         pb->tune.rect_maps = value;
@@ -734,6 +752,7 @@ int pennant_get_tuning(pennant_problem* pb, const char* key) {
     if (!strcmp(key, "xcd")) return pb->tune.xcd;
     if (!strcmp(key, "graph")) return pb->tune.graph;
     if (!strcmp(key, "pipeline")) return pb->tune.pipeline;
+    if (!strcmp(key, "tiles")) return (pb->tune.tiles && pb->tile.nzx > 0) ? 1 : 0;
     // whether the fused kernels compute the zones' points and corner slots
     if (!strcmp(key, "rect_maps")) return (pb->tune.rect_maps && pb->rect_nzx > 0) ? 1 : 0;
     return PENNANT_EINVAL;
@@ -784,6 +803,22 @@ int pennant_autotune(pennant_problem* pb, int mode, int cycles, double* best_ms)
     // the mixed forms also try the pipelined cycle (it pays where the
     // volume-change limit seldom sets dt)
     const int npipe = (form == FORM_FP64 || pb->cap_buf) ? 1 : 2;
+    auto timed = [&]() {
+        rc = restore();
+        if (!rc) rc = pennant_launch_cycles(pb, 2, mode);
+        double ms = 0.;
+        if (!rc) rc = pennant_time_cycles(pb, cycles, mode, &ms, nullptr);
+        if (rc == PENNANT_EBADSIDES) rc = 0;
+        if (!rc && ms < bms) { bms = ms; best = pb->tune; }
+    };
+    pb->tune.graph = 0;                           // direct launches while shapes change
+    // the tile cycle (its grid follows from the mesh), then the separate
+    // passes' shapes
+    pb->tune.k1_layout = 0;
+    pb->tune.pipeline = 0;
+    pb->tune.tiles = keep.tiles;
+    if (tiled(pb, form)) timed();
+    pb->tune.tiles = 0;
     for (int layout = 0; layout <= (form == FORM_FP64 ? 1 : 0) && !rc; ++layout)
       for (int pipe = 0; pipe < npipe && !rc; ++pipe)
         for (int xcd = 0; xcd <= 1 && !rc; ++xcd)
@@ -793,13 +828,7 @@ int pennant_autotune(pennant_problem* pb, int mode, int cycles, double* best_ms)
                 pb->tune.pipeline = (npipe == 2) ? pipe : keep.pipeline;
                 pb->tune.xcd = xcd;
                 pb->tune.max_blocks = g;
-                pb->tune.graph = 0;               // direct launches while shapes change
-                rc = restore();
-                if (!rc) rc = pennant_launch_cycles(pb, 1, mode);
-                double ms = 0.;
-                if (!rc) rc = pennant_time_cycles(pb, cycles, mode, &ms, nullptr);
-                if (rc == PENNANT_EBADSIDES) rc = 0;
-                if (!rc && ms < bms) { bms = ms; best = pb->tune; }
+                timed();
             }
     pb->tune = (bms < 1e300) ? best : keep;
     pb->tune.graph = keep.graph;

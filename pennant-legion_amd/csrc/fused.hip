@@ -66,6 +66,7 @@ struct FusedArgs {
     int la_npred;              // pipelined cycle: K2's last block folds a redone predictor's partials
     // state (in place)
     double* pxx; double* pxy; double* pux; double* puy;
+    double* oxx; double* oxy; double* oux; double* ouy;   // K2's new point state (the arrays above, or a tile cycle's others)
     double* zr; double* ze; double* zetot; double* zwrate; double* zvol; double* zp;
     const double* zm;
     double* zpn;               // pipelined mixed cycle: the look-ahead predictor's zp
@@ -327,7 +328,6 @@ struct ZoneIn {
     d2 x[NS], u[NS];
     double zm, zr, ze, zvol, zwr;
     double mf[NS];
-    int slot[NS];
 };
 template <int NS>
 __device__ __forceinline__ void load_zone(const FusedArgs& a, int z, int sb, const int (&pp)[NS],
@@ -344,22 +344,47 @@ __device__ __forceinline__ void load_zone(const FusedArgs& a, int z, int sb, con
     in.zwr = a.zwrate[z];
 #pragma unroll
     for (int k = 0; k < NS; ++k) in.mf[k] = a.smf[sb + k];
-    load_slots<NS>(a, sb, in.slot);
 }
 
+// Where a predictor puts its results: the arrays that K2 and K3 read (a
+// corner's values at its slot, side work forces pair-major).
 template <int NS>
-__device__ __forceinline__ double zone_pred_core(const FusedArgs& a, int z, SideW sw, const ZoneIn<NS>& in,
-                                                 double dt, int& bad) {
+struct ZoneToArrays {
+    const FusedArgs& a;
+    int z;
+    SideW sw;
+    int slot[NS];
+    __device__ __forceinline__ void zp(double v) { a.zp[z] = v; }
+    __device__ __forceinline__ void mass(int k, double v) { a.cmass[slot[k]] = v; }
+    __device__ __forceinline__ void force(int k, d2 f) {
+        a.cfx[slot[k]] = f.x;
+        a.cfy[slot[k]] = f.y;
+    }
+    // the work forces of sides k and k + 1, and of a lone last side
+    __device__ __forceinline__ void sides(int k, d2 f0, d2 f1) {
+        const int sl = sw_slot<NS>(sw, k);
+        const f64x2u vx = {f0.x, f1.x}, vy = {f0.y, f1.y};
+        __builtin_nontemporal_store(vx, reinterpret_cast<f64x2u*>(a.sfwx + sl));
+        __builtin_nontemporal_store(vy, reinterpret_cast<f64x2u*>(a.sfwy + sl));
+    }
+    __device__ __forceinline__ void side(int k, d2 f) {
+        const int sl = sw_slot<NS>(sw, k);
+        st_nt(f.x, a.sfwx + sl);
+        st_nt(f.y, a.sfwy + sl);
+    }
+};
+
+template <int NS, class Out>
+__device__ __forceinline__ double zone_pred_core(const FusedArgs& a, const ZoneIn<NS>& in, double dt, int& bad,
+                                                 Out& out) {
     const double dth = 0.5 * dt;
     const double n = (double)NS;
     d2 u0[NS], xp[NS];
     double mf[NS];
-    int slot[NS];
 #pragma unroll
     for (int k = 0; k < NS; ++k) {
         u0[k] = in.u[k];
         mf[k] = in.mf[k];
-        slot[k] = in.slot[k];
     }
     const double zm = in.zm;
     const double zr0 = in.zr;
@@ -415,11 +440,11 @@ __device__ __forceinline__ double zone_pred_core(const FusedArgs& a, int z, Side
     const double denom = 1. + 0.5 * per * dv;
     const double src = zwr * dth * minv;
     const double zp = p + (per * src - r * bulk * dv) / denom;
-    a.zp[z] = zp;
+    out.zp(zp);
     // calcCrnrMass's corner mass
     const double mzz = zrp * zarea;
 #pragma unroll
-    for (int k = 0; k < NS; ++k) a.cmass[slot[k]] = mzz * 0.5 * (mf[k] + mf[prv<NS>(k)]);
+    for (int k = 0; k < NS; ++k) out.mass(k, mzz * 0.5 * (mf[k] + mf[prv<NS>(k)]));
     // calcSurfVecs, calcForcePGas, calcForceTTS per side (below)
     double sstmp = smax(zss, a.ssmin);
     sstmp = a.alfa * sstmp * sstmp;
@@ -465,30 +490,16 @@ __device__ __forceinline__ double zone_pred_core(const FusedArgs& a, int z, Side
         if (k == 0) {
             tot0 = tot;
         } else {
-            const d2 cf = sub(tot, totk);
-            a.cfx[slot[k]] = cf.x;
-            a.cfy[slot[k]] = cf.y;
+            out.force(k, sub(tot, totk));
         }
         totk = tot;
-        // the work forces of a side pair together (pair-major slots)
-        if (k & 1) {
-            const int sl = sw_slot<NS>(sw, k - 1);
-            const f64x2u vx = {sfw_prev.x, sfw.x}, vy = {sfw_prev.y, sfw.y};
-            __builtin_nontemporal_store(vx, reinterpret_cast<f64x2u*>(a.sfwx + sl));
-            __builtin_nontemporal_store(vy, reinterpret_cast<f64x2u*>(a.sfwy + sl));
-        } else if (k + 1 == NS) {
-            const int sl = sw_slot<NS>(sw, k);
-            st_nt(sfw.x, a.sfwx + sl);
-            st_nt(sfw.y, a.sfwy + sl);
-        }
+        // the work forces of a side pair together
+        if (k & 1) out.sides(k - 1, sfw_prev, sfw);
+        else if (k + 1 == NS) out.side(k, sfw);
         sfw_prev = sfw;
         ck = cn;
     }
-    {
-        const d2 cf = sub(tot0, totk);
-        a.cfx[slot[0]] = cf.x;
-        a.cfy[slot[0]] = cf.y;
-    }
+    out.force(0, sub(tot0, totk));
     const double zdu = a.q1 * zss + 2. * a.q2 * ztmp;
     // calcDtNew for this zone
     const double fuzz = 1.e-99;
@@ -501,7 +512,9 @@ __device__ __forceinline__ double zone_pred(const FusedArgs& a, int z, int sb, S
                                             const int (&pp)[NS], double dt, int& bad) {
     ZoneIn<NS> in;
     load_zone<NS>(a, z, sb, pp, in);      // every load of the zone first
-    return zone_pred_core<NS>(a, z, sw, in, dt, bad);
+    ZoneToArrays<NS> out{a, z, sw, {}};
+    load_slots<NS>(a, sb, out.slot);
+    return zone_pred_core<NS>(a, in, dt, bad, out);
 }
 
 template <int NS>
@@ -633,12 +646,14 @@ __device__ __forceinline__ void load_sides(const float* w, const SideW& sw, f2 (
 //   CL_RECOMP   CL_LEARNED for a zone that a CL_FLAG pass has already handled:
 //               stores only what the coefficient changes (corner and work
 //               forces);
-//   CL_CAPTURE  the exact coefficient, recording training tuples.
+//   CL_CAPTURE  the exact coefficient, recording training tuples;
+//   CL_PACKED   CL_LEARNED with the wave's gated corners packed into as few
+//               evaluations as possible, as CL_RECOMP does.
 // The gate: a compressing corner (cdiv < 0) whose quadratic term matters,
 // G du > PN_GATE (q1 zss + G du), i.e. f9 > PN_GATE.  Below it the exact
 // coefficient equals its acoustic limit q1 zss + G du to within 0.1%; the
 // round-off velocities of a quiescent region stay far below it.
-enum { CL_EXACT = 0, CL_LEARNED = 1, CL_CAPTURE = 2, CL_FLAG = 3, CL_RECOMP = 4 };
+enum { CL_EXACT = 0, CL_LEARNED = 1, CL_CAPTURE = 2, CL_FLAG = 3, CL_RECOMP = 4, CL_PACKED = 5 };
 #define PN_GATE 1.e-3f
 
 // Zone counters of the learned form, summed per thread.
@@ -660,7 +675,6 @@ struct ZoneState {
 template <int NS>
 struct MixedFrame {
     float mf[NS];     // FP32 side mass fractions
-    int slot[NS];     // corner-record slots
     f2 ul[NS];        // point velocities relative to the zone-mean velocity zuc
     f2 xl[NS];        // half-step positions relative to the zone centre
     f2 exl[NS];       // edge midpoints, same frame
@@ -668,30 +682,26 @@ struct MixedFrame {
     f2 sfp[NS];       // pressure side forces
     f2 sft[NS];       // TTS side forces
     d2 zuc;
-    double zss, zrp, zarea, r;
+    double zss, zrp, zarea, r, zp;
     float zdl;
 };
 
-// The frame of zone z (sides sb..sb+NS-1) from its points' positions x0 and
-// velocities u0 and its state st; writes zp to a.zp when store_zp.
+// The frame of a zone from its points' positions x0 and velocities u0, its
+// state st and its side fractions (F.mf, set by the caller).
 template <int NS>
-__device__ __forceinline__ void mixed_frame(MixedFrame<NS>& F, const FusedArgs& a, int z, int sb,
-                                            const d2 (&x0)[NS], const d2 (&u0)[NS],
-                                            const ZoneState& st, double dt, int& bad, bool valid,
-                                            bool store_zp) {
+__device__ __forceinline__ void mixed_frame(MixedFrame<NS>& F, const FusedArgs& a, const d2 (&x0)[NS],
+                                            const d2 (&u0)[NS], const ZoneState& st, double dt, int& bad,
+                                            bool valid) {
     const double dth = 0.5 * dt;
     const double n = (double)NS;
     d2 xp[NS];
-    float (&mf)[NS] = F.mf;
+    const float (&mf)[NS] = F.mf;
     const double zm = st.zm;
     const double r = st.zr;
     const double ze0 = st.ze;
     const double zvol0 = st.zvol;
     const double zwr = st.zwrate;
     F.r = r;
-#pragma unroll
-    for (int k = 0; k < NS; ++k) mf[k] = ld_nt(a.fsmf + sb + k);
-    load_slots<NS>(a, sb, F.slot);
 #pragma unroll
     for (int k = 0; k < NS; ++k)
         xp[k] = mk(__builtin_fma(dth, u0[k].x, x0[k].x), __builtin_fma(dth, u0[k].y, x0[k].y));
@@ -753,7 +763,7 @@ __device__ __forceinline__ void mixed_frame(MixedFrame<NS>& F, const FusedArgs& 
     const double denom = 1. + 0.5 * per * dv;
     const double src = zwr * dth * minv;
     const double zp = pz + (per * src - r * bulk * dv) * drcp(denom);
-    if (valid && store_zp) a.zp[z] = zp;
+    F.zp = zp;
     // pressure and TTS side forces
     const float zpf = (float)zp;
     double sstmp = smax(zss, a.ssmin);
@@ -838,20 +848,39 @@ __device__ __forceinline__ void corner_features(const MixedFrame<NS>& F, int k, 
     f[9] = (tl + tq > 0.f) ? tq * frcp(tl + tq) : 0.f;
 }
 
-// The mixed-precision predictor half of zone z (sides sb..sb+NS-1), from its
-// points' positions x0 and velocities u0 and its state st.  With CL !=
+// Where a mixed predictor puts its results: the arrays that K2 and K3 read.
+template <int NS>
+struct MixedToArrays {
+    const FusedArgs& a;
+    int z;
+    SideW sw;
+    int slot[NS];
+    __device__ __forceinline__ void zp(double v) { a.zp[z] = v; }
+    __device__ __forceinline__ void sides(const f2 (&f)[NS]) { store_sides<NS>(a.fsfw, sw, f); }
+    __device__ __forceinline__ void force(int k, float fx, float fy) {
+        a.fcrn[3 * slot[k]] = fx;
+        a.fcrn[3 * slot[k] + 1] = fy;
+    }
+    __device__ __forceinline__ void mass(int k, float m) { a.fcrn[3 * slot[k] + 2] = m; }
+};
+
+// The mixed-precision predictor half of a zone, from its points' positions x0
+// and velocities u0, its state st and its FP32 side fractions mf.  With CL !=
 // CL_EXACT it must be called by all 64 lanes of a wave together (the network
 // runs across the wave); `valid` false marks a lane that only takes part in
-// the wave-wide steps and stores nothing.  Writes zp to a.zp.
-template <int NS, int CL>
-__device__ __forceinline__ double zone_pred_mixed_core(const FusedArgs& a, int z, int sb, SideW sw,
-                                                       const d2 (&x0)[NS], const d2 (&u0)[NS],
-                                                       const ZoneState& st, double dt, int& bad,
-                                                       bool valid, ClCount& cnt) {
+// the wave-wide steps and stores nothing.
+template <int NS, int CL, class Out>
+__device__ __forceinline__ double zone_pred_mixed_core(const FusedArgs& a, const d2 (&x0)[NS],
+                                                       const d2 (&u0)[NS], const ZoneState& st,
+                                                       const float (&mf0)[NS], double dt, int& bad,
+                                                       bool valid, ClCount& cnt, Out& out) {
+    constexpr bool NET = CL == CL_LEARNED || CL == CL_RECOMP || CL == CL_PACKED;
     MixedFrame<NS> F;
-    mixed_frame<NS>(F, a, z, sb, x0, u0, st, dt, bad, valid, CL != CL_RECOMP);
+#pragma unroll
+    for (int k = 0; k < NS; ++k) F.mf[k] = mf0[k];
+    mixed_frame<NS>(F, a, x0, u0, st, dt, bad, valid);
+    if (CL != CL_RECOMP && valid) out.zp(F.zp);
     const float (&mf)[NS] = F.mf;
-    const int (&slot)[NS] = F.slot;
     const f2 (&ul)[NS] = F.ul;
     const f2 (&xl)[NS] = F.xl;
     const float (&el)[NS] = F.el;
@@ -885,24 +914,24 @@ __device__ __forceinline__ double zone_pred_mixed_core(const FusedArgs& a, int z
         cdiv[k] = div;
         cevol[k] = (div < 0.f) ? evol : 0.f;
         cdu[k] = (div < 0.f) ? du : 0.f;
-        if constexpr (CL == CL_FLAG || CL == CL_LEARNED || CL == CL_RECOMP) {
+        if constexpr (CL == CL_FLAG || NET) {
             // G du > PN_GATE (q1 zss + G du)  <=>  du > gthr zss
             if (div < 0.f && du > gthr * zssf) {
                 gated |= 1u << k;
                 comp = true;
             }
         }
-        if constexpr (CL == CL_LEARNED || CL == CL_RECOMP || CL == CL_CAPTURE) {
+        if constexpr (NET || CL == CL_CAPTURE) {
             float f[PN_MLP_NF];
             corner_features<NS>(F, k, c, zssf, zrpf, q1f, gq, f);
-            if constexpr (CL == CL_LEARNED || CL == CL_RECOMP) {
+            if constexpr (NET) {
                 if (gated & (1u << k)) {
 #pragma unroll
                     for (int j = 0; j < PN_MLP_NF; ++j)
                         inenv = inenv && (f[j] >= a.pack->lo[j]) && (f[j] <= a.pack->hi[j]);
                 }
             }
-            if constexpr (CL == CL_LEARNED || CL == CL_RECOMP) {
+            if constexpr (NET) {
                 u32x4 hi;
                 pack_features(f, flo[k], hi);
                 fhi[k] = hi[0];
@@ -937,7 +966,7 @@ __device__ __forceinline__ double zone_pred_mixed_core(const FusedArgs& a, int z
         crmu[k] = (cdiv[k] > 0.f) ? 0.f : zkur * zrpf * cevol[k];
     }
     if constexpr (CL == CL_FLAG) cnt.flag = comp;
-    if constexpr (CL == CL_RECOMP) {
+    if constexpr (CL == CL_RECOMP || CL == CL_PACKED) {
         // The wave's corners that need the network, packed into as few
         // evaluations as possible: corner k of a lane goes to slot off_k +
         // its rank among the lanes needing corner k, in an LDS row of the
@@ -1058,7 +1087,7 @@ __device__ __forceinline__ double zone_pred_mixed_core(const FusedArgs& a, int z
         const float dux = fabsf(fdot(du, dx)) * frcp(el[k]);
         dux_max = fmaxr(dux_max, (el[k] > 0.f) ? dux : 0.f);
     }
-    if (valid) store_sides<NS>(a.fsfw, sw, sfwk);
+    if (valid) out.sides(sfwk);
     const double zdu = a.q1 * zss + 2. * a.q2 * (double)dux_max;
     const double mzz = zrp * zarea;
     if (valid) {
@@ -1066,14 +1095,27 @@ __device__ __forceinline__ double zone_pred_mixed_core(const FusedArgs& a, int z
         for (int k = 0; k < NS; ++k) {
             const int km = prv<NS>(k);
             const d2 cf = sub(tot[k], tot[km]);
-            a.fcrn[3 * slot[k]] = (float)cf.x;
-            a.fcrn[3 * slot[k] + 1] = (float)cf.y;
-            if constexpr (CL != CL_RECOMP)
-                a.fcrn[3 * slot[k] + 2] = (float)(mzz * 0.5 * ((double)mf[k] + (double)mf[km]));
+            out.force(k, (float)cf.x, (float)cf.y);
+            if constexpr (CL != CL_RECOMP) out.mass(k, (float)(mzz * 0.5 * ((double)mf[k] + (double)mf[km])));
         }
     }
     const double cdt = smax(zdu, smax(zss, 1.e-99));
     return (double)zdl * a.cfl * drcp(cdt);
+}
+
+// zone_pred_mixed_core of zone z (sides sb..sb+NS-1), its results to the
+// arrays that K2 and K3 read.
+template <int NS, int CL>
+__device__ __forceinline__ double zone_pred_mixed_arrays(const FusedArgs& a, int z, int sb, SideW sw,
+                                                         const d2 (&x0)[NS], const d2 (&u0)[NS],
+                                                         const ZoneState& st, double dt, int& bad,
+                                                         bool valid, ClCount& cnt) {
+    float mf[NS];
+#pragma unroll
+    for (int k = 0; k < NS; ++k) mf[k] = ld_nt(a.fsmf + sb + k);
+    MixedToArrays<NS> out{a, z, sw, {}};
+    load_slots<NS>(a, sb, out.slot);
+    return zone_pred_mixed_core<NS, CL>(a, x0, u0, st, mf, dt, bad, valid, cnt, out);
 }
 
 // The predictor of zone z whose points are pp (mapsp1 of its sides); every
@@ -1107,7 +1149,7 @@ __device__ __forceinline__ double zone_pred_mixed(const FusedArgs& a, int z, int
     d2 x0[NS], u0[NS];
     ZoneState st;
     load_zone_mixed<NS>(a, z, pp, zre, x0, u0, st);
-    return zone_pred_mixed_core<NS, CL>(a, z, sb, sw, x0, u0, st, dt, bad, valid, cnt);
+    return zone_pred_mixed_arrays<NS, CL>(a, z, sb, sw, x0, u0, st, dt, bad, valid, cnt);
 }
 
 template <int NS, int CL>
@@ -1511,12 +1553,15 @@ __device__ __forceinline__ PointIn load_point(const FusedArgs& a, int p) {
     return q;
 }
 
-// T = float (the mixed form): calcWork needs (pu0 + pu) only times pxp.x, so
-// that product is stored in vs2 and pxpx is not written.  vs2 holds a point's
-// pair {x, y} together (K3 gathers it as one 16-byte access).
+// A point's new state, and what calcWork reads at it: T = float (the mixed
+// form) needs (pu0 + pu) only times pxp.x, so that product is vs and xpx is
+// not used.
+struct PointOut {
+    d2 x, u, vs;
+    double xpx;
+};
 template <typename T>
-__device__ __forceinline__ void point_update(const FusedArgs& a, int p, const PointIn& q,
-                                             double mass, d2 f, double dt) {
+__device__ __forceinline__ PointOut point_new(const FusedArgs& a, const PointIn& q, double mass, d2 f, double dt) {
     const double dth = 0.5 * dt;
     const d2 x0 = q.x0;
     const d2 uin = q.u0;
@@ -1533,22 +1578,33 @@ __device__ __forceinline__ void point_update(const FusedArgs& a, int p, const Po
     }
     const double fuzz = 1.e-99;
     const d2 acc = dvs(f, smax(mass, fuzz));
-    const d2 u = add(u0, scl(dt, acc));
-    const d2 x = add(x0, scl(dt * 0.5, add(u0, u)));
-    const double xpx = x0.x + dth * uin.x;   // pxp.x for calcWork
-    const d2 vs = add(u0, u);                // pu0 + pu for calcWork
-    if constexpr (sizeof(T) == 4) {
-        const f64x2u v = {vs.x * xpx, vs.y * xpx};
-        *reinterpret_cast<f64x2u*>(a.vs2 + 2 * (int64_t)p) = v;
-    } else {
-        a.pxpx[p] = xpx;
-        const f64x2u v = {vs.x, vs.y};
-        *reinterpret_cast<f64x2u*>(a.vs2 + 2 * (int64_t)p) = v;
-    }
-    a.pxx[p] = x.x;
-    a.pxy[p] = x.y;
-    a.pux[p] = u.x;
-    a.puy[p] = u.y;
+    PointOut r;
+    r.u = add(u0, scl(dt, acc));
+    r.x = add(x0, scl(dt * 0.5, add(u0, r.u)));
+    r.xpx = x0.x + dth * uin.x;              // pxp.x for calcWork
+    r.vs = add(u0, r.u);                     // pu0 + pu for calcWork
+    if constexpr (sizeof(T) == 4) r.vs = mk(r.vs.x * r.xpx, r.vs.y * r.xpx);
+    return r;
+}
+
+// calcWork's values of a point (vs2 holds the pair {x, y} together: K3
+// gathers it as one 16-byte access).
+template <typename T>
+__device__ __forceinline__ void store_work_point(const FusedArgs& a, int p, const PointOut& r) {
+    if constexpr (sizeof(T) == 8) a.pxpx[p] = r.xpx;
+    const f64x2u v = {r.vs.x, r.vs.y};
+    *reinterpret_cast<f64x2u*>(a.vs2 + 2 * (int64_t)p) = v;
+}
+
+template <typename T>
+__device__ __forceinline__ void point_update(const FusedArgs& a, int p, const PointIn& q,
+                                             double mass, d2 f, double dt) {
+    const PointOut r = point_new<T>(a, q, mass, f, dt);
+    store_work_point<T>(a, p, r);
+    a.oxx[p] = r.x.x;
+    a.oxy[p] = r.x.y;
+    a.oux[p] = r.u.x;
+    a.ouy[p] = r.u.y;
 }
 
 // Corner values by corner slot: FP64 arrays for the plain form, FP32 records
@@ -1671,6 +1727,59 @@ __global__ void __launch_bounds__(PN_BLOCK) k_point(FusedArgs a) {
     if (p < a.npown) point_light<T>(a, p, dt);
 }
 
+// The corrector of a zone from its state before the cycle (et, zvol0, zm), its
+// predictor's pressure and side work forces, and its points' new positions x
+// and work values vs, xp; folds the bad-side count and the dvol ratio.
+struct CorrOut {
+    double zwrate, zetot, ze, zr, zvol;
+};
+template <int NS, typename T>
+__device__ __forceinline__ CorrOut corr_core(double et, double zvol0, double zm, double zp, const d2 (&sfw)[NS],
+                                             const d2 (&x)[NS], const d2 (&vs)[NS], const double (&xp)[NS],
+                                             double dt, int& bad, double& dvov) {
+    const double dth = 0.5 * dt;
+    const double n = (double)NS;
+    d2 zx = mk(0., 0.);
+#pragma unroll
+    for (int k = 0; k < NS; ++k) zx = add(zx, dvs(x[k], n));
+    const double third = 1. / 3.;
+    double zvol = 0.;
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        const d2 p1 = x[k], p2 = x[nxt<NS>(k)];
+        const double sa = 0.5 * cross(sub(p2, p1), sub(zx, p1));
+        const double sv = third * sa * (p1.x + p2.x + zx.x);
+        zvol += sv;
+        if (sv <= 0.) bad += 1;
+    }
+    // calcWork
+    double w = 0.;
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        const int k2 = nxt<NS>(k);
+        const d2 sftot = sfw[k];
+        const double sd1 = dot(sftot, vs[k]);
+        const double sd2 = dot(neg(sftot), vs[k2]);
+        const double dwork = (sizeof(T) == 8) ? -dth * (sd1 * xp[k] + sd2 * xp[k2]) : -dth * (sd1 + sd2);
+        et += dwork;
+        w += dwork;
+    }
+    // calcWorkRate, calcEnergy, calcRho (corr), calcDvol
+    const double dtinv = 1. / dt;
+    const double dvol = zvol - zvol0;
+    const double zwr = (w + zp * dvol) * dtinv;
+    const double fuzz = 1.e-99;
+    CorrOut r;
+    r.zwrate = zwr;
+    r.zetot = et;
+    r.ze = et / (zm + fuzz);
+    r.zr = zm / zvol;
+    r.zvol = zvol;
+    const double zdvov = fabs((zvol - zvol0) / zvol0);
+    dvov = (zdvov > dvov) ? zdvov : dvov;
+    return r;
+}
+
 // ---------------------------------------------------------------------------
 // K3: corrector geometry, work, work rate, energy, density, dvol of zone z
 // (sides sb..sb+NS-1, points pp); folds the bad-side count and the dvol
@@ -1715,56 +1824,21 @@ __device__ __forceinline__ void corr_zone_core(const FusedArgs& a, int z, int sb
         vs[k] = mk(v[0], v[1]);
         if constexpr (sizeof(T) == 8) xp[k] = a.pxpx[pp[k]];
     }
-    const double dth = 0.5 * dt;
-    const double n = (double)NS;
-    d2 zx = mk(0., 0.);
-#pragma unroll
-    for (int k = 0; k < NS; ++k) zx = add(zx, dvs(x[k], n));
-    const double third = 1. / 3.;
-    double zvol = 0.;
-#pragma unroll
-    for (int k = 0; k < NS; ++k) {
-        const d2 p1 = x[k], p2 = x[nxt<NS>(k)];
-        const double sa = 0.5 * cross(sub(p2, p1), sub(zx, p1));
-        const double sv = third * sa * (p1.x + p2.x + zx.x);
-        zvol += sv;
-        if (sv <= 0.) bad += 1;
-    }
-    // calcWork
-    double w = 0.;
-#pragma unroll
-    for (int k = 0; k < NS; ++k) {
-        const int k2 = nxt<NS>(k);
-        const d2 sftot = sfw[k];
-        const double sd1 = dot(sftot, vs[k]);
-        const double sd2 = dot(neg(sftot), vs[k2]);
-        const double dwork = (sizeof(T) == 8) ? -dth * (sd1 * xp[k] + sd2 * xp[k2]) : -dth * (sd1 + sd2);
-        et += dwork;
-        w += dwork;
-    }
-    // calcWorkRate, calcEnergy, calcRho (corr), calcDvol
-    const double dtinv = 1. / dt;
-    const double dvol = zvol - zvol0;
-    const double zwr = (w + zp * dvol) * dtinv;
-    a.zwrate[z] = zwr;
-    a.zetot[z] = et;
-    const double fuzz = 1.e-99;
-    const double ze = et / (zm + fuzz);
-    const double zr = zm / zvol;
+    const CorrOut r = corr_core<NS, T>(et, zvol0, zm, zp, sfw, x, vs, xp, dt, bad, dvov);
+    a.zwrate[z] = r.zwrate;
+    a.zetot[z] = r.zetot;
     if constexpr (sizeof(T) == 8) {
         // the mixed form's predictors derive zr and ze from zm, zvol, zetot
-        a.ze[z] = ze;
-        a.zr[z] = zr;
+        a.ze[z] = r.ze;
+        a.zr[z] = r.zr;
     }
-    a.zvol[z] = zvol;
+    a.zvol[z] = r.zvol;
     if (PIPE) a.zp[z] = zp;
-    const double zdvov = fabs((zvol - zvol0) / zvol0);
-    dvov = (zdvov > dvov) ? zdvov : dvov;
     st.zm = zm;
-    st.zr = zr;
-    st.ze = ze;
-    st.zvol = zvol;
-    st.zwrate = zwr;
+    st.zr = r.zr;
+    st.ze = r.ze;
+    st.zvol = r.zvol;
+    st.zwrate = r.zwrate;
 }
 
 template <int NS, typename T>
@@ -1922,7 +1996,7 @@ k_zone_pipe(FusedArgs a, int zbeg, int zend, int sbeg, int poff, int run, DtPara
             ZoneState st;
             corr_zone_core<NS, float, true>(a, z, sb, sw, pp, dt, badc, dvov, x, st);
             if (!last) {
-                const double zdthyd = zone_pred_mixed_core<NS, FLAG ? CL_FLAG : CL_EXACT>(
+                const double zdthyd = zone_pred_mixed_arrays<NS, FLAG ? CL_FLAG : CL_EXACT>(
                     b, z, sb, sw, x, u, st, dtn, badp, true, cnt);
                 dtmin = (zdthyd < dtmin) ? zdthyd : dtmin;
             }
@@ -1982,9 +2056,10 @@ __device__ __forceinline__ int blk_sum_fin(int v) {
 // The four folds of a finalize in one pass over the block: wave folds, one
 // LDS row per wave, and thread 0 folds the rows in wave order (the result is
 // thread 0's).
+template <int BS>
 __device__ __forceinline__ void blk_fold_fin(double& mn, double& mx, int& bp, int& bc) {
-    __shared__ double pmn[PN_FIN_BLOCK / 64], pmx[PN_FIN_BLOCK / 64];
-    __shared__ int pbp[PN_FIN_BLOCK / 64], pbc[PN_FIN_BLOCK / 64];
+    __shared__ double pmn[BS / 64], pmx[BS / 64];
+    __shared__ int pbp[BS / 64], pbc[BS / 64];
     mn = wave_min(mn);
     mx = wave_max(mx);
     bp = wave_sum(bp);
@@ -1998,7 +2073,7 @@ __device__ __forceinline__ void blk_fold_fin(double& mn, double& mx, int& bp, in
     }
     __syncthreads();
     if (threadIdx.x == 0)
-        for (int i = 1; i < PN_FIN_BLOCK / 64; ++i) {
+        for (int i = 1; i < BS / 64; ++i) {
             mn = (pmn[i] < mn) ? pmn[i] : mn;
             mx = (pmx[i] > mx) ? pmx[i] : mx;
             bp += pbp[i];
@@ -2013,22 +2088,23 @@ __device__ __forceinline__ int end_cycle(Ctl* c, const CtlSnap& v, double mn, do
                                          double dtfac, double tstop, int zre,
                                          double* next_dt = nullptr);
 
-// Each thread's share of the partials (thread t folds t, t + PN_FIN_BLOCK,
-// ...), loaded PN_FIN_PER per thread at a time with no branch between the
+// Each thread's share of the partials (thread t of BS folds t, t + BS, ...),
+// loaded PN_FIN_PER per thread at a time with no branch between the
 // loads.  Indices past the end read the last partial again: a repeat leaves a
 // min or max unchanged and adds 0 to a count.  npred, ncorr >= 1 (every
 // launch has at least one block, every problem at least one unit).
 #define PN_FIN_PER 8
+template <int BS>
 __device__ __forceinline__ void fold_partials(const double* part_dt, const int* part_bp, int npred,
                                               const double* part_dv, const int* part_bc, int ncorr,
                                               double& mn, int& bp, double& mx, int& bc) {
     const int n = npred > ncorr ? npred : ncorr;
-    for (int base = 0; base < n; base += PN_FIN_PER * PN_FIN_BLOCK) {
+    for (int base = 0; base < n; base += PN_FIN_PER * BS) {
         double dv[PN_FIN_PER], dd[PN_FIN_PER];
         int ip[PN_FIN_PER], ic[PN_FIN_PER];
 #pragma unroll
         for (int j = 0; j < PN_FIN_PER; ++j) {
-            const int i = base + (int)threadIdx.x + j * PN_FIN_BLOCK;
+            const int i = base + (int)threadIdx.x + j * BS;
             const int ipd = min(i, npred - 1), icr = min(i, ncorr - 1);
             dd[j] = part_dt[ipd];
             ip[j] = part_bp[ipd];
@@ -2037,7 +2113,7 @@ __device__ __forceinline__ void fold_partials(const double* part_dt, const int* 
         }
 #pragma unroll
         for (int j = 0; j < PN_FIN_PER; ++j) {
-            const int i = base + (int)threadIdx.x + j * PN_FIN_BLOCK;
+            const int i = base + (int)threadIdx.x + j * BS;
             mn = (dd[j] < mn) ? dd[j] : mn;
             bp += (i < npred) ? ip[j] : 0;
             mx = (dv[j] > mx) ? dv[j] : mx;
@@ -2056,8 +2132,8 @@ __device__ __forceinline__ void finalize_block(Ctl* c, const double* part_dt, co
     const CtlSnap v = snap_ctl(c);
     double mn = 1.e99, mx = 1.e-99;
     int bp = 0, bc = 0;
-    fold_partials(part_dt, part_bp, npred, part_dv, part_bc, ncorr, mn, bp, mx, bc);
-    blk_fold_fin(mn, mx, bp, bc);
+    fold_partials<PN_FIN_BLOCK>(part_dt, part_bp, npred, part_dv, part_bc, ncorr, mn, bp, mx, bc);
+    blk_fold_fin<PN_FIN_BLOCK>(mn, mx, bp, bc);
     if (threadIdx.x != 0 || v.done) return;
     end_cycle(c, v, mn, mx, bp, bc, cflv, cstop, dtmax, dtfac, tstop, zre);
 }
@@ -2128,8 +2204,8 @@ __global__ void __launch_bounds__(PN_FIN_BLOCK) k_finalize_pipe(FusedArgs a, int
     if (c->done) return;
     double mn = 1.e99, mx = 1.e-99;
     int bp = 0, bc = 0;
-    fold_partials(a.part_dt, a.part_bp, npred, a.part_dv, a.part_bc, ncorr, mn, bp, mx, bc);
-    blk_fold_fin(mn, mx, bp, bc);
+    fold_partials<PN_FIN_BLOCK>(a.part_dt, a.part_bp, npred, a.part_dv, a.part_bc, ncorr, mn, bp, mx, bc);
+    blk_fold_fin<PN_FIN_BLOCK>(mn, mx, bp, bc);
     if (threadIdx.x != 0) return;
     if (a.cl_stats) {
         const unsigned long long nl = atomicExch(a.cl_stats + 2, 0ull);
@@ -2183,12 +2259,391 @@ __global__ void __launch_bounds__(PN_FIN_BLOCK) k_finalize_la(FusedArgs a, int n
     fold_lookahead<REDO>(a, npred);
 }
 
+// ---------------------------------------------------------------------------
+// Tile cycle: the whole cycle of a structured mesh in one kernel.
+//
+// On a rect or pie mesh in the generator's numbering a block takes a tile of
+// PN_TILE x PN_TILE quads, one per thread: its (PN_TILE - 2)^2 inner zones and
+// a ring of neighbours.  It runs the predictor of all of them, hands the
+// corner values to the points between them through LDS, and finishes its
+// inner zones' corrector from registers and LDS.  Neither corner records, nor
+// side work forces, nor the points' work values go through memory, and a zone
+// and its points are read once per cycle instead of two or three times: about
+// 190 bytes a zone instead of 690 (FP64) or 460 (mixed).  The ring costs
+// (16 / 14)^2 = 1.31 times the predictor's arithmetic.
+//
+// A block reads its ring from zones that other blocks own, so a cycle never
+// writes what it reads: odd cycles of a launch go from the problem's arrays
+// to a second set, even ones back (Ctl::cur says where the state is, and the
+// second cycle of a pair copies it back when the first ended the run), so the
+// problem's own arrays hold the state after every pair.
+//
+// The triangles of a pie's first row and the origin are not part of a tile:
+// their predictor and corrector run as in the separate passes, before and
+// after, and the tiles of the first row of quads read the triangles' corner
+// records.  Sums run in the order of the separate passes (a point's corners in
+// ascending side order), so the results are the same bits.
+//
+// What bounds it: arithmetic (FP64: 238 VGPRs, two waves per SIMD, VALU issue;
+// mixed: 128 VGPRs, four).  Per cycle, separate passes (for mixed and learned
+// the pipelined ones) -> tiles: FP64 Sedov 1440^2 306 -> 214 us, Noh pie
+// 1024^2 178 -> 132 us; mixed LeBlanc 4096 x 256 87 -> 62 us, 333 x 217 23 ->
+// 14 us; learned Sedov 1440^2 176 -> 159 us; FP64 45^2 21 -> 14 us.  It was
+// faster at every size, so structured meshes always take it.
+#define PN_TILE 16
+#define PN_TIN (PN_TILE - 2)
+
+// A structured mesh in the arrays: zone (i, j) of nzx x nzy has its points
+// (i, j), (i + 1, j), (i + 1, j + 1), (i, j + 1); row 0 of a pie is the
+// triangles, whose first point is the origin.
+struct TileMesh {
+    int nzx, nzy, pie;
+    int zo, so, po;              // first zone, side and point in the arrays
+};
+__device__ __forceinline__ int tile_zone(const TileMesh& g, int i, int j) { return g.zo + j * g.nzx + i; }
+__device__ __forceinline__ int tile_side(const TileMesh& g, int i, int j) {
+    return g.so + 4 * (j * g.nzx + i) - (g.pie ? g.nzx : 0);
+}
+__device__ __forceinline__ int tile_point(const TileMesh& g, int i, int j) {
+    return g.po + j * (g.nzx + 1) + i - (g.pie ? g.nzx : 0);
+}
+
+// Where a tile cycle writes the state (the points' through FusedArgs::oxx..).
+struct TileOut {
+    double* zr; double* ze; double* zetot; double* zwrate; double* zvol;
+};
+
+// A predictor's results kept in the block: corner forces and masses in LDS,
+// [3 k + {0, 1, 2}][thread], the rest in registers.
+template <typename T> struct TileKeep;
+template <> struct TileKeep<double> {
+    double* c;
+    d2 sfw[4];
+    double p;
+    __device__ __forceinline__ void zp(double v) { p = v; }
+    __device__ __forceinline__ void mass(int k, double v) { c[(3 * k + 2) * PN_BLOCK] = v; }
+    __device__ __forceinline__ void force(int k, d2 f) {
+        c[(3 * k) * PN_BLOCK] = f.x;
+        c[(3 * k + 1) * PN_BLOCK] = f.y;
+    }
+    __device__ __forceinline__ void sides(int k, d2 f0, d2 f1) {
+        sfw[k] = f0;
+        sfw[k + 1] = f1;
+    }
+    __device__ __forceinline__ void side(int k, d2 f) { sfw[k] = f; }
+};
+template <> struct TileKeep<float> {
+    float* c;
+    f2 sfw[4];
+    double p;
+    __device__ __forceinline__ void zp(double v) { p = v; }
+    __device__ __forceinline__ void mass(int k, float v) { c[(3 * k + 2) * PN_BLOCK] = v; }
+    __device__ __forceinline__ void force(int k, float fx, float fy) {
+        c[(3 * k) * PN_BLOCK] = fx;
+        c[(3 * k + 1) * PN_BLOCK] = fy;
+    }
+    __device__ __forceinline__ void sides(const f2 (&f)[4]) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) sfw[k] = f[k];
+    }
+};
+
+// The tile whose first zone (ring included) is (i0, j0); its partials go to
+// slot.  Returns whether a CL_FLAG tile has a zone for the network: such a
+// tile is left to the list kernel and stores nothing.
+template <typename T, int CL>
+__device__ __forceinline__ bool tile_body(const FusedArgs& a, const TileOut& o, const TileMesh& g, int i0, int j0,
+                                          int slot, double dt, bool zre, ClCount& total) {
+    __shared__ T crn[12][PN_BLOCK];
+    __shared__ double pts[sizeof(T) == 8 ? 5 : 4][PN_BLOCK];
+    const int tid = threadIdx.x;
+    const int ti = tid & (PN_TILE - 1), tj = tid / PN_TILE;
+    const int i = i0 + ti, j = j0 + tj;
+    const bool zin = i >= 0 && i < g.nzx && j >= 0 && j < g.nzy;
+    const bool tri = zin && j < g.pie;                       // a triangle of its own pass
+    const bool quad = zin && !tri;
+    const bool inner = ti >= 1 && ti <= PN_TIN && tj >= 1 && tj <= PN_TIN;
+    const bool own = quad && inner;
+    const bool pin = i >= 0 && i <= g.nzx && j >= g.pie && j <= g.nzy;   // point (i, j) exists
+    // Every load of the tile first, with no branch: threads outside the mesh
+    // read the nearest zone and use nothing of it.
+    const int ci = min(max(i, 0), g.nzx - 1), cj = min(max(j, g.pie), g.nzy - 1);
+    const int z = tile_zone(g, ci, cj), sb = tile_side(g, ci, cj);
+    const int p00 = tile_point(g, ci, cj);
+    const int pp[4] = {p00, p00 + 1, p00 + g.nzx + 2, p00 + g.nzx + 1};
+    PointIn q;
+    double dtz = 1.e99, et = 0., zm, zvol0;
+    int bad = 0;
+    ClCount cnt;
+    TileKeep<T> keep;
+    keep.c = &crn[0][tid];
+    if constexpr (sizeof(T) == 8) {
+        ZoneIn<4> in;
+        load_zone<4>(a, z, sb, pp, in);
+        q.bits = a.pbc[p00];
+        zm = in.zm;
+        zvol0 = in.zvol;
+        q.x0 = in.x[0];
+        q.u0 = in.u[0];
+        if (own) et = a.zetot[z];
+        if (quad) dtz = zone_pred_core<4>(a, in, dt, bad, keep);
+    } else {
+        d2 x0[4], u0[4];
+        ZoneState st;
+        load_zone_mixed<4>(a, z, pp, zre, x0, u0, st);
+        float mf[4];
+        const f32x4u m4 = *reinterpret_cast<const f32x4u*>(a.fsmf + sb);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) mf[k] = m4[k];
+        q.bits = a.pbc[p00];
+        zm = st.zm;
+        zvol0 = st.zvol;
+        q.x0 = x0[0];
+        q.u0 = u0[0];
+        if (own) et = a.zetot[z];
+        // the network runs across the wave, so every lane takes part
+        if (CL == CL_PACKED || quad)
+            dtz = zone_pred_mixed_core<4, CL>(a, x0, u0, st, mf, dt, bad, quad, cnt, keep);
+    }
+    if (tri) {
+        // the corners of triangle i at points (i + 1, 1) and (i, 1), where a
+        // quad has its corners 2 and 3
+        const int s0 = g.so + 3 * i;
+#pragma unroll
+        for (int k = 2; k < 4; ++k) {
+            const int sl = a.pcpos[s0 + k - 1];
+            if constexpr (sizeof(T) == 8) {
+                keep.force(k, mk(a.cfx[sl], a.cfy[sl]));
+                keep.mass(k, a.cmass[sl]);
+            } else {
+                keep.force(k, a.fcrn[3 * sl], a.fcrn[3 * sl + 1]);
+                keep.mass(k, a.fcrn[3 * sl + 2]);
+            }
+        }
+    }
+    if constexpr (CL == CL_FLAG) {
+        if (__syncthreads_or(quad && cnt.flag)) return true;
+    } else {
+        __syncthreads();
+    }
+    if constexpr (CL == CL_PACKED) {
+        if (own) {
+            total.learned += cnt.learned;
+            total.fallback += cnt.fallback;
+        }
+    }
+    if (pin && ti >= 1 && tj >= 1) {
+        const int p = tile_point(g, i, j);
+        if (!quad) q = load_point(a, p);     // the last column and row of points
+        // the point's corners in ascending side order
+        const bool l = i >= 1, r = i < g.nzx, b = j >= 1, t = j < g.nzy;
+        double mass = 0.;
+        d2 f = mk(0., 0.);
+        auto corner = [&](bool on, int k, int from) {
+            if (on) {
+                mass += (double)crn[3 * k + 2][from];
+                f = add(f, mk((double)crn[3 * k][from], (double)crn[3 * k + 1][from]));
+            }
+        };
+        corner(l && b, 2, tid - PN_TILE - 1);
+        corner(r && b, 3, tid - PN_TILE);
+        corner(l && t, 1, tid - 1);
+        corner(r && t, 0, tid);
+        const PointOut w = point_new<T>(a, q, mass, f, dt);
+        pts[0][tid] = w.x.x;
+        pts[1][tid] = w.x.y;
+        pts[2][tid] = w.vs.x;
+        pts[3][tid] = w.vs.y;
+        if constexpr (sizeof(T) == 8) pts[4][tid] = w.xpx;
+        // a point belongs to the tile whose inner zones it is the first point
+        // of; the mesh's last column and row go with the tiles they end
+        if ((ti <= PN_TIN || i == g.nzx) && (tj <= PN_TIN || j == g.nzy)) {
+            a.oxx[p] = w.x.x;
+            a.oxy[p] = w.x.y;
+            a.oux[p] = w.u.x;
+            a.ouy[p] = w.u.y;
+            if (g.pie && j == 1) store_work_point<T>(a, p, w);   // for the triangles' corrector
+        }
+    }
+    __syncthreads();
+    double dvov = 1.e-99, dtm = 1.e99;
+    int badc = 0;
+    if (own) {
+        const int at[4] = {tid, tid + 1, tid + PN_TILE + 1, tid + PN_TILE};
+        d2 x[4], vs[4], sfw[4];
+        double xp[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            x[k] = mk(pts[0][at[k]], pts[1][at[k]]);
+            vs[k] = mk(pts[2][at[k]], pts[3][at[k]]);
+            if constexpr (sizeof(T) == 8) xp[k] = pts[4][at[k]];
+            sfw[k] = mk((double)keep.sfw[k].x, (double)keep.sfw[k].y);
+        }
+        const CorrOut r = corr_core<4, T>(et, zvol0, zm, keep.p, sfw, x, vs, xp, dt, badc, dvov);
+        o.zwrate[z] = r.zwrate;
+        o.zetot[z] = r.zetot;
+        if constexpr (sizeof(T) == 8) {
+            o.ze[z] = r.ze;
+            o.zr[z] = r.zr;
+        }
+        o.zvol[z] = r.zvol;
+        a.zp[z] = keep.p;
+        dtm = (dtz < dtm) ? dtz : dtm;       // a NaN never replaces the minimum
+    }
+    int badp = own ? bad : 0;
+    blk_fold_fin<PN_BLOCK>(dtm, dvov, badp, badc);
+    if (tid == 0) {
+        a.part_dt[slot] = dtm;
+        a.part_bp[slot] = badp;
+        a.part_dv[slot] = dvov;
+        a.part_bc[slot] = badc;
+    }
+    return false;
+}
+
+// The second cycle of a pair when the first ended the run: the tile's own
+// part of the state goes back to the problem's arrays.
+template <typename T>
+__device__ __forceinline__ void tile_copy(const FusedArgs& a, const TileOut& o, const TileMesh& g, int i0, int j0) {
+    const int ti = threadIdx.x & (PN_TILE - 1), tj = threadIdx.x / PN_TILE;
+    const int i = i0 + ti, j = j0 + tj;
+    if (ti < 1 || tj < 1 || i > g.nzx || j > g.nzy) return;
+    if ((ti <= PN_TIN || i == g.nzx) && (tj <= PN_TIN || j == g.nzy)) {
+        const int p = tile_point(g, i, j);
+        a.oxx[p] = a.pxx[p];
+        a.oxy[p] = a.pxy[p];
+        a.oux[p] = a.pux[p];
+        a.ouy[p] = a.puy[p];
+    }
+    if (ti <= PN_TIN && tj <= PN_TIN && i < g.nzx && j < g.nzy) {
+        const int z = tile_zone(g, i, j);
+        o.zetot[z] = a.zetot[z];
+        o.zwrate[z] = a.zwrate[z];
+        o.zvol[z] = a.zvol[z];
+        if constexpr (sizeof(T) == 8) {
+            o.zr[z] = a.zr[z];
+            o.ze[z] = a.ze[z];
+        }
+    }
+}
+
+struct TileArgs {
+    TileOut o;
+    TileMesh g;
+    int ntx, ntiles;
+    int back;                    // the second cycle of a pair
+    int poff;                    // the tiles' first partial
+    int* list;                   // learned form: tiles left to the list kernel, and their number
+    int* nlist;
+};
+__device__ __forceinline__ void tile_at(const TileArgs& t, int tile, int& i0, int& j0) {
+    const int tj = tile / t.ntx, ti = tile - tj * t.ntx;
+    i0 = ti * PN_TIN - 1;
+    j0 = t.g.pie + tj * PN_TIN - 1;
+}
+
+// One block per tile, the tiles of each XCD a contiguous share in row order
+// (neighbouring tiles share their rings through its L2); a pie's origin takes
+// one block more.  The flagging form needs 147 VGPRs: at four waves per SIMD it
+// spills 9 and takes 142 us on Sedov 1440^2, at three 121 us.
+template <typename T, int CL>
+__global__ void __launch_bounds__(PN_BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 2 : (CL == CL_FLAG ? 3 : 4))))
+k_tile(FusedArgs a, TileArgs t) {
+    const Ctl* c = a.ctl;
+    const int done = c->done;
+    if (done && !(t.back && c->cur)) return;
+    const double dt = c->dt;
+    if ((int)blockIdx.x == t.ntiles) {
+        if (done) {
+            if (threadIdx.x == 0) {
+                const int p = t.g.po;
+                a.oxx[p] = a.pxx[p]; a.oxy[p] = a.pxy[p]; a.oux[p] = a.pux[p]; a.ouy[p] = a.puy[p];
+            }
+        } else {
+            point_heavy<T>(a, t.g.po, dt);
+        }
+        return;
+    }
+    // the XCD shares of the tiles alone (the origin's block comes last)
+    const int n = t.ntiles, b = blockIdx.x, qn = n >> 3, rn = n & 7, x = b & 7;
+    const int tile = x * qn + (x < rn ? x : rn) + (b >> 3);
+    int i0, j0;
+    tile_at(t, tile, i0, j0);
+    if (done) {
+        tile_copy<T>(a, t.o, t.g, i0, j0);
+        return;
+    }
+    ClCount none;
+    const bool left = tile_body<T, CL>(a, t.o, t.g, i0, j0, t.poff + tile, dt, c->zre_valid != 0, none);
+    if (CL == CL_FLAG && left && threadIdx.x == 0) t.list[atomicAdd(t.nlist, 1)] = tile;
+}
+
+// The learned form's tiles that have a zone for the network (in the ring or
+// inside): the whole tile again, the network evaluated for the wave's gated
+// corners packed together.  Their order in the list is not fixed, their
+// results are.
+__global__ void __launch_bounds__(PN_BLOCK) __attribute__((amdgpu_waves_per_eu(2)))
+k_tile_list(FusedArgs a, TileArgs t) {
+    const int done = a.ctl->done, n = *t.nlist;
+    const double dt = a.ctl->dt;
+    const bool zre = a.ctl->zre_valid != 0;
+    if (done || (int)blockIdx.x >= n) return;
+    constexpr int NQ = (int)(sizeof(ClosurePack) / 16);
+    __shared__ ClosurePack wp;
+    {
+        const uint4* src = reinterpret_cast<const uint4*>(a.pack);
+        uint4* dst = reinterpret_cast<uint4*>(&wp);
+        for (int k = threadIdx.x; k < NQ; k += PN_BLOCK) dst[k] = src[k];
+    }
+    __syncthreads();
+    FusedArgs b = a;
+    b.pack = &wp;
+    ClCount cnt;
+    for (int k = blockIdx.x; k < n; k += gridDim.x) {
+        const int tile = t.list[k];
+        int i0, j0;
+        tile_at(t, tile, i0, j0);
+        (void)tile_body<float, CL_PACKED>(b, t.o, t.g, i0, j0, t.poff + tile, dt, zre, cnt);
+    }
+    const int nl = block_sum(cnt.learned);
+    const int nf = block_sum(cnt.fallback);
+    if (threadIdx.x == 0 && (nl | nf)) {
+        atomicAdd(a.cl_stats, (unsigned long long)nl);
+        atomicAdd(a.cl_stats + 1, (unsigned long long)nf);
+    }
+}
+
+// K4 of a tile cycle; also says where the state is now (cur: 1 after the first
+// cycle of a pair) and empties the learned form's lists.
+// Blocks of 256 threads fold 2048 partials in one round of loads; with more, a
+// block of 1024 saves rounds and costs 1.3 us of barriers.
+template <int BS>
+__global__ void __launch_bounds__(BS) k_finalize_tile(FusedArgs a, int npred, int ncorr, DtParams q,
+                                                                 int zre, int cur, int* nlist) {
+    if (nlist && threadIdx.x == 0) *nlist = 0;
+    if (a.zcount)
+        for (int k = threadIdx.x; k < a.nzruns * PN_LSLICES; k += BS) a.zcount[k * PN_LSTRIDE] = 0u;
+    const CtlSnap v = snap_ctl(a.ctl);
+    double mn = 1.e99, mx = 1.e-99;
+    int bp = 0, bc = 0;
+    fold_partials<BS>(a.part_dt, a.part_bp, npred, a.part_dv, a.part_bc, ncorr, mn, bp, mx, bc);
+    blk_fold_fin<BS>(mn, mx, bp, bc);
+    if (threadIdx.x != 0) return;
+    if (v.done) {
+        if (!cur) a.ctl->cur = 0;            // copied back
+        return;
+    }
+    end_cycle(a.ctl, v, mn, mx, bp, bc, q.cflv, q.cstop, q.dtmax, q.dtfac, q.tstop, zre);
+    a.ctl->cur = cur;
+}
+
 FusedArgs make_args(pennant_problem* pb) {
     FusedArgs a;
     const Params& q = pb->prm;
     a.mapsp1 = pb->dm.mapsp1; a.pcbeg = pb->dm.pcbeg; a.pcpos = pb->pcpos;
     a.smf = pb->f("smf"); a.nump = pb->dm.nump; a.npown = own_points(pb); a.la_npred = 0;
     a.pxx = pb->f("px", 0); a.pxy = pb->f("px", 1); a.pux = pb->f("pu", 0); a.puy = pb->f("pu", 1);
+    a.oxx = a.pxx; a.oxy = a.pxy; a.oux = a.pux; a.ouy = a.puy;
     a.zr = pb->f("zr"); a.ze = pb->f("ze"); a.zetot = pb->f("zetot"); a.zwrate = pb->f("zwrate");
     a.zvol = pb->f("zvol"); a.zp = pb->f("zp"); a.zm = pb->f("zm");
     a.cfx = pb->cfx; a.cfy = pb->cfy; a.cmass = pb->cmass; a.sfwx = pb->sfwx; a.sfwy = pb->sfwy;
@@ -2510,6 +2965,7 @@ BatchArgs make_batch_args(pennant_batch* b) {
     a.npown = a.nump;
     a.la_npred = 0;
     a.pxx = b->pxx; a.pxy = b->pxy; a.pux = b->pux; a.puy = b->puy;
+    a.oxx = a.pxx; a.oxy = a.pxy; a.oux = a.pux; a.ouy = a.puy;
     a.zr = b->zr; a.ze = b->ze; a.zetot = b->zetot; a.zwrate = b->zwrate; a.zvol = b->zvol;
     a.zp = b->zp; a.zm = b->zm;
     a.cfx = b->cfx; a.cfy = b->cfy; a.cmass = b->cmass; a.sfwx = b->sfwx; a.sfwy = b->sfwy;
@@ -2674,6 +3130,7 @@ int fused_setup(pennant_problem* pb) {
     pb->bcv_dev = (double*)al(16, 8);
     if (!pb->bcv_dev || hipMemcpy(pb->bcv_dev, bcv, sizeof bcv, hipMemcpyHostToDevice) != hipSuccess)
         return (int)hipErrorOutOfMemory;
+    if (const int rc = tile_setup(pb)) return rc;
     return (int)hipMemcpy(pb->pbc, bits.data(), bits.size(), hipMemcpyHostToDevice);
 }
 
@@ -2881,6 +3338,133 @@ int fused_cycle_pipe(pennant_problem* pb, hipEvent_t* ev, int form) {
         if (rc) return rc;
     }
     if (ev) (void)hipEventRecord(ev[4], s);
+    return (int)hipGetLastError();
+}
+
+namespace {
+
+// The tile cycle's arguments, with the points and zones read from the state
+// that cycle `second` of a pair starts from.
+TileArgs tile_args(const pennant_problem* pb, int second, FusedArgs& a) {
+    TileArgs t;
+    const TileState& q = pb->tile;
+    double* const own[9] = {a.pxx, a.pxy, a.pux, a.puy, a.zr, a.ze, a.zetot, a.zwrate, a.zvol};
+    double* const* src = second ? q.alt : own;
+    double* const* dst = second ? own : q.alt;
+    a.pxx = src[0]; a.pxy = src[1]; a.pux = src[2]; a.puy = src[3];
+    a.zr = src[4]; a.ze = src[5]; a.zetot = src[6]; a.zwrate = src[7]; a.zvol = src[8];
+    a.oxx = dst[0]; a.oxy = dst[1]; a.oux = dst[2]; a.ouy = dst[3];
+    t.o = {dst[4], dst[5], dst[6], dst[7], dst[8]};
+    t.g = {q.nzx, q.nzy, q.pie, 0, 0, 0};
+    t.ntx = (q.nzx + PN_TIN - 1) / PN_TIN;
+    t.ntiles = t.ntx * ((q.nzy - q.pie + PN_TIN - 1) / PN_TIN);
+    t.back = second;
+    t.list = q.list;
+    t.nlist = q.nlist;
+    a.part_dt = q.part_d;
+    a.part_dv = q.part_d + q.npart;
+    a.part_bp = q.part_i;
+    a.part_bc = q.part_i + q.npart;
+    return t;
+}
+
+}  // namespace
+
+int tile_cycle(pennant_problem* pb, int form, int second) {
+    if (!pb->tile.nzx || (form == FORM_LEARNED && !pb->closure)) return PENNANT_EINVAL;
+    FusedArgs a = make_args(pb);
+    FusedArgs tri = a;                       // the triangles' own state stays in the problem's arrays
+    TileArgs t = tile_args(pb, second, a);
+    hipStream_t s = pb->stream;
+    const dim3 blk(PN_BLOCK);
+    const int nt = t.g.pie ? t.g.nzx : 0;    // triangles
+    int npred = 0, ncorr = 0;
+    tri.part_dt = a.part_dt; tri.part_dv = a.part_dv; tri.part_bp = a.part_bp; tri.part_bc = a.part_bc;
+    if (nt) {
+        tri.pxx = a.pxx; tri.pxy = a.pxy; tri.pux = a.pux; tri.puy = a.puy;
+        launch_pred<3>(pb, tri, 0, nt, 0, 0, form, 0, s);
+        npred = pred_grid(pb, nt, 3, form);
+        ncorr = corr_grid(pb, nt);
+        if (form == FORM_LEARNED) {
+            const dim3 g(npred < 512 ? npred : 512);
+            hipLaunchKernelGGL(k_pred_list<3>, g, blk, 0, s, tri, 0, nt, 0, 0);
+        }
+    }
+    // one partial index per tile for both halves
+    t.poff = npred > ncorr ? npred : ncorr;
+    const dim3 grid(t.ntiles + (nt ? 1 : 0));
+    if (form == FORM_FP64)
+        hipLaunchKernelGGL((k_tile<double, CL_EXACT>), grid, blk, 0, s, a, t);
+    else if (form == FORM_MIXED)
+        hipLaunchKernelGGL((k_tile<float, CL_EXACT>), grid, blk, 0, s, a, t);
+    else {
+        hipLaunchKernelGGL((k_tile<float, CL_FLAG>), grid, blk, 0, s, a, t);
+        hipLaunchKernelGGL(k_tile_list, dim3(t.ntiles < 512 ? t.ntiles : 512), blk, 0, s, a, t);
+    }
+    if (nt) {
+        tri.pxx = a.oxx; tri.pxy = a.oxy; tri.pux = a.oux; tri.puy = a.ouy;
+        launch_corr<3>(pb, tri, 0, nt, 0, 0, form, s);
+    }
+    // the triangles' launches use equal grids, so no partial lies between
+    // theirs and the tiles'
+    if (npred != ncorr) return PENNANT_EINVAL;
+    const int np = t.poff + t.ntiles, zre = form == FORM_FP64 ? 1 : 0, cur = second ? 0 : 1;
+    int* nlist = form == FORM_LEARNED ? t.nlist : nullptr;
+    if (np <= PN_FIN_PER * PN_FIN_BLOCK)
+        hipLaunchKernelGGL(k_finalize_tile<PN_FIN_BLOCK>, dim3(1), dim3(PN_FIN_BLOCK), 0, s, a, np, np, dt_params(pb),
+                           zre, cur, nlist);
+    else
+        hipLaunchKernelGGL(k_finalize_tile<1024>, dim3(1), dim3(1024), 0, s, a, np, np, dt_params(pb), zre, cur, nlist);
+    return (int)hipGetLastError();
+}
+
+// Whether the mesh is one the tile cycle takes: a rect (rect_detect has
+// checked every side) or a pie of at least two rows in the generator's
+// numbering, every side's point checked here against the formula the kernel
+// uses.  Allocates the second set of state arrays, the partials and the
+// learned form's list.
+int tile_setup(pennant_problem* pb) {
+    const HostMesh& h = pb->hm;
+    TileState& q = pb->tile;
+    q.nzx = 0;
+    const int64_t nzx = pb->prm.nzx;
+    const bool pie = pb->prm.meshtype == "pie" && own_points(pb) == h.nump;
+    if (!pie && pb->rect_nzx == 0) return 0;
+    const int64_t nzy = nzx > 0 ? h.numz / nzx : 0;
+    if (pie) {
+        if (nzx < 1 || nzy < 2 || nzx * nzy != h.numz || h.nump != (nzx + 1) * nzy + 1 ||
+            (int64_t)h.nums != 3 * nzx + 4 * nzx * (nzy - 1))
+            return 0;
+        for (int64_t j = 0; j < nzy; ++j)
+            for (int64_t i = 0; i < nzx; ++i) {
+                const int64_t z = j * nzx + i, sb = j ? 4 * z - nzx : 3 * i;
+                const int64_t p = j * (nzx + 1) + i - nzx;        // the quad's first point
+                const int64_t quad[4] = {p, p + 1, p + nzx + 2, p + nzx + 1}, tri[3] = {0, i + 2, i + 1};
+                if (h.zsbeg[z] != sb || h.znump[z] != (j ? 4 : 3)) return 0;
+                for (int k = 0; k < (j ? 4 : 3); ++k)
+                    if (h.mapsp1[sb + k] != (j ? quad[k] : tri[k])) return 0;
+            }
+    }
+    const int64_t tiles = ((nzx + PN_TIN - 1) / PN_TIN) * ((nzy - pie + PN_TIN - 1) / PN_TIN);
+    const int64_t P = h.nump, Z = h.numz;
+    q.npart = (int)tiles + PN_MAX_GRID;
+    const size_t bytes = (size_t)(4 * P + 5 * Z + 2 * (int64_t)q.npart) * 8 + (size_t)(2 * (int64_t)q.npart + tiles + 1) * 4;
+    char* m = nullptr;
+    if (hipMalloc((void**)&m, bytes) != hipSuccess) return (int)hipErrorOutOfMemory;
+    pb->allocs.push_back(m);
+    double* d = (double*)m;
+    for (int k = 0; k < 9; ++k) {
+        q.alt[k] = d;
+        d += k < 4 ? P : Z;
+    }
+    q.part_d = d;
+    q.part_i = (int*)(d + 2 * (int64_t)q.npart);
+    q.nlist = q.part_i + 2 * (int64_t)q.npart;
+    q.list = q.nlist + 1;
+    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, pb->stream, (unsigned*)q.nlist, 1);
+    q.nzx = (int)nzx;
+    q.nzy = (int)nzy;
+    q.pie = pie ? 1 : 0;
     return (int)hipGetLastError();
 }
 

@@ -39,6 +39,7 @@ struct Ctl {
     // corrector stored neither, and predictors derive them from zm, zvol and
     // zetot with the same quotients until they are materialised
     int zre_valid;
+    int cur;          // tile cycles: 1 while the state is in the second set of arrays
 };
 
 #define PN_MAX_GRID 4096   // largest grid of a fused K1/K3 launch
@@ -68,6 +69,7 @@ struct Tuning {
     int graph = 1;           // batched cycles through a captured HIP graph
     int pipeline = 0;        // mixed forms: next cycle's predictor in the corrector pass
     int rect_maps = 1;       // structured rect meshes: zone points and corner slots computed, not loaded
+    int tiles = 1;           // structured meshes: the whole cycle in one kernel over tiles of zones
 };
 
 struct Params {
@@ -82,6 +84,20 @@ struct DevField {
     int kind;        // 0 point, 1 zone, 2 side
     int ncomp;       // 1 or 2
     double* c[2];
+};
+
+// What the tile cycle of a structured mesh keeps (tile_setup): the mesh's
+// zones nzx x nzy (nzx 0: not such a mesh), the second set of state arrays
+// (px, pu by component, zr, ze, zetot, zwrate, zvol), block partials, and the
+// tiles that the learned form leaves to its list kernel.
+struct TileState {
+    int nzx = 0, nzy = 0, pie = 0;
+    double* alt[9] = {};
+    double* part_d = nullptr;
+    int* part_i = nullptr;
+    int npart = 0;
+    int* list = nullptr;
+    int* nlist = nullptr;
 };
 
 struct HostMesh {
@@ -139,6 +155,7 @@ struct pennant_problem {
     int rect_nzx = 0;
     unsigned long long rect_m = 0;
     int rect_sh = 0;
+    pn::TileState tile;
     int* zlist = nullptr;            // zones for the learned pass (per run, at the run's zone range)
     unsigned* zcount = nullptr;      // per run and list slice, one 128-byte line each
     pn::Tuning tune;
@@ -247,6 +264,10 @@ int fused_cycle(pennant_problem* pb, hipEvent_t* ev, int form);
 // ev: NULL, or 5 events recorded before K2, the zone pass, K4 and the redo,
 // the learned pass, and after it
 int fused_prologue(pennant_problem* pb, int form);
+// Tile cycle of a structured mesh: cycle `second` (0, 1) of a pair.  The
+// state is in the problem's own arrays before and after every pair.
+int tile_setup(pennant_problem* pb);
+int tile_cycle(pennant_problem* pb, int form, int second);
 int fused_cycle_pipe(pennant_problem* pb, hipEvent_t* ev, int form);
 // Stores zr = zm / zvol and ze = zetot / (zm + 1e-99) where mixed cycles left
 // them to be derived (the mixed corrector does not store them).
