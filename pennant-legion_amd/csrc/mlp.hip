@@ -1,9 +1,9 @@
 // The learned QCS closure's network on the device: parameters, BF16 MFMA
-// GEMM, training (forward, backward, Adam) and batched inference.
+// kernels for training (forward, backward, Adam) and batched inference.
 //
-// Training step on a minibatch of B tuples (all matrices row-major, BF16
-// operands, FP32 accumulation; H1, H2 and the gradients fed to the next GEMM
-// are rounded to BF16 where the MFMA consumes them):
+// Training step on a minibatch of B tuples (BF16 operands, FP32 accumulation;
+// H1, H2 and the gradients fed to the next product are rounded to BF16 where
+// the MFMA consumes them):
 //   Z1 = X W1^T          H1 = relu(Z1)
 //   Z2 = H1 W2^T + b2    H2 = relu(Z2)
 //   Y  = H2 W3^T + b3    loss = sum_b sum_o (Y - T)^2 / B
@@ -11,8 +11,19 @@
 //   dW3 = dY^T H2   db3 = colsum dY    dZ2 = (dY W3) * [H2 > 0]
 //   dW2 = dZ2^T H1  db2 = colsum dZ2   dZ1 = (dZ2 W2) * [H1 > 0]
 //   dW1 = dZ1^T X   (column 10 of X is 1, so dW1[:,10] is the bias gradient)
-// Every reduction runs in a fixed order (one wave per output tile, split-K
-// partials summed in order), so training is deterministic.
+// Three launches a step: k_rows (a wave takes 32 rows through forward and
+// backward in registers), k_grads (the weight gradients over the batch, bias
+// and loss sums), k_update (sums of the partials, Adam, the BF16 copies).
+// Every reduction runs in a fixed order (split-K partials summed in order), so
+// training is deterministic.
+//
+// What bounds a step at B = 8192 is latency: k_rows 9.0 us (the row list over
+// PCIe, the gathered tuples, a chain of 26 products), k_grads 10.8 us (eight
+// rounds of loads of what other XCDs have just written; loading twice or four
+// times as far ahead changed nothing), k_update 5.4 us, and the host's draw of
+// the next step's rows, 30 us, beside them: 32 us a step.  One kernel per
+// product and elementwise step (22 launches, 112 us of kernels, drawing while
+// the GPU waited) took 262 us.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -33,16 +44,21 @@ struct pennant_mlp {
     float* v = nullptr;
     __bf16* w1b = nullptr;     // BF16 copies, row-major [out][in]
     __bf16* w2b = nullptr;
+    __bf16* w2t = nullptr;     // W2 transposed, [in][out]
     __bf16* w3b = nullptr;
     ClosurePack* pack = nullptr;
     float lo[PN_MLP_NF], hi[PN_MLP_NF];
     int adam_t = 0;
-    // minibatch buffers (capacity cap rows)
+    // batch buffers (capacity cap rows, a multiple of 32): per unit a row of
+    // the batch's values
     int64_t cap = 0;
-    int* idx = nullptr;
-    int* idx_host = nullptr;   // pinned
-    __bf16 *xb = nullptr, *h1 = nullptr, *h2 = nullptr, *dyb = nullptr, *dz2 = nullptr, *dz1 = nullptr;
-    float *t = nullptr, *z = nullptr, *y = nullptr, *dh = nullptr, *part = nullptr, *lossp = nullptr;
+    int* idx_host[2] = {};     // pinned: the rows of a step, read by the kernel
+    hipEvent_t read[2] = {};   // when they have been read
+    __bf16 *xt = nullptr, *h1t = nullptr, *h2t = nullptr, *dyt = nullptr, *dz2t = nullptr, *dz1t = nullptr;
+    float *lrow = nullptr, *lossp = nullptr;
+    float* part = nullptr;     // split-K partials
+    float* losses = nullptr;   // per step
+    int loss_cap = 0;
     hipStream_t stream = nullptr;
     std::string err;
 };
@@ -52,225 +68,365 @@ namespace {
 #define MCK(x) do { const int e_ = (int)(x); if (e_ != 0) return e_; } while (0)
 
 // ---------------------------------------------------------------------------
-// GEMM: C[M][N] = sum_k A(i,k) B(k,j), A(i,k) = ta ? A[k*lda+i] : A[i*lda+k],
-// B(k,j) = tb ? B[j*ldb+k] : B[k*ldb+j].  One wave per 32x32 tile of C;
-// blockIdx.z splits K into gridDim.z contiguous ranges whose partial tiles go
-// to C + z*M*N (summed afterwards in order by k_sum_parts).
-__global__ void __launch_bounds__(64) k_gemm(int M, int N, int K, int kper, const __bf16* __restrict__ A,
-                                             int lda, int ta, const __bf16* __restrict__ B, int ldb,
-                                             int tb, float* __restrict__ C) {
-    const int lane = threadIdx.x, h = lane >> 5, r = lane & 31;
-    const int i = blockIdx.y * 32 + r;        // A row of this lane
-    const int j = blockIdx.x * 32 + r;        // B column of this lane
-    const int kb = blockIdx.z * kper;
-    const int ke = (kb + kper < K) ? kb + kper : K;
-    const __bf16 zero = (__bf16)0.f;
-    f32x16 acc = {};
-    for (int k0 = kb; k0 < ke; k0 += 16) {
-        bf16x8 a, b;
+// A wave's rows through the network.
+//
+// The products are taken as C^T = W act^T, so that a lane's accumulator
+// holds one batch row (lane % 32) and the units 8 (q / 4) + 4 (lane / 32) + q
+// % 4 of register q.  The next product wants, per 16 units, units 0-7 in the
+// low half of the wave and 8-15 in the high half: one swap of the halves per
+// register pair, and no pass through LDS.  Within an MFMA the units stay in
+// order, so a result does not depend on how the rows are spread over waves.
+
+// Units 16 c .. 16 c + 15 of an accumulator pair (already rounded: packed
+// pairs of registers), as the B operand of the next product.
+__device__ __forceinline__ bf16x8 next_operand(const unsigned (&v)[2][8], int c) {
+    const unsigned* a = &v[c >> 1][4 * (c & 1)];
+    u32x4 o;
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const int k = k0 + 8 * h + t;
-            const bool kin = k < ke;
-            a[t] = (kin && i < M) ? (ta ? A[(int64_t)k * lda + i] : A[(int64_t)i * lda + k]) : zero;
-            b[t] = (kin && j < N) ? (tb ? B[(int64_t)j * ldb + k] : B[(int64_t)k * ldb + j]) : zero;
+    for (int d = 0; d < 2; ++d) {
+        const auto r = __builtin_amdgcn_permlane32_swap(a[d], a[2 + d], false, false);
+        o[d] = r[0];
+        o[2 + d] = r[1];
+    }
+    return as_bf16x8(o);
+}
+__device__ __forceinline__ float bf_lo(unsigned v) { return __uint_as_float(v << 16); }
+__device__ __forceinline__ float bf_hi(unsigned v) { return __uint_as_float(v & 0xffff0000u); }
+
+// Register pairs (2 d, 2 d + 1) of an accumulator to rows [unit][b] of dst.
+__device__ __forceinline__ void store_units(const unsigned (&v)[2][8], __bf16* dst, int64_t ld, int64_t b, int h) {
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int d = 0; d < 8; ++d) {
+            const int64_t u = 32 * mb + 8 * (d >> 1) + 4 * h + 2 * (d & 1);
+            unsigned short* o = reinterpret_cast<unsigned short*>(dst) + u * ld + b;
+            o[0] = (unsigned short)v[mb][d];
+            o[ld] = (unsigned short)(v[mb][d] >> 16);
         }
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-    }
-    float* Cz = C + (int64_t)blockIdx.z * M * N;
+}
+
+typedef float f32x2a __attribute__((ext_vector_type(2), aligned(4)));
+
+struct RowArgs {
+    const float* p;
+    const __bf16 *w1b, *w2b, *w2t, *w3b;
+    int64_t n;                 // rows
+    const float* x;            // rows of 10 features, or tuples
+    const int* idx;            // training: the tuple of row b (NULL: tuple b)
+    float* y;                  // inference: n x 2
+    int64_t ld;                // training: row length of the buffers below
+    __bf16 *xt, *h1t, *h2t, *dyt, *dz2t, *dz1t;
+    float* lrow;
+};
+
+// 32 rows a wave: forward, and with TRAIN the loss of each row and its
+// backward values; rows past n give zeros.
+template <bool TRAIN>
+__global__ void __launch_bounds__(64) k_rows(RowArgs a) {
+    const int lane = threadIdx.x, h = lane >> 5, r = lane & 31;
+    const int64_t b = (int64_t)blockIdx.x * 32 + r;
+    const bool in = b < a.n;
+    const int64_t bc = in ? b : a.n - 1;
+    const float* row = TRAIN ? a.x + (a.idx ? (int64_t)a.idx[bc] : bc) * PN_MLP_TUPLE : a.x + bc * PN_MLP_NF;
+    // the row's inputs 8 h .. 8 h + 7 (10: the bias slot, 11-15: zeros), and
+    // its targets in the low half
+    f32x2a f[4];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        const int ci = blockIdx.y * 32 + 8 * (q >> 2) + 4 * h + (q & 3);
-        const int cj = blockIdx.x * 32 + r;
-        if (ci < M && cj < N) Cz[(int64_t)ci * N + cj] = acc[q];
+    for (int k = 0; k < 4; ++k) f[k] = *reinterpret_cast<const f32x2a*>(row + (h ? 8 : 2 * k));
+    f32x2a t = {0.f, 0.f};
+    if constexpr (TRAIN) t = *reinterpret_cast<const f32x2a*>(row + PN_MLP_NF);
+    bf16x8 w1[2], w2[2][4];
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb) {
+        w1[mb] = *reinterpret_cast<const bf16x8*>(a.w1b + (32 * mb + r) * PN_MLP_K1 + 8 * h);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            w2[mb][c] = *reinterpret_cast<const bf16x8*>(a.w2b + (32 * mb + r) * PN_MLP_NH + 16 * c + 8 * h);
     }
-}
-
-__global__ void k_sum_parts(int n, int nparts, const float* __restrict__ part, float* __restrict__ out) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float s = 0.f;
-    for (int z = 0; z < nparts; ++z) s += part[(int64_t)z * n + i];
-    out[i] = s;
-}
-
-// C (row-major M x N, FP32) = op(A) op(B).  Uses `part` (M*N*ksplit floats)
-// when K is split.
-int gemm(int M, int N, int K, const __bf16* A, int lda, int ta, const __bf16* B, int ldb, int tb,
-         float* C, float* part, hipStream_t s) {
-    // split long reductions (the weight gradients over the batch) into
-    // chunks of 512 so that more waves share them
-    int ksplit = 1;
-    if (K > 1024 && part) ksplit = (K + 511) / 512;
-    if (ksplit > 64) ksplit = 64;
-    int kper = (K + ksplit - 1) / ksplit;
-    kper = (kper + 15) / 16 * 16;
-    ksplit = (K + kper - 1) / kper;
-    const dim3 grid((N + 31) / 32, (M + 31) / 32, ksplit);
-    if (ksplit == 1) {
-        hipLaunchKernelGGL(k_gemm, grid, dim3(64), 0, s, M, N, K, kper, A, lda, ta, B, ldb, tb, C);
-    } else {
-        hipLaunchKernelGGL(k_gemm, grid, dim3(64), 0, s, M, N, K, kper, A, lda, ta, B, ldb, tb, part);
-        const int n = M * N;
-        hipLaunchKernelGGL(k_sum_parts, dim3((n + 255) / 256), dim3(256), 0, s, n, ksplit, part, C);
+    u32x4 xv;
+    xv[0] = pack_bf16(f[0][0], f[0][1]);
+    xv[1] = h ? pack_bf16(1.f, 0.f) : pack_bf16(f[1][0], f[1][1]);
+    xv[2] = h ? 0u : pack_bf16(f[2][0], f[2][1]);
+    xv[3] = h ? 0u : pack_bf16(f[3][0], f[3][1]);
+    if (!in) xv = u32x4{0u, 0u, 0u, 0u};
+    const bf16x8 x = as_bf16x8(xv);
+    // layer 1
+    unsigned h1[2][8], h2[2][8];
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb) {
+        const f32x16 zero = {};
+        const f32x16 z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w1[mb], x, zero, 0, 0, 0);
+#pragma unroll
+        for (int d = 0; d < 8; ++d) h1[mb][d] = relu_bf16(z[2 * d], z[2 * d + 1]);
     }
-    return (int)hipGetLastError();
+    // layer 2
+    bf16x8 act[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) act[c] = next_operand(h1, c);
+    const float* b2 = a.p + PN_MLP_OFF_B2;
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb) {
+        f32x16 z = {};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w2[mb][c], act[c], z, 0, 0, 0);
+#pragma unroll
+        for (int d = 0; d < 8; ++d) {
+            const float* bu = b2 + 32 * mb + 8 * (d >> 1) + 4 * h + 2 * (d & 1);
+            const unsigned v = relu_bf16(z[2 * d] + bu[0], z[2 * d + 1] + bu[1]);
+            h2[mb][d] = in ? v : 0u;
+        }
+    }
+    // output layer: rows 0 and 1 of W3, the others zero
+    f32x16 z3 = {};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const bf16x8 zero8 = {};
+        const bf16x8 w = r < PN_MLP_NO
+                             ? *reinterpret_cast<const bf16x8*>(a.w3b + r * PN_MLP_NH + 16 * c + 8 * h)
+                             : zero8;
+        z3 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, next_operand(h2, c), z3, 0, 0, 0);
+    }
+    // the outputs of row r are in its low lane
+    const float y0 = z3[0] + a.p[PN_MLP_OFF_B3], y1 = z3[1] + a.p[PN_MLP_OFF_B3 + 1];
+    if constexpr (!TRAIN) {
+        if (in && !h) {
+            const f32x2a y = {y0, y1};
+            *reinterpret_cast<f32x2a*>(a.y + 2 * b) = y;
+        }
+        return;
+    }
+    const float d0 = y0 - t[0], d1 = y1 - t[1];
+    const float inv = 2.f / (float)a.n;
+    const unsigned dy = (in && !h) ? pack_bf16(inv * d0, inv * d1) : 0u;
+    if (!h) {
+        a.lrow[b] = in ? d0 * d0 + d1 * d1 : 0.f;
+        unsigned short* o = reinterpret_cast<unsigned short*>(a.dyt) + b;
+        o[0] = (unsigned short)dy;
+        o[a.ld] = (unsigned short)(dy >> 16);
+    }
+    {
+        unsigned short* o = reinterpret_cast<unsigned short*>(a.xt) + (int64_t)(8 * h) * a.ld + b;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            o[(2 * k) * a.ld] = (unsigned short)xv[k];
+            o[(2 * k + 1) * a.ld] = (unsigned short)(xv[k] >> 16);
+        }
+    }
+    store_units(h1, a.h1t, a.ld, b, h);
+    store_units(h2, a.h2t, a.ld, b, h);
+    // dZ2 = (dY W3) [H2 > 0]: two of the product's 16 inputs
+    u32x4 dyv = {dy, 0u, 0u, 0u};
+    unsigned g2[2][8], g1[2][8];
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb) {
+        const unsigned short* w = reinterpret_cast<const unsigned short*>(a.w3b) + 32 * mb + r;
+        const u32x4 wv = {h ? 0u : ((unsigned)w[0] | ((unsigned)w[PN_MLP_NH] << 16)), 0u, 0u, 0u};
+        const f32x16 zero = {};
+        const f32x16 z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(wv), as_bf16x8(dyv), zero, 0, 0, 0);
+#pragma unroll
+        for (int d = 0; d < 8; ++d)
+            g2[mb][d] = pack_bf16(bf_lo(h2[mb][d]) > 0.f ? z[2 * d] : 0.f, bf_hi(h2[mb][d]) > 0.f ? z[2 * d + 1] : 0.f);
+    }
+    store_units(g2, a.dz2t, a.ld, b, h);
+    // dZ1 = (dZ2 W2) [H1 > 0]
+#pragma unroll
+    for (int c = 0; c < 4; ++c) act[c] = next_operand(g2, c);
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb) {
+        f32x16 z = {};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const bf16x8 w = *reinterpret_cast<const bf16x8*>(a.w2t + (32 * mb + r) * PN_MLP_NH + 16 * c + 8 * h);
+            z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, act[c], z, 0, 0, 0);
+        }
+#pragma unroll
+        for (int d = 0; d < 8; ++d)
+            g1[mb][d] = pack_bf16(bf_lo(h1[mb][d]) > 0.f ? z[2 * d] : 0.f, bf_hi(h1[mb][d]) > 0.f ? z[2 * d + 1] : 0.f);
+    }
+    store_units(g1, a.dz1t, a.ld, b, h);
 }
 
 // ---------------------------------------------------------------------------
-// elementwise and small kernels
+// The gradients over the batch.  Long reductions are split into ranges of kper
+// rows (about 512, at most 64 ranges); a wave takes one 32 x 32 tile of one
+// gradient and one range, and its partial goes to part[range] (in the flat
+// parameter layout).  Blocks after those sum the columns of dY and dZ2 (the
+// bias gradients) and the rows' losses, 256 at a time.
+struct GradArgs {
+    int64_t rows, ld;
+    int kper, ksplit;
+    const __bf16 *xt, *h1t, *h2t, *dyt, *dz2t, *dz1t;
+    const float* lrow;
+    float* part;               // ksplit x PN_MLP_NPARAM
+    float* g;
+    float* lossp;              // per 256 rows
+};
+#define PN_GTILES 8            // dW2: 2 x 2, dW1: 2 x 1, dW3: 1 x 2
 
-// minibatch rows idx[b] of the tuple array: X (BF16, slot 10 = 1) and T
-__global__ void k_gather(int B, const int* __restrict__ idx, const float* __restrict__ tup,
-                         __bf16* __restrict__ X, float* __restrict__ T) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= B) return;
-    const float* r = tup + (int64_t)idx[b] * PN_MLP_TUPLE;
-#pragma unroll
-    for (int k = 0; k < PN_MLP_K1; ++k)
-        X[(int64_t)b * PN_MLP_K1 + k] = (__bf16)(k < PN_MLP_NF ? r[k] : (k == PN_MLP_NF ? 1.f : 0.f));
-    T[2 * b] = r[PN_MLP_NF];
-    T[2 * b + 1] = r[PN_MLP_NF + 1];
-}
-
-// X rows (BF16, slot 10 = 1) from feature rows x (B x 10)
-__global__ void k_x_rows(int B, const float* __restrict__ x, __bf16* __restrict__ X) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= B) return;
-#pragma unroll
-    for (int k = 0; k < PN_MLP_K1; ++k)
-        X[(int64_t)b * PN_MLP_K1 + k] =
-            (__bf16)(k < PN_MLP_NF ? x[(int64_t)b * PN_MLP_NF + k] : (k == PN_MLP_NF ? 1.f : 0.f));
-}
-
-// Y = Z + b3 (inference)
-__global__ void k_out(int B, const float* __restrict__ Z, const float* __restrict__ b3, float* __restrict__ Y) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= B) return;
-    Y[2 * b] = Z[2 * b] + b3[0];
-    Y[2 * b + 1] = Z[2 * b + 1] + b3[1];
-}
-
-// H = bf16(relu(Z + bias)), Z is B x 64
-__global__ void k_bias_relu(int n, const float* __restrict__ Z, const float* __restrict__ bias,
-                            __bf16* __restrict__ H) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float zb = Z[i] + (bias ? bias[i & (PN_MLP_NH - 1)] : 0.f);
-    H[i] = (__bf16)fmaxf(zb, 0.f);
-}
-
-// Y = Z + b3; dY = 2 (Y - T) / B as BF16; per-block partial losses
-__global__ void __launch_bounds__(256) k_out_loss(int B, const float* __restrict__ Z,
-                                                  const float* __restrict__ b3,
-                                                  const float* __restrict__ T, float* __restrict__ Y,
-                                                  __bf16* __restrict__ dYb, float* __restrict__ lossp) {
-    const int b = blockIdx.x * 256 + threadIdx.x;
-    float l = 0.f;
-    if (b < B) {
-        const float inv = 2.f / (float)B;
-#pragma unroll
-        for (int o = 0; o < 2; ++o) {
-            const float y = Z[2 * b + o] + b3[o];
-            Y[2 * b + o] = y;
-            const float d = y - T[2 * b + o];
-            l += d * d;
-            dYb[2 * b + o] = (__bf16)(inv * d);
-        }
-    }
+// The block's sum of v in a fixed tree; thread 0 has it.
+__device__ __forceinline__ float tree256(float v) {
     __shared__ float sh[256];
-    sh[threadIdx.x] = l;
+    sh[threadIdx.x] = v;
     __syncthreads();
     for (int off = 128; off > 0; off >>= 1) {
         if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
         __syncthreads();
     }
-    if (threadIdx.x == 0) lossp[blockIdx.x] = sh[0];
+    return sh[0];
 }
 
-// dZ = bf16(dH * [H > 0])
-__global__ void k_relu_grad(int n, const float* __restrict__ dH, const __bf16* __restrict__ H,
-                            __bf16* __restrict__ dZ) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    dZ[i] = (__bf16)(((float)H[i] > 0.f) ? dH[i] : 0.f);
-}
-
-// out[j] = sum over rows of X[:, j] (X is rows x ncol BF16); one block per
-// column, fixed-order tree
-__global__ void __launch_bounds__(256) k_colsum(int rows, int ncol, const __bf16* __restrict__ X,
-                                                float* __restrict__ out) {
-    const int j = blockIdx.x;
-    float s = 0.f;
-    for (int r = threadIdx.x; r < rows; r += 256) s += (float)X[(int64_t)r * ncol + j];
-    __shared__ float sh[256];
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[j] = sh[0];
-}
-
-__global__ void k_sum_small(int n, const float* __restrict__ x, float* __restrict__ out) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        float s = 0.f;
-        for (int i = 0; i < n; ++i) s += x[i];
-        *out = s;
-    }
-}
-
-// Adam (bias-corrected); W1 input columns 11-15 stay zero
-__global__ void k_adam(int n, float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, float lr, float b1, float b2, float eps, float c1, float c2) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    if (i < PN_MLP_OFF_W2 && (i % PN_MLP_K1) > PN_MLP_NF) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.f - b1) * gi;
-    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-}
-
-// BF16 row-major copies and the A-operand pack of the fused inference
-__global__ void __launch_bounds__(256) k_pack(const float* __restrict__ p, __bf16* __restrict__ w1b,
-                                              __bf16* __restrict__ w2b, __bf16* __restrict__ w3b,
-                                              ClosurePack* __restrict__ pk) {
-    const int tid = blockIdx.x * blockDim.x + threadIdx.x;
-    const float* W1 = p + PN_MLP_OFF_W1;
-    const float* W2 = p + PN_MLP_OFF_W2;
-    const float* b2 = p + PN_MLP_OFF_B2;
-    const float* W3 = p + PN_MLP_OFF_W3;
-    for (int i = tid; i < PN_MLP_NH * PN_MLP_K1; i += gridDim.x * blockDim.x) w1b[i] = (__bf16)W1[i];
-    for (int i = tid; i < PN_MLP_NH * PN_MLP_NH; i += gridDim.x * blockDim.x) w2b[i] = (__bf16)W2[i];
-    for (int i = tid; i < PN_MLP_NO * PN_MLP_NH; i += gridDim.x * blockDim.x) w3b[i] = (__bf16)W3[i];
-    // fragments: 2 (w1) + 8 (w2) + 4 (w3) per lane
-    for (int f = tid; f < 14 * 64; f += gridDim.x * blockDim.x) {
-        const int fr = f >> 6, lane = f & 63, h = lane >> 5, m = lane & 31;
-        bf16x8 v;
-        if (fr < 2) {
-            const int row = 32 * fr + m;
-            for (int t = 0; t < 8; ++t) v[t] = (__bf16)W1[row * PN_MLP_K1 + 8 * h + t];
-            pk->w1[fr][lane] = v;
-        } else if (fr < 10) {
-            const int mb = (fr - 2) >> 2, c = (fr - 2) & 3, row = 32 * mb + m;
-            for (int t = 0; t < 8; ++t) v[t] = (__bf16)W2[row * PN_MLP_NH + 16 * c + 8 * (t >> 2) + 4 * h + (t & 3)];
-            pk->w2[mb][c][lane] = v;
+__global__ void __launch_bounds__(256) k_grads(GradArgs a) {
+    const int gblocks = a.ksplit * PN_GTILES / 4;
+    int blk = blockIdx.x;
+    if (blk < gblocks) {
+        const int item = blk * 4 + (threadIdx.x >> 6);
+        const int tile = item & (PN_GTILES - 1), range = item / PN_GTILES;
+        const int lane = threadIdx.x & 63, h = lane >> 5, r = lane & 31;
+        // gradient C[i][j] = sum_b A[i][b] B[j][b]
+        const __bf16 *A, *B;
+        int i0 = 0, j0 = 0, M = 64, N = 64, off;
+        if (tile < 4) {
+            A = a.dz2t; B = a.h1t; off = PN_MLP_OFF_W2; i0 = 32 * (tile >> 1); j0 = 32 * (tile & 1);
+        } else if (tile < 6) {
+            A = a.dz1t; B = a.xt; off = PN_MLP_OFF_W1; i0 = 32 * (tile & 1); N = PN_MLP_K1;
         } else {
-            const int c = fr - 10;
-            for (int t = 0; t < 8; ++t)
-                v[t] = (__bf16)(m < PN_MLP_NO ? W3[m * PN_MLP_NH + 16 * c + 8 * (t >> 2) + 4 * h + (t & 3)] : 0.f);
-            pk->w3[c][lane] = v;
+            A = a.dyt; B = a.h2t; off = PN_MLP_OFF_W3; j0 = 32 * (tile & 1); M = PN_MLP_NO;
         }
+        const bool ain = i0 + r < M, bin = j0 + r < N;
+        const __bf16* pa = A + (int64_t)(ain ? i0 + r : 0) * a.ld + 8 * h;
+        const __bf16* pb = B + (int64_t)(bin ? j0 + r : 0) * a.ld + 8 * h;
+        const bf16x8 zero8 = {};
+        const int64_t kb = (int64_t)range * a.kper;
+        const int64_t ke = kb + a.kper < a.rows ? kb + a.kper : a.rows;
+        f32x16 acc = {};
+        // rows past the batch hold zeros up to the next multiple of 32; four
+        // products' operands are loaded before the first is used
+        constexpr int AHEAD = 4;
+        for (int64_t k0 = kb; k0 < ke; k0 += 16 * AHEAD) {
+            bf16x8 va[AHEAD], vb[AHEAD];
+#pragma unroll
+            for (int s = 0; s < AHEAD; ++s) {
+                const int64_t k = k0 + 16 * s < ke ? k0 + 16 * s : kb;
+                va[s] = *reinterpret_cast<const bf16x8*>(pa + k);
+                vb[s] = *reinterpret_cast<const bf16x8*>(pb + k);
+            }
+#pragma unroll
+            for (int s = 0; s < AHEAD; ++s)
+                if (k0 + 16 * s < ke)
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ain ? va[s] : zero8, bin ? vb[s] : zero8, acc, 0, 0, 0);
+        }
+        float* C = a.part + (int64_t)range * PN_MLP_NPARAM + off;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const int ci = i0 + 8 * (q >> 2) + 4 * h + (q & 3), cj = j0 + r;
+            if (ci < M && cj < N) C[ci * N + cj] = acc[q];
+        }
+        return;
     }
-    for (int i = tid; i < 64; i += gridDim.x * blockDim.x) {
-        const int mb = i >> 5, h = (i >> 4) & 1, r = i & 15;
-        pk->b2c[mb][h][r] = b2[32 * mb + 8 * (r >> 2) + 4 * h + (r & 3)];
+    blk -= gblocks;
+    if (blk < PN_MLP_NO + PN_MLP_NH) {
+        const __bf16* col = blk < PN_MLP_NO ? a.dyt + blk * a.ld : a.dz2t + (blk - PN_MLP_NO) * a.ld;
+        float s = 0.f;
+#pragma unroll 8
+        for (int64_t b = threadIdx.x; b < a.rows; b += 256) s += (float)col[b];
+        s = tree256(s);
+        if (threadIdx.x == 0) a.g[blk < PN_MLP_NO ? PN_MLP_OFF_B3 + blk : PN_MLP_OFF_B2 + blk - PN_MLP_NO] = s;
+        return;
     }
-    if (tid < PN_MLP_NO) pk->b3[tid] = p[PN_MLP_OFF_B3 + tid];
+    blk -= PN_MLP_NO + PN_MLP_NH;
+    const int64_t b = (int64_t)blk * 256 + threadIdx.x;
+    const float s = tree256(b < a.rows ? a.lrow[b] : 0.f);
+    if (threadIdx.x == 0) a.lossp[blk] = s;
+}
+
+// ---------------------------------------------------------------------------
+// Where a parameter's BF16 copies live: the row-major ones and the A-operand
+// pack of the fused inference (ClosurePack).
+__device__ __forceinline__ void put_param(int i, float v, __bf16* w1b, __bf16* w2b, __bf16* w2t, __bf16* w3b,
+                                          ClosurePack* pk) {
+    const __bf16 e = (__bf16)v;
+    __bf16* q = nullptr;
+    if (i < PN_MLP_OFF_W2) {
+        const int row = i / PN_MLP_K1, k = i % PN_MLP_K1;
+        w1b[i] = e;
+        q = reinterpret_cast<__bf16*>(&pk->w1[row >> 5][(row & 31) + 32 * (k >> 3)]) + (k & 7);
+    } else if (i < PN_MLP_OFF_B2) {
+        const int j = i - PN_MLP_OFF_W2, row = j / PN_MLP_NH, k = j % PN_MLP_NH, kk = k & 15;
+        w2b[j] = e;
+        w2t[k * PN_MLP_NH + row] = e;
+        q = reinterpret_cast<__bf16*>(&pk->w2[row >> 5][k >> 4][(row & 31) + 32 * ((kk >> 2) & 1)]) + 4 * (kk >> 3) + (kk & 3);
+    } else if (i < PN_MLP_OFF_W3) {
+        const int u = i - PN_MLP_OFF_B2, w = u & 31;
+        pk->b2c[u >> 5][(w >> 2) & 1][4 * (w >> 3) + (w & 3)] = v;
+        return;
+    } else if (i < PN_MLP_OFF_B3) {
+        const int j = i - PN_MLP_OFF_W3, row = j / PN_MLP_NH, k = j % PN_MLP_NH, kk = k & 15;
+        w3b[j] = e;
+        q = reinterpret_cast<__bf16*>(&pk->w3[k >> 4][row + 32 * ((kk >> 2) & 1)]) + 4 * (kk >> 3) + (kk & 3);
+    } else {
+        pk->b3[i - PN_MLP_OFF_B3] = v;
+        return;
+    }
+    *q = e;
+}
+
+struct UpdateArgs {
+    int ksplit, nloss;
+    const float* part;
+    const float* lossp;
+    float* g;
+    float* loss;
+    // Adam (ADAM)
+    float *p, *m, *v;
+    float lr, b1, b2, eps, c1, c2;
+    __bf16 *w1b, *w2b, *w2t, *w3b;
+    ClosurePack* pack;
+};
+
+// One thread a parameter: its gradient (the ranges' partials summed in order)
+// and with ADAM its bias-corrected update and BF16 copies; one thread more
+// sums the loss.
+template <bool ADAM>
+__global__ void __launch_bounds__(256) k_update(UpdateArgs a) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i == PN_MLP_NPARAM) {
+        float s = 0.f;
+        for (int k = 0; k < a.nloss; ++k) s += a.lossp[k];
+        *a.loss = s;
+    }
+    if (i >= PN_MLP_NPARAM) return;
+    float gi;
+    if ((i >= PN_MLP_OFF_B2 && i < PN_MLP_OFF_W3) || i >= PN_MLP_OFF_B3) {
+        gi = a.g[i];
+    } else {
+        gi = a.part[i];
+#pragma unroll 16
+        for (int z = 1; z < a.ksplit; ++z) gi += a.part[(int64_t)z * PN_MLP_NPARAM + i];
+        a.g[i] = gi;
+    }
+    if constexpr (ADAM) {
+        if (i < PN_MLP_OFF_W2 && (i % PN_MLP_K1) > PN_MLP_NF) return;   // these inputs are zero
+        const float mi = a.b1 * a.m[i] + (1.f - a.b1) * gi;
+        const float vi = a.b2 * a.v[i] + (1.f - a.b2) * gi * gi;
+        a.m[i] = mi;
+        a.v[i] = vi;
+        const float pi = a.p[i] - a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
+        a.p[i] = pi;
+        put_param(i, pi, a.w1b, a.w2b, a.w2t, a.w3b, a.pack);
+    }
+}
+
+// Every parameter's BF16 copies, and zeros where the output layer's pack has
+// no row.
+__global__ void __launch_bounds__(256) k_pack(const float* __restrict__ p, __bf16* w1b, __bf16* w2b, __bf16* w2t,
+                                              __bf16* w3b, ClosurePack* pk) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < PN_MLP_NPARAM) put_param(i, p[i], w1b, w2b, w2t, w3b, pk);
+    if (i < 4 * 64 && (i & 31) >= PN_MLP_NO) {
+        const bf16x8 zero = {};
+        pk->w3[i >> 6][i & 63] = zero;
+    }
 }
 
 // Batched inference through the same wave routine the fused predictor uses:
@@ -295,68 +451,95 @@ __global__ void __launch_bounds__(256) k_mlp_wave(const ClosurePack* __restrict_
     }
 }
 
-int ensure_batch(pennant_mlp* m, int64_t B) {
-    if (B <= m->cap) return 0;
-    auto fr = [](void* p) { if (p) (void)hipFree(p); };
-    fr(m->idx); fr(m->xb); fr(m->h1); fr(m->h2); fr(m->dyb); fr(m->dz2); fr(m->dz1);
-    fr(m->t); fr(m->z); fr(m->y); fr(m->dh); fr(m->part); fr(m->lossp);
-    if (m->idx_host) (void)hipHostFree(m->idx_host);
-    m->cap = B;
-    MCK(hipMalloc(&m->idx, B * 4));
-    MCK(hipHostMalloc((void**)&m->idx_host, B * 4));
-    MCK(hipMalloc(&m->xb, B * PN_MLP_K1 * 2));
-    MCK(hipMalloc(&m->h1, B * PN_MLP_NH * 2));
-    MCK(hipMalloc(&m->h2, B * PN_MLP_NH * 2));
-    MCK(hipMalloc(&m->dyb, B * PN_MLP_NO * 2));
-    MCK(hipMalloc(&m->dz2, B * PN_MLP_NH * 2));
-    MCK(hipMalloc(&m->dz1, B * PN_MLP_NH * 2));
-    MCK(hipMalloc(&m->t, B * PN_MLP_NO * 4));
-    MCK(hipMalloc(&m->z, B * PN_MLP_NH * 4));
-    MCK(hipMalloc(&m->y, B * PN_MLP_NO * 4));
-    MCK(hipMalloc(&m->dh, B * PN_MLP_NH * 4));
-    // split-K partials: at most 64 parts of the largest gradient (64 x 64)
-    MCK(hipMalloc(&m->part, (size_t)64 * PN_MLP_NH * PN_MLP_NH * 4));
-    MCK(hipMalloc(&m->lossp, ((B + 255) / 256 + 1) * 4));
+inline int nb(int64_t n) { return (int)((n + 255) / 256); }
+
+// Buffers for batches of B rows; with `rows` also the host's lists of them.
+int ensure_batch(pennant_mlp* m, int64_t B, bool rows) {
+    const int64_t ld = (B + 31) / 32 * 32;
+    if (ld > m->cap) {
+        if (m->lrow) (void)hipFree(m->lrow);
+        m->lrow = nullptr;
+        m->cap = 0;
+        // one allocation: two FP32 rows, then the BF16 ones (ld is a multiple
+        // of 32, so each is 16-byte aligned)
+        constexpr size_t HALF = PN_MLP_K1 + 4 * PN_MLP_NH + PN_MLP_NO;
+        MCK(hipMalloc(&m->lrow, (size_t)ld * (2 * 4 + HALF * 2)));
+        m->lossp = m->lrow + ld;
+        m->xt = reinterpret_cast<__bf16*>(m->lossp + ld);
+        m->h1t = m->xt + PN_MLP_K1 * ld;
+        m->h2t = m->h1t + PN_MLP_NH * ld;
+        m->dz2t = m->h2t + PN_MLP_NH * ld;
+        m->dz1t = m->dz2t + PN_MLP_NH * ld;
+        m->dyt = m->dz1t + PN_MLP_NH * ld;
+        for (int*& h : m->idx_host) {
+            if (h) (void)hipHostFree(h);
+            h = nullptr;
+        }
+        if (!m->part) MCK(hipMalloc(&m->part, (size_t)64 * PN_MLP_NPARAM * 4));
+        m->cap = ld;
+    }
+    for (int k = 0; k < 2 && rows; ++k) {
+        if (!m->idx_host[k]) MCK(hipHostMalloc((void**)&m->idx_host[k], (size_t)m->cap * 4));
+        if (!m->read[k]) MCK(hipEventCreateWithFlags(&m->read[k], hipEventDisableTiming));
+    }
     return 0;
 }
 
 int repack(pennant_mlp* m) {
-    hipLaunchKernelGGL(k_pack, dim3(8), dim3(256), 0, m->stream, m->p, m->w1b, m->w2b, m->w3b, m->pack);
+    hipLaunchKernelGGL(k_pack, dim3(nb(PN_MLP_NPARAM)), dim3(256), 0, m->stream, m->p, m->w1b, m->w2b, m->w2t, m->w3b,
+                       m->pack);
     MCK(hipGetLastError());
     MCK(hipMemcpyAsync(m->pack->lo, m->lo, sizeof m->lo, hipMemcpyHostToDevice, m->stream));
     MCK(hipMemcpyAsync(m->pack->hi, m->hi, sizeof m->hi, hipMemcpyHostToDevice, m->stream));
     return 0;
 }
 
-inline int nb(int64_t n) { return (int)((n + 255) / 256); }
+RowArgs row_args(const pennant_mlp* m, int64_t n, const float* x) {
+    RowArgs a = {};
+    a.p = m->p;
+    a.w1b = m->w1b; a.w2b = m->w2b; a.w2t = m->w2t; a.w3b = m->w3b;
+    a.n = n;
+    a.x = x;
+    return a;
+}
 
-// forward + backward on the gathered minibatch (m->xb, m->t, B rows);
-// leaves the gradient in m->g and the loss in m->lossp[nb(B)]
-int fwd_bwd(pennant_mlp* m, int B) {
+// Forward and backward of the B rows idx (NULL: 0 .. B - 1) of the tuples;
+// `read` (may be NULL) is recorded once idx has been read.
+void launch_batch(pennant_mlp* m, const float* tuples, const int* idx, int64_t B, hipEvent_t read) {
     hipStream_t s = m->stream;
-    float* g = m->g;
-    const float* b2 = m->p + PN_MLP_OFF_B2;
-    const float* b3 = m->p + PN_MLP_OFF_B3;
-    const int nh = B * PN_MLP_NH;
-    // forward
-    MCK(gemm(B, PN_MLP_NH, PN_MLP_K1, m->xb, PN_MLP_K1, 0, m->w1b, PN_MLP_K1, 1, m->z, m->part, s));
-    hipLaunchKernelGGL(k_bias_relu, dim3(nb(nh)), dim3(256), 0, s, nh, m->z, (const float*)nullptr, m->h1);
-    MCK(gemm(B, PN_MLP_NH, PN_MLP_NH, m->h1, PN_MLP_NH, 0, m->w2b, PN_MLP_NH, 1, m->z, m->part, s));
-    hipLaunchKernelGGL(k_bias_relu, dim3(nb(nh)), dim3(256), 0, s, nh, m->z, b2, m->h2);
-    MCK(gemm(B, PN_MLP_NO, PN_MLP_NH, m->h2, PN_MLP_NH, 0, m->w3b, PN_MLP_NH, 1, m->z, m->part, s));
-    hipLaunchKernelGGL(k_out_loss, dim3(nb(B)), dim3(256), 0, s, B, m->z, b3, m->t, m->y, m->dyb, m->lossp);
-    hipLaunchKernelGGL(k_sum_small, dim3(1), dim3(64), 0, s, nb(B), m->lossp, m->lossp + nb(B));
-    // backward
-    MCK(gemm(PN_MLP_NO, PN_MLP_NH, B, m->dyb, PN_MLP_NO, 1, m->h2, PN_MLP_NH, 0, g + PN_MLP_OFF_W3, m->part, s));
-    hipLaunchKernelGGL(k_colsum, dim3(PN_MLP_NO), dim3(256), 0, s, B, PN_MLP_NO, m->dyb, g + PN_MLP_OFF_B3);
-    MCK(gemm(B, PN_MLP_NH, PN_MLP_NO, m->dyb, PN_MLP_NO, 0, m->w3b, PN_MLP_NH, 0, m->dh, m->part, s));
-    hipLaunchKernelGGL(k_relu_grad, dim3(nb(nh)), dim3(256), 0, s, nh, m->dh, m->h2, m->dz2);
-    MCK(gemm(PN_MLP_NH, PN_MLP_NH, B, m->dz2, PN_MLP_NH, 1, m->h1, PN_MLP_NH, 0, g + PN_MLP_OFF_W2, m->part, s));
-    hipLaunchKernelGGL(k_colsum, dim3(PN_MLP_NH), dim3(256), 0, s, B, PN_MLP_NH, m->dz2, g + PN_MLP_OFF_B2);
-    MCK(gemm(B, PN_MLP_NH, PN_MLP_NH, m->dz2, PN_MLP_NH, 0, m->w2b, PN_MLP_NH, 0, m->dh, m->part, s));
-    hipLaunchKernelGGL(k_relu_grad, dim3(nb(nh)), dim3(256), 0, s, nh, m->dh, m->h1, m->dz1);
-    MCK(gemm(PN_MLP_NH, PN_MLP_K1, B, m->dz1, PN_MLP_NH, 1, m->xb, PN_MLP_K1, 0, g + PN_MLP_OFF_W1, m->part, s));
-    return (int)hipGetLastError();
+    RowArgs a = row_args(m, B, tuples);
+    a.idx = idx;
+    a.ld = m->cap;
+    a.xt = m->xt; a.h1t = m->h1t; a.h2t = m->h2t; a.dyt = m->dyt; a.dz2t = m->dz2t; a.dz1t = m->dz1t;
+    a.lrow = m->lrow;
+    hipLaunchKernelGGL(k_rows<true>, dim3((unsigned)((B + 31) / 32)), dim3(64), 0, s, a);
+    if (read) (void)hipEventRecord(read, s);
+    GradArgs g;
+    g.rows = B;
+    g.ld = m->cap;
+    int64_t ksplit = B > 1024 ? (B + 511) / 512 : 1;
+    if (ksplit > 64) ksplit = 64;
+    g.kper = (int)((B + ksplit - 1) / ksplit + 15) / 16 * 16;
+    g.ksplit = (int)((B + g.kper - 1) / g.kper);
+    g.xt = m->xt; g.h1t = m->h1t; g.h2t = m->h2t; g.dyt = m->dyt; g.dz2t = m->dz2t; g.dz1t = m->dz1t;
+    g.lrow = m->lrow;
+    g.part = m->part;
+    g.g = m->g;
+    g.lossp = m->lossp;
+    hipLaunchKernelGGL(k_grads, dim3(g.ksplit * PN_GTILES / 4 + PN_MLP_NO + PN_MLP_NH + nb(B)), dim3(256), 0, s, g);
+}
+UpdateArgs update_args(pennant_mlp* m, int64_t B, float* loss) {
+    UpdateArgs u = {};
+    int64_t ksplit = B > 1024 ? (B + 511) / 512 : 1;
+    if (ksplit > 64) ksplit = 64;
+    const int kper = (int)((B + ksplit - 1) / ksplit + 15) / 16 * 16;
+    u.ksplit = (int)((B + kper - 1) / kper);
+    u.nloss = nb(B);
+    u.part = m->part;
+    u.lossp = m->lossp;
+    u.g = m->g;
+    u.loss = loss;
+    return u;
 }
 
 }  // namespace
@@ -368,14 +551,22 @@ int pennant_mlp_num_params(void) { return PN_MLP_NPARAM; }
 pennant_mlp* pennant_mlp_create(uint64_t seed) {
     pennant_mlp* m = new pennant_mlp();
     bool ok = hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) == hipSuccess;
-    ok = ok && hipMalloc(&m->p, PN_MLP_NPARAM * 4) == hipSuccess;
-    ok = ok && hipMalloc(&m->g, PN_MLP_NPARAM * 4) == hipSuccess;
-    ok = ok && hipMalloc(&m->m, PN_MLP_NPARAM * 4) == hipSuccess;
-    ok = ok && hipMalloc(&m->v, PN_MLP_NPARAM * 4) == hipSuccess;
-    ok = ok && hipMalloc(&m->w1b, PN_MLP_NH * PN_MLP_K1 * 2) == hipSuccess;
-    ok = ok && hipMalloc(&m->w2b, PN_MLP_NH * PN_MLP_NH * 2) == hipSuccess;
-    ok = ok && hipMalloc(&m->w3b, PN_MLP_NO * PN_MLP_NH * 2) == hipSuccess;
-    ok = ok && hipMalloc(&m->pack, sizeof(ClosurePack)) == hipSuccess;
+    // one allocation: the pack, the FP32 vectors, the BF16 copies (each
+    // 16-byte aligned)
+    constexpr size_t NP = (PN_MLP_NPARAM + 3) / 4 * 4;
+    ok = ok && hipMalloc(&m->pack, sizeof(ClosurePack) + 4 * NP * 4 +
+                                       (PN_MLP_NH * (PN_MLP_K1 + 2 * PN_MLP_NH) + PN_MLP_NO * PN_MLP_NH) * 2) == hipSuccess;
+    if (ok) {
+        static_assert(sizeof(ClosurePack) % 16 == 0, "the FP32 vectors follow the pack");
+        m->p = reinterpret_cast<float*>(m->pack + 1);
+        m->g = m->p + NP;
+        m->m = m->g + NP;
+        m->v = m->m + NP;
+        m->w1b = reinterpret_cast<__bf16*>(m->v + NP);
+        m->w2b = m->w1b + PN_MLP_NH * PN_MLP_K1;
+        m->w2t = m->w2b + PN_MLP_NH * PN_MLP_NH;
+        m->w3b = m->w2t + PN_MLP_NH * PN_MLP_NH;
+    }
     if (!ok) { pennant_mlp_destroy(m); return nullptr; }
     // He-uniform initial weights from a seeded generator; zero biases
     std::vector<float> h(PN_MLP_NPARAM, 0.f);
@@ -394,11 +585,13 @@ pennant_mlp* pennant_mlp_create(uint64_t seed) {
 void pennant_mlp_destroy(pennant_mlp* m) {
     if (!m) return;
     if (m->stream) (void)hipStreamSynchronize(m->stream);
-    void* bufs[] = {m->p, m->g, m->m, m->v, m->w1b, m->w2b, m->w3b, m->pack, m->idx, m->xb, m->h1,
-                    m->h2, m->dyb, m->dz2, m->dz1, m->t, m->z, m->y, m->dh, m->part, m->lossp};
+    void* bufs[] = {m->pack, m->lrow, m->part, m->losses};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
-    if (m->idx_host) (void)hipHostFree(m->idx_host);
+    for (int* h : m->idx_host)
+        if (h) (void)hipHostFree(h);
+    for (hipEvent_t e : m->read)
+        if (e) (void)hipEventDestroy(e);
     if (m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
 }
@@ -441,34 +634,23 @@ int pennant_mlp_forward(pennant_mlp* m, const float* x, int64_t n, float* y, int
         MCK(hipGetLastError());
         return (int)hipStreamSynchronize(m->stream);
     }
-    // GEMM path, in chunks of the batch capacity
-    const int64_t chunk = 65536;
-    MCK(ensure_batch(m, chunk));
-    hipStream_t s = m->stream;
-    for (int64_t b0 = 0; b0 < n; b0 += chunk) {
-        const int B = (int)((n - b0 < chunk) ? n - b0 : chunk);
-        const int nh = B * PN_MLP_NH;
-        hipLaunchKernelGGL(k_x_rows, dim3(nb(B)), dim3(256), 0, s, B, x + b0 * PN_MLP_NF, m->xb);
-        MCK(gemm(B, PN_MLP_NH, PN_MLP_K1, m->xb, PN_MLP_K1, 0, m->w1b, PN_MLP_K1, 1, m->z, m->part, s));
-        hipLaunchKernelGGL(k_bias_relu, dim3(nb(nh)), dim3(256), 0, s, nh, m->z, (const float*)nullptr, m->h1);
-        MCK(gemm(B, PN_MLP_NH, PN_MLP_NH, m->h1, PN_MLP_NH, 0, m->w2b, PN_MLP_NH, 1, m->z, m->part, s));
-        hipLaunchKernelGGL(k_bias_relu, dim3(nb(nh)), dim3(256), 0, s, nh, m->z, m->p + PN_MLP_OFF_B2, m->h2);
-        MCK(gemm(B, PN_MLP_NO, PN_MLP_NH, m->h2, PN_MLP_NH, 0, m->w3b, PN_MLP_NH, 1, m->z, m->part, s));
-        hipLaunchKernelGGL(k_out, dim3(nb(B)), dim3(256), 0, s, B, m->z, m->p + PN_MLP_OFF_B3, y + 2 * b0);
-        MCK(hipGetLastError());
-    }
-    return (int)hipStreamSynchronize(s);
+    RowArgs a = row_args(m, n, x);
+    a.y = y;
+    if ((n + 31) / 32 > 0x7fffffff) return PENNANT_EINVAL;
+    hipLaunchKernelGGL(k_rows<false>, dim3((unsigned)((n + 31) / 32)), dim3(64), 0, m->stream, a);
+    MCK(hipGetLastError());
+    return (int)hipStreamSynchronize(m->stream);
 }
 
 int pennant_mlp_loss_grad(pennant_mlp* m, const float* tuples, int64_t n, float* grad, float* loss) {
     if (n <= 0 || n > (1 << 30)) return PENNANT_EINVAL;
-    MCK(ensure_batch(m, n));
-    for (int64_t b = 0; b < n; ++b) m->idx_host[b] = (int)b;
-    MCK(hipMemcpyAsync(m->idx, m->idx_host, n * 4, hipMemcpyHostToDevice, m->stream));
-    hipLaunchKernelGGL(k_gather, dim3(nb(n)), dim3(256), 0, m->stream, (int)n, m->idx, tuples, m->xb, m->t);
-    MCK(fwd_bwd(m, (int)n));
+    MCK(ensure_batch(m, n, false));
+    launch_batch(m, tuples, nullptr, n, nullptr);
+    const UpdateArgs u = update_args(m, n, m->lossp + nb(n));
+    hipLaunchKernelGGL(k_update<false>, dim3(nb(PN_MLP_NPARAM + 1)), dim3(256), 0, m->stream, u);
+    MCK(hipGetLastError());
     MCK(hipMemcpyAsync(grad, m->g, PN_MLP_NPARAM * 4, hipMemcpyDeviceToHost, m->stream));
-    MCK(hipMemcpyAsync(loss, m->lossp + nb(n), 4, hipMemcpyDeviceToHost, m->stream));
+    MCK(hipMemcpyAsync(loss, u.loss, 4, hipMemcpyDeviceToHost, m->stream));
     MCK(hipStreamSynchronize(m->stream));
     *loss /= (float)n;
     return 0;
@@ -477,26 +659,38 @@ int pennant_mlp_loss_grad(pennant_mlp* m, const float* tuples, int64_t n, float*
 int pennant_mlp_train(pennant_mlp* m, const float* tuples, int64_t n, int steps, int batch, float lr,
                       uint64_t seed, float* loss_out) {
     if (n <= 0 || n > (1 << 30) || steps < 0 || batch <= 0 || batch > (1 << 22)) return PENNANT_EINVAL;
-    MCK(ensure_batch(m, batch));
-    MCK(hipMemsetAsync(m->g, 0, PN_MLP_NPARAM * 4, m->stream));
+    MCK(ensure_batch(m, batch, true));
+    if (steps > m->loss_cap) {
+        if (m->losses) (void)hipFree(m->losses);
+        m->losses = nullptr;
+        m->loss_cap = 0;
+        MCK(hipMalloc(&m->losses, (size_t)steps * 4));
+        m->loss_cap = steps;
+    }
     std::mt19937_64 rng(seed);
     std::uniform_int_distribution<int64_t> pick(0, n - 1);
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     for (int st = 0; st < steps; ++st) {
-        MCK(hipStreamSynchronize(m->stream));    // the pinned index buffer is reused
-        for (int b = 0; b < batch; ++b) m->idx_host[b] = (int)pick(rng);
-        MCK(hipMemcpyAsync(m->idx, m->idx_host, (size_t)batch * 4, hipMemcpyHostToDevice, m->stream));
-        hipLaunchKernelGGL(k_gather, dim3(nb(batch)), dim3(256), 0, m->stream, batch, m->idx, tuples, m->xb, m->t);
-        MCK(fwd_bwd(m, batch));
+        // a step's rows are drawn while the steps before it run; the kernel
+        // reads them from the host's list, which is free again two steps later
+        int* idx = m->idx_host[st & 1];
+        if (st >= 2) MCK(hipEventSynchronize(m->read[st & 1]));
+        for (int b = 0; b < batch; ++b) idx[b] = (int)pick(rng);
+        launch_batch(m, tuples, idx, batch, m->read[st & 1]);
         m->adam_t += 1;
-        const float c1 = 1.f - std::pow(b1, (float)m->adam_t), c2 = 1.f - std::pow(b2, (float)m->adam_t);
+        UpdateArgs u = update_args(m, batch, m->losses + st);
+        u.c1 = 1.f - std::pow(b1, (float)m->adam_t);
+        u.c2 = 1.f - std::pow(b2, (float)m->adam_t);
         // cosine decay from lr to lr/50 over the call's steps
-        const float lrt = lr * (0.02f + 0.98f * 0.5f * (1.f + std::cos(3.14159265f * (float)st / (float)steps)));
-        hipLaunchKernelGGL(k_adam, dim3(nb(PN_MLP_NPARAM)), dim3(256), 0, m->stream, PN_MLP_NPARAM, m->p, m->g,
-                           m->m, m->v, lrt, b1, b2, eps, c1, c2);
-        hipLaunchKernelGGL(k_pack, dim3(8), dim3(256), 0, m->stream, m->p, m->w1b, m->w2b, m->w3b, m->pack);
-        if (loss_out) MCK(hipMemcpyAsync(loss_out + st, m->lossp + nb(batch), 4, hipMemcpyDeviceToHost, m->stream));
+        u.lr = lr * (0.02f + 0.98f * 0.5f * (1.f + std::cos(3.14159265f * (float)st / (float)steps)));
+        u.b1 = b1; u.b2 = b2; u.eps = eps;
+        u.p = m->p; u.m = m->m; u.v = m->v;
+        u.w1b = m->w1b; u.w2b = m->w2b; u.w2t = m->w2t; u.w3b = m->w3b; u.pack = m->pack;
+        hipLaunchKernelGGL(k_update<true>, dim3(nb(PN_MLP_NPARAM + 1)), dim3(256), 0, m->stream, u);
     }
+    MCK(hipGetLastError());
+    if (loss_out && steps > 0)
+        MCK(hipMemcpyAsync(loss_out, m->losses, (size_t)steps * 4, hipMemcpyDeviceToHost, m->stream));
     MCK(hipStreamSynchronize(m->stream));
     if (loss_out)
         for (int st = 0; st < steps; ++st) loss_out[st] /= (float)batch;
