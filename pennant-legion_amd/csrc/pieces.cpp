@@ -73,8 +73,8 @@ int sync_ctl(pennant_pieces* pp) {
 
 #define PN_PIECES_GRAPH_CYCLES 16
 
-// Captures PN_PIECES_GRAPH_CYCLES cycles of `form` as one HIP graph (the
-// pieces' kernels of a phase on parallel branches, kernel nodes only).
+// Captures PN_PIECES_GRAPH_CYCLES cycles of `form` as one HIP graph (kernel
+// nodes only).
 int build_pieces_graph(pennant_pieces* pp, int form) {
     if (pp->gexec) (void)hipGraphExecDestroy(pp->gexec);
     pp->gexec = nullptr;
@@ -325,13 +325,6 @@ pennant_pieces* pennant_pieces_create(const char* deck_text, int numpcs, char* e
         pb->tune.pipeline = 0;
         pp->pc.push_back(pb);
     }
-    // fork and join events of the piece cycle's phases
-    pp->ev_fork.assign(3, nullptr);
-    pp->ev_join.assign((size_t)3 * npc, nullptr);
-    for (hipEvent_t& e : pp->ev_fork)
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return fail("hipEventCreate failed");
-    for (hipEvent_t& e : pp->ev_join)
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return fail("hipEventCreate failed");
     // corner exchange: the slot a ghost's corner is written to, and the
     // owner's slot for it (both as corner_slot places them)
     std::vector<XEnt> cx;
@@ -375,12 +368,7 @@ pennant_pieces* pennant_pieces_create(const char* deck_text, int numpcs, char* e
     pp->ncx = (int)cx.size();
     pp->halo = upload_to(pp, halo);
     pp->nhalo = (int)halo.size();
-    int nruns = 0;
-    for (pennant_problem* pb : pp->pc) nruns += (int)pb->zruns.size() / 3;
-    pp->npart = nruns * PN_MAX_GRID;
-    pp->part_d = upload_to(pp, std::vector<double>((size_t)2 * pp->npart, 0.));
-    pp->part_i = upload_to(pp, std::vector<int>((size_t)2 * pp->npart, 0));
-    if (!pp->tab || !pp->cx || !pp->halo || !pp->part_d || !pp->part_i) return fail("device allocation failed");
+    if (!pp->tab || !pp->cx || !pp->halo || pieces_setup(pp)) return fail("piece set-up failed");
     if (hipDeviceSynchronize() != hipSuccess) return fail("piece set-up failed");
     return pp;
 }
@@ -424,10 +412,6 @@ void pennant_pieces_destroy(pennant_pieces* pp) {
     if (!pp) return;
     if (!pp->pc.empty()) (void)hipStreamSynchronize(pp->pc[0]->stream);
     if (pp->gexec) (void)hipGraphExecDestroy(pp->gexec);
-    for (hipEvent_t e : pp->ev_fork)
-        if (e) (void)hipEventDestroy(e);
-    for (hipEvent_t e : pp->ev_join)
-        if (e) (void)hipEventDestroy(e);
     for (pennant_problem* pb : pp->pc) pennant_destroy(pb);
     for (void* p : pp->allocs) (void)hipFree(p);
     delete pp;

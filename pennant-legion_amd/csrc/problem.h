@@ -327,13 +327,16 @@ struct pennant_pieces {
     int nhalo = 0;
     pn::XEnt* cx = nullptr;                       // corner slot at a ghost point -> owner's slot
     int ncx = 0;
-    double* part_d = nullptr;                     // partials: [0, npart) K1's, [npart, 2 npart) K3's
+    // work of a launch over all pieces (pieces_setup): zone units, units of the
+    // pieces' own points, heavy points, and each piece's kernel arguments
+    pn::BUnit* units = nullptr;
+    pn::PUnit* punits = nullptr;
+    pn::BHeavy* heavy = nullptr;
+    void* args = nullptr;
+    int nunits = 0, npunits = 0, nheavy = 0;
+    double* part_d = nullptr;                     // partials per zone unit: K1's, then K3's
     int* part_i = nullptr;
-    int npart = 0;
     bool zre_stale = false;                       // mixed cycles ran since zr, ze were stored
-    // the pieces' kernels of a phase run on their own streams (fork and join
-    // events on piece 0's stream); runs of 16 cycles replay a captured graph
-    std::vector<hipEvent_t> ev_fork, ev_join;     // 3 forks; 3 joins per piece
     hipGraphExec_t gexec = nullptr;
     int graph_form = -1;
     std::vector<void*> allocs;
@@ -341,8 +344,9 @@ struct pennant_pieces {
 };
 
 namespace pn {
-// one cycle of every piece (fused.hip): K1 per piece, the corner exchange, K2
-// per piece, the halo, K3 per piece, one finalize
+// one cycle of every piece (fused.hip): K1, the corner exchange, K2, the halo
+// and K3, each one launch over all pieces, and one finalize
+int pieces_setup(pennant_pieces* pp);
 int pieces_cycle(pennant_pieces* pp, int form);
 // zr and ze stored in every piece where mixed cycles left them derived
 int pieces_materialize_zre(pennant_pieces* pp);
