@@ -2299,12 +2299,18 @@ __global__ void __launch_bounds__(PN_FIN_BLOCK) k_finalize_la(FusedArgs a, int n
 // records.  Sums run in the order of the separate passes (a point's corners in
 // ascending side order), so the results are the same bits.
 //
-// What bounds it: arithmetic (FP64: 238 VGPRs, two waves per SIMD, VALU issue;
-// mixed: 128 VGPRs, four).  Per cycle, separate passes (for mixed and learned
-// the pipelined ones) -> tiles: FP64 Sedov 1440^2 306 -> 214 us, Noh pie
-// 1024^2 178 -> 132 us; mixed LeBlanc 4096 x 256 87 -> 62 us, 333 x 217 23 ->
-// 14 us; learned Sedov 1440^2 176 -> 159 us; FP64 45^2 21 -> 14 us.  It was
-// faster at every size, so structured meshes always take it.
+// What bounds it: a tile's chain of loads, arithmetic and barriers, with few
+// waves to hide it (FP64: 241 VGPRs, two waves per SIMD, vector unit 0.8 busy;
+// mixed: 128 VGPRs, four, 0.86 busy).  Larger tiles have less ring but more
+// waves in step: 32 x 16 zones took 258 us where 16 x 16 takes 212 (FP64), and
+// 139 where it takes 117 (mixed).  FP64 square roots and quotients without the
+// scaling of their operands (9% fewer instructions) gained 1 to 3%; blocks
+// that loop over tiles, loading the next one early, spilled (265 us).
+// Per cycle, separate passes (for mixed and learned the pipelined ones) ->
+// tiles: FP64 Sedov 1440^2 306 -> 209 us, Noh pie 1024^2 178 -> 120 us; mixed
+// LeBlanc 4096 x 256 87 -> 58 us, 333 x 217 23 -> 12.6 us; learned Sedov
+// 1440^2 176 -> 153 us; FP64 45^2 21 -> 14 us.  It was faster at every size, so
+// structured meshes always take it.
 #define PN_TILE 16
 #define PN_TIN (PN_TILE - 2)
 
@@ -2363,12 +2369,53 @@ template <> struct TileKeep<float> {
     }
 };
 
-// The tile whose first zone (ring included) is (i0, j0); its partials go to
-// slot.  Returns whether a CL_FLAG tile has a zone for the network: such a
+// What a thread reads of its tile, as loaded.
+template <typename T> struct TileIn;
+template <> struct TileIn<double> {
+    ZoneIn<4> z;
+    double et;
+    unsigned bits;
+};
+template <> struct TileIn<float> {
+    d2 x[4], u[4];
+    double zm, zvol, zwrate, et;
+    f32x4u mf;
+    unsigned bits;
+};
+
+// Every load of a thread for the tile whose first zone (ring included) is (i0,
+// j0), with no branch: threads outside the mesh read the nearest zone and use
+// nothing of it.
+template <typename T>
+__device__ __forceinline__ void tile_load(const FusedArgs& a, const TileMesh& g, int i0, int j0, TileIn<T>& in) {
+    const int i = i0 + ((int)threadIdx.x & (PN_TILE - 1)), j = j0 + (int)threadIdx.x / PN_TILE;
+    const int ci = min(max(i, 0), g.nzx - 1), cj = min(max(j, g.pie), g.nzy - 1);
+    const int z = tile_zone(g, ci, cj), sb = tile_side(g, ci, cj);
+    const int p00 = tile_point(g, ci, cj);
+    const int pp[4] = {p00, p00 + 1, p00 + g.nzx + 2, p00 + g.nzx + 1};
+    if constexpr (sizeof(T) == 8) {
+        load_zone<4>(a, z, sb, pp, in.z);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            in.x[k] = mk(a.pxx[pp[k]], a.pxy[pp[k]]);
+            in.u[k] = mk(a.pux[pp[k]], a.puy[pp[k]]);
+        }
+        in.zm = a.zm[z];
+        in.zvol = a.zvol[z];
+        in.zwrate = a.zwrate[z];
+        in.mf = *reinterpret_cast<const f32x4u*>(a.fsmf + sb);
+    }
+    in.et = a.zetot[z];
+    in.bits = a.pbc[p00];
+}
+
+// The tile whose first zone (ring included) is (i0, j0), loaded in `in`; its
+// partials go to slot.  Returns whether a CL_FLAG tile has a zone for the network: such a
 // tile is left to the list kernel and stores nothing.
 template <typename T, int CL>
 __device__ __forceinline__ bool tile_body(const FusedArgs& a, const TileOut& o, const TileMesh& g, int i0, int j0,
-                                          int slot, double dt, bool zre, ClCount& total) {
+                                          const TileIn<T>& in, int slot, double dt, bool zre, ClCount& total) {
     __shared__ T crn[12][PN_BLOCK];
     __shared__ double pts[sizeof(T) == 8 ? 5 : 4][PN_BLOCK];
     const int tid = threadIdx.x;
@@ -2380,45 +2427,42 @@ __device__ __forceinline__ bool tile_body(const FusedArgs& a, const TileOut& o, 
     const bool inner = ti >= 1 && ti <= PN_TIN && tj >= 1 && tj <= PN_TIN;
     const bool own = quad && inner;
     const bool pin = i >= 0 && i <= g.nzx && j >= g.pie && j <= g.nzy;   // point (i, j) exists
-    // Every load of the tile first, with no branch: threads outside the mesh
-    // read the nearest zone and use nothing of it.
-    const int ci = min(max(i, 0), g.nzx - 1), cj = min(max(j, g.pie), g.nzy - 1);
-    const int z = tile_zone(g, ci, cj), sb = tile_side(g, ci, cj);
-    const int p00 = tile_point(g, ci, cj);
-    const int pp[4] = {p00, p00 + 1, p00 + g.nzx + 2, p00 + g.nzx + 1};
     PointIn q;
-    double dtz = 1.e99, et = 0., zm, zvol0;
+    double dtz = 1.e99, zm, zvol0;
+    const double et = in.et;
     int bad = 0;
     ClCount cnt;
     TileKeep<T> keep;
     keep.c = &crn[0][tid];
+    q.bits = in.bits;
     if constexpr (sizeof(T) == 8) {
-        ZoneIn<4> in;
-        load_zone<4>(a, z, sb, pp, in);
-        q.bits = a.pbc[p00];
-        zm = in.zm;
-        zvol0 = in.zvol;
+        zm = in.z.zm;
+        zvol0 = in.z.zvol;
+        q.x0 = in.z.x[0];
+        q.u0 = in.z.u[0];
+        if (quad) dtz = zone_pred_core<4>(a, in.z, dt, bad, keep);
+    } else {
+        ZoneState st;
+        st.zm = zm = in.zm;
+        st.zvol = zvol0 = in.zvol;
+        st.zwrate = in.zwrate;
+        if (zre) {
+            const int z = tile_zone(g, min(max(i, 0), g.nzx - 1), min(max(j, g.pie), g.nzy - 1));
+            st.zr = a.zr[z];
+            st.ze = a.ze[z];
+        } else {
+            // the mixed corrector stored neither; these are its quotients
+            st.zr = zm / zvol0;
+            st.ze = et / (zm + 1.e-99);
+        }
+        float mf[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) mf[k] = in.mf[k];
         q.x0 = in.x[0];
         q.u0 = in.u[0];
-        if (own) et = a.zetot[z];
-        if (quad) dtz = zone_pred_core<4>(a, in, dt, bad, keep);
-    } else {
-        d2 x0[4], u0[4];
-        ZoneState st;
-        load_zone_mixed<4>(a, z, pp, zre, x0, u0, st);
-        float mf[4];
-        const f32x4u m4 = *reinterpret_cast<const f32x4u*>(a.fsmf + sb);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) mf[k] = m4[k];
-        q.bits = a.pbc[p00];
-        zm = st.zm;
-        zvol0 = st.zvol;
-        q.x0 = x0[0];
-        q.u0 = u0[0];
-        if (own) et = a.zetot[z];
         // the network runs across the wave, so every lane takes part
         if (CL == CL_PACKED || quad)
-            dtz = zone_pred_mixed_core<4, CL>(a, x0, u0, st, mf, dt, bad, quad, cnt, keep);
+            dtz = zone_pred_mixed_core<4, CL>(a, in.x, in.u, st, mf, dt, bad, quad, cnt, keep);
     }
     if (tri) {
         // the corners of triangle i at points (i + 1, 1) and (i, 1), where a
@@ -2494,6 +2538,7 @@ __device__ __forceinline__ bool tile_body(const FusedArgs& a, const TileOut& o, 
             if constexpr (sizeof(T) == 8) xp[k] = pts[4][at[k]];
             sfw[k] = mk((double)keep.sfw[k].x, (double)keep.sfw[k].y);
         }
+        const int z = tile_zone(g, i, j);
         const CorrOut r = corr_core<4, T>(et, zvol0, zm, keep.p, sfw, x, vs, xp, dt, badc, dvov);
         o.zwrate[z] = r.zwrate;
         o.zetot[z] = r.zetot;
@@ -2565,10 +2610,10 @@ template <typename T, int CL>
 __global__ void __launch_bounds__(PN_BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 2 : (CL == CL_FLAG ? 3 : 4))))
 k_tile(FusedArgs a, TileArgs t) {
     const Ctl* c = a.ctl;
-    const int done = c->done;
-    if (done && !(t.back && c->cur)) return;
-    const double dt = c->dt;
     if ((int)blockIdx.x == t.ntiles) {
+        const int done = c->done;
+        if (done && !(t.back && c->cur)) return;
+        const double dt = c->dt;
         if (done) {
             if (threadIdx.x == 0) {
                 const int p = t.g.po;
@@ -2584,12 +2629,18 @@ k_tile(FusedArgs a, TileArgs t) {
     const int tile = x * qn + (x < rn ? x : rn) + (b >> 3);
     int i0, j0;
     tile_at(t, tile, i0, j0);
+    // the loads do not wait for the control block, which the last finalize has
+    // just written in another XCD's L2: Sedov 1440^2 FP64 217 -> 209 us a
+    // cycle, mixed 116 -> 108, learned 158 -> 153
+    TileIn<T> in;
+    tile_load<T>(a, t.g, i0, j0, in);
+    const int done = c->done;
     if (done) {
-        tile_copy<T>(a, t.o, t.g, i0, j0);
+        if (t.back && c->cur) tile_copy<T>(a, t.o, t.g, i0, j0);
         return;
     }
     ClCount none;
-    const bool left = tile_body<T, CL>(a, t.o, t.g, i0, j0, t.poff + tile, dt, c->zre_valid != 0, none);
+    const bool left = tile_body<T, CL>(a, t.o, t.g, i0, j0, in, t.poff + tile, c->dt, c->zre_valid != 0, none);
     if (CL == CL_FLAG && left && threadIdx.x == 0) t.list[atomicAdd(t.nlist, 1)] = tile;
 }
 
@@ -2618,7 +2669,9 @@ k_tile_list(FusedArgs a, TileArgs t) {
         const int tile = t.list[k];
         int i0, j0;
         tile_at(t, tile, i0, j0);
-        (void)tile_body<float, CL_PACKED>(b, t.o, t.g, i0, j0, t.poff + tile, dt, zre, cnt);
+        TileIn<float> in;
+        tile_load<float>(b, t.g, i0, j0, in);
+        (void)tile_body<float, CL_PACKED>(b, t.o, t.g, i0, j0, in, t.poff + tile, dt, zre, cnt);
     }
     const int nl = block_sum(cnt.learned);
     const int nf = block_sum(cnt.fallback);
