@@ -588,11 +588,15 @@ int pennant_batch_set_capture(pennant_batch* b, float* dev_buf, int64_t cap);
 int pennant_batch_capture_count(pennant_batch* b, int64_t* count);
 /* "max_blocks" (1..65535, default 2048), "xcd" (0/1), "graph" (0/1),
  * "rect_maps" (0/1, default 1: the zone kernels compute the points and corner
- * slots of the batch's rect problems, as pennant_set_tuning's "rect_maps"). */
+ * slots of the batch's rect problems, as pennant_set_tuning's "rect_maps"),
+ * "tiles" (0/1, default 1: when every problem is structured, a cycle of the
+ * FP64 and mixed forms is one kernel over the tiles of all of them, as
+ * pennant_set_tuning's "tiles"; "rect_maps" 0, a capture buffer and the odd
+ * cycle of a launch take the separate passes). */
 int pennant_batch_set_tuning(pennant_batch* b, const char* key, int value);
 int pennant_batch_get_tuning(pennant_batch* b, const char* key);
-/* Times `cycles` cycles at each grid shape (grid cap x XCD mapping) from the
- * same snapshot of the state, keeps the fastest and restores the snapshot:
+/* Times `cycles` cycles as tiles and at each grid shape of the separate passes
+ * (grid cap x XCD mapping) from the same snapshot of the state, keeps the fastest and restores the snapshot:
  * the problems do not advance.  best_ms (may be NULL) receives its time. */
 int pennant_batch_autotune(pennant_batch* b, int mode, int cycles, double* best_ms);
 /* Parameters of an ensemble of `count` problems: for k even a Sedov blast on

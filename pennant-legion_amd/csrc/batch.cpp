@@ -48,12 +48,18 @@ void drop_graph(pennant_batch* b) {
     b->graph_cycles = 0;
 }
 
+// Whether cycles of `form` run as tile cycles (as `tiled` in driver.cpp).
+bool tiled(const pennant_batch* b, int form) {
+    return b->ntiles > 0 && b->tune.tiles && b->tune.rect_maps && form != FORM_LEARNED && !b->cap_buf;
+}
+
 int build_graph(pennant_batch* b, int form) {
     drop_graph(b);
     hipGraph_t g = nullptr;
     BCK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
     int rc = 0;
-    for (int k = 0; k < PN_GRAPH_CYCLES && !rc; ++k) rc = batch_cycle(b, form);
+    for (int k = 0; k < PN_GRAPH_CYCLES && !rc; ++k)
+        rc = tiled(b, form) ? batch_tile_cycle(b, form, k & 1) : batch_cycle(b, form);
     const int rc2 = (int)hipStreamEndCapture(b->stream, &g);
     if (rc || rc2) {
         if (g) (void)hipGraphDestroy(g);
@@ -179,6 +185,7 @@ pennant_batch* pennant_batch_create(const char* const* decks, int n, char* errbu
     std::vector<PUnit> punits;
     std::vector<BHeavy> heavy;
     std::vector<BProb> probs(n);
+    std::vector<TileState> meshes(n);
     for (int i = 0; i < n; ++i) {
         pennant_problem* pb = pennant_create(decks[i], e, sizeof e);
         if (!pb) return fail(b, "deck " + std::to_string(i) + ": " + e);
@@ -219,6 +226,7 @@ pennant_batch* pennant_batch_create(const char* const* decks, int n, char* errbu
         q.rect_sh = pb->rect_sh;
         q.so = (int)so;
         q.po = (int)po;
+        meshes[i] = pb->tile;
         q.ubeg = (int)units.size();
         for (size_t r = 0; r < pb->zruns.size(); r += 3) {
             const int zb = pb->zruns[r], ze = pb->zruns[r + 1], nsd = pb->zruns[r + 2];
@@ -231,6 +239,7 @@ pennant_batch* pennant_batch_create(const char* const* decks, int n, char* errbu
                 U.sb = (int)(so + h.zsbeg[zb] + (int64_t)(u0 - zb) * nsd);
                 U.ns = nsd;
                 U.pid = i;
+                U.slot = (int)units.size();
                 units.push_back(U);
             }
         }
@@ -249,6 +258,7 @@ pennant_batch* pennant_batch_create(const char* const* decks, int n, char* errbu
     b->part_d = (double*)al(2 * units.size(), 8);
     b->part_i = (int*)al(2 * units.size(), 4);
     if (!ok) return fail(b, "device allocation failed");
+    if (batch_tile_setup(b, meshes, probs)) return fail(b, "device allocation failed");
     int rc = (int)hipMemcpy(b->mapsp1, mapsp1.data(), S * 4, hipMemcpyHostToDevice);
     if (!rc) rc = (int)hipMemcpy(b->pcbeg, pcbeg.data(), (P + 1) * 4, hipMemcpyHostToDevice);
     if (!rc) rc = (int)hipMemcpy(b->pcpos, pcpos.data(), S * 4, hipMemcpyHostToDevice);
@@ -296,6 +306,11 @@ int pennant_batch_launch_cycles(pennant_batch* b, int ncycles, int mode) {
     if (b->tune.graph && left >= PN_GRAPH_CYCLES) {
         if (b->graph_form != form || !b->gexec) BCK(build_graph(b, form));
         for (; left >= b->graph_cycles; left -= b->graph_cycles) BCK(hipGraphLaunch(b->gexec, b->stream));
+    }
+    // tile cycles come in pairs; an odd cycle runs as separate passes
+    for (; left > 1 && tiled(b, form); left -= 2) {
+        BCK(batch_tile_cycle(b, form, 0));
+        BCK(batch_tile_cycle(b, form, 1));
     }
     for (; left > 0; --left) BCK(batch_cycle(b, form));
     return 0;
@@ -432,6 +447,9 @@ int pennant_batch_set_tuning(pennant_batch* b, const char* key, int value) {
     } else if (!strcmp(key, "rect_maps")) {
         if (value != 0 && value != 1) return PENNANT_EINVAL;
         b->tune.rect_maps = value;
+    } else if (!strcmp(key, "tiles")) {
+        if (value != 0 && value != 1) return PENNANT_EINVAL;
+        b->tune.tiles = value;
     } else {
         return PENNANT_EINVAL;
     }
@@ -444,6 +462,7 @@ int pennant_batch_get_tuning(pennant_batch* b, const char* key) {
     if (!strcmp(key, "xcd")) return b->tune.xcd;
     if (!strcmp(key, "graph")) return b->tune.graph;
     if (!strcmp(key, "rect_maps")) return b->tune.rect_maps;
+    if (!strcmp(key, "tiles")) return (b->tune.tiles && b->ntiles > 0) ? 1 : 0;
     return PENNANT_EINVAL;
 }
 
@@ -457,22 +476,29 @@ int pennant_batch_autotune(pennant_batch* b, int mode, int cycles, double* best_
     Tuning best = keep;
     double bms = 1e300;
     const int grids[] = {512, 1024, 2048, 4096, 8192, 16384};
-    for (int xcd = 0; xcd <= 1 && !rc; ++xcd) {
+    auto timed = [&]() {
+        b->tune.graph = 0;
+        drop_graph(b);
+        rc = snap_restore(b, sn);
+        b->zre_stale = true;
+        // two untimed cycles, then the timed ones
+        if (!rc) rc = pennant_batch_launch_cycles(b, 2, mode);
+        double ms = 0.;
+        if (!rc) rc = pennant_batch_time_cycles(b, cycles, mode, &ms);
+        if (rc == PENNANT_EBADSIDES) rc = 0;
+        if (!rc && ms < bms) { bms = ms; best = b->tune; }
+    };
+    // the tile cycle (its grid follows from the meshes), then the separate
+    // passes' grids
+    if (!rc && tiled(b, form)) timed();
+    for (int xcd = 0; xcd <= 1; ++xcd) {
         for (int g : grids) {
             if (rc) break;
             b->tune = keep;
+            b->tune.tiles = 0;
             b->tune.max_blocks = g;
             b->tune.xcd = xcd;
-            b->tune.graph = 0;
-            drop_graph(b);
-            rc = snap_restore(b, sn);
-            b->zre_stale = true;
-            // one untimed cycle, then the timed ones
-            if (!rc) rc = pennant_batch_launch_cycles(b, 1, mode);
-            double ms = 0.;
-            if (!rc) rc = pennant_batch_time_cycles(b, cycles, mode, &ms);
-            if (rc == PENNANT_EBADSIDES) rc = 0;
-            if (!rc && ms < bms) { bms = ms; best = b->tune; }
+            timed();
         }
     }
     best.graph = keep.graph;

@@ -185,7 +185,12 @@ namespace pn {
 // of one problem), point units (at most PN_BLOCK points of one problem),
 // heavy points and the per-problem parameters.
 struct BUnit {
-    int zb, ze, sb, ns, pid, pad0, pad1, pad2;
+    int zb, ze, sb, ns, pid, slot, pad1, pad2;   // slot: of its block partials
+};
+// A tile of a structured problem (fused.hip, tile_body): the first zone of its
+// ring, the mesh and its place in the arena, its problem and partials.
+struct BTile {
+    int i0, j0, nzx, nzy, pie, zo, so, po, pid, slot;
 };
 struct PUnit {
     int pb, pe, pid, pad;
@@ -201,6 +206,7 @@ struct BProb {
     // problem's own zone z; so, po: its first side and point in the arena
     unsigned long long rect_m;
     int rect_nzx, rect_sh, so, po;
+    int tbeg, tend;              // the problem's partials in a tile cycle
 };
 }  // namespace pn
 
@@ -227,6 +233,19 @@ struct pennant_batch {
     int npunits = 0;
     pn::BHeavy* heavy = nullptr;
     int nheavy = 0;
+    // tile cycles, when every problem is structured (ntiles > 0): the tiles, the
+    // pies' triangles as zone units and their origins, partials, and the
+    // second set of state arrays (as pennant_problem::tile)
+    pn::BTile* tiles = nullptr;
+    int ntiles = 0;
+    pn::BUnit* tunits = nullptr;
+    int ntunits = 0;
+    pn::BHeavy* origins = nullptr;
+    int norigins = 0;
+    int ntparts = 0;
+    double* tpart_d = nullptr;
+    int* tpart_i = nullptr;
+    double* alt[9] = {};
     pn::BProb* probs = nullptr;
     pn::Ctl* ctls = nullptr;
     pn::Ctl* ctls_host = nullptr;                // pinned mirror
@@ -249,6 +268,10 @@ struct pennant_batch {
 namespace pn {
 // one cycle of every unfinished problem of a batch (fused.hip)
 int batch_cycle(pennant_batch* b, int form);
+// tile cycles of a batch of structured problems: the set-up from the problems'
+// meshes (nzx, nzy, pie), and cycle `second` (0, 1) of a pair
+int batch_tile_setup(pennant_batch* b, const std::vector<TileState>& meshes, std::vector<BProb>& probs);
+int batch_tile_cycle(pennant_batch* b, int form, int second);
 int launch_to_float(const double* src, float* dst, int64_t n, hipStream_t s);
 // fused cycle (fused.hip)
 int fused_setup(pennant_problem* pb);

@@ -98,7 +98,30 @@ def test_tiles_stop_on_bad_sides_as_the_separate_passes():
         assert np.array_equal(bits(a[~nan]), bits(b[~nan])), f
 
 
+@pytest.mark.parametrize("mode", [pa.MODE_FUSED, pa.MODE_MIXED])
+def test_batch_tiles_match_single_runs(mode):
+    """Rect and pie meshes at the edges of tiles in one arena (non-zero zone,
+    side and point offsets), stopping at different cycles."""
+    names = sorted(DECKS)
+    texts = [DECKS[n](20 + k) for k, n in enumerate(names)]
+    for steps in ([60], [1, 2, 3, 60]):
+        with pa.Batch(texts) as b:
+            assert b.get_tuning("tiles") == 1
+            for n in steps:
+                b.run(n, mode)
+            for i, t in enumerate(texts):
+                st, sc, _ = state(t, mode, 0, [100])
+                got = b.scalars(i)
+                for k in SCAL:
+                    assert bits(got[k]) == bits(sc[k]), (names[i], steps, k)
+                for f in STATE:
+                    assert np.array_equal(bits(b.get(i, f)), bits(st[f])), (names[i], steps, f)
+
+
 def test_a_mesh_that_does_not_qualify():
     with pa.Problem(wd.noh_pie(1, 7, cstop=3, dtinit=1e-4)) as pb:      # triangles only
         assert pb.get_tuning("tiles") == 0
         assert pb.run(5, pa.MODE_FUSED) == 3
+    with pa.Batch([wd.sedov_rect(8, cstop=3), wd.noh_pie(1, 7, cstop=3, dtinit=1e-4)]) as b:
+        assert b.get_tuning("tiles") == 0
+        b.run(5, pa.MODE_FUSED)
