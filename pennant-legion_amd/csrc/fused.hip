@@ -2308,16 +2308,19 @@ __global__ void __launch_bounds__(PN_FIN_BLOCK) k_finalize_la(FusedArgs a, int n
 // ascending side order), so the results are the same bits.
 //
 // What bounds it: a tile's chain of loads, arithmetic and barriers, with few
-// waves to hide it (FP64: 241 VGPRs, two waves per SIMD, vector unit 0.8 busy;
+// waves to hide it (FP64: 229 VGPRs, two waves per SIMD, vector unit 0.8 busy;
 // mixed: 128 VGPRs, four, 0.86 busy).  Larger tiles have less ring but more
 // waves in step: 32 x 16 zones took 258 us where 16 x 16 takes 212 (FP64), and
 // 139 where it takes 117 (mixed).  FP64 square roots and quotients without the
 // scaling of their operands (9% fewer instructions) gained 1 to 3%; blocks
-// that loop over tiles, loading the next one early, spilled (265 us).
+// that loop over tiles, loading the next one early, spilled (265 us).  Corner
+// sums without branches (zones outside the mesh give zeros), 32-bit byte
+// offsets and one fold of both counts together took Sedov 1440^2 from 211 to
+// 205 us (FP64), 108.5 to 106.6 (mixed) and 154 to 149 (learned).
 // Per cycle, separate passes (for mixed and learned the pipelined ones) ->
-// tiles: FP64 Sedov 1440^2 306 -> 209 us, Noh pie 1024^2 178 -> 120 us; mixed
-// LeBlanc 4096 x 256 87 -> 58 us, 333 x 217 23 -> 12.6 us; learned Sedov
-// 1440^2 176 -> 153 us; FP64 45^2 21 -> 14 us.  It was faster at every size, so
+// tiles: FP64 Sedov 1440^2 306 -> 205 us, Noh pie 1024^2 178 -> 120 us; mixed
+// LeBlanc 4096 x 256 87 -> 57 us, 333 x 217 23 -> 12.2 us; learned Sedov
+// 1440^2 176 -> 149 us; FP64 45^2 21 -> 14 us.  It was faster at every size, so
 // structured meshes always take it.
 #define PN_TILE 16
 #define PN_TIN (PN_TILE - 2)
@@ -2377,6 +2380,18 @@ template <> struct TileKeep<float> {
     }
 };
 
+// The element at a byte offset (and a constant) from an array's start.  A
+// scalar base, a 32-bit offset and the constant are one access's address,
+// where an index takes a 64-bit addition and two registers per access; the
+// arrays of a structured mesh are below 4 GiB (corner_slots_fit).
+template <typename E, int C = 0, typename A>
+__device__ __forceinline__ E at_byte(const A* p, unsigned off) {
+    return *reinterpret_cast<const E*>(reinterpret_cast<const char*>(p) + off + C);
+}
+__device__ __forceinline__ void put_byte(double* p, unsigned off, double v) {
+    *reinterpret_cast<double*>(reinterpret_cast<char*>(p) + off) = v;
+}
+
 // What a thread reads of its tile, as loaded.
 template <typename T> struct TileIn;
 template <> struct TileIn<double> {
@@ -2398,24 +2413,34 @@ template <typename T>
 __device__ __forceinline__ void tile_load(const FusedArgs& a, const TileMesh& g, int i0, int j0, TileIn<T>& in) {
     const int i = i0 + ((int)threadIdx.x & (PN_TILE - 1)), j = j0 + (int)threadIdx.x / PN_TILE;
     const int ci = min(max(i, 0), g.nzx - 1), cj = min(max(j, g.pie), g.nzy - 1);
-    const int z = tile_zone(g, ci, cj), sb = tile_side(g, ci, cj);
-    const int p00 = tile_point(g, ci, cj);
-    const int pp[4] = {p00, p00 + 1, p00 + g.nzx + 2, p00 + g.nzx + 1};
+    const unsigned z = 8u * (unsigned)tile_zone(g, ci, cj), sb = (unsigned)tile_side(g, ci, cj);
+    const unsigned p = (unsigned)tile_point(g, ci, cj), p0 = 8u * p, p3 = p0 + 8u * (unsigned)(g.nzx + 1);
+    auto points = [&](const double* x, const double* y, d2 (&v)[4]) {
+        v[0] = mk(at_byte<double>(x, p0), at_byte<double>(y, p0));
+        v[1] = mk(at_byte<double, 8>(x, p0), at_byte<double, 8>(y, p0));
+        v[2] = mk(at_byte<double, 8>(x, p3), at_byte<double, 8>(y, p3));
+        v[3] = mk(at_byte<double>(x, p3), at_byte<double>(y, p3));
+    };
     if constexpr (sizeof(T) == 8) {
-        load_zone<4>(a, z, sb, pp, in.z);
+        points(a.pxx, a.pxy, in.z.x);
+        points(a.pux, a.puy, in.z.u);
+        in.z.zm = at_byte<double>(a.zm, z);
+        in.z.zr = at_byte<double>(a.zr, z);
+        in.z.ze = at_byte<double>(a.ze, z);
+        in.z.zvol = at_byte<double>(a.zvol, z);
+        in.z.zwr = at_byte<double>(a.zwrate, z);
+        const f64x2u m0 = at_byte<f64x2u>(a.smf, 8u * sb), m1 = at_byte<f64x2u, 16>(a.smf, 8u * sb);
+        in.z.mf[0] = m0[0]; in.z.mf[1] = m0[1]; in.z.mf[2] = m1[0]; in.z.mf[3] = m1[1];
     } else {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            in.x[k] = mk(a.pxx[pp[k]], a.pxy[pp[k]]);
-            in.u[k] = mk(a.pux[pp[k]], a.puy[pp[k]]);
-        }
-        in.zm = a.zm[z];
-        in.zvol = a.zvol[z];
-        in.zwrate = a.zwrate[z];
-        in.mf = *reinterpret_cast<const f32x4u*>(a.fsmf + sb);
+        points(a.pxx, a.pxy, in.x);
+        points(a.pux, a.puy, in.u);
+        in.zm = at_byte<double>(a.zm, z);
+        in.zvol = at_byte<double>(a.zvol, z);
+        in.zwrate = at_byte<double>(a.zwrate, z);
+        in.mf = at_byte<f32x4u>(a.fsmf, 4u * sb);
     }
-    in.et = a.zetot[z];
-    in.bits = a.pbc[p00];
+    in.et = at_byte<double>(a.zetot, z);
+    in.bits = at_byte<unsigned char>(a.pbc, p);
 }
 
 // The tile whose first zone (ring included) is (i0, j0), loaded in `in`; its
@@ -2426,6 +2451,10 @@ __device__ __forceinline__ bool tile_body(const FusedArgs& a, const TileOut& o, 
                                           const TileIn<T>& in, int slot, double dt, bool zre, ClCount& total) {
     __shared__ T crn[12][PN_BLOCK];
     __shared__ double pts[sizeof(T) == 8 ? 5 : 4][PN_BLOCK];
+    __shared__ struct {
+        double dt[PN_BLOCK / 64], dv[PN_BLOCK / 64];
+        int bad[PN_BLOCK / 64];
+    } lds;
     const int tid = threadIdx.x;
     const int ti = tid & (PN_TILE - 1), tj = tid / PN_TILE;
     const int i = i0 + ti, j = j0 + tj;
@@ -2488,6 +2517,11 @@ __device__ __forceinline__ bool tile_body(const FusedArgs& a, const TileOut& o, 
             }
         }
     }
+    if (!zin) {
+        // outside the mesh: corners that add nothing
+#pragma unroll
+        for (int k = 0; k < 12; ++k) crn[k][tid] = (T)0;
+    }
     if constexpr (CL == CL_FLAG) {
         if (__syncthreads_or(quad && cnt.flag)) return true;
     } else {
@@ -2502,20 +2536,25 @@ __device__ __forceinline__ bool tile_body(const FusedArgs& a, const TileOut& o, 
     if (pin && ti >= 1 && tj >= 1) {
         const int p = tile_point(g, i, j);
         if (!quad) q = load_point(a, p);     // the last column and row of points
-        // the point's corners in ascending side order
-        const bool l = i >= 1, r = i < g.nzx, b = j >= 1, t = j < g.nzy;
+        // the point's corners in ascending side order, every read first; one
+        // that does not exist is zero, and adding zero to a sum that starts
+        // from zero leaves its bits
+        const int from[4] = {tid - PN_TILE - 1, tid - PN_TILE, tid - 1, tid};
+        constexpr int at[4] = {2, 3, 1, 0};
+        T cx[4], cy[4], cm[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            cx[k] = crn[3 * at[k]][from[k]];
+            cy[k] = crn[3 * at[k] + 1][from[k]];
+            cm[k] = crn[3 * at[k] + 2][from[k]];
+        }
         double mass = 0.;
         d2 f = mk(0., 0.);
-        auto corner = [&](bool on, int k, int from) {
-            if (on) {
-                mass += (double)crn[3 * k + 2][from];
-                f = add(f, mk((double)crn[3 * k][from], (double)crn[3 * k + 1][from]));
-            }
-        };
-        corner(l && b, 2, tid - PN_TILE - 1);
-        corner(r && b, 3, tid - PN_TILE);
-        corner(l && t, 1, tid - 1);
-        corner(r && t, 0, tid);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            mass += (double)cm[k];
+            f = add(f, mk((double)cx[k], (double)cy[k]));
+        }
         const PointOut w = point_new<T>(a, q, mass, f, dt);
         pts[0][tid] = w.x.x;
         pts[1][tid] = w.x.y;
@@ -2525,10 +2564,11 @@ __device__ __forceinline__ bool tile_body(const FusedArgs& a, const TileOut& o, 
         // a point belongs to the tile whose inner zones it is the first point
         // of; the mesh's last column and row go with the tiles they end
         if ((ti <= PN_TIN || i == g.nzx) && (tj <= PN_TIN || j == g.nzy)) {
-            a.oxx[p] = w.x.x;
-            a.oxy[p] = w.x.y;
-            a.oux[p] = w.u.x;
-            a.ouy[p] = w.u.y;
+            const unsigned o8 = 8u * (unsigned)p;
+            put_byte(a.oxx, o8, w.x.x);
+            put_byte(a.oxy, o8, w.x.y);
+            put_byte(a.oux, o8, w.u.x);
+            put_byte(a.ouy, o8, w.u.y);
             if (g.pie && j == 1) store_work_point<T>(a, p, w);   // for the triangles' corrector
         }
     }
@@ -2546,25 +2586,41 @@ __device__ __forceinline__ bool tile_body(const FusedArgs& a, const TileOut& o, 
             if constexpr (sizeof(T) == 8) xp[k] = pts[4][at[k]];
             sfw[k] = mk((double)keep.sfw[k].x, (double)keep.sfw[k].y);
         }
-        const int z = tile_zone(g, i, j);
+        const unsigned z = 8u * (unsigned)tile_zone(g, i, j);
         const CorrOut r = corr_core<4, T>(et, zvol0, zm, keep.p, sfw, x, vs, xp, dt, badc, dvov);
-        o.zwrate[z] = r.zwrate;
-        o.zetot[z] = r.zetot;
+        put_byte(o.zwrate, z, r.zwrate);
+        put_byte(o.zetot, z, r.zetot);
         if constexpr (sizeof(T) == 8) {
-            o.ze[z] = r.ze;
-            o.zr[z] = r.zr;
+            put_byte(o.ze, z, r.ze);
+            put_byte(o.zr, z, r.zr);
         }
-        o.zvol[z] = r.zvol;
-        a.zp[z] = keep.p;
+        put_byte(o.zvol, z, r.zvol);
+        put_byte(a.zp, z, keep.p);
         dtm = (dtz < dtm) ? dtz : dtm;       // a NaN never replaces the minimum
     }
-    int badp = own ? bad : 0;
-    blk_fold_fin<PN_BLOCK>(dtm, dvov, badp, badc);
+    // the tile's partials; the counts share a register (at most 784 each), and
+    // their fold is skipped by a wave that has none
+    int bads = (own ? bad : 0) + (badc << 16);
+    dtm = wave_min(dtm);
+    dvov = wave_max(dvov);
+    if (__any(bads)) bads = wave_sum(bads);
+    if ((tid & 63) == 0) {
+        lds.dt[tid >> 6] = dtm;
+        lds.dv[tid >> 6] = dvov;
+        lds.bad[tid >> 6] = bads;
+    }
+    __syncthreads();
     if (tid == 0) {
+#pragma unroll
+        for (int w = 1; w < PN_BLOCK / 64; ++w) {
+            dtm = (lds.dt[w] < dtm) ? lds.dt[w] : dtm;
+            dvov = (lds.dv[w] > dvov) ? lds.dv[w] : dvov;
+            bads += lds.bad[w];
+        }
         a.part_dt[slot] = dtm;
-        a.part_bp[slot] = badp;
+        a.part_bp[slot] = bads & 0xffff;
         a.part_dv[slot] = dvov;
-        a.part_bc[slot] = badc;
+        a.part_bc[slot] = bads >> 16;
     }
     return false;
 }
