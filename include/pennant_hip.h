@@ -13,8 +13,9 @@
  *  2. Driver entry points, pennant_*(): a whole-problem driver (deck parsing,
  *     mesh generation, initialisation, the cycle loop with dt kept on the
  *     device) mirroring Driver/Hydro (src/Driver.cc, src/Hydro.cc).  It runs
- *     the cycle either through the task entry points (one launch per task, the
- *     reference's structure) or through the fused cycle kernels.
+ *     the cycle either in task form (every task's fields in memory after each
+ *     cycle; pennant_step runs single tasks) or through the fused cycle
+ *     kernels.
  *
  * Conventions for every task entry point:
  *   - all array arguments are device pointers; a vector (double2) field is a
@@ -287,7 +288,8 @@ int pennant_hip_calc_global_dt(const double* dtlast, const double* dtrec,
 typedef struct pennant_problem pennant_problem;
 
 enum pennant_mode {
-    PENNANT_MODE_TASKS = 0,   /* one launch per task ID, src/Hydro.cc:342-983 order */
+    PENNANT_MODE_TASKS = 0,   /* every task ID's fields written each cycle (src/Hydro.cc:342-983),
+                                 tasks on the same zones or points sharing a launch */
     PENNANT_MODE_FUSED = 1,   /* fused cycle kernels (same arithmetic, fewer HBM passes) */
     PENNANT_MODE_MIXED = 2,   /* fused cycle, mixed precision: FP32 side/corner/QCS math,
                                  FP64 positions, volumes, EOS state, energy, work and dt */

@@ -8,6 +8,7 @@
 // arrays and keeps dt, time and the stop test on the device.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -402,7 +403,7 @@ pennant_problem* pn::create_problem(const Params& prm, HostMesh&& hm, int npown,
         }
         pb->fields[fs.name] = d;
     }
-    pb->ws = dalloc<double>(pb, pennant_hip_reduce_workspace_bytes() / sizeof(double));
+    pb->ws = dalloc<char>(pb, std::max(pennant_hip_reduce_workspace_bytes(), cycle_parts_bytes(cycle_blocks(&m))));
     pb->ctl = dalloc<Ctl>(pb, 1);
     if (hipHostMalloc((void**)&pb->ctl_host, sizeof(Ctl), hipHostMallocDefault) != hipSuccess)
         return fail("hipHostMalloc failed");
@@ -551,40 +552,13 @@ static int build_graph(pennant_problem* pb, int form) {
     return 0;
 }
 
-// One task-mode cycle: the 30 doCycle steps through the task entry points,
-// then the end-of-cycle update (time, cycle, stop test, next dt).
-static int task_cycle(pennant_problem* pb) {
-    for (int st = 0; st < 30; ++st) CK(task_step(pb, st));
-    return launch_end_cycle(pb, 0);
-}
-
-// Whether `n` task-mode cycles from the state in ctl_host all run before the
-// stop condition.  cstop is exact.  For tstop: the next cycle's dt is known,
-// and each later dt is at most dtfac times the one before
-// (calcGlobalDt, src/Driver.cc:225-231) and at most dtmax, so the time after
-// n cycles is bounded; a margin covers the rounding of the time sums.
-static bool task_run_is_safe(const pennant_problem* pb, int n) {
-    const Ctl& c = *pb->ctl_host;
-    const Params& q = pb->prm;
-    if (c.done || (long long)c.cycle + n > (long long)q.cstop) return false;
-    const double f = q.dtfac > 1. ? q.dtfac : 1.;
-    double dt = c.dt, span = 0.;
-    for (int k = 0; k < n; ++k) {
-        span += dt;
-        dt = std::fmin(dt * f, q.dtmax);
-    }
-    if (!(span >= 0.) || !std::isfinite(span)) return false;
-    return c.time + span * (1. + 1.e-6) + 1.e-12 * std::fabs(q.tstop) < q.tstop;
-}
-
-// Captures PN_GRAPH_CYCLES task-mode cycles as one HIP graph (kernel nodes
-// only: the copies and fills of doCycle are kernels too).
+// Captures PN_GRAPH_CYCLES task-mode cycles as one HIP graph.
 static int build_task_graph(pennant_problem* pb) {
     drop_graph(pb);
     hipGraph_t g = nullptr;
     CK(hipStreamBeginCapture(pb->stream, hipStreamCaptureModeThreadLocal));
     int rc = 0;
-    for (int k = 0; k < PN_GRAPH_CYCLES && !rc; ++k) rc = task_cycle(pb);
+    for (int k = 0; k < PN_GRAPH_CYCLES && !rc; ++k) rc = launch_task_cycle(pb);
     const int rc2 = (int)hipStreamEndCapture(pb->stream, &g);
     if (rc || rc2) {
         if (g) (void)hipGraphDestroy(g);
@@ -633,24 +607,12 @@ int pennant_launch_cycles(pennant_problem* pb, int ncycles, int mode) {
     }
     if (mode != PENNANT_MODE_TASKS) return PENNANT_EINVAL;
     drop_lookahead(pb);
-    // Task mode mirrors Driver::run, one launch per task.  The task entry
-    // points have no stop predicate, so the host reads the control block
-    // before every run of cycles it queues: a run of PN_GRAPH_CYCLES cycles
-    // replays one captured HIP graph when no cycle of it can reach the stop
-    // condition (task_run_is_safe), otherwise cycles go one at a time.
-    for (int k = 0; k < ncycles;) {
-        CK(copy_ctl_to_host(pb));
-        if (pb->ctl_host->done) break;
-        if (pb->tune.graph && ncycles - k >= PN_GRAPH_CYCLES &&
-            task_run_is_safe(pb, PN_GRAPH_CYCLES)) {
-            if (pb->graph_form != PN_GRAPH_TASKS || !pb->gexec) CK(build_task_graph(pb));
-            CK(hipGraphLaunch(pb->gexec, pb->stream));
-            k += PN_GRAPH_CYCLES;
-            continue;
-        }
-        CK(task_cycle(pb));
-        ++k;
+    int left = ncycles;
+    if (pb->tune.graph && left >= PN_GRAPH_CYCLES) {
+        if (pb->graph_form != PN_GRAPH_TASKS || !pb->gexec) CK(build_task_graph(pb));
+        for (; left >= PN_GRAPH_CYCLES; left -= PN_GRAPH_CYCLES) CK(hipGraphLaunch(pb->gexec, pb->stream));
     }
+    for (; left > 0; --left) CK(launch_task_cycle(pb));
     return 0;
 }
 
@@ -1146,7 +1108,7 @@ int pennant_step(pennant_problem* pb, int step) {
 int pennant_end_cycle(pennant_problem* pb) {
     drop_lookahead(pb);
     CK(materialize_zre(pb));
-    CK(launch_end_cycle(pb, 0));
+    CK(launch_end_cycle(pb));
     return pennant_sync(pb);
 }
 

@@ -1643,8 +1643,8 @@ __device__ __forceinline__ int corner_slot(const FusedArgs& a, int p, int c, int
     return (c < 4) ? c * a.nump + p : 4 * a.nump + k;
 }
 
-template <typename T>
-__device__ __forceinline__ void point_heavy(const FusedArgs& a, int p, double dt) {
+template <typename T, class Update>
+__device__ __forceinline__ void point_heavy(const FusedArgs& a, int p, const Update& update) {
     using C = Corners<T>;
     __shared__ double sv[3][PN_BLOCK];
     const int kb = a.pcbeg[p], ke = a.pcbeg[p + 1], t = threadIdx.x;
@@ -1680,7 +1680,11 @@ __device__ __forceinline__ void point_heavy(const FusedArgs& a, int p, double dt
     }
     if (t < 3) sv[t][0] = acc;
     __syncthreads();
-    if (t == 0) point_update<T>(a, p, load_point(a, p), sv[0][0], mk(sv[1][0], sv[2][0]), dt);
+    if (t == 0) update(p, load_point(a, p), sv[0][0], mk(sv[1][0], sv[2][0]));
+}
+template <typename T>
+__device__ __forceinline__ void point_heavy(const FusedArgs& a, int p, double dt) {
+    point_heavy<T>(a, p, [&](int p, const PointIn& q, double mass, d2 f) { point_update<T>(a, p, q, mass, f, dt); });
 }
 
 // An ordinary point, one thread; points with more than PN_HEAVY corners are
@@ -1688,8 +1692,8 @@ __device__ __forceinline__ void point_heavy(const FusedArgs& a, int p, double dt
 //
 // The point's state and its first four corners (most points have at most
 // four) are loaded together, then summed in ascending order.
-template <typename T>
-__device__ __forceinline__ void point_light(const FusedArgs& a, int p, double dt) {
+template <typename T, class Update>
+__device__ __forceinline__ void point_light(const FusedArgs& a, int p, const Update& update) {
     using C = Corners<T>;
     const int kb = a.pcbeg[p], ke = a.pcbeg[p + 1];
     const int n = ke - kb;
@@ -1719,7 +1723,52 @@ __device__ __forceinline__ void point_light(const FusedArgs& a, int p, double dt
         mass += C::mass(a, sl);
         f = add(f, mk(C::fx(a, sl), C::fy(a, sl)));
     }
-    point_update<T>(a, p, q, mass, f, dt);
+    update(p, q, mass, f);
+}
+template <typename T>
+__device__ __forceinline__ void point_light(const FusedArgs& a, int p, double dt) {
+    point_light<T>(a, p, [&](int p, const PointIn& q, double mass, d2 f) { point_update<T>(a, p, q, mass, f, dt); });
+}
+
+// The point pass of a task-mode cycle: the sums of k_point over the same
+// corner slots, then the fields that the point tasks leave: copies and half
+// step (advPosHalf), corner mass and force sums, the force and start velocity
+// with the fixed velocities applied, calcAccel and advPosFull.
+struct TaskPoints {
+    pennant_vec px0, pu0, pxp, pf, pap;
+    double* pmaswt;
+};
+__global__ void __launch_bounds__(PN_BLOCK) k_cycle_points(FusedArgs a, TaskPoints t) {
+    if (a.ctl->done) return;
+    const double dt = a.ctl->dt;
+    auto update = [&](int p, const PointIn& q, double mass, d2 f) {
+        st(t.px0, p, q.x0);
+        st(t.pxp, p, add(q.x0, scl(0.5 * dt, q.u0)));
+        d2 u0 = q.u0;
+        if (q.bits)
+            for (int b = 0; b < a.nbcs; ++b)
+                if (q.bits & (1u << b)) {
+                    const d2 v = mk(a.bcv[b], a.bcv[8 + b]);
+                    u0 = project(u0, v);
+                    f = project(f, v);
+                }
+        const d2 acc = dvs(f, smax(mass, 1.e-99));
+        const d2 u = add(u0, scl(dt, acc)), x = add(q.x0, scl(dt * 0.5, add(u0, u)));
+        t.pmaswt[p] = mass;
+        st(t.pf, p, f);
+        st(t.pu0, p, u0);
+        st(t.pap, p, acc);
+        a.pxx[p] = x.x;
+        a.pxy[p] = x.y;
+        a.pux[p] = u.x;
+        a.puy[p] = u.y;
+    };
+    if ((int)blockIdx.x < a.nheavy) {
+        point_heavy<double>(a, a.heavy[blockIdx.x], update);
+        return;
+    }
+    const int p = (blockIdx.x - a.nheavy) * PN_BLOCK + threadIdx.x;
+    if (p < a.npown) point_light<double>(a, p, update);
 }
 
 // K2: blocks [0, nheavy) take the heavy points, the rest one point per thread.
@@ -3370,6 +3419,14 @@ int launch_learned_pass(const pennant_problem* pb, const FusedArgs& a, bool pend
 }
 
 }  // namespace
+
+int launch_cycle_points(pennant_problem* pb) {
+    const FusedArgs a = make_args(pb);
+    const TaskPoints t = {pb->vv("px0"), pb->vv("pu0"), pb->vv("pxp"), pb->vv("pf"), pb->vv("pap"), pb->f("pmaswt")};
+    const int nb = pb->nheavy + nblocks(own_points(pb));
+    if (nb > 0) hipLaunchKernelGGL(k_cycle_points, dim3(nb), dim3(PN_BLOCK), 0, pb->stream, a, t);
+    return (int)hipGetLastError();
+}
 
 int fused_cycle(pennant_problem* pb, hipEvent_t* ev, int form) {
     if (form == FORM_LEARNED && !pb->closure) return PENNANT_EINVAL;

@@ -304,12 +304,29 @@ int refresh_side_fracs(pennant_problem* pb);
 int batch_materialize_zre(pennant_batch* b);
 // device init and end-of-cycle kernels (driver_kernels.hip)
 int launch_init_state(pennant_problem* pb);
-int launch_end_cycle(pennant_problem* pb, int compute_dtrec);
+int launch_end_cycle(pennant_problem* pb);
 int launch_first_dt(pennant_problem* pb);
-// doCycle's copies and fills (src/Hydro.cc:361-368,389-418) as kernels, so
-// that a captured task-mode cycle holds kernel nodes only: zvol0 = zvol;
-// px0 = px, pu0 = pu, pmaswt = 0, pf = 0
+// doCycle's copies and fills (src/Hydro.cc:361-368,389-418) for its steps one
+// at a time: zvol0 = zvol; px0 = px, pu0 = pu, pmaswt = 0, pf = 0
 int launch_copy_zvol0(pennant_problem* pb);
+// A task-mode cycle, every task's fields written, in four launches
+// (task_kernels.hip), and its end: the folds of the zone kernels' block
+// partials, calcDt and the end-of-cycle update (driver_kernels.hip).  The
+// partials of nb blocks lie in the reduction workspace.
+struct CycleParts {
+    double *dt, *dv;   // dt minima, dvol maxima
+    int *bp, *bc;      // bad sides of the predictor and the corrector
+};
+inline size_t cycle_parts_bytes(int nb) { return (size_t)nb * (2 * sizeof(double) + 2 * sizeof(int)); }
+inline CycleParts cycle_parts(void* ws, int nb) {
+    double* d = static_cast<double*>(ws);
+    int* i = reinterpret_cast<int*>(d + 2 * (size_t)nb);
+    return {d, d + nb, i, i + nb};
+}
+int cycle_blocks(const pennant_mesh* m);
+int launch_task_cycle(pennant_problem* pb);
+int launch_cycle_points(pennant_problem* pb);   // its point pass (fused.hip)
+int launch_task_end(pennant_problem* pb, const CycleParts& part, int nb);
 int launch_point_begin(pennant_problem* pb);
 // Multi-piece runs (pieces.cpp, fused.hip): per-piece device pointers the
 // exchange kernels use, and one exchange entry (element src of piece sp to

@@ -39,6 +39,7 @@
 #include <stdint.h>
 
 #include "common.h"
+#include "problem.h"
 #include "reduce.h"
 
 using namespace pn;
@@ -156,6 +157,128 @@ __device__ __forceinline__ int wide_zone_end(const Tile& t, const int* zsb, int 
 #define SIDEC(j) (t.s0 + min(SIDE(j), t.ns - 1))
 
 // ---------------------------------------------------------------------------
+// Formulas of one side, corner or zone, as the task kernels and the task-mode
+// cycle's kernels (below) both evaluate them
+
+// area and volume of the side from p1 to p2 of the zone with centre z
+__device__ __forceinline__ void side_volume(d2 p1, d2 p2, d2 z, double& sa, double& sv) {
+    const double third = 1. / 3.;
+    sa = 0.5 * cross(sub(p2, p1), sub(z, p1));
+    sv = third * sa * (p1.x + p2.x + z.x);
+}
+
+// calcStateHalfTask's pressure and sound speed of a zone
+__device__ __forceinline__ void state_half(double r, double zvolp, double zvol0, double ze,
+                                           double zwrate, double zm, double gamma, double ssmin,
+                                           double dth, double& zp, double& zss) {
+    const double gm1 = gamma - 1.;
+    const double ssmin2 = smax(ssmin * ssmin, 1.e-99);
+    const double e = smax(ze, 0.);
+    const double p = gm1 * r * e;
+    const double pre = gm1 * e;
+    const double per = gm1 * r;
+    const double csqd = smax(ssmin2, pre + per * p / (r * r));
+    const double ss = __builtin_sqrt(csqd);
+    const double minv = 1. / zm;
+    const double dv = (zvolp - zvol0) * minv;
+    const double bulk = r * csqd;
+    const double denom = 1. + 0.5 * per * dv;
+    const double src = zwrate * dth * minv;
+    zp = p + (per * src - r * bulk * dv) / denom;
+    zss = ss;
+}
+
+// TTS::calcForceTask's pressure difference of a side
+__device__ __forceinline__ double tts_sdp(double sarea, double smf, double zarea, double zr,
+                                          double zss, double alfa, double ssmin) {
+    const double vfacinv = zarea / sarea;
+    const double srho = zr * smf * vfacinv;
+    double sstmp = smax(zss, ssmin);
+    sstmp = alfa * sstmp * sstmp;
+    return sstmp * (srho - zr);
+}
+
+// QCS::setCornerDivTask for the corner at a side's first point (position
+// xp0, velocity up0): xp1 and xp3 are the midpoints of this side and the one
+// before, up1 and up3 their velocities, de2 and de1 their lengths; xp2, up2
+// the zone's centre and velocity.
+struct CornerDiv {
+    double area, cos, div, evol, du;
+};
+__device__ __forceinline__ CornerDiv corner_div(d2 xp0, d2 xp1, d2 xp2, d2 xp3, d2 up0, d2 up1,
+                                                d2 up2, d2 up3, double de1, double de2) {
+    CornerDiv o;
+    const double cvolume = 0.5 * cross(sub(xp2, xp0), sub(xp3, xp1));
+    o.area = cvolume;
+    const d2 v1 = sub(xp3, xp0);
+    const d2 v2 = sub(xp1, xp0);
+    const double minelen = smin(de1, de2);
+    o.cos = ((minelen < 1.e-12) ? 0. : 4. * dot(v1, v2) / (de1 * de2));
+    const double div =
+        (cross(sub(up2, up0), sub(xp3, xp1)) - cross(sub(up3, up1), sub(xp2, xp0))) / (2.0 * cvolume);
+    o.div = div;
+    const d2 dxx1 = scl(0.5, sub(sub(add(xp1, xp2), xp0), xp3));
+    const d2 dxx2 = scl(0.5, sub(sub(add(xp2, xp3), xp0), xp1));
+    const double dx1 = len(dxx1);
+    const double dx2 = len(dxx2);
+    const d2 duav = scl(0.25, add(add(add(up0, up1), up2), up3));
+    const double test1 = fabs(dot(dxx1, duav) * dx2);
+    const double test2 = fabs(dot(dxx2, duav) * dx1);
+    const double num = (test1 > test2 ? dx1 : dx2);
+    const double den = (test1 > test2 ? dx2 : dx1);
+    const double r = num / den;
+    double evol = __builtin_sqrt(4.0 * cvolume * r);
+    evol = smin(evol, 2.0 * minelen);
+    const double dv1 = len2(sub(sub(add(up1, up2), up0), up3));
+    const double dv2 = len2(sub(sub(add(up2, up3), up0), up1));
+    const double du = __builtin_sqrt(smax(dv1, dv2));
+    o.evol = (div < 0.0 ? evol : 0.);
+    o.du = (div < 0.0 ? du : 0.);
+    return o;
+}
+
+// QCS::setQCnForceTask's viscosity of a corner
+__device__ __forceinline__ double corner_mu(double cdu, double cevol, double cdiv, double zrp,
+                                            double zss, double qgamma, double q1, double q2) {
+    const double gammap1 = qgamma + 1.0;
+    const double ztmp2 = q2 * 0.25 * gammap1 * cdu;
+    const double ztmp1 = q1 * zss;
+    const double zkur = ztmp2 + __builtin_sqrt(ztmp2 * ztmp2 + ztmp1 * ztmp1);
+    const double mu = zkur * zrp * cevol;
+    return (cdiv > 0.0) ? 0. : mu;
+}
+
+// QCS::setForceTask: a corner's weight, and its cosine cleared where the
+// corner is nearly straight
+__device__ __forceinline__ double corner_weight(double carea, double& ccos) {
+    const double csin2 = 1.0 - ccos * ccos;
+    const double w = ((csin2 < 1.e-4) ? 0. : carea / csin2);
+    ccos = ((csin2 < 1.e-4) ? 0. : ccos);
+    return w;
+}
+// ... and a side's force from its corner (1) and the next (2): weights,
+// cosines and edge forces cqe1, cqe2
+__device__ __forceinline__ d2 qcs_force(double cw1, double cw2, double ccos1, double ccos2,
+                                        d2 cqe11, d2 cqe21, d2 cqe12, d2 cqe22, double elen) {
+    const d2 f = add(scl(cw1, add(cqe21, scl(ccos1, cqe11))), scl(cw2, add(cqe12, scl(ccos2, cqe22))));
+    return dvs(f, elen);
+}
+
+// QCS::setVelDiffTask's velocity difference along a side
+__device__ __forceinline__ double vel_diff(d2 dx, d2 du, double elen) {
+    const double dux = dot(du, dx);
+    return elen > 0. ? fabs(dux) / elen : 0.;
+}
+
+// calcWorkTask's work of a side: sftot = sfp + sfq; v1, v2 = pu0 + pu and x1,
+// x2 = pxp.x at its points
+__device__ __forceinline__ double side_work(d2 sftot, d2 v1, d2 v2, double x1, double x2, double dth) {
+    const double sd1 = dot(sftot, v1);
+    const double sd2 = dot(neg(sftot), v2);
+    return -dth * (sd1 * x1 + sd2 * x2);
+}
+
+// ---------------------------------------------------------------------------
 // Mesh tasks
 
 // calcCtrsTask, src/Mesh.cc:797-837: ex = (px1 + px2) / 2 per side; zx =
@@ -221,10 +344,8 @@ __global__ void __launch_bounds__(PN_TB) k_calc_vols(pennant_mesh m, int tz, pen
         const int i = SIDE(j);
         if (i < t.ns) {
             const SideAt c = side_at(t, zsb, zof, i);
-            const double third = 1. / 3.;
-            const d2 p1 = x[j], p2 = x1[wide_next<R>(c)], z = zc[c.zi];
-            const double sa = 0.5 * cross(sub(p2, p1), sub(z, p1));
-            const double sv = third * sa * (p1.x + p2.x + z.x);
+            double sa, sv;
+            side_volume(x[j], x1[wide_next<R>(c)], zc[c.zi], sa, sv);
             sarea[t.s0 + i] = sa;
             svol[t.s0 + i] = sv;
             sa_[i] = sa;
@@ -732,10 +853,7 @@ __global__ void __launch_bounds__(PN_TB) k_calc_work(pennant_mesh m, int tz, pen
         if (i < t.ns) {
             const SideAt c = side_at(t, zsb, zof, i);
             const int n2 = wide_next<R>(c);
-            const d2 sftot = add(sp[j], sq[j]);
-            const double sd1 = dot(sftot, v[j]);
-            const double sd2 = dot(neg(sftot), vs[n2]);
-            dw[i] = -dth * (sd1 * xv[j] + sd2 * xx[n2]);
+            dw[i] = side_work(add(sp[j], sq[j]), v[j], vs[n2], xv[j], xx[n2], dth);
         }
     }
     __syncthreads();
@@ -816,22 +934,9 @@ __global__ void __launch_bounds__(PN_BLOCK) k_calc_state_half(int numz, const do
                                                               double ssmin, const double* dtp) {
     const int z = blockIdx.x * PN_BLOCK + threadIdx.x;
     if (z >= numz) return;
-    const double dth = 0.5 * (*dtp);
-    const double gm1 = gamma - 1.;
-    const double ssmin2 = smax(ssmin * ssmin, 1.e-99);
-    const double r = zr[z];
-    const double e = smax(ze[z], 0.);
-    const double p = gm1 * r * e;
-    const double pre = gm1 * e;
-    const double per = gm1 * r;
-    const double csqd = smax(ssmin2, pre + per * p / (r * r));
-    const double ss = __builtin_sqrt(csqd);
-    const double minv = 1. / zm[z];
-    const double dv = (zvolp[z] - zvol0[z]) * minv;
-    const double bulk = r * csqd;
-    const double denom = 1. + 0.5 * per * dv;
-    const double src = zwrate[z] * dth * minv;
-    zp[z] = p + (per * src - r * bulk * dv) / denom;
+    double p, ss;
+    state_half(zr[z], zvolp[z], zvol0[z], ze[z], zwrate[z], zm[z], gamma, ssmin, 0.5 * (*dtp), p, ss);
+    zp[z] = p;
     zss[z] = ss;
 }
 
@@ -888,12 +993,7 @@ __global__ void __launch_bounds__(PN_TB) k_calc_force_tts(pennant_mesh m, int tz
         const int i = SIDE(j);
         if (i < t.ns) {
             const SideAt c = side_at(t, zsb, zof, i);
-            const double vfacinv = za[c.zi] / sa[j];
-            const double r = zrl[c.zi];
-            const double srho = r * mf[j] * vfacinv;
-            double sstmp = smax(zsl[c.zi], ssmin);
-            sstmp = alfa * sstmp * sstmp;
-            const double sdp = sstmp * (srho - r);
+            const double sdp = tts_sdp(sa[j], mf[j], za[c.zi], zrl[c.zi], zsl[c.zi], alfa, ssmin);
             VIO<L>::st(sf, t.s0 + i, scl(-sdp, ss[j]));
         }
     }
@@ -961,44 +1061,14 @@ __global__ void __launch_bounds__(PN_TB) k_set_corner_div(pennant_mesh m, int tz
         const SideAt c = side_at(t, zsb, zof, i);
         const int ip = wide_prev<R>(c), in = wide_next<R>(c);
         const int cc = t.s0 + i;
-        const d2 up0 = u[j];
-        const d2 xp0 = x[j];
-        const d2 up1 = scl(0.5, add(up0, u1[in]));
-        const d2 xp1 = e[j];
-        const d2 up2 = zul[c.zi];
-        const d2 xp2 = zxl[c.zi];
-        const d2 up3 = scl(0.5, add(u1[ip], up0));
-        const d2 xp3 = e1[ip];
-        const double cvolume = 0.5 * cross(sub(xp2, xp0), sub(xp3, xp1));
-        carea[cc] = cvolume;
-        const d2 v1 = sub(xp3, xp0);
-        const d2 v2 = sub(xp1, xp0);
-        const double de1 = el[ip];
-        const double de2 = l[j];
-        const double minelen = smin(de1, de2);
-        ccos[cc] = ((minelen < 1.e-12) ? 0. : 4. * dot(v1, v2) / (de1 * de2));
-        const double div =
-            (cross(sub(up2, up0), sub(xp3, xp1)) - cross(sub(up3, up1), sub(xp2, xp0))) / (2.0 * cvolume);
-        cdiv[cc] = div;
-        const d2 dxx1 = scl(0.5, sub(sub(add(xp1, xp2), xp0), xp3));
-        const d2 dxx2 = scl(0.5, sub(sub(add(xp2, xp3), xp0), xp1));
-        const double dx1 = len(dxx1);
-        const double dx2 = len(dxx2);
-        const d2 duav = scl(0.25, add(add(add(up0, up1), up2), up3));
-        const double test1 = fabs(dot(dxx1, duav) * dx2);
-        const double test2 = fabs(dot(dxx2, duav) * dx1);
-        const double num = (test1 > test2 ? dx1 : dx2);
-        const double den = (test1 > test2 ? dx2 : dx1);
-        const double r = num / den;
-        double evol = __builtin_sqrt(4.0 * cvolume * r);
-        evol = smin(evol, 2.0 * minelen);
-        const double dv1 = len2(sub(sub(add(up1, up2), up0), up3));
-        const double dv2 = len2(sub(sub(add(up2, up3), up0), up1));
-        double du = __builtin_sqrt(smax(dv1, dv2));
-        evol = (div < 0.0 ? evol : 0.);
-        du = (div < 0.0 ? du : 0.);
-        cevol[cc] = evol;
-        cdu[cc] = du;
+        const d2 up1 = scl(0.5, add(u[j], u1[in]));
+        const d2 up3 = scl(0.5, add(u1[ip], u[j]));
+        const CornerDiv o = corner_div(x[j], e[j], zxl[c.zi], e1[ip], u[j], up1, zul[c.zi], up3, el[ip], l[j]);
+        carea[cc] = o.area;
+        ccos[cc] = o.cos;
+        cdiv[cc] = o.div;
+        cevol[cc] = o.evol;
+        cdu[cc] = o.du;
     }
 }
 
@@ -1043,7 +1113,6 @@ __global__ void __launch_bounds__(PN_TB) k_set_qcn_force(pennant_mesh m, int tz,
         }
     }
     __syncthreads();
-    const double gammap1 = qgamma + 1.0;
 #pragma unroll
     for (int j = 0; j < R; ++j) {
         const int i = SIDE(j);
@@ -1051,11 +1120,7 @@ __global__ void __launch_bounds__(PN_TB) k_set_qcn_force(pennant_mesh m, int tz,
         const SideAt c = side_at(t, zsb, zof, i);
         const int cc = t.s0 + i;
         const int ip = wide_prev<R>(c), in = wide_next<R>(c);
-        const double ztmp2 = q2 * 0.25 * gammap1 * du[j];
-        const double ztmp1 = q1 * zsl[c.zi];
-        const double zkur = ztmp2 + __builtin_sqrt(ztmp2 * ztmp2 + ztmp1 * ztmp1);
-        const double mu = zkur * zrl[c.zi] * ev[j];
-        const double cm = ((dv[j] > 0.0) ? 0. : mu);
+        const double cm = corner_mu(du[j], ev[j], dv[j], zrl[c.zi], zsl[c.zi], qgamma, q1, q2);
         crmu[cc] = cm;
         VIO<L>::st(cqe1, cc, dvs(scl(cm, sub(u[j], u1[ip])), el[ip]));
         VIO<L>::st(cqe2, cc, dvs(scl(cm, sub(u1[in], u[j])), l[j]));
@@ -1087,9 +1152,8 @@ __global__ void __launch_bounds__(PN_TB) k_set_force_qcs(pennant_mesh m, int tz,
     double w[R], cl[R];
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-        const double csin2 = 1.0 - cc0[j] * cc0[j];
-        w[j] = ((csin2 < 1.e-4) ? 0. : ca[j] / csin2);
-        cl[j] = ((csin2 < 1.e-4) ? 0. : cc0[j]);
+        cl[j] = cc0[j];
+        w[j] = corner_weight(ca[j], cl[j]);
         const int i = SIDE(j);
         if (i < t.ns) {
             cw[t.s0 + i] = w[j];
@@ -1107,13 +1171,7 @@ __global__ void __launch_bounds__(PN_TB) k_set_force_qcs(pennant_mesh m, int tz,
         if (i >= t.ns) continue;
         const SideAt c = side_at(t, zsb, zof, i);
         const int i2 = wide_next<R>(c);
-        const double cw1 = w[j], cw2 = cwl[i2];
-        const double ccos1 = cl[j], ccos2 = ccl[i2];
-        const d2 cqe11 = qa[j], cqe12 = q1l[i2];
-        const d2 cqe21 = qb[j], cqe22 = q2l[i2];
-        const d2 f = add(scl(cw1, add(cqe21, scl(ccos1, cqe11))),
-                         scl(cw2, add(cqe12, scl(ccos2, cqe22))));
-        VIO<L>::st(sfq, t.s0 + i, dvs(f, el[j]));
+        VIO<L>::st(sfq, t.s0 + i, qcs_force(w[j], cwl[i2], cl[j], ccl[i2], qa[j], qb[j], q1l[i2], q2l[i2], el[j]));
     }
 }
 
@@ -1158,12 +1216,7 @@ __global__ void __launch_bounds__(PN_TB) k_set_vel_diff(pennant_mesh m, int tz, 
         if (i < t.ns) {
             const SideAt c = side_at(t, zsb, zof, i);
             const int i2 = wide_next<R>(c);
-            const d2 dx = sub(x1[i2], x[j]);
-            const d2 du = sub(u1[i2], u[j]);
-            const double lenx = l[j];
-            double dux = dot(du, dx);
-            dux = (lenx > 0. ? fabs(dux) / lenx : 0.);
-            dux_[i] = dux;
+            dux_[i] = vel_diff(sub(x1[i2], x[j]), sub(u1[i2], u[j]), l[j]);
         }
     }
     __syncthreads();
@@ -1189,6 +1242,326 @@ __global__ void __launch_bounds__(PN_BLOCK) k_apply_fixed_bc(const int32_t* mapb
     const d2 u = mk(vx, vy);
     VIO<L>::st(pu0, p, project(VIO<L>::ld(pu0, p), u));
     VIO<L>::st(pf, p, project(VIO<L>::ld(pf, p), u));
+}
+
+// ---------------------------------------------------------------------------
+// A task-mode cycle of the driver
+//
+// Steps 0 to 29 of doCycle in four launches, every task's fields in memory as
+// the tasks leave them.  One launch per task moves 688 bytes a side, 536 a
+// zone and 512 a point, most of them fields that the task before has just
+// written; here the tasks that follow each other on the same zones or points
+// share a kernel and pass those on in registers and LDS, which leaves what has
+// to be written and the first reads: about 360, 290 and 220 bytes.  The task
+// entry points stay one kernel a task.  Bound by those bytes on large meshes
+// (Sedov 1440^2: 1466 -> 753 us a cycle, 5.1 TB/s), by the four launches'
+// latencies on small ones (97 x 61: 111 -> 21 us).
+//
+//   k_cycle_pred    zones: steps 0, 2-7, 9-15 and 26's block minima, with the
+//                   half-step positions computed from px and pu; also each
+//                   corner's force and mass in its corner slot, so that the
+//                   point pass reads them coalesced
+//   k_cycle_points  points: steps 1, 8, 16, 17, 19 (fused.hip)
+//   k_cycle_corr    zones: steps 20-25 and 27's block maxima
+//   end             the folds of 26 and 27, 28 and the end of the cycle
+//                   (driver_kernels.hip)
+//
+// Sums, minima and maxima are formed as in the tasks' kernels, in the same
+// order: the same bits.  The fields are the driver's own (two arrays per
+// vector field).
+struct CycleArgs {
+    pennant_mesh m;
+    int tz;
+    const Ctl* ctl;              // dt, and whether the run has stopped: then nothing is done
+    double gamma, ssmin, alfa, qgamma, q1, q2, cfl;
+    pennant_cvec px, pu, pu0, pxp;
+    // zones
+    pennant_vec zx, zxp, zuc;
+    double *zarea, *zvol, *zareap, *zvolp, *zvol0, *zdl, *zr, *zrp, *ze, *zetot, *zw, *zwrate, *zp,
+        *zss, *zdu, *ztmp;
+    const double* zm;
+    // sides
+    pennant_vec ex, exp, ssurfp, sfp, sfq, sft, cqe1, cqe2;
+    double *sarea, *svol, *sareap, *svolp, *elen, *carea, *cevol, *cdu, *cdiv, *ccos, *crmu, *cw;
+    const double* smf;
+    const int32_t* pcpos;        // corner slots, and the corners' values there
+    double *cfx, *cfy, *cmass;
+    CycleParts part;
+};
+using V = VIO<VL_SOA>;
+// The zone kernels' fields pass through memory once a kernel and are too many
+// for the caches on all but small meshes: non-temporal accesses leave those to
+// the point values.  Sedov 1440^2 957 -> 753 us a cycle, 700^2 229 -> 193, 500^2
+// the same, 97 x 61 20.0 -> 20.6.
+__device__ __forceinline__ void put(double* a, int64_t i, double v) { __builtin_nontemporal_store(v, a + i); }
+__device__ __forceinline__ void put(const pennant_vec& a, int64_t i, d2 v) {
+    put(a.x, i, v.x);
+    put(a.y, i, v.y);
+}
+
+#define PN_CYC_TZ (PN_TB / 3 + 1)     // most zones of a tile of one side per thread
+
+__device__ __forceinline__ double get(const double* a, int64_t i) { return __builtin_nontemporal_load(a + i); }
+__device__ __forceinline__ d2 get(const pennant_vec& a, int64_t i) { return mk(get(a.x, i), get(a.y, i)); }
+
+// This thread's side of a tile and its neighbours in the zone
+struct CycSide {
+    SideAt c;
+    int s, prev, next;   // mesh index; tile-local indices
+};
+__device__ __forceinline__ CycSide cyc_side(const Tile& t, const int* zsb, const unsigned char* zof, int lane) {
+    CycSide o;
+    o.c = side_at(t, zsb, zof, min(lane, t.ns - 1));
+    o.s = t.s0 + o.c.i;
+    o.prev = wide_prev<1>(o.c);
+    o.next = wide_next<1>(o.c);
+    return o;
+}
+
+__global__ void __launch_bounds__(PN_TB) k_cycle_pred(CycleArgs a) {
+    const pennant_mesh& m = a.m;
+    const int tz = a.tz;
+    if (a.ctl->done) return;
+    PN_WIDE_SHARED(1);
+    // later x1, e1, sa_ and sv_ hold cqe1, cqe2, cw and ccos, dl_ the side
+    // fractions and u1 the sides' forces
+    __shared__ d2 x1[PN_TB], u1[PN_TB], e1[PN_TB];
+    __shared__ double el[PN_TB], sa_[PN_TB], sv_[PN_TB], dl_[PN_TB], dux_[PN_TB];
+    __shared__ d2 zxl[PN_CYC_TZ], zul[PN_CYC_TZ];
+    __shared__ double zal[PN_CYC_TZ], zrl[PN_CYC_TZ], zpl[PN_CYC_TZ], zsl[PN_CYC_TZ];
+    const double dth = 0.5 * a.ctl->dt;
+    const int z = t.z0 + lane;
+    const bool on = lane < t.ns;
+    const CycSide d = cyc_side(t, zsb, zof, lane);
+    // the corner that this thread stores (below): of zone qz of the tile, its side qk
+    const int qk = lane / t.nz, qz = lane - qk * t.nz;
+    const int qb = zsb[qz] - t.s0, qn = zsb[qz + 1] - zsb[qz], qi = qb + qk;
+    const bool qon = qk < qn && qi < PN_TB;
+    const int p = m.mapsp1[d.s], slot = a.pcpos[qon ? t.s0 + qi : d.s];
+    const double mf = get(a.smf, d.s);
+    double zr0 = 0., ze = 0., zwr = 0., zm = 0., zv0 = 0.;
+    if (has_zone) {
+        zr0 = a.zr[z];
+        ze = a.ze[z];
+        zwr = a.zwrate[z];
+        zm = a.zm[z];
+        zv0 = a.zvol[z];
+    }
+    const d2 u = V::ld(a.pu, p);
+    const d2 x = add(V::ld(a.px, p), scl(dth, u));          // advPosHalf
+    if (on) {
+        x1[lane] = x;
+        u1[lane] = u;
+    }
+    __syncthreads();
+    // zone centres and mean velocities; edges (calcCtrs, calcEdgeLen, setVelDiff)
+    const int zb = has_zone ? zsb[lane] - t.s0 : 0, zend = has_zone ? wide_zone_end<1>(t, zsb, lane) : 0;
+    if (has_zone) {
+        const double n = (double)(zsb[lane + 1] - zsb[lane]);
+        d2 cx = mk(0., 0.), cu = mk(0., 0.);
+        for (int i = zb; i < zend; ++i) {
+            cx = add(cx, dvs(x1[i], n));
+            cu = add(cu, dvs(u1[i], n));
+        }
+        zxl[lane] = cx;
+        zul[lane] = cu;
+        put(a.zxp, z, cx);
+        put(a.zuc, z, cu);
+    }
+    const d2 dx = sub(x1[d.next], x), e = scl(0.5, add(x, x1[d.next]));
+    const double l = len(dx);
+    if (on) {
+        e1[lane] = e;
+        el[lane] = l;
+        dux_[lane] = vel_diff(dx, sub(u1[d.next], u), l);
+        put(a.exp, d.s, e);
+        put(a.elen, d.s, l);
+    }
+    __syncthreads();
+    // sides and corners (calcVols, calcSurfVecs, calcCharLen, setCornerDiv)
+    const d2 zx = zxl[d.c.zi], ss = rot_ccw(sub(e, zx));
+    double sa, sv;
+    side_volume(x, x1[d.next], zx, sa, sv);
+    int bad = (on && sv <= 0.) ? 1 : 0;
+    CornerDiv cd;
+    {
+        const d2 up1 = scl(0.5, add(u, u1[d.next])), up3 = scl(0.5, add(u1[d.prev], u));
+        cd = corner_div(x, e, zx, e1[d.prev], u, up1, zul[d.c.zi], up3, el[d.prev], l);
+    }
+    if (on) {
+        const double fac = (d.c.n == 3 ? 3. : 4.);
+        sa_[lane] = sa;
+        sv_[lane] = sv;
+        dl_[lane] = fac * sa / l;
+        put(a.sareap, d.s, sa);
+        put(a.svolp, d.s, sv);
+        put(a.ssurfp, d.s, ss);
+        put(a.carea, d.s, cd.area);
+        put(a.cdiv, d.s, cd.div);
+        put(a.cevol, d.s, cd.evol);
+        put(a.cdu, d.s, cd.du);
+    }
+    __syncthreads();
+    // zone sums, density, pressure and time step limit
+    double dtm = 1.e99;
+    if (has_zone) {
+        double za = 0., zv = 0., dl = 1.e99, tm = 0.;
+        for (int i = zb; i < zend; ++i) {
+            za += sa_[i];
+            zv += sv_[i];
+            dl = smin(dl, dl_[i]);
+            tm = smax(tm, dux_[i]);
+        }
+        const double zr = zm / zv;
+        double zp, zss;
+        state_half(zr0, zv, zv0, ze, zwr, zm, a.gamma, a.ssmin, dth, zp, zss);
+        const double zdu = a.q1 * zss + 2. * a.q2 * tm;
+        zal[lane] = za;
+        zrl[lane] = zr;
+        zpl[lane] = zp;
+        zsl[lane] = zss;
+        put(a.zvol0, z, zv0);
+        put(a.zareap, z, za);
+        put(a.zvolp, z, zv);
+        put(a.zdl, z, dl);
+        put(a.zrp, z, zr);
+        put(a.zp, z, zp);
+        put(a.zss, z, zss);
+        put(a.ztmp, z, tm);
+        put(a.zdu, z, zdu);
+        const double cdu = smax(zdu, smax(zss, 1.e-99));      // calcDtNew
+        const double zdthyd = dl * a.cfl / cdu;
+        dtm = (zdthyd < dtm) ? zdthyd : dtm;
+    }
+    __syncthreads();
+    // forces (calcForcePGas, calcForceTTS, setQCnForce, setForceQCS)
+    const double zr = zrl[d.c.zi], zs = zsl[d.c.zi];
+    const d2 fp = scl(-zpl[d.c.zi], ss);
+    const d2 ft = scl(-tts_sdp(sa, mf, zal[d.c.zi], zr, zs, a.alfa, a.ssmin), ss);
+    const double cm = corner_mu(cd.du, cd.evol, cd.div, zr, zs, a.qgamma, a.q1, a.q2);
+    const d2 qa = dvs(scl(cm, sub(u, u1[d.prev])), el[d.prev]);
+    const d2 qb2 = dvs(scl(cm, sub(u1[d.next], u)), l);
+    double cl = cd.cos;
+    const double w = corner_weight(cd.area, cl);
+    if (on) {
+        put(a.sfp, d.s, fp);
+        put(a.sft, d.s, ft);
+        put(a.crmu, d.s, cm);
+        put(a.cqe1, d.s, qa);
+        put(a.cqe2, d.s, qb2);
+        put(a.cw, d.s, w);
+        put(a.ccos, d.s, cl);
+        x1[lane] = qa;
+        e1[lane] = qb2;
+        sa_[lane] = w;
+        sv_[lane] = cl;
+        dl_[lane] = mf;
+    }
+    __syncthreads();
+    if (on) {
+        const d2 fq = qcs_force(w, sa_[d.next], cl, sv_[d.next], qa, qb2, x1[d.next], e1[d.next], l);
+        put(a.sfq, d.s, fq);
+        u1[lane] = add(add(fp, fq), ft);
+    }
+    __syncthreads();
+    // corner forces and masses (calcCrnrMass, sumCrnrForce): a wave takes one
+    // corner of consecutive zones, whose slots follow each other (stored side
+    // by side, each wave's stores are four runs of 16 slots: 606 -> 575 us)
+    if (qon) {
+        const int prev = min(qk == 0 ? qb + qn - 1 : qi - 1, PN_TB - 1);
+        const d2 fc = sub(u1[qi], u1[prev]);
+        put(a.cfx, slot, fc.x);
+        put(a.cfy, slot, fc.y);
+        put(a.cmass, slot, zrl[qz] * zal[qz] * 0.5 * (dl_[qi] + dl_[prev]));
+    }
+    dtm = block_min(dtm);
+    bad = block_sum(bad);
+    if (threadIdx.x == 0) {
+        a.part.dt[blockIdx.x] = dtm;
+        a.part.bp[blockIdx.x] = bad;
+    }
+}
+
+__global__ void __launch_bounds__(PN_TB) k_cycle_corr(CycleArgs a) {
+    const pennant_mesh& m = a.m;
+    const int tz = a.tz;
+    if (a.ctl->done) return;
+    PN_WIDE_SHARED(1);
+    __shared__ d2 x1[PN_TB], vs[PN_TB], zxl[PN_CYC_TZ];
+    __shared__ double xx[PN_TB], sa_[PN_TB], sv_[PN_TB], dw[PN_TB];
+    const double dt = a.ctl->dt;
+    const int z = t.z0 + lane;
+    const bool on = lane < t.ns;
+    const CycSide d = cyc_side(t, zsb, zof, lane);
+    const int p = m.mapsp1[d.s];
+    const d2 sf = add(get(a.sfp, d.s), get(a.sfq, d.s));
+    double et = 0., zm = 0., zv0 = 0., zp = 0.;
+    if (has_zone) {
+        et = a.zetot[z];
+        zm = a.zm[z];
+        zv0 = a.zvol0[z];
+        zp = a.zp[z];
+    }
+    const d2 x = V::ld(a.px, p), v = add(V::ld(a.pu0, p), V::ld(a.pu, p));
+    const double xv = V::ldx(a.pxp, p);
+    if (on) {
+        x1[lane] = x;
+        vs[lane] = v;
+        xx[lane] = xv;
+    }
+    __syncthreads();
+    // calcCtrs, calcWork
+    const int zb = has_zone ? zsb[lane] - t.s0 : 0, zend = has_zone ? wide_zone_end<1>(t, zsb, lane) : 0;
+    if (has_zone) {
+        const double n = (double)(zsb[lane + 1] - zsb[lane]);
+        d2 cx = mk(0., 0.);
+        for (int i = zb; i < zend; ++i) cx = add(cx, dvs(x1[i], n));
+        zxl[lane] = cx;
+        put(a.zx, z, cx);
+    }
+    const d2 x2 = x1[d.next];
+    if (on) {
+        put(a.ex, d.s, scl(0.5, add(x, x2)));
+        dw[lane] = side_work(sf, v, vs[d.next], xv, xx[d.next], 0.5 * dt);
+    }
+    __syncthreads();
+    // calcVols
+    double sa, sv;
+    side_volume(x, x2, zxl[d.c.zi], sa, sv);
+    int bad = (on && sv <= 0.) ? 1 : 0;
+    if (on) {
+        put(a.sarea, d.s, sa);
+        put(a.svol, d.s, sv);
+        sa_[lane] = sa;
+        sv_[lane] = sv;
+    }
+    __syncthreads();
+    double dvov = 1.e-99;
+    if (has_zone) {
+        double za = 0., zv = 0., w = 0.;
+        for (int i = zb; i < zend; ++i) {
+            za += sa_[i];
+            zv += sv_[i];
+            et += dw[i];
+            w += dw[i];
+        }
+        const double dvol = zv - zv0;
+        put(a.zarea, z, za);
+        put(a.zvol, z, zv);
+        put(a.zetot, z, et);
+        put(a.zw, z, w);
+        put(a.zwrate, z, (w + zp * dvol) * (1. / dt));            // calcWorkRate
+        put(a.ze, z, et / (zm + 1.e-99));                         // calcEnergy
+        put(a.zr, z, zm / zv);                                    // calcRho
+        const double zdvov = fabs(dvol / zv0);                // calcDvol
+        dvov = (zdvov > dvov) ? zdvov : dvov;
+    }
+    dvov = block_max(dvov);
+    bad = block_sum(bad);
+    if (threadIdx.x == 0) {
+        a.part.dv[blockIdx.x] = dvov;
+        a.part.bc[blockIdx.x] = bad;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1545,3 +1918,48 @@ int pennant_hip_apply_fixed_bc(const int32_t* mapbp, int32_t numb, double vfix_x
 }
 
 }  // extern "C"
+
+namespace pn {
+
+int cycle_blocks(const pennant_mesh* m) {
+    const int tz = wide_tile_zones(m, 1);
+    return tz ? tile_blocks(m, tz) : 0;
+}
+
+int launch_task_cycle(pennant_problem* pb) {
+    const pennant_mesh& m = pb->dm;
+    const Params& q = pb->prm;
+    const int nb = cycle_blocks(&m);
+    CycleArgs a;
+    a.m = m;
+    a.tz = wide_tile_zones(&m, 1);
+    a.ctl = pb->ctl;
+    a.gamma = q.gamma; a.ssmin = q.ssmin; a.alfa = q.alfa; a.qgamma = q.qgamma;
+    a.q1 = q.q1; a.q2 = q.q2; a.cfl = q.cfl;
+    a.px = pb->cv("px"); a.pu = pb->cv("pu"); a.pu0 = pb->cv("pu0"); a.pxp = pb->cv("pxp");
+    a.pcpos = pb->pcpos; a.cfx = pb->cfx; a.cfy = pb->cfy; a.cmass = pb->cmass;
+    const struct { const char* name; pennant_vec* v; } vecs[] = {
+        {"zx", &a.zx}, {"zxp", &a.zxp}, {"zuc", &a.zuc},
+        {"ex", &a.ex}, {"exp", &a.exp}, {"ssurfp", &a.ssurfp}, {"sfp", &a.sfp}, {"sfq", &a.sfq},
+        {"sft", &a.sft}, {"cqe1", &a.cqe1}, {"cqe2", &a.cqe2}};
+    for (const auto& e : vecs) *e.v = pb->vv(e.name);
+    const struct { const char* name; double** d; } vals[] = {
+        {"zarea", &a.zarea}, {"zvol", &a.zvol}, {"zareap", &a.zareap},
+        {"zvolp", &a.zvolp}, {"zvol0", &a.zvol0}, {"zdl", &a.zdl}, {"zr", &a.zr}, {"zrp", &a.zrp},
+        {"ze", &a.ze}, {"zetot", &a.zetot}, {"zw", &a.zw}, {"zwrate", &a.zwrate}, {"zp", &a.zp},
+        {"zss", &a.zss}, {"zdu", &a.zdu}, {"ztmp", &a.ztmp}, {"sarea", &a.sarea}, {"svol", &a.svol},
+        {"sareap", &a.sareap}, {"svolp", &a.svolp}, {"elen", &a.elen}, {"carea", &a.carea},
+        {"cevol", &a.cevol}, {"cdu", &a.cdu}, {"cdiv", &a.cdiv}, {"ccos", &a.ccos},
+        {"crmu", &a.crmu}, {"cw", &a.cw}};
+    for (const auto& e : vals) *e.d = pb->f(e.name);
+    a.zm = pb->f("zm");
+    a.smf = pb->f("smf");
+    a.part = cycle_parts(pb->ws, nb);
+    if (nb > 0) hipLaunchKernelGGL(k_cycle_pred, dim3(nb), dim3(PN_TB), 0, pb->stream, a);
+    if (const int rc = launch_cycle_points(pb)) return rc;
+    if (nb > 0) hipLaunchKernelGGL(k_cycle_corr, dim3(nb), dim3(PN_TB), 0, pb->stream, a);
+    if (const int rc = launch_status()) return rc;
+    return launch_task_end(pb, a.part, nb);
+}
+
+}  // namespace pn
