@@ -43,6 +43,14 @@ __device__ __forceinline__ d2 ld(pennant_cvec v, int64_t i) { return mk(v.x[i], 
 __device__ __forceinline__ d2 ld(pennant_vec v, int64_t i) { return mk(v.x[i], v.y[i]); }
 __device__ __forceinline__ void st(pennant_vec v, int64_t i, d2 a) { v.x[i] = a.x; v.y[i] = a.y; }
 
+// A value that is the same in every lane, in scalar registers.
+__device__ __forceinline__ double uni(double v) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
 __device__ __forceinline__ double wave_min(double v) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {

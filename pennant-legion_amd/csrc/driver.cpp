@@ -8,7 +8,6 @@
 // arrays and keeps dt, time and the stop test on the device.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -403,7 +402,7 @@ pennant_problem* pn::create_problem(const Params& prm, HostMesh&& hm, int npown,
         }
         pb->fields[fs.name] = d;
     }
-    pb->ws = dalloc<char>(pb, std::max(pennant_hip_reduce_workspace_bytes(), cycle_parts_bytes(cycle_blocks(&m))));
+    pb->ws = dalloc<char>(pb, pennant_hip_reduce_workspace_bytes() + task_chain_bytes());
     pb->ctl = dalloc<Ctl>(pb, 1);
     if (hipHostMalloc((void**)&pb->ctl_host, sizeof(Ctl), hipHostMallocDefault) != hipSuccess)
         return fail("hipHostMalloc failed");
@@ -453,6 +452,7 @@ pennant_problem* pn::create_problem(const Params& prm, HostMesh&& hm, int npown,
     if (!rc) rc = launch_init_state(pb);
     if (!rc) rc = launch_first_dt(pb);
     if (!rc) rc = fused_setup(pb);
+    if (!rc) rc = task_chain_setup(pb);
     if (!rc) rc = (int)hipStreamSynchronize(s);
     if (rc) return fail(std::string("initialisation failed: ") + hipGetErrorString((hipError_t)rc));
     return pb;
@@ -536,10 +536,9 @@ static int build_graph(pennant_problem* pb, int form) {
     hipGraph_t g = nullptr;
     const bool pipe = pipelined(pb, form), tile = tiled(pb, form);
     CK(hipStreamBeginCapture(pb->stream, hipStreamCaptureModeThreadLocal));
-    int rc = 0;
-    for (int k = 0; k < PN_GRAPH_CYCLES && !rc; ++k)
-        rc = pipe ? fused_cycle_pipe(pb, nullptr, form)
-                  : (tile ? tile_cycle(pb, form, k & 1) : fused_cycle(pb, nullptr, form));
+    int rc = tile ? tile_cycles(pb, form, PN_GRAPH_CYCLES) : 0;
+    for (int k = 0; k < PN_GRAPH_CYCLES && !rc && !tile; ++k)
+        rc = pipe ? fused_cycle_pipe(pb, nullptr, form) : fused_cycle(pb, nullptr, form);
     const int rc2 = (int)hipStreamEndCapture(pb->stream, &g);
     if (rc || rc2) {
         if (g) (void)hipGraphDestroy(g);
@@ -557,16 +556,15 @@ static int build_task_graph(pennant_problem* pb) {
     drop_graph(pb);
     hipGraph_t g = nullptr;
     CK(hipStreamBeginCapture(pb->stream, hipStreamCaptureModeThreadLocal));
-    int rc = 0;
-    for (int k = 0; k < PN_GRAPH_CYCLES && !rc; ++k) rc = launch_task_cycle(pb);
+    const int rc = launch_task_cycles(pb, PN_GRAPH_CYCLES);
     const int rc2 = (int)hipStreamEndCapture(pb->stream, &g);
     if (rc || rc2) {
         if (g) (void)hipGraphDestroy(g);
         return rc ? rc : rc2;
     }
-    rc = (int)hipGraphInstantiate(&pb->gexec, g, nullptr, nullptr, 0);
+    const int rc3 = (int)hipGraphInstantiate(&pb->gexec, g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
-    if (rc) { pb->gexec = nullptr; return rc; }
+    if (rc3) { pb->gexec = nullptr; return rc3; }
     pb->graph_form = PN_GRAPH_TASKS;
     return 0;
 }
@@ -598,9 +596,9 @@ int pennant_launch_cycles(pennant_problem* pb, int ncycles, int mode) {
         }
         if (left > 0) CK(ensure_lookahead(pb, form));
         // tile cycles come in pairs; an odd cycle runs as separate passes
-        for (; left > 1 && tiled(pb, form); left -= 2) {
-            CK(tile_cycle(pb, form, 0));
-            CK(tile_cycle(pb, form, 1));
+        if (left > 1 && tiled(pb, form)) {
+            CK(tile_cycles(pb, form, left & ~1));
+            left &= 1;
         }
         for (; left > 0; --left) CK(one_cycle(pb, nullptr, form));
         return 0;
@@ -612,7 +610,7 @@ int pennant_launch_cycles(pennant_problem* pb, int ncycles, int mode) {
         if (pb->graph_form != PN_GRAPH_TASKS || !pb->gexec) CK(build_task_graph(pb));
         for (; left >= PN_GRAPH_CYCLES; left -= PN_GRAPH_CYCLES) CK(hipGraphLaunch(pb->gexec, pb->stream));
     }
-    for (; left > 0; --left) CK(launch_task_cycle(pb));
+    CK(launch_task_cycles(pb, left));
     return 0;
 }
 

@@ -75,10 +75,11 @@ __global__ void k_first_dt(Ctl* c, int cstop, double dtmax, double dtinit, doubl
     c->done = (c->cycle >= cstop || c->time >= tstop) ? 1 : 0;
 }
 
-// End of cycle: checkBadSides (src/Mesh.cc:1531-1550), updateTime/updateCycle
-// (src/Driver.cc:266-295), the PENNANT stop test (time >= tstop or
-// cycle >= cstop) and calcGlobalDt for the next cycle.
-__device__ void end_cycle(Ctl* c, int cstop, double dtmax, double dtinit, double dtfac, double tstop) {
+// End of a cycle of single task steps, whose calcDt has run: checkBadSides
+// (src/Mesh.cc:1531-1550), updateTime/updateCycle (src/Driver.cc:266-295), the
+// PENNANT stop test (time >= tstop or cycle >= cstop) and calcGlobalDt for the
+// next cycle.
+__global__ void k_end_cycle(Ctl* c, int cstop, double dtmax, double dtinit, double dtfac, double tstop) {
     if (c->done) return;
     if (c->numsbad_pred > 0 || c->numsbad_corr > 0) {
         c->err_cycle = c->cycle;
@@ -91,75 +92,6 @@ __device__ void end_cycle(Ctl* c, int cstop, double dtmax, double dtinit, double
     c->dtlast = c->dt;
     c->done = (c->cycle >= cstop || c->time >= tstop) ? 1 : 0;
     c->dt = global_dt(c->cycle, c->time, c->dtlast, c->dtrec, dtmax, dtinit, dtfac, tstop);
-}
-__global__ void k_end_cycle(Ctl* c, int cstop, double dtmax, double dtinit, double dtfac, double tstop) {
-    end_cycle(c, cstop, dtmax, dtinit, dtfac, tstop);
-}
-
-// The end of a task-mode cycle: the folds of calcDtNew's and calcDvol's block
-// partials and of the bad-side counts, calcDt, and the end of the cycle.  One
-// block; eight partials of each array are loaded before any is used.
-#define PN_END_BLOCK 1024
-__global__ void __launch_bounds__(PN_END_BLOCK) k_task_end(Ctl* c, CycleParts q, int nb, double cflv, int cstop,
-                                                           double dtmax, double dtinit, double dtfac,
-                                                           double tstop) {
-    if (c->done) return;
-    constexpr int U = 8;
-    double mn = 1.e99, mx = 1.e-99;
-    int bp = 0, bc = 0;
-    for (int i0 = threadIdx.x; i0 < nb; i0 += U * PN_END_BLOCK) {
-        double a[U], b[U];
-        int d[U], e[U];
-#pragma unroll
-        for (int k = 0; k < U; ++k) {
-            const int i = min(i0 + k * PN_END_BLOCK, nb - 1);
-            a[k] = q.dt[i];
-            b[k] = q.dv[i];
-            d[k] = q.bp[i];
-            e[k] = q.bc[i];
-        }
-#pragma unroll
-        for (int k = 0; k < U; ++k) {
-            mn = (a[k] < mn) ? a[k] : mn;
-            mx = (b[k] > mx) ? b[k] : mx;
-            if (i0 + k * PN_END_BLOCK < nb) {
-                bp += d[k];
-                bc += e[k];
-            }
-        }
-    }
-    mn = wave_min(mn);
-    mx = wave_max(mx);
-    bp = wave_sum(bp);
-    bc = wave_sum(bc);
-    __shared__ double pmn[PN_END_BLOCK / 64], pmx[PN_END_BLOCK / 64];
-    __shared__ int pbp[PN_END_BLOCK / 64], pbc[PN_END_BLOCK / 64];
-    if ((threadIdx.x & 63) == 0) {
-        const int w = threadIdx.x >> 6;
-        pmn[w] = mn;
-        pmx[w] = mx;
-        pbp[w] = bp;
-        pbc[w] = bc;
-    }
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    for (int w = 1; w < PN_END_BLOCK / 64; ++w) {
-        mn = (pmn[w] < mn) ? pmn[w] : mn;
-        mx = (pmx[w] > mx) ? pmx[w] : mx;
-        bp += pbp[w];
-        bc += pbc[w];
-    }
-    // calcDtTask, src/Hydro.cc:1647-1667
-    double r = 1.e99;
-    if (mn < r) r = mn;
-    const double b = c->dt * cflv / mx;
-    if (b < r) r = b;
-    c->dtnew = mn;
-    c->dvovmax = mx;
-    c->numsbad_pred = bp;
-    c->numsbad_corr = bc;
-    c->dtrec = r;
-    end_cycle(c, cstop, dtmax, dtinit, dtfac, tstop);
 }
 
 // Hydro::doCycle's copies and fills, src/Hydro.cc:361-368 and 389-418
@@ -261,13 +193,6 @@ int launch_end_cycle(pennant_problem* pb) {
     const Params& q = pb->prm;
     hipLaunchKernelGGL(k_end_cycle, dim3(1), dim3(1), 0, pb->stream, pb->ctl, q.cstop, q.dtmax,
                        q.dtinit, q.dtfac, q.tstop);
-    return (int)hipGetLastError();
-}
-
-int launch_task_end(pennant_problem* pb, const CycleParts& part, int nb) {
-    const Params& q = pb->prm;
-    hipLaunchKernelGGL(k_task_end, dim3(1), dim3(PN_END_BLOCK), 0, pb->stream, pb->ctl, part, nb, q.cflv,
-                       q.cstop, q.dtmax, q.dtinit, q.dtfac, q.tstop);
     return (int)hipGetLastError();
 }
 

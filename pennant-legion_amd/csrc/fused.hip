@@ -47,6 +47,7 @@
 
 #include "closure.h"
 #include "common.h"
+#include "cycle_end.h"
 #include "problem.h"
 
 using namespace pn;
@@ -137,14 +138,6 @@ template <int NS>
 __device__ __forceinline__ int nxt(int k) { return (k + 1 == NS) ? 0 : k + 1; }
 template <int NS>
 __device__ __forceinline__ int prv(int k) { return (k == 0) ? NS - 1 : k - 1; }
-
-// A value that is the same in every lane, in scalar registers.
-__device__ __forceinline__ double uni(double v) {
-    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
 
 // Streaming accesses (each element touched once per kernel): nontemporal
 // loads and stores, which a plain copy kernel measures 9% faster than
@@ -1974,36 +1967,6 @@ __global__ void __launch_bounds__(PN_BLOCK) k_corr(FusedArgs a, int zbeg, int ze
 // unpipelined cycle.
 
 // The control-block values the end of a cycle and the look-ahead dt start from.
-struct CtlSnap {
-    double time, dt, la_dtnew;
-    int cycle, la_bp, done;
-};
-// Relaxed atomic loads: vector loads (never scalar-cache loads), issued
-// back to back with no wait between them.
-__device__ __forceinline__ double ld_vec(const double* p) {
-    return __builtin_bit_cast(double, __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p),
-                                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-}
-__device__ __forceinline__ int ld_vec(const int* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// Read through vector loads: the caller stores to the block later.
-__device__ __forceinline__ CtlSnap snap_ctl(const Ctl* c) {
-    CtlSnap v;
-    v.time = ld_vec(&c->time);
-    v.dt = ld_vec(&c->dt);
-    v.la_dtnew = ld_vec(&c->la_dtnew);
-    v.cycle = ld_vec(&c->cycle);
-    v.la_bp = ld_vec(&c->la_bp);
-    v.done = ld_vec(&c->done);
-    return v;
-}
-
-struct DtParams {
-    double cflv, dtmax, dtfac, tstop;
-    int cstop;
-};
-
 // dt of the cycle after the current one as the finalize computes it
 // (src/Hydro.cc:1647-1667, src/Driver.cc:213-245) when the volume-change
 // limit does not bind; `last` when the current cycle ends the run.
@@ -2153,13 +2116,6 @@ __device__ __forceinline__ void blk_fold_fin(double& mn, double& mx, int& bp, in
         }
 }
 
-// The end of the cycle for one problem, by one block of PN_FIN_BLOCK threads,
-// from npred predictor and ncorr corrector partials.
-__device__ __forceinline__ int end_cycle(Ctl* c, const CtlSnap& v, double mn, double mx, int bp,
-                                         int bc, double cflv, int cstop, double dtmax,
-                                         double dtfac, double tstop, int zre,
-                                         double* next_dt = nullptr);
-
 // Each thread's share of the partials (thread t of BS folds t, t + BS, ...),
 // loaded PN_FIN_PER per thread at a time with no branch between the
 // loads.  Indices past the end read the last partial again: a repeat leaves a
@@ -2207,51 +2163,8 @@ __device__ __forceinline__ void finalize_block(Ctl* c, const double* part_dt, co
     fold_partials<PN_FIN_BLOCK>(part_dt, part_bp, npred, part_dv, part_bc, ncorr, mn, bp, mx, bc);
     blk_fold_fin<PN_FIN_BLOCK>(mn, mx, bp, bc);
     if (threadIdx.x != 0 || v.done) return;
-    end_cycle(c, v, mn, mx, bp, bc, cflv, cstop, dtmax, dtfac, tstop, zre);
-}
-
-// The end of a cycle from its predictor's dt limit and bad-side count (mn,
-// bp) and its corrector's dvol ratio and bad-side count (mx, bc).  v is the
-// control block as read through vector loads before any store to it (a
-// scalar-cache load is not ordered with a later vector store to the same
-// address).
-// Returns the new done flag; *next_dt (when given) receives the next dt.
-// zre: whether this cycle's corrector stored zr and ze (Ctl::zre_valid).
-__device__ __forceinline__ int end_cycle(Ctl* c, const CtlSnap& v, double mn, double mx, int bp,
-                                         int bc, double cflv, int cstop, double dtmax,
-                                         double dtfac, double tstop, int zre, double* next_dt) {
     c->zre_valid = zre;
-    double r = 1.e99;
-    if (mn < r) r = mn;
-    const double d2v = v.dt * cflv / mx;
-    if (d2v < r) r = d2v;
-    c->dtnew = mn;
-    c->dvovmax = mx;
-    c->numsbad_pred = bp;
-    c->numsbad_corr = bc;
-    c->dtrec = r;
-    if (bp > 0 || bc > 0) {
-        c->err_cycle = v.cycle;
-        c->err_pred = bp > 0 ? 1 : 0;
-        c->done = 1;
-        return 1;
-    }
-    const double time = v.time + v.dt;
-    const int cycle = v.cycle + 1;
-    const double dtlast = v.dt;
-    double dt = dtmax;
-    const double dtrecover = dtfac * dtlast;
-    if (dtrecover < dt) dt = dtrecover;
-    if ((tstop - time) < dt) dt = tstop - time;
-    if (r < dt) dt = r;
-    const int done = (cycle >= cstop || time >= tstop) ? 1 : 0;
-    c->time = time;
-    c->cycle = cycle;
-    c->dtlast = dtlast;
-    c->done = done;
-    c->dt = dt;
-    if (next_dt) *next_dt = dt;
-    return done;
+    end_cycle(c, v, mn, mx, bp, bc, {cflv, dtmax, dtfac, tstop, cstop});
 }
 
 __global__ void __launch_bounds__(PN_FIN_BLOCK) k_finalize(FusedArgs a, int npred, int ncorr,
@@ -2289,9 +2202,8 @@ __global__ void __launch_bounds__(PN_FIN_BLOCK) k_finalize_pipe(FusedArgs a, int
     bool last;
     const double dtn = lookahead_dt(v, q, last);
     double dt1 = 0.;
-    if (end_cycle(c, v, v.la_dtnew, mx, v.la_bp, bc, q.cflv, q.cstop, q.dtmax, q.dtfac, q.tstop, 0,
-                  &dt1))
-        return;
+    c->zre_valid = 0;
+    if (end_cycle(c, v, v.la_dtnew, mx, v.la_bp, bc, q, &dt1)) return;
     if (!last && dt1 == dtn) {
         c->la_dtnew = mn;
         c->la_bp = bp;
@@ -2350,6 +2262,13 @@ __global__ void __launch_bounds__(PN_FIN_BLOCK) k_finalize_la(FusedArgs a, int n
 // second cycle of a pair copies it back when the first ended the run), so the
 // problem's own arrays hold the state after every pair.
 //
+// Tiles hand their dt limits and dvol ratios on in slots (cycle_end.h).  On a
+// rect of few tiles, all of them at work together, each tile of the next cycle
+// ends the cycle from them by itself while its loads are under way (linked
+// cycles: no launch between two tile kernels).  With many tiles each would pay
+// for that, and one wave ends the cycle between the two: 3.5 us, where folding
+// an array of 10600 partials took 9.5.
+//
 // The triangles of a pie's first row and the origin are not part of a tile:
 // their predictor and corrector run as in the separate passes, before and
 // after, and the tiles of the first row of quads read the triangles' corner
@@ -2367,12 +2286,17 @@ __global__ void __launch_bounds__(PN_FIN_BLOCK) k_finalize_la(FusedArgs a, int n
 // offsets and one fold of both counts together took Sedov 1440^2 from 211 to
 // 205 us (FP64), 108.5 to 106.6 (mixed) and 154 to 149 (learned).
 // Per cycle, separate passes (for mixed and learned the pipelined ones) ->
-// tiles: FP64 Sedov 1440^2 306 -> 205 us, Noh pie 1024^2 178 -> 120 us; mixed
-// LeBlanc 4096 x 256 87 -> 57 us, 333 x 217 23 -> 12.2 us; learned Sedov
-// 1440^2 176 -> 149 us; FP64 45^2 21 -> 14 us.  It was faster at every size, so
+// tiles: FP64 Sedov 1440^2 306 -> 201 us, Noh pie 1024^2 178 -> 119 us; mixed
+// LeBlanc 4096 x 256 87 -> 55 us, 333 x 217 23 -> 10.1 us; learned Sedov
+// 1440^2 176 -> 147 us; FP64 90^2 12.6 -> 10.1 us by the linking alone.  It was faster at every size, so
 // structured meshes always take it.
 #define PN_TILE 16
 #define PN_TIN (PN_TILE - 2)
+// Most tiles of linked cycles (tile_cycles).  Linked and not, us a cycle, FP64
+// and mixed: 90^2 (49 tiles) 10.1 and 12.7, 7.6 and 10.1; 333 x 217 (384) 14.9
+// and 17.1, 10.1 and 12.4; 420^2 (900) 25.8 and 27.3, 16.1 and 17.8; 500^2
+// (1296) 35.4 both, 21.4 and 21.3; 1440^2 (10609) 213 and 200, 120 and 102.
+#define PN_LINK_TILES 1024
 
 // A structured mesh in the arrays: zone (i, j) of nzx x nzy has its points
 // (i, j), (i + 1, j), (i + 1, j + 1), (i, j + 1); row 0 of a pie is the
@@ -2492,12 +2416,18 @@ __device__ __forceinline__ void tile_load(const FusedArgs& a, const TileMesh& g,
     in.bits = at_byte<unsigned char>(a.pbc, p);
 }
 
-// The tile whose first zone (ring included) is (i0, j0), loaded in `in`; its
-// partials go to slot.  Returns whether a CL_FLAG tile has a zone for the network: such a
+// Where a tile's dt limit, dvol ratio and bad sides go: into slots, or (a batch,
+// whose problems have few tiles each) into the block partials a.part_*.
+struct TileSink {
+    slot_t* slots;
+    int at;
+};
+
+// The tile whose first zone (ring included) is (i0, j0), loaded in `in`.  Returns whether a CL_FLAG tile has a zone for the network: such a
 // tile is left to the list kernel and stores nothing.
 template <typename T, int CL>
 __device__ __forceinline__ bool tile_body(const FusedArgs& a, const TileOut& o, const TileMesh& g, int i0, int j0,
-                                          const TileIn<T>& in, int slot, double dt, bool zre, ClCount& total) {
+                                          const TileIn<T>& in, const TileSink& sink, double dt, bool zre, ClCount& total) {
     __shared__ T crn[12][PN_BLOCK];
     __shared__ double pts[sizeof(T) == 8 ? 5 : 4][PN_BLOCK];
     __shared__ struct {
@@ -2666,10 +2596,15 @@ __device__ __forceinline__ bool tile_body(const FusedArgs& a, const TileOut& o, 
             dvov = (lds.dv[w] > dvov) ? lds.dv[w] : dvov;
             bads += lds.bad[w];
         }
-        a.part_dt[slot] = dtm;
-        a.part_bp[slot] = bads & 0xffff;
-        a.part_dv[slot] = dvov;
-        a.part_bc[slot] = bads >> 16;
+        if (sink.slots) {
+            slots_dt(sink.slots, sink.at, dtm, bads & 0xffff);
+            slots_dv(sink.slots, sink.at, dvov, bads >> 16);
+        } else {
+            a.part_dt[sink.at] = dtm;
+            a.part_bp[sink.at] = bads & 0xffff;
+            a.part_dv[sink.at] = dvov;
+            a.part_bc[sink.at] = bads >> 16;
+        }
     }
     return false;
 }
@@ -2705,9 +2640,11 @@ struct TileArgs {
     TileMesh g;
     int ntx, ntiles;
     int back;                    // the second cycle of a pair
-    int poff;                    // the tiles' first partial
+    CycleStep step;              // linked cycles: the place in their chain; others: `in` is current
+    int linked;
     int* list;                   // learned form: tiles left to the list kernel, and their number
     int* nlist;
+    int* nlist_clear;            // a chain's next cycle's number
 };
 __device__ __forceinline__ void tile_at(const TileArgs& t, int tile, int& i0, int& j0) {
     const int tj = tile / t.ntx, ti = tile - tj * t.ntx;
@@ -2726,11 +2663,17 @@ __device__ __forceinline__ int xcd_tile(int n) {
 // (neighbouring tiles share their rings through its L2); a pie's origin takes
 // one block more.  The flagging form needs 147 VGPRs: at four waves per SIMD it
 // spills 9 and takes 142 us on Sedov 1440^2, at three 121 us.
-template <typename T, int CL>
-__global__ void __launch_bounds__(PN_BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 2 : (CL == CL_FLAG ? 3 : 4))))
+template <typename T, int CL, bool LINK>
+__global__ void __launch_bounds__(PN_BLOCK)
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 2 : (LINK || CL == CL_FLAG ? 3 : 4))))
 k_tile(FusedArgs a, TileArgs t) {
-    const Ctl* c = a.ctl;
     if ((int)blockIdx.x == t.ntiles) {
+        const Ctl* c = t.step.in;
+        if (LINK) {
+            cycle_step(t.step);
+            if (CL == CL_FLAG && threadIdx.x == 0) *t.nlist_clear = 0;
+            return;
+        }
         const int done = c->done;
         if (done && !(t.back && c->cur)) return;
         const double dt = c->dt;
@@ -2747,19 +2690,31 @@ k_tile(FusedArgs a, TileArgs t) {
     const int tile = xcd_tile(t.ntiles);
     int i0, j0;
     tile_at(t, tile, i0, j0);
-    // the loads do not wait for the control block, which the last finalize has
-    // just written in another XCD's L2: Sedov 1440^2 FP64 217 -> 209 us a
-    // cycle, mixed 116 -> 108, learned 158 -> 153
+    // the loads do not wait for the control block, which another XCD has just
+    // written: Sedov 1440^2 FP64 217 -> 209 us a cycle, mixed 116 -> 108,
+    // learned 158 -> 153
     TileIn<T> in;
     tile_load<T>(a, t.g, i0, j0, in);
-    const int done = c->done;
-    if (done) {
-        if (t.back && c->cur) tile_copy<T>(a, t.o, t.g, i0, j0);
-        return;
+    auto body = [&](double dt, bool zre) {
+        ClCount none;
+        const bool left = tile_body<T, CL>(a, t.o, t.g, i0, j0, in, {t.step.put, tile}, dt, zre, none);
+        if (CL == CL_FLAG && left && threadIdx.x == 0) t.list[atomicAdd(t.nlist, 1)] = tile;
+    };
+    if constexpr (LINK) {
+        const CycleNow now = cycle_now(t.step);
+        if (!now.done)
+            body(now.dt, now.zre != 0);
+        else if (t.back && now.ended)
+            tile_copy<T>(a, t.o, t.g, i0, j0);
+    } else {
+        // (dt and zre_valid are read here and not before the branch: held
+        // across it, the mixed kernel spills 8 registers)
+        const Ctl* c = t.step.in;
+        if (!c->done)
+            body(c->dt, c->zre_valid != 0);
+        else if (t.back && c->cur)
+            tile_copy<T>(a, t.o, t.g, i0, j0);
     }
-    ClCount none;
-    const bool left = tile_body<T, CL>(a, t.o, t.g, i0, j0, in, t.poff + tile, c->dt, c->zre_valid != 0, none);
-    if (CL == CL_FLAG && left && threadIdx.x == 0) t.list[atomicAdd(t.nlist, 1)] = tile;
 }
 
 // The learned form's tiles that have a zone for the network (in the ring or
@@ -2768,9 +2723,10 @@ k_tile(FusedArgs a, TileArgs t) {
 // results are.
 __global__ void __launch_bounds__(PN_BLOCK) __attribute__((amdgpu_waves_per_eu(2)))
 k_tile_list(FusedArgs a, TileArgs t) {
-    const int done = a.ctl->done, n = *t.nlist;
-    const double dt = a.ctl->dt;
-    const bool zre = a.ctl->zre_valid != 0;
+    const Ctl* c = t.linked ? t.step.out : t.step.in;
+    const int done = c->done, n = *t.nlist;
+    const double dt = c->dt;
+    const bool zre = c->zre_valid != 0;
     if (done || (int)blockIdx.x >= n) return;
     constexpr int NQ = (int)(sizeof(ClosurePack) / 16);
     __shared__ ClosurePack wp;
@@ -2789,7 +2745,7 @@ k_tile_list(FusedArgs a, TileArgs t) {
         tile_at(t, tile, i0, j0);
         TileIn<float> in;
         tile_load<float>(b, t.g, i0, j0, in);
-        (void)tile_body<float, CL_PACKED>(b, t.o, t.g, i0, j0, in, t.poff + tile, dt, zre, cnt);
+        (void)tile_body<float, CL_PACKED>(b, t.o, t.g, i0, j0, in, {t.step.put, tile}, dt, zre, cnt);
     }
     const int nl = block_sum(cnt.learned);
     const int nf = block_sum(cnt.fallback);
@@ -2799,39 +2755,45 @@ k_tile_list(FusedArgs a, TileArgs t) {
     }
 }
 
-// K4 of a tile cycle; also says where the state is now (cur: 1 after the first
-// cycle of a pair) and empties the learned form's lists.
-// The end of a tile cycle by one block of BS threads, from its npart partials;
-// also says where the state is now (cur: 1 after the first cycle of a pair).
-template <int BS>
+// The end of a tile cycle that is not linked, by one block of PN_FIN_BLOCK
+// threads (without partials 64 do): from npart partials and (slots given) a set
+// of slots, which it empties; also says where the state is now (cur: 1 after
+// the first cycle of a pair).
 __device__ __forceinline__ void finalize_tile_block(Ctl* c, const double* part_dt, const int* part_bp,
                                                     const double* part_dv, const int* part_bc, int npart,
-                                                    double cflv, int cstop, double dtmax, double dtfac, double tstop,
-                                                    int zre, int cur) {
+                                                    slot_t* slots, const DtParams& q, int zre, int cur) {
     const CtlSnap v = snap_ctl(c);
     double mn = 1.e99, mx = 1.e-99;
     int bp = 0, bc = 0;
-    fold_partials<BS>(part_dt, part_bp, npart, part_dv, part_bc, npart, mn, bp, mx, bc);
-    blk_fold_fin<BS>(mn, mx, bp, bc);
+    SlotFold f = {1.e99, 1.e-99, 0, 0};
+    if (slots && threadIdx.x < 64) f = slots_fold(slots_load(slots));
+    if (npart > 0) {
+        fold_partials<PN_FIN_BLOCK>(part_dt, part_bp, npart, part_dv, part_bc, npart, mn, bp, mx, bc);
+        blk_fold_fin<PN_FIN_BLOCK>(mn, mx, bp, bc);
+    }
+    if (slots) slots_reset(slots);
     if (threadIdx.x != 0) return;
+    mn = (f.mn < mn) ? f.mn : mn;
+    mx = (f.mx > mx) ? f.mx : mx;
+    bp += f.bp;
+    bc += f.bc;
     if (v.done) {
         if (!cur) c->cur = 0;                // copied back
         return;
     }
-    end_cycle(c, v, mn, mx, bp, bc, cflv, cstop, dtmax, dtfac, tstop, zre);
+    c->zre_valid = zre;
+    end_cycle(c, v, mn, mx, bp, bc, q);
     c->cur = cur;
 }
 
-// K4 of a tile cycle; empties the learned form's lists.  Blocks of 256 threads
-// fold 2048 partials in one round of loads; with more, a block of 1024 saves
-// rounds and costs 1.3 us of barriers.
-template <int BS>
-__global__ void __launch_bounds__(BS) k_finalize_tile(FusedArgs a, int npart, DtParams q, int zre, int cur, int* nlist) {
+// K4 of a tile cycle that is not linked, from the tiles' slots and a pie's
+// triangles' partials; empties the learned form's lists.
+__global__ void __launch_bounds__(PN_FIN_BLOCK) k_finalize_tile(FusedArgs a, int npart, slot_t* slots, DtParams q, int zre,
+                                                                int cur, int* nlist) {
     if (nlist && threadIdx.x == 0) *nlist = 0;
     if (a.zcount)
-        for (int k = threadIdx.x; k < a.nzruns * PN_LSLICES; k += BS) a.zcount[k * PN_LSTRIDE] = 0u;
-    finalize_tile_block<BS>(a.ctl, a.part_dt, a.part_bp, a.part_dv, a.part_bc, npart, q.cflv, q.cstop, q.dtmax,
-                            q.dtfac, q.tstop, zre, cur);
+        for (int k = threadIdx.x; k < a.nzruns * PN_LSLICES; k += blockDim.x) a.zcount[k * PN_LSTRIDE] = 0u;
+    finalize_tile_block(a.ctl, a.part_dt, a.part_bp, a.part_dv, a.part_bc, npart, slots, q, zre, cur);
 }
 
 FusedArgs make_args(pennant_problem* pb) {
@@ -3187,14 +3149,14 @@ k_tile_batch(BatchArgs B, TileBatch t) {
     a.q1 = uni(a.q1); a.q2 = uni(a.q2); a.cfl = uni(a.cfl);
     const double dt = uni(c->dt);
     ClCount none;
-    (void)tile_body<T, CL_EXACT>(a, t.o, g, U.i0, U.j0, in, U.slot, dt, c->zre_valid != 0, none);
+    (void)tile_body<T, CL_EXACT>(a, t.o, g, U.i0, U.j0, in, {nullptr, U.slot}, dt, c->zre_valid != 0, none);
 }
 
 __global__ void __launch_bounds__(PN_FIN_BLOCK) k_finalize_batch_tile(BatchArgs B, int zre, int cur) {
     const BProb& q = B.probs[blockIdx.x];
-    finalize_tile_block<PN_FIN_BLOCK>(B.ctls + blockIdx.x, B.a.part_dt + q.tbeg, B.a.part_bp + q.tbeg,
-                                      B.a.part_dv + q.tbeg, B.a.part_bc + q.tbeg, q.tend - q.tbeg, q.cflv, q.cstop,
-                                      q.dtmax, q.dtfac, q.tstop, zre, cur);
+    finalize_tile_block(B.ctls + blockIdx.x, B.a.part_dt + q.tbeg, B.a.part_bp + q.tbeg, B.a.part_dv + q.tbeg,
+                        B.a.part_bc + q.tbeg, q.tend - q.tbeg, nullptr, {q.cflv, q.dtmax, q.dtfac, q.tstop, q.cstop},
+                        zre, cur);
 }
 
 // k_zre over the units of every problem whose flag is clear.
@@ -3420,8 +3382,9 @@ int launch_learned_pass(const pennant_problem* pb, const FusedArgs& a, bool pend
 
 }  // namespace
 
-int launch_cycle_points(pennant_problem* pb) {
-    const FusedArgs a = make_args(pb);
+int launch_cycle_points(pennant_problem* pb, Ctl* ctl) {
+    FusedArgs a = make_args(pb);
+    a.ctl = ctl;
     const TaskPoints t = {pb->vv("px0"), pb->vv("pu0"), pb->vv("pxp"), pb->vv("pf"), pb->vv("pap"), pb->f("pmaswt")};
     const int nb = pb->nheavy + nblocks(own_points(pb));
     if (nb > 0) hipLaunchKernelGGL(k_cycle_points, dim3(nb), dim3(PN_BLOCK), 0, pb->stream, a, t);
@@ -3488,13 +3451,6 @@ int fused_cycle(pennant_problem* pb, hipEvent_t* ev, int form) {
 }
 
 namespace {
-
-DtParams dt_params(const pennant_problem* pb) {
-    const Params& q = pb->prm;
-    DtParams d;
-    d.cflv = q.cflv; d.dtmax = q.dtmax; d.dtfac = q.dtfac; d.tstop = q.tstop; d.cstop = q.cstop;
-    return d;
-}
 
 // Predictor launches of the pipelined cycle (the prologue's, or with REDO
 // the redo), writing zp to zpn; returns the number of partials.
@@ -3623,7 +3579,6 @@ TileArgs tile_args(const pennant_problem* pb, int second, FusedArgs& a) {
     t.ntiles = t.ntx * ((q.nzy - q.pie + PN_TIN - 1) / PN_TIN);
     t.back = second;
     t.list = q.list;
-    t.nlist = q.nlist;
     a.part_dt = q.part_d;
     a.part_dv = q.part_d + q.npart;
     a.part_bp = q.part_i;
@@ -3633,52 +3588,66 @@ TileArgs tile_args(const pennant_problem* pb, int second, FusedArgs& a) {
 
 }  // namespace
 
-int tile_cycle(pennant_problem* pb, int form, int second) {
-    if (!pb->tile.nzx || (form == FORM_LEARNED && !pb->closure)) return PENNANT_EINVAL;
+template <bool LINK>
+static void launch_tiles(const FusedArgs& a, const TileArgs& t, int blocks, int form, hipStream_t s) {
+    const dim3 grid(blocks), blk(PN_BLOCK);
+    if (form == FORM_FP64)
+        hipLaunchKernelGGL((k_tile<double, CL_EXACT, LINK>), grid, blk, 0, s, a, t);
+    else if (form == FORM_MIXED)
+        hipLaunchKernelGGL((k_tile<float, CL_EXACT, LINK>), grid, blk, 0, s, a, t);
+    else {
+        hipLaunchKernelGGL((k_tile<float, CL_FLAG, LINK>), grid, blk, 0, s, a, t);
+        hipLaunchKernelGGL(k_tile_list, dim3(t.ntiles < 512 ? t.ntiles : 512), blk, 0, s, a, t);
+    }
+}
+
+// Cycle k of n.  Linked cycles are a chain: each tile kernel ends the cycle
+// before it by itself, one block more writes the control block, and the last
+// is ended when the run of n is.
+static int tile_cycle(pennant_problem* pb, int form, int k, bool linked) {
+    const int second = k & 1, zre = form == FORM_FP64 ? 1 : 0;
     FusedArgs a = make_args(pb);
     FusedArgs tri = a;                       // the triangles' own state stays in the problem's arrays
     TileArgs t = tile_args(pb, second, a);
     hipStream_t s = pb->stream;
-    const dim3 blk(PN_BLOCK);
+    t.linked = linked ? 1 : 0;
+    t.step = chain_step(pb, pb->tile.chain, linked ? k : 0, zre);
+    t.nlist = pb->tile.nlist + (linked ? k & 1 : 0);
+    t.nlist_clear = pb->tile.nlist + ((k + 1) & 1);
+    if (linked) {
+        launch_tiles<true>(a, t, t.ntiles + 1, form, s);
+        return (int)hipGetLastError();
+    }
     const int nt = t.g.pie ? t.g.nzx : 0;    // triangles
-    int npred = 0, ncorr = 0;
+    int npart = 0;
     tri.part_dt = a.part_dt; tri.part_dv = a.part_dv; tri.part_bp = a.part_bp; tri.part_bc = a.part_bc;
     if (nt) {
         tri.pxx = a.pxx; tri.pxy = a.pxy; tri.pux = a.pux; tri.puy = a.puy;
         launch_pred<3>(pb, tri, 0, nt, 0, 0, form, 0, s);
-        npred = pred_grid(pb, nt, 3, form);
-        ncorr = corr_grid(pb, nt);
-        if (form == FORM_LEARNED) {
-            const dim3 g(npred < 512 ? npred : 512);
-            hipLaunchKernelGGL(k_pred_list<3>, g, blk, 0, s, tri, 0, nt, 0, 0);
-        }
+        // one partial index per block of both halves
+        npart = pred_grid(pb, nt, 3, form);
+        if (npart != corr_grid(pb, nt)) return PENNANT_EINVAL;
+        if (form == FORM_LEARNED)
+            hipLaunchKernelGGL(k_pred_list<3>, dim3(npart < 512 ? npart : 512), dim3(PN_BLOCK), 0, s, tri, 0, nt, 0, 0);
     }
-    // one partial index per tile for both halves
-    t.poff = npred > ncorr ? npred : ncorr;
-    const dim3 grid(t.ntiles + (nt ? 1 : 0));
-    if (form == FORM_FP64)
-        hipLaunchKernelGGL((k_tile<double, CL_EXACT>), grid, blk, 0, s, a, t);
-    else if (form == FORM_MIXED)
-        hipLaunchKernelGGL((k_tile<float, CL_EXACT>), grid, blk, 0, s, a, t);
-    else {
-        hipLaunchKernelGGL((k_tile<float, CL_FLAG>), grid, blk, 0, s, a, t);
-        hipLaunchKernelGGL(k_tile_list, dim3(t.ntiles < 512 ? t.ntiles : 512), blk, 0, s, a, t);
-    }
+    launch_tiles<false>(a, t, t.ntiles + (nt ? 1 : 0), form, s);
     if (nt) {
         tri.pxx = a.oxx; tri.pxy = a.oxy; tri.pux = a.oux; tri.puy = a.ouy;
         launch_corr<3>(pb, tri, 0, nt, 0, 0, form, s);
     }
-    // the triangles' launches use equal grids, so no partial lies between
-    // theirs and the tiles'
-    if (npred != ncorr) return PENNANT_EINVAL;
-    const int np = t.poff + t.ntiles, zre = form == FORM_FP64 ? 1 : 0, cur = second ? 0 : 1;
-    int* nlist = form == FORM_LEARNED ? t.nlist : nullptr;
-    if (np <= PN_FIN_PER * PN_FIN_BLOCK)
-        hipLaunchKernelGGL(k_finalize_tile<PN_FIN_BLOCK>, dim3(1), dim3(PN_FIN_BLOCK), 0, s, a, np, dt_params(pb),
-                           zre, cur, nlist);
-    else
-        hipLaunchKernelGGL(k_finalize_tile<1024>, dim3(1), dim3(1024), 0, s, a, np, dt_params(pb), zre, cur, nlist);
+    hipLaunchKernelGGL(k_finalize_tile, dim3(1), dim3(npart ? PN_FIN_BLOCK : 64), 0, s, a, npart, t.step.put, t.step.q, zre,
+                       second ? 0 : 1, form == FORM_LEARNED ? t.nlist : nullptr);
     return (int)hipGetLastError();
+}
+
+int tile_cycles(pennant_problem* pb, int form, int n) {
+    const TileState& q = pb->tile;
+    if (!q.nzx || (n & 1) || (form == FORM_LEARNED && !pb->closure)) return PENNANT_EINVAL;
+    const int64_t tiles = (int64_t)((q.nzx + PN_TIN - 1) / PN_TIN) * ((q.nzy - q.pie + PN_TIN - 1) / PN_TIN);
+    const bool linked = n > 0 && !q.pie && tiles <= PN_LINK_TILES;
+    for (int k = 0; k < n; ++k)
+        if (const int rc = tile_cycle(pb, form, k, linked)) return rc;
+    return linked ? chain_end(pb, q.chain, n, form == FORM_FP64 ? 1 : 0) : 0;
 }
 
 // Whether the mesh is one the tile cycle takes: a rect (rect_detect has
@@ -3710,12 +3679,14 @@ int tile_setup(pennant_problem* pb) {
     }
     const int64_t tiles = ((nzx + PN_TIN - 1) / PN_TIN) * ((nzy - pie + PN_TIN - 1) / PN_TIN);
     const int64_t P = h.nump, Z = h.numz;
-    q.npart = (int)tiles + PN_MAX_GRID;
-    const size_t bytes = (size_t)(4 * P + 5 * Z + 2 * (int64_t)q.npart) * 8 + (size_t)(2 * (int64_t)q.npart + tiles + 1) * 4;
+    q.npart = pie ? PN_MAX_GRID : 0;         // the triangles'
+    const size_t bytes = PN_CHAIN_BYTES + (size_t)(4 * P + 5 * Z + 2 * (int64_t)q.npart) * 8 +
+                         (size_t)(2 * (int64_t)q.npart + tiles + 2) * 4;
     char* m = nullptr;
     if (hipMalloc((void**)&m, bytes) != hipSuccess) return (int)hipErrorOutOfMemory;
     pb->allocs.push_back(m);
-    double* d = (double*)m;
+    q.chain = m;
+    double* d = (double*)(m + PN_CHAIN_BYTES);
     for (int k = 0; k < 9; ++k) {
         q.alt[k] = d;
         d += k < 4 ? P : Z;
@@ -3723,8 +3694,9 @@ int tile_setup(pennant_problem* pb) {
     q.part_d = d;
     q.part_i = (int*)(d + 2 * (int64_t)q.npart);
     q.nlist = q.part_i + 2 * (int64_t)q.npart;
-    q.list = q.nlist + 1;
-    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, pb->stream, (unsigned*)q.nlist, 1);
+    q.list = q.nlist + 2;
+    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, pb->stream, (unsigned*)q.nlist, 2);
+    hipLaunchKernelGGL(k_chain_begin, dim3(1), dim3(64), 0, pb->stream, chain_sets(q.chain));
     q.nzx = (int)nzx;
     q.nzy = (int)nzy;
     q.pie = pie ? 1 : 0;

@@ -93,7 +93,8 @@ struct DevField {
 struct TileState {
     int nzx = 0, nzy = 0, pie = 0;
     double* alt[9] = {};
-    double* part_d = nullptr;
+    void* chain = nullptr;       // slots and the second control block of a chain (cycle_end.h)
+    double* part_d = nullptr;    // the triangles' partials
     int* part_i = nullptr;
     int npart = 0;
     int* list = nullptr;
@@ -287,10 +288,10 @@ int fused_cycle(pennant_problem* pb, hipEvent_t* ev, int form);
 // ev: NULL, or 5 events recorded before K2, the zone pass, K4 and the redo,
 // the learned pass, and after it
 int fused_prologue(pennant_problem* pb, int form);
-// Tile cycle of a structured mesh: cycle `second` (0, 1) of a pair.  The
-// state is in the problem's own arrays before and after every pair.
+// Tile cycles of a structured mesh, an even number n of them.  The state is in
+// the problem's own arrays before and after.
 int tile_setup(pennant_problem* pb);
-int tile_cycle(pennant_problem* pb, int form, int second);
+int tile_cycles(pennant_problem* pb, int form, int n);
 int fused_cycle_pipe(pennant_problem* pb, hipEvent_t* ev, int form);
 // Stores zr = zm / zvol and ze = zetot / (zm + 1e-99) where mixed cycles left
 // them to be derived (the mixed corrector does not store them).
@@ -309,24 +310,13 @@ int launch_first_dt(pennant_problem* pb);
 // doCycle's copies and fills (src/Hydro.cc:361-368,389-418) for its steps one
 // at a time: zvol0 = zvol; px0 = px, pu0 = pu, pmaswt = 0, pf = 0
 int launch_copy_zvol0(pennant_problem* pb);
-// A task-mode cycle, every task's fields written, in four launches
-// (task_kernels.hip), and its end: the folds of the zone kernels' block
-// partials, calcDt and the end-of-cycle update (driver_kernels.hip).  The
-// partials of nb blocks lie in the reduction workspace.
-struct CycleParts {
-    double *dt, *dv;   // dt minima, dvol maxima
-    int *bp, *bc;      // bad sides of the predictor and the corrector
-};
-inline size_t cycle_parts_bytes(int nb) { return (size_t)nb * (2 * sizeof(double) + 2 * sizeof(int)); }
-inline CycleParts cycle_parts(void* ws, int nb) {
-    double* d = static_cast<double*>(ws);
-    int* i = reinterpret_cast<int*>(d + 2 * (size_t)nb);
-    return {d, d + nb, i, i + nb};
-}
-int cycle_blocks(const pennant_mesh* m);
-int launch_task_cycle(pennant_problem* pb);
-int launch_cycle_points(pennant_problem* pb);   // its point pass (fused.hip)
-int launch_task_end(pennant_problem* pb, const CycleParts& part, int nb);
+// n task-mode cycles, every task's fields written each (task_kernels.hip); they
+// keep their slots and second control block behind the reduction workspace
+// (task_chain_setup, at creation).
+size_t task_chain_bytes();
+int task_chain_setup(pennant_problem* pb);
+int launch_task_cycles(pennant_problem* pb, int n);
+int launch_cycle_points(pennant_problem* pb, Ctl* ctl);   // a cycle's point pass (fused.hip)
 int launch_point_begin(pennant_problem* pb);
 // Multi-piece runs (pieces.cpp, fused.hip): per-piece device pointers the
 // exchange kernels use, and one exchange entry (element src of piece sp to

@@ -39,6 +39,7 @@
 #include <stdint.h>
 
 #include "common.h"
+#include "cycle_end.h"
 #include "problem.h"
 #include "reduce.h"
 
@@ -201,13 +202,14 @@ __device__ __forceinline__ double tts_sdp(double sarea, double smf, double zarea
 // QCS::setCornerDivTask for the corner at a side's first point (position
 // xp0, velocity up0): xp1 and xp3 are the midpoints of this side and the one
 // before, up1 and up3 their velocities, de2 and de1 their lengths; xp2, up2
-// the zone's centre and velocity.
+// the zone's centre and velocity.  Each result goes to out as it is known (a
+// CornerDiv keeps them).
 struct CornerDiv {
     double area, cos, div, evol, du;
 };
-__device__ __forceinline__ CornerDiv corner_div(d2 xp0, d2 xp1, d2 xp2, d2 xp3, d2 up0, d2 up1,
-                                                d2 up2, d2 up3, double de1, double de2) {
-    CornerDiv o;
+template <class Out>
+__device__ __forceinline__ void corner_div(d2 xp0, d2 xp1, d2 xp2, d2 xp3, d2 up0, d2 up1, d2 up2,
+                                           d2 up3, double de1, double de2, Out&& o) {
     const double cvolume = 0.5 * cross(sub(xp2, xp0), sub(xp3, xp1));
     o.area = cvolume;
     const d2 v1 = sub(xp3, xp0);
@@ -234,8 +236,11 @@ __device__ __forceinline__ CornerDiv corner_div(d2 xp0, d2 xp1, d2 xp2, d2 xp3, 
     const double du = __builtin_sqrt(smax(dv1, dv2));
     o.evol = (div < 0.0 ? evol : 0.);
     o.du = (div < 0.0 ? du : 0.);
-    return o;
 }
+// A CornerDiv in the tasks' arrays
+struct CornerRefs {
+    double &area, &cos, &div, &evol, &du;
+};
 
 // QCS::setQCnForceTask's viscosity of a corner
 __device__ __forceinline__ double corner_mu(double cdu, double cevol, double cdiv, double zrp,
@@ -1063,12 +1068,8 @@ __global__ void __launch_bounds__(PN_TB) k_set_corner_div(pennant_mesh m, int tz
         const int cc = t.s0 + i;
         const d2 up1 = scl(0.5, add(u[j], u1[in]));
         const d2 up3 = scl(0.5, add(u1[ip], u[j]));
-        const CornerDiv o = corner_div(x[j], e[j], zxl[c.zi], e1[ip], u[j], up1, zul[c.zi], up3, el[ip], l[j]);
-        carea[cc] = o.area;
-        ccos[cc] = o.cos;
-        cdiv[cc] = o.div;
-        cevol[cc] = o.evol;
-        cdu[cc] = o.du;
+        corner_div(x[j], e[j], zxl[c.zi], e1[ip], u[j], up1, zul[c.zi], up3, el[ip], l[j],
+                   CornerRefs{carea[cc], ccos[cc], cdiv[cc], cevol[cc], cdu[cc]});
     }
 }
 
@@ -1247,24 +1248,26 @@ __global__ void __launch_bounds__(PN_BLOCK) k_apply_fixed_bc(const int32_t* mapb
 // ---------------------------------------------------------------------------
 // A task-mode cycle of the driver
 //
-// Steps 0 to 29 of doCycle in four launches, every task's fields in memory as
+// Steps 0 to 29 of doCycle in three launches, every task's fields in memory as
 // the tasks leave them.  One launch per task moves 688 bytes a side, 536 a
 // zone and 512 a point, most of them fields that the task before has just
 // written; here the tasks that follow each other on the same zones or points
 // share a kernel and pass those on in registers and LDS, which leaves what has
 // to be written and the first reads: about 360, 290 and 220 bytes.  The task
 // entry points stay one kernel a task.  Bound by those bytes on large meshes
-// (Sedov 1440^2: 1466 -> 753 us a cycle, 5.1 TB/s), by the four launches'
-// latencies on small ones (97 x 61: 111 -> 21 us).
+// (Sedov 1440^2: 1466 -> 750 us a cycle, 5.1 TB/s), by the launches' latencies
+// on small ones (97 x 61: 111 -> 18 us).
 //
-//   k_cycle_pred    zones: steps 0, 2-7, 9-15 and 26's block minima, with the
-//                   half-step positions computed from px and pu; also each
-//                   corner's force and mass in its corner slot, so that the
-//                   point pass reads them coalesced
+//   k_cycle_pred    zones: steps 0, 2-7, 9-15 and 26, with the half-step
+//                   positions computed from px and pu; also each corner's
+//                   force and mass in its corner slot, so that the point pass
+//                   reads them coalesced
 //   k_cycle_points  points: steps 1, 8, 16, 17, 19 (fused.hip)
-//   k_cycle_corr    zones: steps 20-25 and 27's block maxima
-//   end             the folds of 26 and 27, 28 and the end of the cycle
-//                   (driver_kernels.hip)
+//   k_cycle_corr    zones: steps 20-25 and 27
+//
+// Steps 26 and 27 go into slots, and the next cycle's first kernel does 28 and
+// the end of the cycle from them (cycle_now); on meshes of many tiles, where
+// each would pay for it, one wave does it between the cycles (PN_LINK_TASKS).
 //
 // Sums, minima and maxima are formed as in the tasks' kernels, in the same
 // order: the same bits.  The fields are the driver's own (two arrays per
@@ -1272,7 +1275,9 @@ __global__ void __launch_bounds__(PN_BLOCK) k_apply_fixed_bc(const int32_t* mapb
 struct CycleArgs {
     pennant_mesh m;
     int tz;
-    const Ctl* ctl;              // dt, and whether the run has stopped: then nothing is done
+    CycleStep step;              // the cycle's dt, and whether the run has stopped: then nothing is done
+    int linked;
+    const Ctl* ctl;              // the same for the cycle's later kernels
     double gamma, ssmin, alfa, qgamma, q1, q2, cfl;
     pennant_cvec px, pu, pu0, pxp;
     // zones
@@ -1286,7 +1291,6 @@ struct CycleArgs {
     const double* smf;
     const int32_t* pcpos;        // corner slots, and the corners' values there
     double *cfx, *cfy, *cmass;
-    CycleParts part;
 };
 using V = VIO<VL_SOA>;
 // The zone kernels' fields pass through memory once a kernel and are too many
@@ -1299,6 +1303,10 @@ __device__ __forceinline__ void put(const pennant_vec& a, int64_t i, d2 v) {
     put(a.y, i, v.y);
 }
 
+// Most tiles of linked cycles.  Linked and not, us a cycle: 16^2 16.8 and 17.9,
+// 97 x 61 (93 tiles) 17.8 and 18.9, 200^2 (625) 26.8 and 27.9, 333 x 217 (1130)
+// 46.3 and 45.3, 1440^2 780 and 750.
+#define PN_LINK_TASKS 1024
 #define PN_CYC_TZ (PN_TB / 3 + 1)     // most zones of a tile of one side per thread
 
 __device__ __forceinline__ double get(const double* a, int64_t i) { return __builtin_nontemporal_load(a + i); }
@@ -1321,7 +1329,12 @@ __device__ __forceinline__ CycSide cyc_side(const Tile& t, const int* zsb, const
 __global__ void __launch_bounds__(PN_TB) k_cycle_pred(CycleArgs a) {
     const pennant_mesh& m = a.m;
     const int tz = a.tz;
-    if (a.ctl->done) return;
+    if (a.linked && blockIdx.x == gridDim.x - 1) {
+        cycle_step(a.step);
+        return;
+    }
+    const CycleNow now = cycle_now(a.step);
+    if (now.done) return;
     PN_WIDE_SHARED(1);
     // later x1, e1, sa_ and sv_ hold cqe1, cqe2, cw and ccos, dl_ the side
     // fractions and u1 the sides' forces
@@ -1329,7 +1342,7 @@ __global__ void __launch_bounds__(PN_TB) k_cycle_pred(CycleArgs a) {
     __shared__ double el[PN_TB], sa_[PN_TB], sv_[PN_TB], dl_[PN_TB], dux_[PN_TB];
     __shared__ d2 zxl[PN_CYC_TZ], zul[PN_CYC_TZ];
     __shared__ double zal[PN_CYC_TZ], zrl[PN_CYC_TZ], zpl[PN_CYC_TZ], zsl[PN_CYC_TZ];
-    const double dth = 0.5 * a.ctl->dt;
+    const double dth = 0.5 * now.dt;
     const int z = t.z0 + lane;
     const bool on = lane < t.ns;
     const CycSide d = cyc_side(t, zsb, zof, lane);
@@ -1386,7 +1399,7 @@ __global__ void __launch_bounds__(PN_TB) k_cycle_pred(CycleArgs a) {
     CornerDiv cd;
     {
         const d2 up1 = scl(0.5, add(u, u1[d.next])), up3 = scl(0.5, add(u1[d.prev], u));
-        cd = corner_div(x, e, zx, e1[d.prev], u, up1, zul[d.c.zi], up3, el[d.prev], l);
+        corner_div(x, e, zx, e1[d.prev], u, up1, zul[d.c.zi], up3, el[d.prev], l, cd);
     }
     if (on) {
         const double fac = (d.c.n == 3 ? 3. : 4.);
@@ -1476,10 +1489,7 @@ __global__ void __launch_bounds__(PN_TB) k_cycle_pred(CycleArgs a) {
     }
     dtm = block_min(dtm);
     bad = block_sum(bad);
-    if (threadIdx.x == 0) {
-        a.part.dt[blockIdx.x] = dtm;
-        a.part.bp[blockIdx.x] = bad;
-    }
+    if (threadIdx.x == 0) slots_dt(a.step.put, blockIdx.x, dtm, bad);
 }
 
 __global__ void __launch_bounds__(PN_TB) k_cycle_corr(CycleArgs a) {
@@ -1558,10 +1568,7 @@ __global__ void __launch_bounds__(PN_TB) k_cycle_corr(CycleArgs a) {
     }
     dvov = block_max(dvov);
     bad = block_sum(bad);
-    if (threadIdx.x == 0) {
-        a.part.dv[blockIdx.x] = dvov;
-        a.part.bc[blockIdx.x] = bad;
-    }
+    if (threadIdx.x == 0) slots_dv(a.step.put, blockIdx.x, dvov, bad);
 }
 
 // ---------------------------------------------------------------------------
@@ -1921,19 +1928,26 @@ int pennant_hip_apply_fixed_bc(const int32_t* mapbp, int32_t numb, double vfix_x
 
 namespace pn {
 
-int cycle_blocks(const pennant_mesh* m) {
-    const int tz = wide_tile_zones(m, 1);
-    return tz ? tile_blocks(m, tz) : 0;
+size_t task_chain_bytes() { return PN_CHAIN_BYTES; }
+
+static void* task_chain(pennant_problem* pb) {
+    return static_cast<char*>(pb->ws) + pennant_hip_reduce_workspace_bytes();
 }
 
-int launch_task_cycle(pennant_problem* pb) {
+int task_chain_setup(pennant_problem* pb) {
+    hipLaunchKernelGGL(k_chain_begin, dim3(1), dim3(64), 0, pb->stream, chain_sets(task_chain(pb)));
+    return launch_status();
+}
+
+int launch_task_cycles(pennant_problem* pb, int n) {
+    if (n < 1) return 0;
     const pennant_mesh& m = pb->dm;
     const Params& q = pb->prm;
-    const int nb = cycle_blocks(&m);
+    const int tz = wide_tile_zones(&m, 1), nb = tz ? tile_blocks(&m, tz) : 0;
     CycleArgs a;
     a.m = m;
-    a.tz = wide_tile_zones(&m, 1);
-    a.ctl = pb->ctl;
+    a.tz = tz;
+    a.linked = (nb > 0 && nb <= PN_LINK_TASKS) ? 1 : 0;
     a.gamma = q.gamma; a.ssmin = q.ssmin; a.alfa = q.alfa; a.qgamma = q.qgamma;
     a.q1 = q.q1; a.q2 = q.q2; a.cfl = q.cfl;
     a.px = pb->cv("px"); a.pu = pb->cv("pu"); a.pu0 = pb->cv("pu0"); a.pxp = pb->cv("pxp");
@@ -1954,12 +1968,19 @@ int launch_task_cycle(pennant_problem* pb) {
     for (const auto& e : vals) *e.d = pb->f(e.name);
     a.zm = pb->f("zm");
     a.smf = pb->f("smf");
-    a.part = cycle_parts(pb->ws, nb);
-    if (nb > 0) hipLaunchKernelGGL(k_cycle_pred, dim3(nb), dim3(PN_TB), 0, pb->stream, a);
-    if (const int rc = launch_cycle_points(pb)) return rc;
-    if (nb > 0) hipLaunchKernelGGL(k_cycle_corr, dim3(nb), dim3(PN_TB), 0, pb->stream, a);
-    if (const int rc = launch_status()) return rc;
-    return launch_task_end(pb, a.part, nb);
+    // the driver's zr and ze are current (materialize_zre): zre stays 1
+    for (int k = 0; k < n; ++k) {
+        a.step = chain_step(pb, task_chain(pb), a.linked ? k : 0, 1);
+        Ctl* ctl = a.linked ? a.step.out : pb->ctl;
+        a.ctl = ctl;
+        if (nb > 0) hipLaunchKernelGGL(k_cycle_pred, dim3(nb + a.linked), dim3(PN_TB), 0, pb->stream, a);
+        if (const int rc = launch_cycle_points(pb, ctl)) return rc;
+        if (nb > 0) hipLaunchKernelGGL(k_cycle_corr, dim3(nb), dim3(PN_TB), 0, pb->stream, a);
+        if (const int rc = launch_status()) return rc;
+        if (!a.linked)
+            if (const int rc = chain_end(pb, task_chain(pb), 0, 1)) return rc;
+    }
+    return a.linked ? chain_end(pb, task_chain(pb), n, 1) : 0;
 }
 
 }  // namespace pn
