@@ -43,6 +43,7 @@
 // one partial per reduction (no same-address atomics on the hot path).  The
 // host launches K1 and K3 once per run of consecutive zones with equal side
 // count (rect: one run of quads; pie: triangles, then quads).
+#include <algorithm>
 #include <cstring>
 
 #include "closure.h"
@@ -3296,8 +3297,10 @@ int fused_setup(pennant_problem* pb) {
         return p;
     };
     const size_t S = h.nums, P = h.nump;
-    if (!corner_slots_fit((int64_t)P, (int64_t)S)) return PENNANT_EINVAL;
-    const size_t NC = (size_t)corner_slots((int64_t)P, (int64_t)S);
+    // (a piece's master points list other pieces' corners too: more than its sides)
+    const int64_t K = std::max((int64_t)S, (int64_t)h.pcside.size());
+    if (!corner_slots_fit((int64_t)P, K)) return PENNANT_EINVAL;
+    const size_t NC = (size_t)corner_slots((int64_t)P, K);
     pb->cfx = (double*)al(NC, 8); pb->cfy = (double*)al(NC, 8); pb->cmass = (double*)al(NC, 8);
     pb->sfwx = (double*)al(S, 8); pb->sfwy = (double*)al(S, 8);
     pb->vs2 = (double*)al(2 * P, 8); pb->pxpx = (double*)al(P, 8);

@@ -50,14 +50,15 @@ struct Ctl {
 // corner-major, c * nump + p: neighbouring zones write the records of
 // neighbouring points at one position, and neighbouring points read them,
 // so both sides touch whole cache lines.  Later positions (points with more
-// than four corners) take 4 * nump + k.  A mesh needs corner_slots() slots.
+// than four corners) take 4 * nump + k.  A mesh needs corner_slots() slots for
+// the entries of its corner lists (a whole mesh: its sides).
 inline int64_t corner_slot(int64_t nump, int64_t p, int64_t c, int64_t k) {
     return c < 4 ? c * nump + p : 4 * nump + k;
 }
-inline int64_t corner_slots(int64_t nump, int64_t nums) { return 4 * nump + nums; }
+inline int64_t corner_slots(int64_t nump, int64_t entries) { return 4 * nump + entries; }
 // The kernels index FP32 corner records {fx, fy, mass} as 3 * slot + j in int.
-inline bool corner_slots_fit(int64_t nump, int64_t nums) {
-    return 3 * corner_slots(nump, nums) < (int64_t)0x7fffffff;
+inline bool corner_slots_fit(int64_t nump, int64_t entries) {
+    return 3 * corner_slots(nump, entries) < (int64_t)0x7fffffff;
 }
 #define PN_HEAVY 64        // points with more corners get a whole block in K2
 
