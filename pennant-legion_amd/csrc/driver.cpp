@@ -201,15 +201,38 @@ void build_mesh(const Params& q, HostMesh& h) {
 
 }  // namespace pn
 
+// A problem has about a hundred arrays, and an allocation, a fill and a release
+// of each are most of what creating and destroying a small one takes: those of
+// a problem below PN_ARENA_MAX come from one allocation (arena_begin).  A larger
+// one's each have their own, as what the arena has no room for.  45^2 zones: 1050
+// -> 650 us to create and 150 -> 105 to destroy; 180^2: 2500 -> 1300 and 3600 ->
+// 100.
+#define PN_ARENA_MAX ((size_t)512 << 20)
+#define PN_ARENA_ALIGN 256
+
+static bool zeroed(pennant_problem* pb, size_t bytes, char** out) {
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) return false;
+    if (hipMemset(p, 0, bytes) != hipSuccess) { (void)hipFree(p); return false; }
+    pb->allocs.push_back(p);
+    *out = static_cast<char*>(p);
+    return true;
+}
+
+void* pn::problem_alloc(pennant_problem* pb, size_t bytes) {
+    const size_t n = (bytes + PN_ARENA_ALIGN - 1) / PN_ARENA_ALIGN * PN_ARENA_ALIGN;
+    if (n > 0 && n <= pb->arena_size - pb->arena_used) {
+        pb->arena_used += n;
+        return pb->arena + pb->arena_used - n;
+    }
+    char* p = nullptr;
+    return zeroed(pb, bytes > 0 ? bytes : 8, &p) ? p : nullptr;
+}
+
 namespace {
 
 template <class T> T* dalloc(pennant_problem* pb, size_t n) {
-    void* p = nullptr;
-    const size_t bytes = n * sizeof(T) > 0 ? n * sizeof(T) : sizeof(T);
-    if (hipMalloc(&p, bytes) != hipSuccess) return nullptr;
-    if (hipMemset(p, 0, bytes) != hipSuccess) { (void)hipFree(p); return nullptr; }
-    pb->allocs.push_back(p);
-    return static_cast<T*>(p);
+    return static_cast<T*>(problem_alloc(pb, n * sizeof(T)));
 }
 
 template <class T> T* upload(pennant_problem* pb, const std::vector<T>& v) {
@@ -236,6 +259,20 @@ const FieldSpec kFields[] = {
 
 int64_t count_of(const pennant_problem* pb, int kind) {
     return kind == 0 ? pb->dm.nump : (kind == 1 ? pb->dm.numz : pb->dm.nums);
+}
+
+// The arena of a small problem, from what its fields, maps, fused and tile
+// cycles take (too small an estimate costs allocations, nothing else).
+bool arena_begin(pennant_problem* pb) {
+    const size_t P = pb->dm.nump, Z = pb->dm.numz, S = pb->dm.nums, C = (size_t)corner_slots((int64_t)P, (int64_t)S);
+    size_t n = 24 * S + 12 * Z + 4 * P                       // maps
+               + 36 * C + 32 * S + 32 * P + 16 * Z           // corner records, side forces, point values, lists
+               + 32 * P + 42 * Z                             // the tile cycle's second state
+               + ((size_t)512 << 10);                        // partials, workspaces, rounding
+    for (const FieldSpec& fs : kFields) n += (size_t)fs.ncomp * count_of(pb, fs.kind) * sizeof(double);
+    if (n > PN_ARENA_MAX) return true;
+    pb->arena_size = n;
+    return zeroed(pb, n, &pb->arena);
 }
 
 #define CK(x) do { int _e = (int)(x); if (_e) return _e; } while (0)
@@ -388,6 +425,7 @@ pennant_problem* pn::create_problem(const Params& prm, HostMesh&& hm, int npown,
 
     pennant_mesh& m = pb->dm;
     m.nump = h.nump; m.numz = h.numz; m.nums = h.nums; m.maxznump = h.maxznump;
+    if (!arena_begin(pb)) return fail("device allocation failed");
     m.mapsp1 = upload(pb, h.mapsp1); m.mapsp2 = upload(pb, h.mapsp2); m.mapsz = upload(pb, h.mapsz);
     m.mapss3 = upload(pb, h.mapss3); m.mapss4 = upload(pb, h.mapss4); m.znump = upload(pb, h.znump);
     m.zsbeg = upload(pb, h.zsbeg); m.pcbeg = upload(pb, h.pcbeg); m.pcside = upload(pb, h.pcside);

@@ -3289,13 +3289,7 @@ int fused_setup(pennant_problem* pb) {
     std::vector<int> heavy;
     for (int p = 0; p < own_points(pb); ++p)
         if (h.pcbeg[p + 1] - h.pcbeg[p] > PN_HEAVY) heavy.push_back(p);
-    auto al = [&](size_t n, size_t sz) -> void* {
-        void* p = nullptr;
-        if (hipMalloc(&p, n * sz > 0 ? n * sz : sz) != hipSuccess) return nullptr;
-        if (hipMemset(p, 0, n * sz > 0 ? n * sz : sz) != hipSuccess) { (void)hipFree(p); return nullptr; }
-        pb->allocs.push_back(p);
-        return p;
-    };
+    auto al = [&](size_t n, size_t sz) -> void* { return problem_alloc(pb, n * sz); };
     const size_t S = h.nums, P = h.nump;
     // (a piece's master points list other pieces' corners too: more than its sides)
     const int64_t K = std::max((int64_t)S, (int64_t)h.pcside.size());
@@ -3685,9 +3679,8 @@ int tile_setup(pennant_problem* pb) {
     q.npart = pie ? PN_MAX_GRID : 0;         // the triangles'
     const size_t bytes = PN_CHAIN_BYTES + (size_t)(4 * P + 5 * Z + 2 * (int64_t)q.npart) * 8 +
                          (size_t)(2 * (int64_t)q.npart + tiles + 2) * 4;
-    char* m = nullptr;
-    if (hipMalloc((void**)&m, bytes) != hipSuccess) return (int)hipErrorOutOfMemory;
-    pb->allocs.push_back(m);
+    char* m = (char*)problem_alloc(pb, bytes);
+    if (!m) return (int)hipErrorOutOfMemory;
     q.chain = m;
     double* d = (double*)(m + PN_CHAIN_BYTES);
     for (int k = 0; k < 9; ++k) {

@@ -122,6 +122,9 @@ struct pennant_problem {
     pn::HostMesh hm;
     pennant_mesh dm;                 // device pointers
     std::vector<void*> allocs;
+    // device memory of a small problem, given out in pieces (problem_alloc)
+    char* arena = nullptr;
+    size_t arena_size = 0, arena_used = 0;
     std::map<std::string, pn::DevField> fields;
     std::vector<pn::BCList> bcs;
     pn::Ctl* ctl = nullptr;          // device
@@ -183,6 +186,10 @@ struct pennant_problem {
 };
 
 namespace pn {
+// Zeroed device memory that lives as long as the problem (driver.cpp); NULL
+// when there is none.
+void* problem_alloc(pennant_problem* pb, size_t bytes);
+
 // Batched problems: zone units (at most PN_BLOCK zones of one side-count run
 // of one problem), point units (at most PN_BLOCK points of one problem),
 // heavy points and the per-problem parameters.
