@@ -213,17 +213,20 @@ __device__ __forceinline__ CycleNow cycle_now(const CycleStep& s) {
     }
     return n;
 }
-// The step's writes, by one block.
-__device__ __forceinline__ void cycle_step(const CycleStep& s) {
+// The step's writes, by one block.  back: the state, where the cycle before
+// ended the run, is in the second set of arrays and this one copies it back
+// (Ctl::cur).
+__device__ __forceinline__ void cycle_step(const CycleStep& s, int back = 0) {
     if (threadIdx.x < 64) {
         const CtlSnap v = snap_ctl(s.in);
         SlotFold f = {};
         if (s.prev) f = slots_fold(slots_load(s.prev));
         if (threadIdx.x == 0) {
             *s.out = *s.in;
+            s.out->cur = 0;
             if (s.prev && !v.done) {
                 s.out->zre_valid = s.zre;
-                end_cycle(s.out, v, f.mn, f.mx, f.bp, f.bc, s.q);
+                s.out->cur = end_cycle(s.out, v, f.mn, f.mx, f.bp, f.bc, s.q) && back;
             }
         }
     }
@@ -239,6 +242,7 @@ __device__ __forceinline__ void cycle_chain_end(Ctl* c, const Ctl* in, slot_t* s
         const SlotFold f = slots_fold(slots_load(sets + last * PN_SLOT_SET));
         if (threadIdx.x == 0) {
             if (c != in) *c = *in;
+            c->cur = 0;
             if (!v.done) {
                 c->zre_valid = zre;
                 end_cycle(c, v, f.mn, f.mx, f.bp, f.bc, q);

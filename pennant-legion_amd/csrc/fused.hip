@@ -2268,7 +2268,8 @@ __global__ void __launch_bounds__(PN_FIN_BLOCK) k_finalize_la(FusedArgs a, int n
 // ends the cycle from them by itself while its loads are under way (linked
 // cycles: no launch between two tile kernels).  With many tiles each would pay
 // for that, and one wave ends the cycle between the two: 3.5 us, where folding
-// an array of 10600 partials took 9.5.
+// an array of 10600 partials took 9.5.  On a pie the triangles' few blocks end
+// the cycle, whatever the number of tiles.
 //
 // The triangles of a pie's first row and the origin are not part of a tile:
 // their predictor and corrector run as in the separate passes, before and
@@ -2287,7 +2288,7 @@ __global__ void __launch_bounds__(PN_FIN_BLOCK) k_finalize_la(FusedArgs a, int n
 // offsets and one fold of both counts together took Sedov 1440^2 from 211 to
 // 205 us (FP64), 108.5 to 106.6 (mixed) and 154 to 149 (learned).
 // Per cycle, separate passes (for mixed and learned the pipelined ones) ->
-// tiles: FP64 Sedov 1440^2 306 -> 201 us, Noh pie 1024^2 178 -> 119 us; mixed
+// tiles: FP64 Sedov 1440^2 306 -> 201 us, Noh pie 1024^2 178 -> 115 us; mixed
 // LeBlanc 4096 x 256 87 -> 55 us, 333 x 217 23 -> 10.1 us; learned Sedov
 // 1440^2 176 -> 147 us; FP64 90^2 12.6 -> 10.1 us by the linking alone.  It was faster at every size, so
 // structured meshes always take it.
@@ -2716,6 +2717,50 @@ k_tile(FusedArgs a, TileArgs t) {
         else if (t.back && c->cur)
             tile_copy<T>(a, t.o, t.g, i0, j0);
     }
+}
+
+// The triangles of a pie's linked cycle, before and after its tiles: their
+// predictor, which also ends the cycle before (one block more writes the
+// control block), and their corrector.  A finalize of its own had taken 4.6 us
+// and a launch (Noh pie 1024^2 FP64 118.6 -> 114.7 us a
+// cycle, mixed 68 -> 64; 300^2 27.4 -> 24.4 and 20.9 -> 17.9).
+template <typename T>
+__global__ void __launch_bounds__(PN_BLOCK) k_tri_pred(FusedArgs a, CycleStep s, int nt, int back) {
+    if (blockIdx.x == gridDim.x - 1) {
+        cycle_step(s, back);
+        return;
+    }
+    const CycleNow now = cycle_now(s);
+    if (now.done) return;
+    const int z = blockIdx.x * PN_BLOCK + threadIdx.x;
+    double m = 1.e99;
+    int bad = 0;
+    if (z < nt) {
+        int pp[3];
+        load_pp<3>(a, 3 * z, pp);
+        const SideW sw = side_w(z, 0, nt, 0, 3);
+        ClCount cnt;
+        double v;
+        if constexpr (sizeof(T) == 8)
+            v = zone_pred<3>(a, z, 3 * z, sw, pp, now.dt, bad);
+        else
+            v = zone_pred_mixed<3, CL_EXACT>(a, z, 3 * z, sw, pp, now.dt, bad, true, cnt, now.zre != 0);
+        m = (v < m) ? v : m;
+    }
+    m = block_min(m);
+    bad = block_sum(bad);
+    if (threadIdx.x == 0) slots_dt(s.put, blockIdx.x, m, bad);
+}
+template <typename T>
+__global__ void __launch_bounds__(PN_BLOCK) k_tri_corr(FusedArgs a, CycleStep s, int nt) {
+    if (s.out->done) return;
+    const int z = blockIdx.x * PN_BLOCK + threadIdx.x;
+    double m = 1.e-99;
+    int bad = 0;
+    if (z < nt) corr_zone<3, T>(a, z, 3 * z, side_w(z, 0, nt, 0, 3), s.out->dt, bad, m);
+    m = block_max(m);
+    bad = block_sum(bad);
+    if (threadIdx.x == 0) slots_dv(s.put, blockIdx.x, m, bad);
 }
 
 // The learned form's tiles that have a zone for the network (in the ring or
@@ -3598,9 +3643,9 @@ static void launch_tiles(const FusedArgs& a, const TileArgs& t, int blocks, int 
     }
 }
 
-// Cycle k of n.  Linked cycles are a chain: each tile kernel ends the cycle
-// before it by itself, one block more writes the control block, and the last
-// is ended when the run of n is.
+// Cycle k of n.  Linked cycles are a chain: each ends the cycle before it by
+// itself (a rect's tile kernel, a pie's triangles' predictor), one block more
+// writes the control block, and the last is ended when the run of n is.
 static int tile_cycle(pennant_problem* pb, int form, int k, bool linked) {
     const int second = k & 1, zre = form == FORM_FP64 ? 1 : 0;
     FusedArgs a = make_args(pb);
@@ -3611,21 +3656,36 @@ static int tile_cycle(pennant_problem* pb, int form, int k, bool linked) {
     t.step = chain_step(pb, pb->tile.chain, linked ? k : 0, zre);
     t.nlist = pb->tile.nlist + (linked ? k & 1 : 0);
     t.nlist_clear = pb->tile.nlist + ((k + 1) & 1);
-    if (linked) {
+    const int nt = t.g.pie ? t.g.nzx : 0;    // triangles
+    if (linked && !nt) {
         launch_tiles<true>(a, t, t.ntiles + 1, form, s);
         return (int)hipGetLastError();
     }
-    const int nt = t.g.pie ? t.g.nzx : 0;    // triangles
-    int npart = 0;
     tri.part_dt = a.part_dt; tri.part_dv = a.part_dv; tri.part_bp = a.part_bp; tri.part_bc = a.part_bc;
-    if (nt) {
-        tri.pxx = a.pxx; tri.pxy = a.pxy; tri.pux = a.pux; tri.puy = a.puy;
+    tri.pxx = a.pxx; tri.pxy = a.pxy; tri.pux = a.pux; tri.puy = a.puy;
+    if (linked) {
+        const CycleStep step = t.step;
+        const dim3 blk(PN_BLOCK), g(nblocks(nt)), g1(nblocks(nt) + 1);
+        if (form == FORM_FP64)
+            hipLaunchKernelGGL(k_tri_pred<double>, g1, blk, 0, s, tri, step, nt, second);
+        else
+            hipLaunchKernelGGL(k_tri_pred<float>, g1, blk, 0, s, tri, step, nt, second);
+        t.step.in = step.out;                // as the triangles' kernel left it
+        launch_tiles<false>(a, t, t.ntiles + 1, form, s);
+        tri.pxx = a.oxx; tri.pxy = a.oxy; tri.pux = a.oux; tri.puy = a.ouy;
+        if (form == FORM_FP64)
+            hipLaunchKernelGGL(k_tri_corr<double>, g, blk, 0, s, tri, step, nt);
+        else
+            hipLaunchKernelGGL(k_tri_corr<float>, g, blk, 0, s, tri, step, nt);
+        return (int)hipGetLastError();
+    }
+    int npart = 0;
+    if (nt) {                                // (the learned form's)
         launch_pred<3>(pb, tri, 0, nt, 0, 0, form, 0, s);
         // one partial index per block of both halves
         npart = pred_grid(pb, nt, 3, form);
         if (npart != corr_grid(pb, nt)) return PENNANT_EINVAL;
-        if (form == FORM_LEARNED)
-            hipLaunchKernelGGL(k_pred_list<3>, dim3(npart < 512 ? npart : 512), dim3(PN_BLOCK), 0, s, tri, 0, nt, 0, 0);
+        hipLaunchKernelGGL(k_pred_list<3>, dim3(npart < 512 ? npart : 512), dim3(PN_BLOCK), 0, s, tri, 0, nt, 0, 0);
     }
     launch_tiles<false>(a, t, t.ntiles + (nt ? 1 : 0), form, s);
     if (nt) {
@@ -3641,7 +3701,9 @@ int tile_cycles(pennant_problem* pb, int form, int n) {
     const TileState& q = pb->tile;
     if (!q.nzx || (n & 1) || (form == FORM_LEARNED && !pb->closure)) return PENNANT_EINVAL;
     const int64_t tiles = (int64_t)((q.nzx + PN_TIN - 1) / PN_TIN) * ((q.nzy - q.pie + PN_TIN - 1) / PN_TIN);
-    const bool linked = n > 0 && !q.pie && tiles <= PN_LINK_TILES;
+    // a pie's few blocks of triangles always pay for the fold; the learned
+    // form's triangles have a list pass of their own
+    const bool linked = n > 0 && (q.pie ? form != FORM_LEARNED : tiles <= PN_LINK_TILES);
     for (int k = 0; k < n; ++k)
         if (const int rc = tile_cycle(pb, form, k, linked)) return rc;
     return linked ? chain_end(pb, q.chain, n, form == FORM_FP64 ? 1 : 0) : 0;
