@@ -18,17 +18,16 @@ Prints ONE JSON line on stdout:
               library's stream around exactly --steps cycles)
   roofline    dominant kernel of the timed form: algorithmic bytes per launch
               / its average duration (HIP events between the launches, in
-              further cycles right after the timed ones) against 8 TB/s;
+              further cycles right after the timed ones) against 8 TB/s; for
+              cycles that ran as tiles, the cycle's bytes over its time;
               roofline_fp64: the same for the plain FP64 form
   accuracy    speedup over plain FP64; density/energy/pressure L1 and Linf
               errors, shock radius at tstop; the 1% density gate
   energy      total energy (internal + kinetic) at t = 0 and at tstop, and
               its relative drift, per form
-  drop_in_tasks  the task-by-task FP64 cycle (one kernel launch per
-              reference task ID, through the C ABI's per-task entry points) on
-              the same workload from t = 0: us per cycle and the reference
-              decomposition's bytes per cycle (688 S + 536 Z + 512 P) over that
-              time, against 8 TB/s
+  drop_in_tasks  the task form (FP64; every reference task's fields in memory
+              after each cycle) on the same workload from t = 0: us per cycle
+              and its compulsory bytes over that time, against 8 TB/s
   cpu_baseline  the CPU oracle (a serial C++ restatement of the reference's
               CPU task bodies, and its OpenMP variant) on a bounded sample of
               the same workload, on this host (lscpu model, sockets, cores)
@@ -191,11 +190,14 @@ def bench_pieces(args, pa, text, wname):
 
 
 PROFILE_KERNELS = {
-    "fp64": {"zone_pred": "k_pred_zone<4>", "point": "k_point<double>", "zone_corr": "k_corr<4, double>"},
+    "fp64": {"zone_pred": "k_pred_zone<4>", "point": "k_point<double>", "zone_corr": "k_corr<4, double>",
+             "tile": "k_tile<double, 0, false>"},
     "mixed": {"zone_pred": "k_pred_mixed<4, false, false>", "point": "k_point<float>",
-              "zone_corr": "k_corr<4, float>", "zone": "k_zone_pipe<4, false>"},
+              "zone_corr": "k_corr<4, float>", "zone": "k_zone_pipe<4, false>",
+              "tile": "k_tile<float, 0, false>"},
     "learned": {"zone_pred": "k_pred_mixed<4, true, false>", "point": "k_point<float>",
-                "zone_corr": "k_corr<4, float>", "zone": "k_zone_pipe<4, true>"},
+                "zone_corr": "k_corr<4, float>", "zone": "k_zone_pipe<4, true>",
+                "tile": "k_tile<float, 3, false>"},
 }
 
 
@@ -253,6 +255,14 @@ def cpu_baseline(deck_text: str, numz: int, budget_s: float):
     return out, threads
 
 
+def tile_bytes(S: int, Z: int, P: int, mixed: bool):
+    """Compulsory bytes of a tile cycle, the whole cycle in one kernel: px, pu
+    read and written 64 per point; FP64: zm zr ze zetot zwrate zvol read, zr ze
+    zetot zwrate zvol zp written 96 per zone, smf 8 per side; mixed: zr and ze
+    neither, 64 per zone, and smf in FP32."""
+    return 64 * P + 64 * Z + 4 * S if mixed else 64 * P + 96 * Z + 8 * S
+
+
 def kernel_roofline(kb: dict, per_ms: dict, names) -> dict:
     """Roofline of the dominant (longest) kernel: its algorithmic bytes per
     launch over its average launch duration, against 8 TB/s."""
@@ -299,7 +309,7 @@ def main():
                     help="trained closure (.npz from pennant_amd.train_closure); default: the "
                          "package's closure_ensemble.npz")
     ap.add_argument("--tasks-steps", type=int, default=20,
-                    help="cycles of the task-by-task FP64 form timed for drop_in_tasks (0: skip)")
+                    help="cycles of the FP64 task form timed for drop_in_tasks (0: skip)")
     ap.add_argument("--copy-mb", type=int, default=512,
                     help="size of the streaming-copy calibration (0 disables)")
     ap.add_argument("--k1", type=int, default=None, help="fused K1 layout: 0 zone/thread, 1 corner/lane")
@@ -381,7 +391,8 @@ def main():
             tune_cycles = 16
             ms = pb.autotune(mode, cycles=tune_cycles)
             log(f"autotune: {ms / tune_cycles * 1e3:.1f} us/cycle at the best shape")
-        tune = {k: pb.get_tuning(k) for k in ("k1_layout", "max_blocks", "xcd", "pipeline", "graph", "rect_maps")}
+        tune = {k: pb.get_tuning(k) for k in ("k1_layout", "max_blocks", "xcd", "pipeline", "graph", "rect_maps",
+                                                "tiles")}
         log(f"tuning {tune}")
         sc0 = pb.scalars()
         cl0 = pb.closure_stats() if mode == pa.MODE_LEARNED else None
@@ -433,6 +444,15 @@ def main():
             gbs = kb[n] / (per[n] * 1e-3) / 1e9 if n in kb else 0.0
             log(f"  {n:12s} {per[n] * 1e3:8.1f} us/launch" +
                 (f"  {kb[n] / 1e6:8.1f} MB  {gbs:8.1f} GB/s" if n in kb else ""))
+        if r["tune"]["tiles"] == 1 and not pipelined and r["tune"]["k1_layout"] == 0:
+            # the timed cycles ran as tiles (every workload's mesh is structured):
+            # one kernel a cycle, and what ends it, in the cycle's time; the
+            # phases above are those of the separate passes
+            passes = {n: round(per[n] * 1e3, 2) for n in names if n != "unused"}
+            kb, per, names = {"tile": tile_bytes(S, Z, P, mixed)}, {"tile": r["total_ms"] / args.steps}, ("tile",)
+            roof = kernel_roofline(kb, per, names)
+            roof["separate_passes_us"] = passes
+            return roof, (kb, per, names, pipelined)
         return kernel_roofline(kb, per, names), (kb, per, names, pipelined)
 
     mode = modes[args.mode]
@@ -533,8 +553,11 @@ def main():
     else:
         energy = None
 
-    # the drop-in path: one launch per reference task ID, from t = 0 (its
-    # kernels move the same bytes at any time of the run)
+    # the task form: every task's fields written each cycle, from t = 0 (its
+    # kernels move the same bytes at any time of the run).  Its compulsory
+    # bytes: per side mapsp1, pcpos, smf, then mapsp1, sfp, sfq read, 192 + 24
+    # + 32 written, corner records 24 read; per zone 80 read, 176 written; per
+    # point 133 read, 120 written, less what the caches hold of px, pu
     tasks = None
     if args.tasks_steps > 0 and mode != pa.MODE_TASKS:
         with pa.Problem(text) as pt:
@@ -543,13 +566,13 @@ def main():
             tms, _ = pt.time_cycles(args.tasks_steps, pa.MODE_TASKS, phases=False)
             sct1 = pt.scalars()
         us = tms / args.tasks_steps * 1e3
-        tb = 688 * S + 536 * Z + 512 * P
+        tb = 324 * S + 256 * Z + 245 * P
         gbs = tb / (us * 1e-6) / 1e9
-        log(f"drop-in tasks fp64: {us:.1f} us/cycle, {tb / 1e9:.3f} GB of task bytes per cycle, "
+        log(f"drop-in tasks fp64: {us:.1f} us/cycle, {tb / 1e9:.3f} GB per cycle, "
             f"{gbs:.1f} GB/s ({gbs / HBM_PEAK_GBS:.3f} of peak)")
         tasks = {"form": "plain-fp64-tasks", "us_per_cycle": round(us, 2),
                  "zone_cycles_per_s": round(Z / (us * 1e-6), 1),
-                 "task_bytes_per_cycle": tb, "effective_GBs": round(gbs, 1),
+                 "bytes_per_cycle": tb, "achieved_GBs": round(gbs, 1),
                  "peak_GBs": HBM_PEAK_GBS, "frac": round(gbs / HBM_PEAK_GBS, 4),
                  "t_window": [round(sct0["time"], 9), round(sct1["time"], 9)]}
 

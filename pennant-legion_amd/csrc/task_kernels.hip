@@ -1253,9 +1253,9 @@ __global__ void __launch_bounds__(PN_BLOCK) k_apply_fixed_bc(const int32_t* mapb
 // zone and 512 a point, most of them fields that the task before has just
 // written; here the tasks that follow each other on the same zones or points
 // share a kernel and pass those on in registers and LDS, which leaves what has
-// to be written and the first reads: about 360, 290 and 220 bytes.  The task
+// to be written and the first reads: 324, 256 and 245 bytes.  The task
 // entry points stay one kernel a task.  Bound by those bytes on large meshes
-// (Sedov 1440^2: 1466 -> 750 us a cycle, 5.1 TB/s), by the launches' latencies
+// (Sedov 1440^2: 1466 -> 750 us a cycle, 5.0 TB/s), by the launches' latencies
 // on small ones (97 x 61: 111 -> 18 us).
 //
 //   k_cycle_pred    zones: steps 0, 2-7, 9-15 and 26, with the half-step
