@@ -57,9 +57,9 @@ int build_graph(pennant_batch* b, int form) {
     drop_graph(b);
     hipGraph_t g = nullptr;
     BCK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    int rc = 0;
-    for (int k = 0; k < PN_GRAPH_CYCLES && !rc; ++k)
-        rc = tiled(b, form) ? batch_tile_cycle(b, form, k & 1) : batch_cycle(b, form);
+    const bool tile = tiled(b, form);
+    int rc = tile ? batch_tile_cycles(b, form, PN_GRAPH_CYCLES) : 0;
+    for (int k = 0; k < PN_GRAPH_CYCLES && !rc && !tile; ++k) rc = batch_cycle(b, form);
     const int rc2 = (int)hipStreamEndCapture(b->stream, &g);
     if (rc || rc2) {
         if (g) (void)hipGraphDestroy(g);
@@ -258,7 +258,7 @@ pennant_batch* pennant_batch_create(const char* const* decks, int n, char* errbu
     b->part_d = (double*)al(2 * units.size(), 8);
     b->part_i = (int*)al(2 * units.size(), 4);
     if (!ok) return fail(b, "device allocation failed");
-    if (batch_tile_setup(b, meshes, probs)) return fail(b, "device allocation failed");
+    if (batch_tile_setup(b, meshes)) return fail(b, "device allocation failed");
     int rc = (int)hipMemcpy(b->mapsp1, mapsp1.data(), S * 4, hipMemcpyHostToDevice);
     if (!rc) rc = (int)hipMemcpy(b->pcbeg, pcbeg.data(), (P + 1) * 4, hipMemcpyHostToDevice);
     if (!rc) rc = (int)hipMemcpy(b->pcpos, pcpos.data(), S * 4, hipMemcpyHostToDevice);
@@ -308,9 +308,9 @@ int pennant_batch_launch_cycles(pennant_batch* b, int ncycles, int mode) {
         for (; left >= b->graph_cycles; left -= b->graph_cycles) BCK(hipGraphLaunch(b->gexec, b->stream));
     }
     // tile cycles come in pairs; an odd cycle runs as separate passes
-    for (; left > 1 && tiled(b, form); left -= 2) {
-        BCK(batch_tile_cycle(b, form, 0));
-        BCK(batch_tile_cycle(b, form, 1));
+    if (left > 1 && tiled(b, form)) {
+        BCK(batch_tile_cycles(b, form, left & ~1));
+        left &= 1;
     }
     for (; left > 0; --left) BCK(batch_cycle(b, form));
     return 0;

@@ -2418,18 +2418,13 @@ __device__ __forceinline__ void tile_load(const FusedArgs& a, const TileMesh& g,
     in.bits = at_byte<unsigned char>(a.pbc, p);
 }
 
-// Where a tile's dt limit, dvol ratio and bad sides go: into slots, or (a batch,
-// whose problems have few tiles each) into the block partials a.part_*.
-struct TileSink {
-    slot_t* slots;
-    int at;
-};
-
-// The tile whose first zone (ring included) is (i0, j0), loaded in `in`.  Returns whether a CL_FLAG tile has a zone for the network: such a
+// The tile whose first zone (ring included) is (i0, j0), loaded in `in`; its
+// dt limit, dvol ratio and bad sides go into slots as block `at`'s.  Returns whether a CL_FLAG tile has a zone for the network: such a
 // tile is left to the list kernel and stores nothing.
 template <typename T, int CL>
 __device__ __forceinline__ bool tile_body(const FusedArgs& a, const TileOut& o, const TileMesh& g, int i0, int j0,
-                                          const TileIn<T>& in, const TileSink& sink, double dt, bool zre, ClCount& total) {
+                                          const TileIn<T>& in, slot_t* slots, int at, double dt, bool zre,
+                                          ClCount& total) {
     __shared__ T crn[12][PN_BLOCK];
     __shared__ double pts[sizeof(T) == 8 ? 5 : 4][PN_BLOCK];
     __shared__ struct {
@@ -2598,15 +2593,8 @@ __device__ __forceinline__ bool tile_body(const FusedArgs& a, const TileOut& o, 
             dvov = (lds.dv[w] > dvov) ? lds.dv[w] : dvov;
             bads += lds.bad[w];
         }
-        if (sink.slots) {
-            slots_dt(sink.slots, sink.at, dtm, bads & 0xffff);
-            slots_dv(sink.slots, sink.at, dvov, bads >> 16);
-        } else {
-            a.part_dt[sink.at] = dtm;
-            a.part_bp[sink.at] = bads & 0xffff;
-            a.part_dv[sink.at] = dvov;
-            a.part_bc[sink.at] = bads >> 16;
-        }
+        slots_dt(slots, at, dtm, bads & 0xffff);
+        slots_dv(slots, at, dvov, bads >> 16);
     }
     return false;
 }
@@ -2699,7 +2687,7 @@ k_tile(FusedArgs a, TileArgs t) {
     tile_load<T>(a, t.g, i0, j0, in);
     auto body = [&](double dt, bool zre) {
         ClCount none;
-        const bool left = tile_body<T, CL>(a, t.o, t.g, i0, j0, in, {t.step.put, tile}, dt, zre, none);
+        const bool left = tile_body<T, CL>(a, t.o, t.g, i0, j0, in, t.step.put, tile, dt, zre, none);
         if (CL == CL_FLAG && left && threadIdx.x == 0) t.list[atomicAdd(t.nlist, 1)] = tile;
     };
     if constexpr (LINK) {
@@ -2791,7 +2779,7 @@ k_tile_list(FusedArgs a, TileArgs t) {
         tile_at(t, tile, i0, j0);
         TileIn<float> in;
         tile_load<float>(b, t.g, i0, j0, in);
-        (void)tile_body<float, CL_PACKED>(b, t.o, t.g, i0, j0, in, {t.step.put, tile}, dt, zre, cnt);
+        (void)tile_body<float, CL_PACKED>(b, t.o, t.g, i0, j0, in, t.step.put, tile, dt, zre, cnt);
     }
     const int nl = block_sum(cnt.learned);
     const int nf = block_sum(cnt.fallback);
@@ -2801,45 +2789,36 @@ k_tile_list(FusedArgs a, TileArgs t) {
     }
 }
 
-// The end of a tile cycle that is not linked, by one block of PN_FIN_BLOCK
-// threads (without partials 64 do): from npart partials and (slots given) a set
-// of slots, which it empties; also says where the state is now (cur: 1 after
-// the first cycle of a pair).
-__device__ __forceinline__ void finalize_tile_block(Ctl* c, const double* part_dt, const int* part_bp,
-                                                    const double* part_dv, const int* part_bc, int npart,
-                                                    slot_t* slots, const DtParams& q, int zre, int cur) {
+// K4 of a tile cycle that is not linked, from the tiles' slots, which it
+// empties, and npart partials of a pie's triangles (none: 64 threads do); says
+// where the state is now (cur: 1 after the first cycle of a pair) and empties
+// the learned form's lists.
+__global__ void __launch_bounds__(PN_FIN_BLOCK) k_finalize_tile(FusedArgs a, int npart, slot_t* slots, DtParams q, int zre,
+                                                                int cur, int* nlist) {
+    Ctl* c = a.ctl;
     const CtlSnap v = snap_ctl(c);
     double mn = 1.e99, mx = 1.e-99;
     int bp = 0, bc = 0;
     SlotFold f = {1.e99, 1.e-99, 0, 0};
-    if (slots && threadIdx.x < 64) f = slots_fold(slots_load(slots));
+    if (threadIdx.x < 64) f = slots_fold(slots_load(slots));
     if (npart > 0) {
-        fold_partials<PN_FIN_BLOCK>(part_dt, part_bp, npart, part_dv, part_bc, npart, mn, bp, mx, bc);
+        fold_partials<PN_FIN_BLOCK>(a.part_dt, a.part_bp, npart, a.part_dv, a.part_bc, npart, mn, bp, mx, bc);
         blk_fold_fin<PN_FIN_BLOCK>(mn, mx, bp, bc);
     }
-    if (slots) slots_reset(slots);
+    slots_reset(slots);
+    if (a.zcount)
+        for (int k = threadIdx.x; k < a.nzruns * PN_LSLICES; k += blockDim.x) a.zcount[k * PN_LSTRIDE] = 0u;
     if (threadIdx.x != 0) return;
-    mn = (f.mn < mn) ? f.mn : mn;
-    mx = (f.mx > mx) ? f.mx : mx;
-    bp += f.bp;
-    bc += f.bc;
+    if (nlist) *nlist = 0;
     if (v.done) {
         if (!cur) c->cur = 0;                // copied back
         return;
     }
+    mn = (f.mn < mn) ? f.mn : mn;
+    mx = (f.mx > mx) ? f.mx : mx;
     c->zre_valid = zre;
-    end_cycle(c, v, mn, mx, bp, bc, q);
+    end_cycle(c, v, mn, mx, bp + f.bp, bc + f.bc, q);
     c->cur = cur;
-}
-
-// K4 of a tile cycle that is not linked, from the tiles' slots and a pie's
-// triangles' partials; empties the learned form's lists.
-__global__ void __launch_bounds__(PN_FIN_BLOCK) k_finalize_tile(FusedArgs a, int npart, slot_t* slots, DtParams q, int zre,
-                                                                int cur, int* nlist) {
-    if (nlist && threadIdx.x == 0) *nlist = 0;
-    if (a.zcount)
-        for (int k = threadIdx.x; k < a.nzruns * PN_LSLICES; k += blockDim.x) a.zcount[k * PN_LSTRIDE] = 0u;
-    finalize_tile_block(a.ctl, a.part_dt, a.part_bp, a.part_dv, a.part_bc, npart, slots, q, zre, cur);
 }
 
 FusedArgs make_args(pennant_problem* pb) {
@@ -3161,12 +3140,97 @@ struct TileBatch {
     const BHeavy* origins;
     int back;                    // the second cycle of a pair
 };
+
+// A cycle's place in the problems' chains (CycleStep): control blocks by
+// problem, three sets of slots a problem, and which of them.
+struct BatchChain {
+    const Ctl* in;
+    Ctl* out;
+    slot_t* sets;
+    int prev, put, clear;        // prev -1: the chains' first cycle
+    int zre;
+};
+__device__ __forceinline__ slot_t* batch_slots(const BatchChain& c, int pid, int set) {
+    return c.sets + ((size_t)pid * 3 + set) * PN_SLOT_SET;
+}
+__device__ __forceinline__ DtParams batch_dt(const BProb& q) { return {q.cflv, q.dtmax, q.dtfac, q.tstop, q.cstop}; }
+__device__ __forceinline__ CycleStep batch_step(const BatchArgs& B, const BatchChain& c, int pid) {
+    CycleStep s;
+    s.in = c.in + pid;
+    s.out = c.out + pid;
+    s.prev = c.prev < 0 ? nullptr : batch_slots(c, pid, c.prev);
+    s.put = batch_slots(c, pid, c.put);
+    s.clear = batch_slots(c, pid, c.clear);
+    s.q = batch_dt(B.probs[pid]);
+    s.zre = c.zre;
+    return s;
+}
+
+// Before and after the tiles.  First the end of every problem's cycle before
+// (a block each) and the predictor of the pies' triangles, whose blocks end their
+// problem's by themselves; then the triangles' corrector.  With a K4 of partials
+// between the cycles instead, 32 problems took 53.0 us a cycle instead of 51.0
+// (mixed), 16 others 75.5 instead of 73.1 (FP64).
+template <typename T>
+__global__ void __launch_bounds__(PN_BLOCK) k_head_batch(BatchArgs B, BatchChain c, int nprob, int back) {
+    if ((int)blockIdx.x < nprob) {
+        cycle_step(batch_step(B, c, blockIdx.x), back);
+        return;
+    }
+    const BUnit U = B.units[blockIdx.x - nprob];
+    const CycleStep s = batch_step(B, c, U.pid);
+    const CycleNow now = cycle_now(s);
+    if (now.done) return;
+    FusedArgs a = B.a;
+    apply_prob(a, B.probs[U.pid]);
+    const int z = U.zb + (int)threadIdx.x, sb = U.sb + 3 * (int)threadIdx.x;
+    double m = 1.e99;
+    int bad = 0;
+    if (z < U.ze) {
+        ClCount cnt;
+        double v;
+        if constexpr (sizeof(T) == 8) {
+            v = zone_pred<3>(a, z, sb, unit_w(U, z), now.dt, bad);
+        } else {
+            int pp[3];
+            load_pp<3>(a, sb, pp);
+            v = zone_pred_mixed<3, CL_EXACT>(a, z, sb, unit_w(U, z), pp, now.dt, bad, true, cnt, now.zre != 0);
+        }
+        m = (v < m) ? v : m;
+    }
+    m = block_min(m);
+    bad = block_sum(bad);
+    if (threadIdx.x == 0) slots_dt(s.put, blockIdx.x, m, bad);
+}
+template <typename T>
+__global__ void __launch_bounds__(PN_BLOCK) k_tail_batch(BatchArgs B, BatchChain c) {
+    const BUnit U = B.units[blockIdx.x];
+    const Ctl* q = c.out + U.pid;
+    if (q->done) return;
+    const int z = U.zb + (int)threadIdx.x;
+    double m = 1.e-99;
+    int bad = 0;
+    if (z < U.ze) corr_zone<3, T>(B.a, z, U.sb + 3 * (int)threadIdx.x, unit_w(U, z), q->dt, bad, m);
+    m = block_max(m);
+    bad = block_sum(bad);
+    if (threadIdx.x == 0) slots_dv(batch_slots(c, U.pid, c.put), blockIdx.x, m, bad);
+}
+// The ends of the problems' chains, a block each: c.in as the last cycle left
+// it, c.put the set it filled.
+__global__ void __launch_bounds__(64) k_chain_end_batch(BatchArgs B, BatchChain c) {
+    const int pid = blockIdx.x;
+    cycle_chain_end(B.ctls + pid, c.in + pid, batch_slots(c, pid, 0), c.put, batch_dt(B.probs[pid]), c.zre);
+}
+__global__ void __launch_bounds__(64) k_chain_begin_batch(slot_t* sets) {
+    for (int k = 0; k < 3; ++k) slots_reset(sets + ((size_t)blockIdx.x * 3 + k) * PN_SLOT_SET);
+}
+
 template <typename T>
 __global__ void __launch_bounds__(PN_BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 2 : 3)))
-k_tile_batch(BatchArgs B, TileBatch t) {
+k_tile_batch(BatchArgs B, TileBatch t, BatchChain q) {
     if ((int)blockIdx.x >= t.ntiles) {
         const BHeavy h = t.origins[blockIdx.x - t.ntiles];
-        const Ctl* c = B.ctls + h.pid;
+        const Ctl* c = q.out + h.pid;
         FusedArgs a = B.a;
         if (c->done) {
             if (t.back && c->cur && threadIdx.x == 0) {
@@ -3178,11 +3242,12 @@ k_tile_batch(BatchArgs B, TileBatch t) {
         point_heavy<T>(a, h.p, c->dt);
         return;
     }
-    const BTile U = t.tiles[xcd_tile(t.ntiles)];
+    const int tile = xcd_tile(t.ntiles);
+    const BTile U = t.tiles[tile];
     const TileMesh g = {U.nzx, U.nzy, U.pie, U.zo, U.so, U.po};
     TileIn<T> in;
     tile_load<T>(B.a, g, U.i0, U.j0, in);
-    const Ctl* c = B.ctls + U.pid;
+    const Ctl* c = q.out + U.pid;
     FusedArgs a = B.a;
     if (c->done) {
         if (t.back && c->cur) tile_copy<T>(a, t.o, g, U.i0, U.j0);
@@ -3195,14 +3260,8 @@ k_tile_batch(BatchArgs B, TileBatch t) {
     a.q1 = uni(a.q1); a.q2 = uni(a.q2); a.cfl = uni(a.cfl);
     const double dt = uni(c->dt);
     ClCount none;
-    (void)tile_body<T, CL_EXACT>(a, t.o, g, U.i0, U.j0, in, {nullptr, U.slot}, dt, c->zre_valid != 0, none);
-}
-
-__global__ void __launch_bounds__(PN_FIN_BLOCK) k_finalize_batch_tile(BatchArgs B, int zre, int cur) {
-    const BProb& q = B.probs[blockIdx.x];
-    finalize_tile_block(B.ctls + blockIdx.x, B.a.part_dt + q.tbeg, B.a.part_bp + q.tbeg, B.a.part_dv + q.tbeg,
-                        B.a.part_bc + q.tbeg, q.tend - q.tbeg, nullptr, {q.cflv, q.dtmax, q.dtfac, q.tstop, q.cstop},
-                        zre, cur);
+    (void)tile_body<T, CL_EXACT>(a, t.o, g, U.i0, U.j0, in, batch_slots(q, U.pid, q.put), tile, dt, c->zre_valid != 0,
+                                 none);
 }
 
 // k_zre over the units of every problem whose flag is clear.
@@ -3820,18 +3879,16 @@ int batch_cycle(pennant_batch* b, int form) {
     return (int)hipGetLastError();
 }
 
-int batch_tile_setup(pennant_batch* b, const std::vector<TileState>& meshes, std::vector<BProb>& probs) {
+int batch_tile_setup(pennant_batch* b, const std::vector<TileState>& meshes) {
     b->ntiles = 0;
     for (const TileState& m : meshes)
         if (m.nzx == 0) return 0;            // some problem needs the separate passes
     std::vector<BTile> tiles;
     std::vector<BUnit> tri;
     std::vector<BHeavy> origins;
-    int slot = 0;
     for (size_t k = 0; k < meshes.size(); ++k) {
         const TileState& m = meshes[k];
         const int zo = (int)b->zoff[k], so = (int)b->soff[k], po = (int)b->poff[k], pid = (int)k;
-        probs[k].tbeg = slot;
         if (m.pie) {
             for (int z = 0; z < m.nzx; z += PN_BLOCK) {
                 BUnit U = {};
@@ -3840,39 +3897,38 @@ int batch_tile_setup(pennant_batch* b, const std::vector<TileState>& meshes, std
                 U.sb = so + 3 * z;
                 U.ns = 3;
                 U.pid = pid;
-                U.slot = slot++;
                 tri.push_back(U);
             }
             origins.push_back({po, pid});
         }
         for (int j = 0; j < m.nzy - m.pie; j += PN_TIN)
             for (int i = 0; i < m.nzx; i += PN_TIN)
-                tiles.push_back({i - 1, m.pie + j - 1, m.nzx, m.nzy, m.pie, zo, so, po, pid, slot++});
-        probs[k].tend = slot;
+                tiles.push_back({i - 1, m.pie + j - 1, m.nzx, m.nzy, m.pie, zo, so, po, pid});
     }
     const size_t P = (size_t)b->nump, Z = (size_t)b->numz;
-    const size_t bytes = (4 * P + 5 * Z + 2 * (size_t)slot) * 8 + 2 * (size_t)slot * 4 + tiles.size() * sizeof(BTile) +
+    const size_t N = meshes.size();
+    const size_t bytes = N * PN_CHAIN_BYTES + (4 * P + 5 * Z) * 8 + tiles.size() * sizeof(BTile) +
                          tri.size() * sizeof(BUnit) + origins.size() * sizeof(BHeavy);
     char* m = nullptr;
     if (hipMalloc((void**)&m, bytes) != hipSuccess) return (int)hipErrorOutOfMemory;
     b->allocs.push_back(m);
-    double* d = (double*)m;
+    b->chain = m;                            // the problems' slots, then their second control blocks
+    double* d = (double*)(m + N * PN_CHAIN_BYTES);
     for (int k = 0; k < 9; ++k) {
         b->alt[k] = d;
         d += k < 4 ? P : Z;
     }
-    b->tpart_d = d;
-    b->tpart_i = (int*)(d + 2 * (size_t)slot);
-    b->tiles = (BTile*)(b->tpart_i + 2 * (size_t)slot);
+    b->tiles = (BTile*)d;
     b->tunits = (BUnit*)(b->tiles + tiles.size());
     b->origins = (BHeavy*)(b->tunits + tri.size());
-    b->ntparts = slot;
     b->ntunits = (int)tri.size();
     b->norigins = (int)origins.size();
     int rc = (int)hipMemcpy(b->tiles, tiles.data(), tiles.size() * sizeof(BTile), hipMemcpyHostToDevice);
     if (!rc && !tri.empty()) rc = (int)hipMemcpy(b->tunits, tri.data(), tri.size() * sizeof(BUnit), hipMemcpyHostToDevice);
     if (!rc && !origins.empty())
         rc = (int)hipMemcpy(b->origins, origins.data(), origins.size() * sizeof(BHeavy), hipMemcpyHostToDevice);
+    hipLaunchKernelGGL(k_chain_begin_batch, dim3((unsigned)N), dim3(64), 0, b->stream, (slot_t*)b->chain);
+    if (!rc) rc = (int)hipGetLastError();
     if (!rc) b->ntiles = (int)tiles.size();
     return rc;
 }
@@ -3880,12 +3936,17 @@ int batch_tile_setup(pennant_batch* b, const std::vector<TileState>& meshes, std
 // Cycle `second` of a pair.  The triangles' own state stays in the batch's
 // arrays, as in tile_cycle; their point values come from the state the cycle
 // starts from and go with the one it writes.
-int batch_tile_cycle(pennant_batch* b, int form, int second) {
-    if (!b->ntiles || form == FORM_LEARNED) return PENNANT_EINVAL;
+// Step k of the problems' chains (as chain_step).
+static BatchChain batch_chain(pennant_batch* b, int k, int zre) {
+    slot_t* sets = (slot_t*)b->chain;
+    Ctl* c[2] = {b->ctls, (Ctl*)(sets + (size_t)b->nprob * 3 * PN_SLOT_SET)};
+    return {c[k & 1], c[(k + 1) & 1], sets, k ? (k - 1) % 3 : -1, k % 3, (k + 1) % 3, zre};
+}
+
+static int batch_tile_cycle(pennant_batch* b, int form, int k) {
+    const int second = k & 1;
     BatchArgs B = make_batch_args(b);
     FusedArgs& a = B.a;
-    a.part_dt = b->tpart_d; a.part_dv = b->tpart_d + b->ntparts;
-    a.part_bp = b->tpart_i; a.part_bc = b->tpart_i + b->ntparts;
     BatchArgs T = B;                         // triangles
     double* const own[9] = {a.pxx, a.pxy, a.pux, a.puy, a.zr, a.ze, a.zetot, a.zwrate, a.zvol};
     double* const* src = second ? b->alt : own;
@@ -3897,21 +3958,30 @@ int batch_tile_cycle(pennant_batch* b, int form, int second) {
     T.units = b->tunits;
     T.nunits = b->ntunits;
     hipStream_t s = b->stream;
-    const dim3 blk(PN_BLOCK), tg(b->ntunits), grid(b->ntiles + b->norigins);
+    const dim3 blk(PN_BLOCK), head(b->nprob + b->ntunits), tail(b->ntunits), grid(b->ntiles + b->norigins);
     const bool fp64 = form == FORM_FP64;
-    if (b->ntunits) {
-        T.a.pxx = src[0]; T.a.pxy = src[1]; T.a.pux = src[2]; T.a.puy = src[3];
-        if (fp64) hipLaunchKernelGGL((k_pred_batch<FORM_FP64, CL_EXACT>), tg, blk, 0, s, T);
-        else hipLaunchKernelGGL((k_pred_batch<FORM_MIXED, CL_EXACT>), tg, blk, 0, s, T);
-    }
-    if (fp64) hipLaunchKernelGGL(k_tile_batch<double>, grid, blk, 0, s, B, t);
-    else hipLaunchKernelGGL(k_tile_batch<float>, grid, blk, 0, s, B, t);
+    const BatchChain c = batch_chain(b, k, fp64 ? 1 : 0);
+    T.a.pxx = src[0]; T.a.pxy = src[1]; T.a.pux = src[2]; T.a.puy = src[3];
+    if (fp64) hipLaunchKernelGGL(k_head_batch<double>, head, blk, 0, s, T, c, b->nprob, second);
+    else hipLaunchKernelGGL(k_head_batch<float>, head, blk, 0, s, T, c, b->nprob, second);
+    if (fp64) hipLaunchKernelGGL(k_tile_batch<double>, grid, blk, 0, s, B, t, c);
+    else hipLaunchKernelGGL(k_tile_batch<float>, grid, blk, 0, s, B, t, c);
     if (b->ntunits) {
         T.a.pxx = dst[0]; T.a.pxy = dst[1]; T.a.pux = dst[2]; T.a.puy = dst[3];
-        if (fp64) hipLaunchKernelGGL(k_corr_batch<double>, tg, blk, 0, s, T);
-        else hipLaunchKernelGGL(k_corr_batch<float>, tg, blk, 0, s, T);
+        if (fp64) hipLaunchKernelGGL(k_tail_batch<double>, tail, blk, 0, s, T, c);
+        else hipLaunchKernelGGL(k_tail_batch<float>, tail, blk, 0, s, T, c);
     }
-    hipLaunchKernelGGL(k_finalize_batch_tile, dim3(b->nprob), dim3(PN_FIN_BLOCK), 0, s, B, fp64 ? 1 : 0, second ? 0 : 1);
+    return (int)hipGetLastError();
+}
+
+int batch_tile_cycles(pennant_batch* b, int form, int n) {
+    if (!b->ntiles || (n & 1) || form == FORM_LEARNED) return PENNANT_EINVAL;
+    if (n < 1) return 0;
+    for (int k = 0; k < n; ++k)
+        if (const int rc = batch_tile_cycle(b, form, k)) return rc;
+    BatchChain c = batch_chain(b, n, form == FORM_FP64 ? 1 : 0);
+    c.put = c.prev;
+    hipLaunchKernelGGL(k_chain_end_batch, dim3(b->nprob), dim3(64), 0, b->stream, make_batch_args(b), c);
     return (int)hipGetLastError();
 }
 

@@ -197,9 +197,9 @@ struct BUnit {
     int zb, ze, sb, ns, pid, slot, pad1, pad2;   // slot: of its block partials
 };
 // A tile of a structured problem (fused.hip, tile_body): the first zone of its
-// ring, the mesh and its place in the arena, its problem and partials.
+// ring, the mesh and its place in the arena, its problem.
 struct BTile {
-    int i0, j0, nzx, nzy, pie, zo, so, po, pid, slot;
+    int i0, j0, nzx, nzy, pie, zo, so, po, pid;
 };
 struct PUnit {
     int pb, pe, pid, pad;
@@ -215,7 +215,6 @@ struct BProb {
     // problem's own zone z; so, po: its first side and point in the arena
     unsigned long long rect_m;
     int rect_nzx, rect_sh, so, po;
-    int tbeg, tend;              // the problem's partials in a tile cycle
 };
 }  // namespace pn
 
@@ -243,17 +242,15 @@ struct pennant_batch {
     pn::BHeavy* heavy = nullptr;
     int nheavy = 0;
     // tile cycles, when every problem is structured (ntiles > 0): the tiles, the
-    // pies' triangles as zone units and their origins, partials, and the
-    // second set of state arrays (as pennant_problem::tile)
+    // pies' triangles as zone units and their origins, the problems' chains
+    // (cycle_end.h), and the second set of state arrays
     pn::BTile* tiles = nullptr;
     int ntiles = 0;
     pn::BUnit* tunits = nullptr;
     int ntunits = 0;
     pn::BHeavy* origins = nullptr;
     int norigins = 0;
-    int ntparts = 0;
-    double* tpart_d = nullptr;
-    int* tpart_i = nullptr;
+    void* chain = nullptr;
     double* alt[9] = {};
     pn::BProb* probs = nullptr;
     pn::Ctl* ctls = nullptr;
@@ -278,9 +275,9 @@ namespace pn {
 // one cycle of every unfinished problem of a batch (fused.hip)
 int batch_cycle(pennant_batch* b, int form);
 // tile cycles of a batch of structured problems: the set-up from the problems'
-// meshes (nzx, nzy, pie), and cycle `second` (0, 1) of a pair
-int batch_tile_setup(pennant_batch* b, const std::vector<TileState>& meshes, std::vector<BProb>& probs);
-int batch_tile_cycle(pennant_batch* b, int form, int second);
+// meshes (nzx, nzy, pie), and an even number n of cycles
+int batch_tile_setup(pennant_batch* b, const std::vector<TileState>& meshes);
+int batch_tile_cycles(pennant_batch* b, int form, int n);
 int launch_to_float(const double* src, float* dst, int64_t n, hipStream_t s);
 // fused cycle (fused.hip)
 int fused_setup(pennant_problem* pb);
