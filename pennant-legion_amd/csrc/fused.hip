@@ -2631,7 +2631,6 @@ struct TileArgs {
     int ntx, ntiles;
     int back;                    // the second cycle of a pair
     CycleStep step;              // linked cycles: the place in their chain; others: `in` is current
-    int linked;
     int* list;                   // learned form: tiles left to the list kernel, and their number
     int* nlist;
     int* nlist_clear;            // a chain's next cycle's number
@@ -2754,10 +2753,14 @@ __global__ void __launch_bounds__(PN_BLOCK) k_tri_corr(FusedArgs a, CycleStep s,
 // The learned form's tiles that have a zone for the network (in the ring or
 // inside): the whole tile again, the network evaluated for the wave's gated
 // corners packed together.  Their order in the list is not fixed, their
-// results are.
-__global__ void __launch_bounds__(PN_BLOCK) __attribute__((amdgpu_waves_per_eu(2)))
+// results are.  Two waves per SIMD, for which it spills 31 registers, where many
+// tiles may be listed; one, without, on the small rects of linked cycles, whose
+// listed tiles all run at once: learned 333 x 217 26.6 -> 24.8 us a cycle, 420^2
+// 36.5 -> 32.9, tube 1024 x 128 32.6 -> 29.6 (1440^2 145 -> 147, not taken).
+template <bool LINK>
+__global__ void __launch_bounds__(PN_BLOCK) __attribute__((amdgpu_waves_per_eu(LINK ? 1 : 2)))
 k_tile_list(FusedArgs a, TileArgs t) {
-    const Ctl* c = t.linked ? t.step.out : t.step.in;
+    const Ctl* c = LINK ? t.step.out : t.step.in;
     const int done = c->done, n = *t.nlist;
     const double dt = c->dt;
     const bool zre = c->zre_valid != 0;
@@ -3698,7 +3701,7 @@ static void launch_tiles(const FusedArgs& a, const TileArgs& t, int blocks, int 
         hipLaunchKernelGGL((k_tile<float, CL_EXACT, LINK>), grid, blk, 0, s, a, t);
     else {
         hipLaunchKernelGGL((k_tile<float, CL_FLAG, LINK>), grid, blk, 0, s, a, t);
-        hipLaunchKernelGGL(k_tile_list, dim3(t.ntiles < 512 ? t.ntiles : 512), blk, 0, s, a, t);
+        hipLaunchKernelGGL(k_tile_list<LINK>, dim3(t.ntiles < 512 ? t.ntiles : 512), blk, 0, s, a, t);
     }
 }
 
@@ -3711,7 +3714,6 @@ static int tile_cycle(pennant_problem* pb, int form, int k, bool linked) {
     FusedArgs tri = a;                       // the triangles' own state stays in the problem's arrays
     TileArgs t = tile_args(pb, second, a);
     hipStream_t s = pb->stream;
-    t.linked = linked ? 1 : 0;
     t.step = chain_step(pb, pb->tile.chain, linked ? k : 0, zre);
     t.nlist = pb->tile.nlist + (linked ? k & 1 : 0);
     t.nlist_clear = pb->tile.nlist + ((k + 1) & 1);
