@@ -1,7 +1,7 @@
 """Task-mode cycles (four launches for the thirty steps of doCycle) against the
 same steps through the task entry points, one launch per task: every field and
 scalar bit for bit, at the edges of the zone tiles (64 quads or triangles) and
-of the point blocks, at points of 1, 2, 4, 5, 255 to 257 and 300 corners, for
+of the point blocks, at origins of 2 to 5, 64, 65, 255 to 257 and 300 corners, for
 runs of single cycles and of captured ones, up to the stop condition and past
 it.
 """
@@ -30,6 +30,15 @@ DECKS = {
     "pie256x3": lambda c: wd.noh_pie(256, 3, cstop=c, dtinit=1e-4),
     "pie257x2": lambda c: wd.noh_pie(257, 2, cstop=c, dtinit=1e-4),
     "pie300x5": lambda c: wd.noh_pie(300, 5, cstop=c, dtinit=1e-4),
+    # radial zones x sectors (the origin's corners)
+    "pie3x4": lambda c: wd.noh_pie(3, 4, cstop=c, dtinit=1e-4),
+    "pie2x5": lambda c: wd.noh_pie(2, 5, cstop=c, dtinit=1e-4),
+    "pie2x64": lambda c: wd.noh_pie(2, 64, cstop=c, dtinit=1e-4),
+    "pie2x65": lambda c: wd.noh_pie(2, 65, cstop=c, dtinit=1e-4),
+    "pie2x255": lambda c: wd.noh_pie(2, 255, cstop=c, dtinit=1e-4),
+    "pie3x256": lambda c: wd.noh_pie(3, 256, cstop=c, dtinit=1e-4),
+    "pie2x257": lambda c: wd.noh_pie(2, 257, cstop=c, dtinit=1e-4),
+    "pie5x300": lambda c: wd.noh_pie(5, 300, cstop=c, dtinit=1e-4),
 }
 
 

@@ -29,6 +29,7 @@ DECKS = {
     "pie15x14": lambda c: wd.noh_pie(15, 14, cstop=c, dtinit=1e-4),
     "pie16x29": lambda c: wd.noh_pie(16, 29, cstop=c, dtinit=1e-4),
     "pie30x80": lambda c: wd.noh_pie(30, 80, cstop=c, dtinit=1e-4),
+    "pie2x600": lambda c: wd.noh_pie(2, 600, cstop=c, dtinit=1e-4),
 }
 
 
