@@ -472,6 +472,12 @@ int pennant_batch_autotune(pennant_batch* b, int mode, int cycles, double* best_
     if (form == FORM_LEARNED && !b->closure) return PENNANT_EINVAL;
     Snap sn;
     int rc = snap_take(b, sn);
+    if (rc) {                                // as pennant_autotune without a snapshot
+        (void)hipStreamSynchronize(b->stream);
+        snap_free(sn);
+        (void)hipGetLastError();
+        return rc;
+    }
     const Tuning keep = b->tune;
     Tuning best = keep;
     double bms = 1e300;
@@ -490,7 +496,7 @@ int pennant_batch_autotune(pennant_batch* b, int mode, int cycles, double* best_
     };
     // the tile cycle (its grid follows from the meshes), then the separate
     // passes' grids
-    if (!rc && tiled(b, form)) timed();
+    if (tiled(b, form)) timed();
     for (int xcd = 0; xcd <= 1; ++xcd) {
         for (int g : grids) {
             if (rc) break;

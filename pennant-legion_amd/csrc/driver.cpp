@@ -784,6 +784,14 @@ int pennant_autotune(pennant_problem* pb, int mode, int cycles, double* best_ms)
         if (!rc) copy.push_back(c);
         if (!rc) rc = (int)hipMemcpyAsync(c, a.first, a.second, hipMemcpyDeviceToDevice, pb->stream);
     }
+    if (rc) {
+        // no snapshot: nothing is timed, and nothing has changed.  (The error is
+        // this call's; left with the runtime it would be the next launch's.)
+        (void)hipStreamSynchronize(pb->stream);
+        for (void* c : copy) (void)hipFree(c);
+        (void)hipGetLastError();
+        return rc;
+    }
     auto restore = [&]() {
         drop_lookahead(pb);
         pb->zre_stale = true;        // the restored flag decides; materialising checks it

@@ -1,0 +1,36 @@
+"""The autotuners' decisions, on a HIP runtime without a device: which cycles
+they time, what they leave behind, and that a snapshot that cannot be taken is
+an error with nothing run."""
+from fake_hip import run_fake  # noqa: F401
+
+
+def test_a_failed_snapshot_runs_nothing(run_fake):
+    """Every allocation and every copy of the snapshot in turn fails: the call
+    returns the error, no kernel has run, the tuning and the memory in use are
+    what they were, and the next launch is not told of the error."""
+    run_fake("""
+def check(h, tune, launch, tuning):
+    for what in ("malloc", "copy"):
+        for k in range(1, 13):
+            launch(2, pa.MODE_MIXED)
+            before, live = [tuning(key) for key in ("tiles", "xcd", "max_blocks", "graph")], fake.live
+            clear()
+            fake.fail_bytes = 0
+            setattr(fake, "fail_" + what, k)
+            ms = ctypes.c_double()
+            rc = tune(h, pa.MODE_MIXED, 4, ctypes.byref(ms))
+            setattr(fake, "fail_" + what, 0)
+            assert rc == 2, (what, k, rc)
+            assert names() == [], (what, k, names())
+            assert [tuning(key) for key in ("tiles", "xcd", "max_blocks", "graph")] == before
+            assert fake.live == live, (what, k)
+            launch(2, pa.MODE_MIXED)
+
+L = pa.lib()
+with pa.Problem(wd.sedov_rect(20, cstop=100)) as pb:
+    check(pb._h, L.pennant_autotune, pb.launch, pb.get_tuning)
+    pb.set_tuning("pipeline", 1)                # the look-ahead is current before each call
+    check(pb._h, L.pennant_autotune, pb.launch, pb.get_tuning)
+with pa.Batch([wd.sedov_rect(20, cstop=100), wd.noh_pie(6, 5, cstop=100)]) as b:
+    check(b._h, L.pennant_batch_autotune, b.launch, b.get_tuning)
+""")
