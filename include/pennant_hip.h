@@ -459,7 +459,9 @@ int pennant_get_tuning(pennant_problem* pb, const char* key);
  * shape of the separate passes (K1 layout for the FP64 form, grid cap
  * 256..4096, XCD mapping, the pipelined cycle for the mixed forms) from one
  * snapshot of the state, keeps the fastest and restores the snapshot (the
- * problem does not advance).  best_ms (may be NULL) receives its time. */
+ * problem does not advance).  best_ms (may be NULL) receives its time for
+ * `cycles` cycles (an odd number is timed as one more where tiles, which run in
+ * pairs, are among the shapes). */
 int pennant_autotune(pennant_problem* pb, int mode, int cycles, double* best_ms);
 
 /* Writes <path> in the reference's .xy format (src/WriteXY.cc:28-53). */
@@ -598,8 +600,9 @@ int pennant_batch_capture_count(pennant_batch* b, int64_t* count);
 int pennant_batch_set_tuning(pennant_batch* b, const char* key, int value);
 int pennant_batch_get_tuning(pennant_batch* b, const char* key);
 /* Times `cycles` cycles as tiles and at each grid shape of the separate passes
- * (grid cap x XCD mapping) from the same snapshot of the state, keeps the fastest and restores the snapshot:
- * the problems do not advance.  best_ms (may be NULL) receives its time. */
+ * (grid cap x XCD mapping) from the same snapshot of the state, keeps the
+ * fastest and restores the snapshot: the problems do not advance.  best_ms (may
+ * be NULL) receives its time for `cycles` cycles, as pennant_autotune's. */
 int pennant_batch_autotune(pennant_batch* b, int mode, int cycles, double* best_ms);
 /* Parameters of an ensemble of `count` problems: for k even a Sedov blast on
  * an n[k] x n[k] rect mesh with energy param[k] in [0.1, 1.0], for k odd a

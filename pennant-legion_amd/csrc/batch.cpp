@@ -482,6 +482,8 @@ int pennant_batch_autotune(pennant_batch* b, int mode, int cycles, double* best_
     Tuning best = keep;
     double bms = 1e300;
     const int grids[] = {512, 1024, 2048, 4096, 8192, 16384};
+    // an even number where tiles are one of the shapes, as pennant_autotune
+    const int n = cycles + (tiled(b, form) ? cycles & 1 : 0);
     auto timed = [&]() {
         b->tune.graph = 0;
         drop_graph(b);
@@ -490,7 +492,7 @@ int pennant_batch_autotune(pennant_batch* b, int mode, int cycles, double* best_
         // two untimed cycles, then the timed ones
         if (!rc) rc = pennant_batch_launch_cycles(b, 2, mode);
         double ms = 0.;
-        if (!rc) rc = pennant_batch_time_cycles(b, cycles, mode, &ms);
+        if (!rc) rc = pennant_batch_time_cycles(b, n, mode, &ms);
         if (rc == PENNANT_EBADSIDES) rc = 0;
         if (!rc && ms < bms) { bms = ms; best = b->tune; }
     };
@@ -513,7 +515,7 @@ int pennant_batch_autotune(pennant_batch* b, int mode, int cycles, double* best_
     const int rc2 = snap_restore(b, sn);
     b->zre_stale = true;
     snap_free(sn);
-    if (best_ms) *best_ms = bms;
+    if (best_ms) *best_ms = bms < 1e300 ? bms * cycles / n : bms;
     return rc ? rc : rc2;
 }
 

@@ -761,10 +761,11 @@ int pennant_sync(pennant_problem* pb) {
     return bad_sides_error(pb);
 }
 
-// Times `cycles` cycles (after one untimed cycle) at every launch shape from
+// Times `cycles` cycles (after two untimed ones) at every launch shape from
 // the same snapshot of the state, keeps the fastest shape and restores the
 // snapshot, so the problem does not advance.  Results do not depend on the
-// shape, only the time does.
+// shape, only the time does.  Where tiles are one of the shapes every shape is
+// timed over an even number of cycles: an odd cycle takes the separate passes.
 int pennant_autotune(pennant_problem* pb, int mode, int cycles, double* best_ms) {
     const int form = fused_form(mode);
     if (form < 0 || cycles < 1) return PENNANT_EINVAL;
@@ -809,11 +810,12 @@ int pennant_autotune(pennant_problem* pb, int mode, int cycles, double* best_ms)
     // the mixed forms also try the pipelined cycle (it pays where the
     // volume-change limit seldom sets dt)
     const int npipe = (form == FORM_FP64 || pb->cap_buf) ? 1 : 2;
+    int n = cycles;
     auto timed = [&]() {
         rc = restore();
         if (!rc) rc = pennant_launch_cycles(pb, 2, mode);
         double ms = 0.;
-        if (!rc) rc = pennant_time_cycles(pb, cycles, mode, &ms, nullptr);
+        if (!rc) rc = pennant_time_cycles(pb, n, mode, &ms, nullptr);
         if (rc == PENNANT_EBADSIDES) rc = 0;
         if (!rc && ms < bms) { bms = ms; best = pb->tune; }
     };
@@ -823,7 +825,10 @@ int pennant_autotune(pennant_problem* pb, int mode, int cycles, double* best_ms)
     pb->tune.k1_layout = 0;
     pb->tune.pipeline = 0;
     pb->tune.tiles = keep.tiles;
-    if (tiled(pb, form)) timed();
+    if (tiled(pb, form)) {
+        n += n & 1;
+        timed();
+    }
     pb->tune.tiles = 0;
     for (int layout = 0; layout <= (form == FORM_FP64 ? 1 : 0) && !rc; ++layout)
       for (int pipe = 0; pipe < npipe && !rc; ++pipe)
@@ -841,7 +846,7 @@ int pennant_autotune(pennant_problem* pb, int mode, int cycles, double* best_ms)
     drop_graph(pb);
     const int rc2 = restore();
     for (void* c : copy) (void)hipFree(c);
-    if (best_ms) *best_ms = bms;
+    if (best_ms) *best_ms = bms < 1e300 ? bms * cycles / n : bms;
     return rc ? rc : rc2;
 }
 

@@ -34,3 +34,21 @@ with pa.Problem(wd.sedov_rect(20, cstop=100)) as pb:
 with pa.Batch([wd.sedov_rect(20, cstop=100), wd.noh_pie(6, 5, cstop=100)]) as b:
     check(b._h, L.pennant_batch_autotune, b.launch, b.get_tuning)
 """)
+
+
+def test_an_odd_number_of_cycles_times_tiles(run_fake):
+    """Tiles run in pairs.  With a cycle's time its number of kernels (four as
+    separate passes, one as tiles and one more a run), the time of an odd number
+    of cycles is that of tile cycles alone, scaled, and tiles are kept."""
+    run_fake("""
+for cycles in (1, 3, 4, 7):
+    even = cycles + cycles % 2
+    with pa.Problem(wd.sedov_rect(20, cstop=100)) as pb:
+        best = pb.autotune(pa.MODE_FUSED, cycles)
+        assert best == (even + 1) * cycles / even, (cycles, best)
+        assert pb.get_tuning("tiles") == 1
+    with pa.Batch([wd.sedov_rect(20, cstop=100), wd.leblanc_rect(15, 7, cstop=100)]) as b:
+        best = b.autotune(pa.MODE_FUSED, cycles)
+        assert best == (2 * even + 1) * cycles / even, (cycles, best)
+        assert b.get_tuning("tiles") == 1
+""")
