@@ -448,10 +448,12 @@ int pennant_bench_copy(size_t nbytes, int reps, double* ms_per_copy);
  *   "tiles"      1: on a structured mesh (rect, or pie of two rows or more, in
  *                the generator's numbering) a cycle is one kernel over tiles of
  *                zones (default; pennant_get_tuning reports 1 only when the
- *                mesh qualifies), 0: separate passes.  Cycles for which
- *                "k1_layout" 1, "pipeline" 1, "rect_maps" 0 (rect) or a capture
- *                buffer is set, and the odd cycle of a launch, run as separate
- *                passes
+ *                mesh qualifies and no form's tiles are off), 0: separate
+ *                passes.  Set for all forms; the autotuner switches tiles off for
+ *                the form that it times, where another shape was faster.  Cycles
+ *                for which "k1_layout" 1 (FP64), "pipeline" 1 (mixed, learned),
+ *                "rect_maps" 0 (rect) or a capture buffer is set, and the odd
+ *                cycle of a launch, run as separate passes
  * pennant_set_tuning returns PENNANT_EINVAL for an unknown key or value. */
 int pennant_set_tuning(pennant_problem* pb, const char* key, int value);
 int pennant_get_tuning(pennant_problem* pb, const char* key);

@@ -50,7 +50,7 @@ void drop_graph(pennant_batch* b) {
 
 // Whether cycles of `form` run as tile cycles (as `tiled` in driver.cpp).
 bool tiled(const pennant_batch* b, int form) {
-    return b->ntiles > 0 && b->tune.tiles && b->tune.rect_maps && form != FORM_LEARNED && !b->cap_buf;
+    return b->ntiles > 0 && (b->tune.tiles >> form & 1) && b->tune.rect_maps && form != FORM_LEARNED && !b->cap_buf;
 }
 
 int build_graph(pennant_batch* b, int form) {
@@ -449,7 +449,7 @@ int pennant_batch_set_tuning(pennant_batch* b, const char* key, int value) {
         b->tune.rect_maps = value;
     } else if (!strcmp(key, "tiles")) {
         if (value != 0 && value != 1) return PENNANT_EINVAL;
-        b->tune.tiles = value;
+        b->tune.tiles = value ? PN_TILES_ALL : 0;
     } else {
         return PENNANT_EINVAL;
     }
@@ -462,7 +462,7 @@ int pennant_batch_get_tuning(pennant_batch* b, const char* key) {
     if (!strcmp(key, "xcd")) return b->tune.xcd;
     if (!strcmp(key, "graph")) return b->tune.graph;
     if (!strcmp(key, "rect_maps")) return b->tune.rect_maps;
-    if (!strcmp(key, "tiles")) return (b->tune.tiles && b->ntiles > 0) ? 1 : 0;
+    if (!strcmp(key, "tiles")) return (b->tune.tiles == PN_TILES_ALL && b->ntiles > 0) ? 1 : 0;
     return PENNANT_EINVAL;
 }
 
@@ -483,7 +483,8 @@ int pennant_batch_autotune(pennant_batch* b, int mode, int cycles, double* best_
     double bms = 1e300;
     const int grids[] = {512, 1024, 2048, 4096, 8192, 16384};
     // an even number where tiles are one of the shapes, as pennant_autotune
-    const int n = cycles + (tiled(b, form) ? cycles & 1 : 0);
+    const bool tile = tiled(b, form);
+    const int n = cycles + (tile ? cycles & 1 : 0);
     auto timed = [&]() {
         b->tune.graph = 0;
         drop_graph(b);
@@ -497,13 +498,14 @@ int pennant_batch_autotune(pennant_batch* b, int mode, int cycles, double* best_
         if (!rc && ms < bms) { bms = ms; best = b->tune; }
     };
     // the tile cycle (its grid follows from the meshes), then the separate
-    // passes' grids
-    if (tiled(b, form)) timed();
+    // passes' grids; as in pennant_autotune tiles are switched off for this form
+    // only, and only where they were timed
+    if (tile) timed();
     for (int xcd = 0; xcd <= 1; ++xcd) {
         for (int g : grids) {
             if (rc) break;
             b->tune = keep;
-            b->tune.tiles = 0;
+            if (tile) b->tune.tiles &= ~(1 << form);
             b->tune.max_blocks = g;
             b->tune.xcd = xcd;
             timed();

@@ -539,10 +539,11 @@ static bool pipelined(const pennant_problem* pb, int form) {
 }
 
 // Whether cycles of `form` run as tile cycles: on structured meshes, unless a
-// tuning asks for one of the separate passes' own forms.
+// tuning asks for one of the separate passes' own forms (k1_layout is the FP64
+// form's alone).
 static bool tiled(const pennant_problem* pb, int form) {
-    return pb->tile.nzx > 0 && pb->tune.tiles && pb->tune.k1_layout == 0 && !pb->cap_buf &&
-           (pb->tile.pie || pb->tune.rect_maps) && !pipelined(pb, form);
+    return pb->tile.nzx > 0 && (pb->tune.tiles >> form & 1) && (form != FORM_FP64 || pb->tune.k1_layout == 0) &&
+           !pb->cap_buf && (pb->tile.pie || pb->tune.rect_maps) && !pipelined(pb, form);
 }
 
 // One cycle of `form` (ev as for fused_cycle / fused_cycle_pipe).  A
@@ -733,7 +734,7 @@ int pennant_set_tuning(pennant_problem* pb, const char* key, int value) {
     }
     if (!strcmp(key, "tiles")) {
         if (value != 0 && value != 1) return PENNANT_EINVAL;
-        pb->tune.tiles = value;
+        pb->tune.tiles = value ? PN_TILES_ALL : 0;
         return 0;
     }
     if (!strcmp(key, "rect_maps")) {
@@ -750,7 +751,7 @@ int pennant_get_tuning(pennant_problem* pb, const char* key) {
     if (!strcmp(key, "xcd")) return pb->tune.xcd;
     if (!strcmp(key, "graph")) return pb->tune.graph;
     if (!strcmp(key, "pipeline")) return pb->tune.pipeline;
-    if (!strcmp(key, "tiles")) return (pb->tune.tiles && pb->tile.nzx > 0) ? 1 : 0;
+    if (!strcmp(key, "tiles")) return (pb->tune.tiles == PN_TILES_ALL && pb->tile.nzx > 0) ? 1 : 0;
     // whether the fused kernels compute the zones' points and corner slots
     if (!strcmp(key, "rect_maps")) return (pb->tune.rect_maps && pb->rect_nzx > 0) ? 1 : 0;
     return PENNANT_EINVAL;
@@ -821,15 +822,16 @@ int pennant_autotune(pennant_problem* pb, int mode, int cycles, double* best_ms)
     };
     pb->tune.graph = 0;                           // direct launches while shapes change
     // the tile cycle (its grid follows from the mesh), then the separate
-    // passes' shapes
+    // passes' shapes.  What is decided about tiles is decided for this form, and
+    // where they were not timed (a capture buffer, a mesh that does not qualify)
+    // nothing is.
     pb->tune.k1_layout = 0;
-    pb->tune.pipeline = 0;
-    pb->tune.tiles = keep.tiles;
+    if (form != FORM_FP64) pb->tune.pipeline = 0;
     if (tiled(pb, form)) {
         n += n & 1;
         timed();
+        pb->tune.tiles &= ~(1 << form);
     }
-    pb->tune.tiles = 0;
     for (int layout = 0; layout <= (form == FORM_FP64 ? 1 : 0) && !rc; ++layout)
       for (int pipe = 0; pipe < npipe && !rc; ++pipe)
         for (int xcd = 0; xcd <= 1 && !rc; ++xcd)

@@ -63,6 +63,7 @@ inline bool corner_slots_fit(int64_t nump, int64_t entries) {
 #define PN_HEAVY 64        // points with more corners get a whole block in K2
 
 // Launch-shape choices of the fused cycle (pennant_set_tuning).
+#define PN_TILES_ALL 7     // Tuning::tiles: bit 1 << FORM_* for each form
 struct Tuning {
     int k1_layout = 0;       // 0 zone per thread, 1 corner per lane
     int max_blocks = 4096;   // grid cap of the grid-stride K1/K3 launches
@@ -70,7 +71,7 @@ struct Tuning {
     int graph = 1;           // batched cycles through a captured HIP graph
     int pipeline = 0;        // mixed forms: next cycle's predictor in the corrector pass
     int rect_maps = 1;       // structured rect meshes: zone points and corner slots computed, not loaded
-    int tiles = 1;           // structured meshes: the whole cycle in one kernel over tiles of zones
+    int tiles = PN_TILES_ALL;  // structured meshes: the whole cycle in one kernel over tiles of zones, by form
 };
 
 struct Params {

@@ -17,11 +17,13 @@ int64_t fake_fail_malloc, fake_fail_bytes, fake_fail_copy;
 int64_t fake_launches;                  /* kernels run so far */
 int64_t fake_live;                      /* device bytes in use */
 int64_t fake_max_threads;               /* most threads of a launch along x */
+char fake_slow[64];                     /* kernels with this in their name take 100 times as long */
+static int64_t fake_time;
 static char fake_log[1 << 20];          /* names of the kernels run */
 static size_t fake_log_len;
 static hipError_t last_error;
 static int capturing;
-static int64_t captured;
+static int64_t captured, cap_time;
 static char cap_log[1 << 16];
 static size_t cap_len;
 
@@ -42,6 +44,7 @@ void fake_clear(void) {
     fake_launches = 0;
     fake_max_threads = 0;
 }
+static int64_t cost(const char* name) { return fake_slow[0] && strstr(name, fake_slow) ? 100 : 1; }
 static void put(char* log, size_t cap, size_t* len, const char* s, size_t n) {
     if (*len + n + 2 < cap) {
         memcpy(log + *len, s, n);
@@ -81,11 +84,13 @@ hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** args, size_t sh
     if ((int64_t)threads > fake_max_threads) fake_max_threads = (int64_t)threads;
     if (capturing) {
         ++captured;
+        cap_time += cost(name);
         put(cap_log, sizeof cap_log, &cap_len, name, strlen(name));
         put(cap_log, sizeof cap_log, &cap_len, "\n", 1);
         return OK;
     }
     ++fake_launches;
+    fake_time += cost(name);
     put(fake_log, sizeof fake_log, &fake_log_len, name, strlen(name));
     put(fake_log, sizeof fake_log, &fake_log_len, "\n", 1);
     return OK;
@@ -126,16 +131,17 @@ hipError_t hipDeviceSynchronize(void) { return OK; }
 hipError_t hipStreamBeginCapture(hipStream_t s, int m) {
     (void)s; (void)m;
     capturing = 1;
-    captured = 0;
+    captured = cap_time = 0;
     cap_len = 0;
     return OK;
 }
-typedef struct { int64_t n; size_t len; char log[sizeof cap_log]; } graph;
+typedef struct { int64_t n, time; size_t len; char log[sizeof cap_log]; } graph;
 hipError_t hipStreamEndCapture(hipStream_t s, void** g) {
     (void)s;
     graph* q = malloc(sizeof *q);
     capturing = 0;
     q->n = captured;
+    q->time = cap_time;
     q->len = cap_len;
     memcpy(q->log, cap_log, cap_len);
     *g = q;
@@ -153,13 +159,14 @@ hipError_t hipGraphLaunch(void* e, hipStream_t s) {
     (void)s;
     graph* q = e;
     fake_launches += q->n;
+    fake_time += q->time;
     put(fake_log, sizeof fake_log, &fake_log_len, q->log, q->len);
     return OK;
 }
 hipError_t hipEventCreate(void** e) { *e = calloc(1, 8); return OK; }
 hipError_t hipEventCreateWithFlags(void** e, unsigned f) { (void)f; return hipEventCreate(e); }
 hipError_t hipEventDestroy(void* e) { free(e); return OK; }
-hipError_t hipEventRecord(void* e, hipStream_t s) { (void)s; *(int64_t*)e = fake_launches; return OK; }
+hipError_t hipEventRecord(void* e, hipStream_t s) { (void)s; *(int64_t*)e = fake_time; return OK; }
 hipError_t hipEventSynchronize(void* e) { (void)e; return OK; }
 hipError_t hipEventElapsedTime(float* ms, void* a, void* b) {
     *ms = (float)(*(int64_t*)b - *(int64_t*)a);

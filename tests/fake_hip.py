@@ -3,6 +3,7 @@
 run, allocations and copies that fail where a test says so, and time counted in
 kernels.  The code sees `pa` (the binding), `wd` (its decks), `fake` (the
 runtime: fail_malloc, fail_bytes, fail_copy, launches, live, max_threads),
+`slow(name)`, which makes kernels of that name take 100 times as long, and
 `clear()` and `names()`, the kernels run since."""
 import subprocess
 import sys
@@ -23,6 +24,7 @@ class _Fake:
     def __setattr__(self, k, v): ctypes.c_int64.in_dll(_f, "fake_" + k).value = v
 fake = _Fake()
 clear = _f.fake_clear
+def slow(name): (ctypes.c_char * 64).in_dll(_f, "fake_slow").value = name.encode()
 def names(): return _f.fake_names().decode().split()
 import pennant_amd as pa
 from pennant_amd import decks as wd
