@@ -258,7 +258,7 @@ pennant_batch* pennant_batch_create(const char* const* decks, int n, char* errbu
     b->part_d = (double*)al(2 * units.size(), 8);
     b->part_i = (int*)al(2 * units.size(), 4);
     if (!ok) return fail(b, "device allocation failed");
-    if (batch_tile_setup(b, meshes)) return fail(b, "device allocation failed");
+    if (batch_tile_setup(b, meshes)) return fail(b, "batch upload failed");
     int rc = (int)hipMemcpy(b->mapsp1, mapsp1.data(), S * 4, hipMemcpyHostToDevice);
     if (!rc) rc = (int)hipMemcpy(b->pcbeg, pcbeg.data(), (P + 1) * 4, hipMemcpyHostToDevice);
     if (!rc) rc = (int)hipMemcpy(b->pcpos, pcpos.data(), S * 4, hipMemcpyHostToDevice);

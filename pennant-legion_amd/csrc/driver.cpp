@@ -262,17 +262,18 @@ int64_t count_of(const pennant_problem* pb, int kind) {
 }
 
 // The arena of a small problem, from what its fields, maps, fused and tile
-// cycles take (too small an estimate costs allocations, nothing else).
-bool arena_begin(pennant_problem* pb) {
+// cycles take (too small an estimate costs allocations, nothing else; so does an
+// arena that cannot be had).
+void arena_begin(pennant_problem* pb) {
     const size_t P = pb->dm.nump, Z = pb->dm.numz, S = pb->dm.nums, C = (size_t)corner_slots((int64_t)P, (int64_t)S);
     size_t n = 24 * S + 12 * Z + 4 * P                       // maps
                + 36 * C + 32 * S + 32 * P + 16 * Z           // corner records, side forces, point values, lists
                + 32 * P + 42 * Z                             // the tile cycle's second state
                + ((size_t)512 << 10);                        // partials, workspaces, rounding
     for (const FieldSpec& fs : kFields) n += (size_t)fs.ncomp * count_of(pb, fs.kind) * sizeof(double);
-    if (n > PN_ARENA_MAX) return true;
-    pb->arena_size = n;
-    return zeroed(pb, n, &pb->arena);
+    if (n > PN_ARENA_MAX) return;
+    if (zeroed(pb, n, &pb->arena)) pb->arena_size = n;
+    else (void)hipGetLastError();
 }
 
 #define CK(x) do { int _e = (int)(x); if (_e) return _e; } while (0)
@@ -425,7 +426,7 @@ pennant_problem* pn::create_problem(const Params& prm, HostMesh&& hm, int npown,
 
     pennant_mesh& m = pb->dm;
     m.nump = h.nump; m.numz = h.numz; m.nums = h.nums; m.maxznump = h.maxznump;
-    if (!arena_begin(pb)) return fail("device allocation failed");
+    arena_begin(pb);
     m.mapsp1 = upload(pb, h.mapsp1); m.mapsp2 = upload(pb, h.mapsp2); m.mapsz = upload(pb, h.mapsz);
     m.mapss3 = upload(pb, h.mapss3); m.mapss4 = upload(pb, h.mapss4); m.znump = upload(pb, h.znump);
     m.zsbeg = upload(pb, h.zsbeg); m.pcbeg = upload(pb, h.pcbeg); m.pcside = upload(pb, h.pcside);

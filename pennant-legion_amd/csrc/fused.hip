@@ -3774,7 +3774,8 @@ int tile_cycles(pennant_problem* pb, int form, int n) {
 // checked every side) or a pie of at least two rows in the generator's
 // numbering, every side's point checked here against the formula the kernel
 // uses.  Allocates the second set of state arrays, the partials and the
-// learned form's list.
+// learned form's list; where there is no memory for them (72 bytes a zone) the
+// problem runs as separate passes.
 int tile_setup(pennant_problem* pb) {
     const HostMesh& h = pb->hm;
     TileState& q = pb->tile;
@@ -3803,7 +3804,10 @@ int tile_setup(pennant_problem* pb) {
     const size_t bytes = PN_CHAIN_BYTES + (size_t)(4 * P + 5 * Z + 2 * (int64_t)q.npart) * 8 +
                          (size_t)(2 * (int64_t)q.npart + tiles + 2) * 4;
     char* m = (char*)problem_alloc(pb, bytes);
-    if (!m) return (int)hipErrorOutOfMemory;
+    if (!m) {
+        (void)hipGetLastError();
+        return 0;
+    }
     q.chain = m;
     double* d = (double*)(m + PN_CHAIN_BYTES);
     for (int k = 0; k < 9; ++k) {
@@ -3912,7 +3916,10 @@ int batch_tile_setup(pennant_batch* b, const std::vector<TileState>& meshes) {
     const size_t bytes = N * PN_CHAIN_BYTES + (4 * P + 5 * Z) * 8 + tiles.size() * sizeof(BTile) +
                          tri.size() * sizeof(BUnit) + origins.size() * sizeof(BHeavy);
     char* m = nullptr;
-    if (hipMalloc((void**)&m, bytes) != hipSuccess) return (int)hipErrorOutOfMemory;
+    if (hipMalloc((void**)&m, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;                            // no memory for a second state: separate passes
+    }
     b->allocs.push_back(m);
     b->chain = m;                            // the problems' slots, then their second control blocks
     double* d = (double*)(m + N * PN_CHAIN_BYTES);
