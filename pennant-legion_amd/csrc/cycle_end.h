@@ -259,8 +259,12 @@ __global__ void __launch_bounds__(64) k_chain_begin(slot_t* sets) {
     for (int k = 0; k < 3; ++k) slots_reset(sets + k * PN_SLOT_SET);
 }
 
-// Memory of a chain: three sets of slots and a second control block.
-#define PN_CHAIN_BYTES (3 * PN_SLOT_SET * 8 + 256)
+// Memory of a chain: three sets of slots and a second control block.  (A
+// batch's chains lie as all their slots and then an array of control blocks,
+// with other arrays after it.)
+#define PN_CHAIN_CTL 256
+#define PN_CHAIN_BYTES (3 * PN_SLOT_SET * 8 + PN_CHAIN_CTL)
+static_assert(sizeof(Ctl) <= PN_CHAIN_CTL, "a chain's second control block");
 inline slot_t* chain_sets(void* m) { return static_cast<slot_t*>(m); }
 inline Ctl* chain_ctl(void* m) { return reinterpret_cast<Ctl*>(static_cast<slot_t*>(m) + 3 * PN_SLOT_SET); }
 // Step k of a chain on the problem's control block.
