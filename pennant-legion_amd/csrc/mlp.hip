@@ -634,10 +634,13 @@ int pennant_mlp_forward(pennant_mlp* m, const float* x, int64_t n, float* y, int
         MCK(hipGetLastError());
         return (int)hipStreamSynchronize(m->stream);
     }
-    RowArgs a = row_args(m, n, x);
-    a.y = y;
-    if ((n + 31) / 32 > 0x7fffffff) return PENNANT_EINVAL;
-    hipLaunchKernelGGL(k_rows<false>, dim3((unsigned)((n + 31) / 32)), dim3(64), 0, m->stream, a);
+    // a launch has fewer than 2^32 threads, two a row
+    constexpr int64_t chunk = (int64_t)1 << 30;
+    for (int64_t b0 = 0; b0 < n; b0 += chunk) {
+        RowArgs a = row_args(m, n - b0 < chunk ? n - b0 : chunk, x + b0 * PN_MLP_NF);
+        a.y = y + 2 * b0;
+        hipLaunchKernelGGL(k_rows<false>, dim3((unsigned)((a.n + 31) / 32)), dim3(64), 0, m->stream, a);
+    }
     MCK(hipGetLastError());
     return (int)hipStreamSynchronize(m->stream);
 }
