@@ -16,6 +16,7 @@ enum { OK = 0, OUT_OF_MEMORY = 2, INVALID_CONFIGURATION = 9 };
 int64_t fake_fail_malloc, fake_fail_bytes, fake_fail_copy;
 int64_t fake_launches;                  /* kernels run so far */
 int64_t fake_live;                      /* device bytes in use */
+int64_t fake_copied;                    /* bytes of the last asynchronous copy */
 int64_t fake_max_threads;               /* most threads of a launch along x */
 char fake_slow[64];                     /* kernels with this in their name take 100 times as long */
 static int64_t fake_time;
@@ -121,6 +122,7 @@ hipError_t hipMemcpy(void* d, const void* s, size_t n, int k) { (void)k; memmove
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, int k, hipStream_t q) {
     (void)q;
     if (fake_fail_copy > 0 && --fake_fail_copy == 0) return ret(OUT_OF_MEMORY);
+    fake_copied = (int64_t)n;
     return hipMemcpy(d, s, n, k);
 }
 hipError_t hipStreamCreate(hipStream_t* s) { *s = calloc(1, 8); return OK; }
