@@ -4075,9 +4075,11 @@ FusedArgs piece_args(pennant_pieces* pp, int q) {
 // unit is at most PN_BLOCK zones of one side-count run, or points, of one
 // piece), which reads its piece's arrays from a table.  What bounds a cycle is
 // the latency of its six dependent launches.  Noh pie 640 x 480 in 6 pieces,
-// FP64, 100 cycles and the results' copies: 179 -> 92 us a cycle.  Before, with
+// FP64, 100 cycles and the results' copies: 179 -> 81 us a cycle.  Before, with
 // a launch per piece and run on the pieces' own streams, forked and joined
-// around each phase, it was 34 launches and 30 event waits.
+// around each phase, it was 34 launches and 30 event waits.  A run in one piece
+// has nothing to gain from the tables and takes the launches of a problem (mixed,
+// Sedov 1440^2: 188 us a cycle through the tables, 170 without).
 namespace {
 
 template <int FORM>
@@ -4189,6 +4191,10 @@ int pieces_setup(pennant_pieces* pp) {
 int pieces_cycle(pennant_pieces* pp, int form) {
     if (form == FORM_LEARNED || pp->pc.empty()) return PENNANT_EINVAL;
     const bool mixed = (form != FORM_FP64);
+    if (pp->pc.size() == 1) {                // the whole mesh: a problem's own passes
+        if (mixed) pp->zre_stale = true;
+        return fused_cycle(pp->pc[0], nullptr, form);
+    }
     hipStream_t s = pp->pc[0]->stream;
     const FusedArgs* A = (const FusedArgs*)pp->args;
     const Ctl* ctl = pp->pc[0]->ctl;
