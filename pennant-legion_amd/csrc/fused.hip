@@ -45,6 +45,7 @@
 // count (rect: one run of quads; pie: triangles, then quads).
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include "closure.h"
 #include "common.h"
@@ -650,12 +651,14 @@ __device__ __forceinline__ void load_sides(const float* w, const SideW& sw, f2 (
 //               forces);
 //   CL_CAPTURE  the exact coefficient, recording training tuples;
 //   CL_PACKED   CL_LEARNED with the wave's gated corners packed into as few
-//               evaluations as possible, as CL_RECOMP does.
+//               evaluations as possible, as CL_RECOMP does;
+//   CL_LEAN     CL_PACKED in fewer registers: 32 corners at a time instead of
+//               two groups in one stream, the weights read at each use.
 // The gate: a compressing corner (cdiv < 0) whose quadratic term matters,
 // G du > PN_GATE (q1 zss + G du), i.e. f9 > PN_GATE.  Below it the exact
 // coefficient equals its acoustic limit q1 zss + G du to within 0.1%; the
 // round-off velocities of a quiescent region stay far below it.
-enum { CL_EXACT = 0, CL_LEARNED = 1, CL_CAPTURE = 2, CL_FLAG = 3, CL_RECOMP = 4, CL_PACKED = 5 };
+enum { CL_EXACT = 0, CL_LEARNED = 1, CL_CAPTURE = 2, CL_FLAG = 3, CL_RECOMP = 4, CL_PACKED = 5, CL_LEAN = 6 };
 #define PN_GATE 1.e-3f
 
 // Zone counters of the learned form, summed per thread.
@@ -876,7 +879,7 @@ __device__ __forceinline__ double zone_pred_mixed_core(const FusedArgs& a, const
                                                        const d2 (&u0)[NS], const ZoneState& st,
                                                        const float (&mf0)[NS], double dt, int& bad,
                                                        bool valid, ClCount& cnt, Out& out) {
-    constexpr bool NET = CL == CL_LEARNED || CL == CL_RECOMP || CL == CL_PACKED;
+    constexpr bool PACK = CL == CL_RECOMP || CL == CL_PACKED || CL == CL_LEAN, NET = CL == CL_LEARNED || PACK;
     MixedFrame<NS> F;
 #pragma unroll
     for (int k = 0; k < NS; ++k) F.mf[k] = mf0[k];
@@ -968,7 +971,7 @@ __device__ __forceinline__ double zone_pred_mixed_core(const FusedArgs& a, const
         crmu[k] = (cdiv[k] > 0.f) ? 0.f : zkur * zrpf * cevol[k];
     }
     if constexpr (CL == CL_FLAG) cnt.flag = comp;
-    if constexpr (CL == CL_RECOMP || CL == CL_PACKED) {
+    if constexpr (PACK) {
         // The wave's corners that need the network, packed into as few
         // evaluations as possible: corner k of a lane goes to slot off_k +
         // its rank among the lanes needing corner k, in an LDS row of the
@@ -1004,9 +1007,10 @@ __device__ __forceinline__ double zone_pred_mixed_core(const FusedArgs& a, const
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
         // the lane's weight fragments, read once for all of the wave's
-        // evaluations
-        MlpRegs wr;
-        if (total > 0) mlp_load_regs(a.pack, lane, wr);
+        // evaluations (CL_LEAN: at each use)
+        typename std::conditional<CL == CL_LEAN, MlpPackSrc, MlpRegs>::type wr;
+        if constexpr (CL == CL_LEAN) wr = {a.pack, lane};
+        else if (total > 0) mlp_load_regs(a.pack, lane, wr);
         for (int e = 0; e < total; e += 64) {
             const int sl = e + lane;
             const bool act = sl < total;
@@ -1019,7 +1023,7 @@ __device__ __forceinline__ double zone_pred_mixed_core(const FusedArgs& a, const
             hi[2] = 0u;
             hi[3] = 0u;
             float y0, y1;
-            mlp_wave_w<MlpRegs, true>(wr, lo, hi, (uint32_t)am != 0u, (am >> 32) != 0u, y0, y1);
+            mlp_wave_w<decltype(wr), CL != CL_LEAN>(wr, lo, hi, (uint32_t)am != 0u, (am >> 32) != 0u, y0, y1);
             if (act) {
                 xw[sl][0] = __float_as_uint(y0);
                 xw[sl][1] = __float_as_uint(y1);
@@ -2474,7 +2478,7 @@ __device__ __forceinline__ bool tile_body(const FusedArgs& a, const TileOut& o, 
         q.x0 = in.x[0];
         q.u0 = in.u[0];
         // the network runs across the wave, so every lane takes part
-        if (CL == CL_PACKED || quad)
+        if (CL == CL_PACKED || CL == CL_LEAN || quad)
             dtz = zone_pred_mixed_core<4, CL>(a, in.x, in.u, st, mf, dt, bad, quad, cnt, keep);
     }
     if (tri) {
@@ -2503,7 +2507,7 @@ __device__ __forceinline__ bool tile_body(const FusedArgs& a, const TileOut& o, 
     } else {
         __syncthreads();
     }
-    if constexpr (CL == CL_PACKED) {
+    if constexpr (CL == CL_PACKED || CL == CL_LEAN) {
         if (own) {
             total.learned += cnt.learned;
             total.fallback += cnt.fallback;
@@ -2753,10 +2757,14 @@ __global__ void __launch_bounds__(PN_BLOCK) k_tri_corr(FusedArgs a, CycleStep s,
 // The learned form's tiles that have a zone for the network (in the ring or
 // inside): the whole tile again, the network evaluated for the wave's gated
 // corners packed together.  Their order in the list is not fixed, their
-// results are.  Two waves per SIMD, for which it spills 31 registers, where many
-// tiles may be listed; one, without, on the small rects of linked cycles, whose
-// listed tiles all run at once: learned 333 x 217 26.6 -> 24.8 us a cycle, 420^2
-// 36.5 -> 32.9, tube 1024 x 128 32.6 -> 29.6 (1440^2 145 -> 147, not taken).
+// results are.  Where many tiles may be listed, two waves per SIMD and the lean
+// evaluation (240 VGPRs; two groups of corners in one stream spilled 31 there).
+// Learned Sedov 1440^2, a cycle after 900 cycles 137 -> 134 us, after 37600 208 ->
+// 187, after 50000 232 -> 203; the separate passes take 192, 202 and 204.  On the
+// small rects of linked cycles, whose listed tiles all run at once, one wave and
+// both groups in one stream, without spills: learned 333 x 217 26.6 -> 24.8 us a
+// cycle, 420^2 36.5 -> 32.9, tube 1024 x 128 32.6 -> 29.6 (lean 31.4 -> 32.7 on
+// 420^2, 29.2 -> 31.0 on the tube).
 template <bool LINK>
 __global__ void __launch_bounds__(PN_BLOCK) __attribute__((amdgpu_waves_per_eu(LINK ? 1 : 2)))
 k_tile_list(FusedArgs a, TileArgs t) {
@@ -2782,7 +2790,7 @@ k_tile_list(FusedArgs a, TileArgs t) {
         tile_at(t, tile, i0, j0);
         TileIn<float> in;
         tile_load<float>(b, t.g, i0, j0, in);
-        (void)tile_body<float, CL_PACKED>(b, t.o, t.g, i0, j0, in, t.step.put, tile, dt, zre, cnt);
+        (void)tile_body<float, LINK ? CL_PACKED : CL_LEAN>(b, t.o, t.g, i0, j0, in, t.step.put, tile, dt, zre, cnt);
     }
     const int nl = block_sum(cnt.learned);
     const int nf = block_sum(cnt.fallback);
