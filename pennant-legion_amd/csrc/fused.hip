@@ -3773,6 +3773,8 @@ int tile_cycles(pennant_problem* pb, int form, int n) {
     // a pie's few blocks of triangles always pay for the fold; the learned
     // form's triangles have a list pass of their own
     const bool linked = n > 0 && (q.pie ? form != FORM_LEARNED : tiles <= PN_LINK_TILES);
+    // an error that another call has left is not to end a pair halfway
+    if (const int rc = (int)hipGetLastError()) return rc;
     for (int k = 0; k < n; ++k)
         if (const int rc = tile_cycle(pb, form, k, linked)) return rc;
     return linked ? chain_end(pb, q.chain, n, form == FORM_FP64 ? 1 : 0) : 0;
@@ -3994,6 +3996,7 @@ static int batch_tile_cycle(pennant_batch* b, int form, int k) {
 int batch_tile_cycles(pennant_batch* b, int form, int n) {
     if (!b->ntiles || (n & 1) || form == FORM_LEARNED) return PENNANT_EINVAL;
     if (n < 1) return 0;
+    if (const int rc = (int)hipGetLastError()) return rc;    // as tile_cycles
     for (int k = 0; k < n; ++k)
         if (const int rc = batch_tile_cycle(b, form, k)) return rc;
     BatchChain c = batch_chain(b, n, form == FORM_FP64 ? 1 : 0);

@@ -1954,6 +1954,8 @@ int task_chain_setup(pennant_problem* pb) {
 
 int launch_task_cycles(pennant_problem* pb, int n) {
     if (n < 1) return 0;
+    // an error that another call has left is not to end a cycle halfway
+    if (const int rc = launch_status()) return rc;
     const pennant_mesh& m = pb->dm;
     const Params& q = pb->prm;
     const int tz = wide_tile_zones(&m, 1), nb = tz ? tile_blocks(&m, tz) : 0;

@@ -22,14 +22,14 @@ char fake_slow[64];                     /* kernels with this in their name take 
 static int64_t fake_time;
 static char fake_log[1 << 20];          /* names of the kernels run */
 static size_t fake_log_len;
-static hipError_t last_error;
+int64_t fake_error;                     /* the error that hipGetLastError returns next */
 static int capturing;
 static int64_t captured, cap_time;
 static char cap_log[1 << 16];
 static size_t cap_len;
 
 static hipError_t ret(hipError_t e) {
-    if (e) last_error = e;
+    if (e) fake_error = e;
     return e;
 }
 
@@ -177,8 +177,8 @@ hipError_t hipEventElapsedTime(float* ms, void* a, void* b) {
 hipError_t hipGetDevice(int* d) { *d = 0; return OK; }
 hipError_t hipGetDeviceCount(int* n) { *n = 1; return OK; }
 hipError_t hipGetLastError(void) {
-    const hipError_t e = last_error;
-    last_error = OK;
+    const hipError_t e = (hipError_t)fake_error;
+    fake_error = OK;
     return e;
 }
 const char* hipGetErrorString(hipError_t e) { return e ? "error" : "no error"; }
