@@ -505,7 +505,7 @@ RowArgs row_args(const pennant_mlp* m, int64_t n, const float* x) {
 
 // Forward and backward of the B rows idx (NULL: 0 .. B - 1) of the tuples;
 // `read` (may be NULL) is recorded once idx has been read.
-void launch_batch(pennant_mlp* m, const float* tuples, const int* idx, int64_t B, hipEvent_t read) {
+int launch_batch(pennant_mlp* m, const float* tuples, const int* idx, int64_t B, hipEvent_t read) {
     hipStream_t s = m->stream;
     RowArgs a = row_args(m, B, tuples);
     a.idx = idx;
@@ -513,7 +513,7 @@ void launch_batch(pennant_mlp* m, const float* tuples, const int* idx, int64_t B
     a.xt = m->xt; a.h1t = m->h1t; a.h2t = m->h2t; a.dyt = m->dyt; a.dz2t = m->dz2t; a.dz1t = m->dz1t;
     a.lrow = m->lrow;
     hipLaunchKernelGGL(k_rows<true>, dim3((unsigned)((B + 31) / 32)), dim3(64), 0, s, a);
-    if (read) (void)hipEventRecord(read, s);
+    if (read) MCK(hipEventRecord(read, s));
     GradArgs g;
     g.rows = B;
     g.ld = m->cap;
@@ -527,6 +527,7 @@ void launch_batch(pennant_mlp* m, const float* tuples, const int* idx, int64_t B
     g.g = m->g;
     g.lossp = m->lossp;
     hipLaunchKernelGGL(k_grads, dim3(g.ksplit * PN_GTILES / 4 + PN_MLP_NO + PN_MLP_NH + nb(B)), dim3(256), 0, s, g);
+    return (int)hipGetLastError();
 }
 UpdateArgs update_args(pennant_mlp* m, int64_t B, float* loss) {
     UpdateArgs u = {};
@@ -648,7 +649,7 @@ int pennant_mlp_forward(pennant_mlp* m, const float* x, int64_t n, float* y, int
 int pennant_mlp_loss_grad(pennant_mlp* m, const float* tuples, int64_t n, float* grad, float* loss) {
     if (n <= 0 || n > (1 << 30)) return PENNANT_EINVAL;
     MCK(ensure_batch(m, n, false));
-    launch_batch(m, tuples, nullptr, n, nullptr);
+    MCK(launch_batch(m, tuples, nullptr, n, nullptr));
     const UpdateArgs u = update_args(m, n, m->lossp + nb(n));
     hipLaunchKernelGGL(k_update<false>, dim3(nb(PN_MLP_NPARAM + 1)), dim3(256), 0, m->stream, u);
     MCK(hipGetLastError());
@@ -662,6 +663,7 @@ int pennant_mlp_loss_grad(pennant_mlp* m, const float* tuples, int64_t n, float*
 int pennant_mlp_train(pennant_mlp* m, const float* tuples, int64_t n, int steps, int batch, float lr,
                       uint64_t seed, float* loss_out) {
     if (n <= 0 || n > (1 << 30) || steps < 0 || batch <= 0 || batch > (1 << 22)) return PENNANT_EINVAL;
+    MCK(hipGetLastError());      // what another call has left is reported before the first step
     MCK(ensure_batch(m, batch, true));
     if (steps > m->loss_cap) {
         if (m->losses) (void)hipFree(m->losses);
@@ -673,13 +675,14 @@ int pennant_mlp_train(pennant_mlp* m, const float* tuples, int64_t n, int steps,
     std::mt19937_64 rng(seed);
     std::uniform_int_distribution<int64_t> pick(0, n - 1);
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    for (int st = 0; st < steps; ++st) {
+    int rc = 0;
+    for (int st = 0; st < steps && !rc; ++st) {
         // a step's rows are drawn while the steps before it run; the kernel
         // reads them from the host's list, which is free again two steps later
         int* idx = m->idx_host[st & 1];
-        if (st >= 2) MCK(hipEventSynchronize(m->read[st & 1]));
+        if (st >= 2 && (rc = (int)hipEventSynchronize(m->read[st & 1]))) break;
         for (int b = 0; b < batch; ++b) idx[b] = (int)pick(rng);
-        launch_batch(m, tuples, idx, batch, m->read[st & 1]);
+        if ((rc = launch_batch(m, tuples, idx, batch, m->read[st & 1]))) break;
         m->adam_t += 1;
         UpdateArgs u = update_args(m, batch, m->losses + st);
         u.c1 = 1.f - std::pow(b1, (float)m->adam_t);
@@ -690,14 +693,16 @@ int pennant_mlp_train(pennant_mlp* m, const float* tuples, int64_t n, int steps,
         u.p = m->p; u.m = m->m; u.v = m->v;
         u.w1b = m->w1b; u.w2b = m->w2b; u.w2t = m->w2t; u.w3b = m->w3b; u.pack = m->pack;
         hipLaunchKernelGGL(k_update<true>, dim3(nb(PN_MLP_NPARAM + 1)), dim3(256), 0, m->stream, u);
+        rc = (int)hipGetLastError();
     }
-    MCK(hipGetLastError());
-    if (loss_out && steps > 0)
-        MCK(hipMemcpyAsync(loss_out, m->losses, (size_t)steps * 4, hipMemcpyDeviceToHost, m->stream));
-    MCK(hipStreamSynchronize(m->stream));
+    if (!rc && loss_out && steps > 0)
+        rc = (int)hipMemcpyAsync(loss_out, m->losses, (size_t)steps * 4, hipMemcpyDeviceToHost, m->stream);
+    // (also after an error: the kernels read the caller's tuples and the row lists)
+    const int rc2 = (int)hipStreamSynchronize(m->stream);
+    if (rc || rc2) return rc ? rc : rc2;
     if (loss_out)
         for (int st = 0; st < steps; ++st) loss_out[st] /= (float)batch;
-    return (int)hipGetLastError();
+    return 0;
 }
 
 }  // extern "C"

@@ -9,11 +9,12 @@
 typedef int hipError_t;
 typedef void* hipStream_t;
 typedef struct { uint32_t x, y, z; } dim3;
-enum { OK = 0, OUT_OF_MEMORY = 2, INVALID_CONFIGURATION = 9 };
+enum { OK = 0, OUT_OF_MEMORY = 2, INVALID_CONFIGURATION = 9, UNKNOWN = 999 };
 
 /* failures: the n-th hipMalloc from now of at least fail_bytes, the n-th
- * hipMemcpyAsync from now; 0: none */
-int64_t fake_fail_malloc, fake_fail_bytes, fake_fail_copy;
+ * hipMemcpyAsync or hipEventSynchronize from now; 0: none */
+int64_t fake_fail_malloc, fake_fail_bytes, fake_fail_copy, fake_fail_wait;
+int64_t fake_queued;                    /* kernels since the last wait for a stream */
 int64_t fake_launches;                  /* kernels run so far */
 int64_t fake_live;                      /* device bytes in use */
 int64_t fake_copied;                    /* bytes of the last asynchronous copy */
@@ -91,6 +92,7 @@ hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** args, size_t sh
         return OK;
     }
     ++fake_launches;
+    ++fake_queued;
     fake_time += cost(name);
     put(fake_log, sizeof fake_log, &fake_log_len, name, strlen(name));
     put(fake_log, sizeof fake_log, &fake_log_len, "\n", 1);
@@ -128,7 +130,7 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, int k, hipStream_t q
 hipError_t hipStreamCreate(hipStream_t* s) { *s = calloc(1, 8); return OK; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned f) { (void)f; return hipStreamCreate(s); }
 hipError_t hipStreamDestroy(hipStream_t s) { free(s); return OK; }
-hipError_t hipStreamSynchronize(hipStream_t s) { (void)s; return OK; }
+hipError_t hipStreamSynchronize(hipStream_t s) { (void)s; fake_queued = 0; return OK; }
 hipError_t hipDeviceSynchronize(void) { return OK; }
 hipError_t hipStreamBeginCapture(hipStream_t s, int m) {
     (void)s; (void)m;
@@ -169,7 +171,11 @@ hipError_t hipEventCreate(void** e) { *e = calloc(1, 8); return OK; }
 hipError_t hipEventCreateWithFlags(void** e, unsigned f) { (void)f; return hipEventCreate(e); }
 hipError_t hipEventDestroy(void* e) { free(e); return OK; }
 hipError_t hipEventRecord(void* e, hipStream_t s) { (void)s; *(int64_t*)e = fake_time; return OK; }
-hipError_t hipEventSynchronize(void* e) { (void)e; return OK; }
+hipError_t hipEventSynchronize(void* e) {
+    (void)e;
+    if (fake_fail_wait > 0 && --fake_fail_wait == 0) return ret(UNKNOWN);
+    return OK;
+}
 hipError_t hipEventElapsedTime(float* ms, void* a, void* b) {
     *ms = (float)(*(int64_t*)b - *(int64_t*)a);
     return OK;

@@ -2,8 +2,8 @@
 (fake_hip.c): the library's host code with kernels that are recorded and not
 run, allocations and copies that fail where a test says so, and time counted in
 kernels.  The code sees `pa` (the binding), `wd` (its decks), `fake` (the
-runtime: fail_malloc, fail_bytes, fail_copy, error, launches, live, copied,
-max_threads),
+runtime: fail_malloc, fail_bytes, fail_copy, fail_wait, error, launches, queued,
+live, copied, max_threads),
 `slow(name)`, which makes kernels of that name take 100 times as long, and
 `clear()` and `names()`, the kernels run since."""
 import subprocess
