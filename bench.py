@@ -25,9 +25,10 @@ Prints ONE JSON line on stdout:
               errors, shock radius at tstop; the 1% density gate
   energy      total energy (internal + kinetic) at t = 0 and at tstop, and
               its relative drift, per form
-  drop_in_tasks  the task form (FP64; every reference task's fields in memory
-              after each cycle) on the same workload from t = 0: us per cycle
-              and its compulsory bytes over that time, against 8 TB/s
+  task_form   the driver's task form (FP64; every reference task's fields in
+              memory after each cycle, tasks on the same zones or points sharing
+              a launch) on the same workload from t = 0: us per cycle and its
+              compulsory bytes over that time, against 8 TB/s
   cpu_baseline  the CPU oracle (a serial C++ restatement of the reference's
               CPU task bodies, and its OpenMP variant) on a bounded sample of
               the same workload, on this host (lscpu model, sockets, cores)
@@ -303,13 +304,13 @@ def main():
     ap.add_argument("--mode", default="learned", choices=["learned", "mixed", "fused", "tasks"],
                     help="learned: mixed precision with the learned QCS closure; mixed: mixed "
                          "precision with the exact QCS (both reported against the plain FP64 fused "
-                         "cycle on the same workload); fused: plain FP64 fused cycle; tasks: one "
-                         "launch per task")
+                         "cycle on the same workload); fused: plain FP64 fused cycle; tasks: every "
+                         "task's fields each cycle")
     ap.add_argument("--closure", default=None,
                     help="trained closure (.npz from pennant_amd.train_closure); default: the "
                          "package's closure_ensemble.npz")
     ap.add_argument("--tasks-steps", type=int, default=20,
-                    help="cycles of the FP64 task form timed for drop_in_tasks (0: skip)")
+                    help="cycles of the FP64 task form timed for task_form (0: skip)")
     ap.add_argument("--copy-mb", type=int, default=512,
                     help="size of the streaming-copy calibration (0 disables)")
     ap.add_argument("--k1", type=int, default=None, help="fused K1 layout: 0 zone/thread, 1 corner/lane")
@@ -568,7 +569,7 @@ def main():
         us = tms / args.tasks_steps * 1e3
         tb = 324 * S + 256 * Z + 245 * P
         gbs = tb / (us * 1e-6) / 1e9
-        log(f"drop-in tasks fp64: {us:.1f} us/cycle, {tb / 1e9:.3f} GB per cycle, "
+        log(f"task form fp64: {us:.1f} us/cycle, {tb / 1e9:.3f} GB per cycle, "
             f"{gbs:.1f} GB/s ({gbs / HBM_PEAK_GBS:.3f} of peak)")
         tasks = {"form": "plain-fp64-tasks", "us_per_cycle": round(us, 2),
                  "zone_cycles_per_s": round(Z / (us * 1e-6), 1),
@@ -604,7 +605,7 @@ def main():
     if roofline_fp64 is not None:
         line["roofline_fp64"] = roofline_fp64
     if tasks is not None:
-        line["drop_in_tasks"] = tasks
+        line["task_form"] = tasks
     if accuracy is not None:
         line["accuracy"] = accuracy
     if energy is not None:

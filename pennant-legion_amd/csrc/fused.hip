@@ -1627,6 +1627,12 @@ template <> struct Corners<float> {
     __device__ static double fy(const FusedArgs& a, int k) { return (double)a.fcrn[3 * k + 1]; }
 };
 
+// The slot of position c (CSR index k) of point p's corner list (the host's
+// corner_slot, with a.nump the mesh's or the batch arena's point count).
+__device__ __forceinline__ int corner_slot(const FusedArgs& a, int p, int c, int k) {
+    return (c < 4) ? c * a.nump + p : 4 * a.nump + k;
+}
+
 // Point gathers, fixed BCs, acceleration and position update.
 //
 // A high-valence point (the pie origin has one corner per centre triangle)
@@ -1635,12 +1641,6 @@ template <> struct Corners<float> {
 // order.  It is a serial chain of additions: with one lane for all three sums,
 // waiting for LDS at every corner, the point pass of a pie with 640 corners at
 // its origin took 18.7 us; now 11.5.  Called by every thread of the block.
-// The slot of position c (CSR index k) of point p's corner list (the host's
-// corner_slot, with a.nump the mesh's or the batch arena's point count).
-__device__ __forceinline__ int corner_slot(const FusedArgs& a, int p, int c, int k) {
-    return (c < 4) ? c * a.nump + p : 4 * a.nump + k;
-}
-
 template <typename T, class Update>
 __device__ __forceinline__ void point_heavy(const FusedArgs& a, int p, const Update& update) {
     using C = Corners<T>;
@@ -2282,8 +2282,8 @@ __global__ void __launch_bounds__(PN_FIN_BLOCK) k_finalize_la(FusedArgs a, int n
 // ascending side order), so the results are the same bits.
 //
 // What bounds it: a tile's chain of loads, arithmetic and barriers, with few
-// waves to hide it (FP64: 229 VGPRs, two waves per SIMD, vector unit 0.8 busy;
-// mixed: 128 VGPRs, four, 0.86 busy).  Larger tiles have less ring but more
+// waves to hide it (Sedov 1440^2 FP64: 240 VGPRs, two waves per SIMD, vector unit
+// 0.86 busy; mixed: 128 VGPRs, four, saturated).  Larger tiles have less ring but more
 // waves in step: 32 x 16 zones took 258 us where 16 x 16 takes 212 (FP64), and
 // 139 where it takes 117 (mixed).  FP64 square roots and quotients without the
 // scaling of their operands (9% fewer instructions) gained 1 to 3%; blocks
@@ -2294,8 +2294,10 @@ __global__ void __launch_bounds__(PN_FIN_BLOCK) k_finalize_la(FusedArgs a, int n
 // Per cycle, separate passes (for mixed and learned the pipelined ones) ->
 // tiles: FP64 Sedov 1440^2 306 -> 201 us, Noh pie 1024^2 178 -> 115 us; mixed
 // LeBlanc 4096 x 256 87 -> 55 us, 333 x 217 23 -> 10.1 us; learned Sedov
-// 1440^2 176 -> 147 us; FP64 90^2 12.6 -> 10.1 us by the linking alone.  It was faster at every size, so
-// structured meshes always take it.
+// 1440^2 176 -> 141 us early in its run, 182 -> 187 with a developed front (see
+// k_tile_list; separate passes unpipelined 202); FP64 90^2 12.6 -> 10.1 us by the
+// linking alone.  Faster at every size but for that front's last tenth of the
+// run, by 4%, so structured meshes take it by default.
 #define PN_TILE 16
 #define PN_TIN (PN_TILE - 2)
 // Most tiles of linked cycles (tile_cycles).  Linked and not, us a cycle, FP64
@@ -2423,8 +2425,9 @@ __device__ __forceinline__ void tile_load(const FusedArgs& a, const TileMesh& g,
 }
 
 // The tile whose first zone (ring included) is (i0, j0), loaded in `in`; its
-// dt limit, dvol ratio and bad sides go into slots as block `at`'s.  Returns whether a CL_FLAG tile has a zone for the network: such a
-// tile is left to the list kernel and stores nothing.
+// dt limit, dvol ratio and bad sides go into slots as block `at`'s.  Returns
+// whether a CL_FLAG tile has a zone for the network: such a tile is left to the
+// list kernel and stores nothing.
 template <typename T, int CL>
 __device__ __forceinline__ bool tile_body(const FusedArgs& a, const TileOut& o, const TileMesh& g, int i0, int j0,
                                           const TileIn<T>& in, slot_t* slots, int at, double dt, bool zre,
@@ -3952,9 +3955,6 @@ int batch_tile_setup(pennant_batch* b, const std::vector<TileState>& meshes) {
     return rc;
 }
 
-// Cycle `second` of a pair.  The triangles' own state stays in the batch's
-// arrays, as in tile_cycle; their point values come from the state the cycle
-// starts from and go with the one it writes.
 // Step k of the problems' chains (as chain_step).
 static BatchChain batch_chain(pennant_batch* b, int k, int zre) {
     slot_t* sets = (slot_t*)b->chain;
@@ -3962,6 +3962,9 @@ static BatchChain batch_chain(pennant_batch* b, int k, int zre) {
     return {c[k & 1], c[(k + 1) & 1], sets, k ? (k - 1) % 3 : -1, k % 3, (k + 1) % 3, zre};
 }
 
+// Cycle k of a run, the second of a pair where k is odd.  The triangles' own
+// state stays in the batch's arrays, as in tile_cycle; their point values come
+// from the state the cycle starts from and go with the one it writes.
 static int batch_tile_cycle(pennant_batch* b, int form, int k) {
     const int second = k & 1;
     BatchArgs B = make_batch_args(b);
