@@ -93,6 +93,11 @@ __device__ __forceinline__ bf16x8 next_operand(const unsigned (&v)[2][8], int c)
 __device__ __forceinline__ float bf_lo(unsigned v) { return __uint_as_float(v << 16); }
 __device__ __forceinline__ float bf_hi(unsigned v) { return __uint_as_float(v & 0xffff0000u); }
 
+// relu(a), relu(b) as a BF16 pair.  max(z, 0) is the number where z is a NaN
+// (relu_bf16, on the rounded bits, keeps a NaN whose sign bit is clear): a unit
+// with a NaN bias or input is off in every row.
+__device__ __forceinline__ unsigned relu_max(float a, float b) { return pack_bf16(fmaxf(a, 0.f), fmaxf(b, 0.f)); }
+
 // Register pairs (2 d, 2 d + 1) of an accumulator to rows [unit][b] of dst.
 __device__ __forceinline__ void store_units(const unsigned (&v)[2][8], __bf16* dst, int64_t ld, int64_t b, int h) {
 #pragma unroll
@@ -158,7 +163,7 @@ __global__ void __launch_bounds__(64) k_rows(RowArgs a) {
         const f32x16 zero = {};
         const f32x16 z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w1[mb], x, zero, 0, 0, 0);
 #pragma unroll
-        for (int d = 0; d < 8; ++d) h1[mb][d] = relu_bf16(z[2 * d], z[2 * d + 1]);
+        for (int d = 0; d < 8; ++d) h1[mb][d] = relu_max(z[2 * d], z[2 * d + 1]);
     }
     // layer 2
     bf16x8 act[4];
@@ -173,7 +178,7 @@ __global__ void __launch_bounds__(64) k_rows(RowArgs a) {
 #pragma unroll
         for (int d = 0; d < 8; ++d) {
             const float* bu = b2 + 32 * mb + 8 * (d >> 1) + 4 * h + 2 * (d & 1);
-            const unsigned v = relu_bf16(z[2 * d] + bu[0], z[2 * d + 1] + bu[1]);
+            const unsigned v = relu_max(z[2 * d] + bu[0], z[2 * d + 1] + bu[1]);
             h2[mb][d] = in ? v : 0u;
         }
     }
